@@ -15,6 +15,7 @@
 
 #include "../../include/mlrs_hip_knn.h"
 #include "knn_common.hpp"
+#include "knn_groupmin.hpp"
 #include "knn_kernels.hpp"
 
 using namespace mlrs;
@@ -516,17 +517,19 @@ static bool small_search(int64_t nq, int64_t nt, int64_t d) {
     return (double)nq * (double)nt * (double)d <= 4294967296.0;
 }
 
-// f32 searches the low-d ALU kernel serves faster than the Gram kernel
-// (timed on 500,000-row self-searches: the ALU kernel's cost grows with d
-// and, past list capacity 16, with one query per lane instead of two; the
-// Gram kernel's is nearly flat for d <= 16): every d at k <= 8, d <= 11 at
-// k <= 16, and for Euclidean d <= 3 at k <= 32 (cosine at d = 3, k = 32:
-// 176 ms against the Gram kernel's 149).  f64 always takes the ALU kernel
-// (its Gram kernel runs 2.4-12x slower there).
-static bool lowd_f32_faster(int64_t d, int64_t k, bool cos) {
-    if (k <= 8) return true;
-    if (k <= 16) return d <= 11;
-    return !cos && d <= 3;
+// Searches the low-d ALU kernel serves faster than the group-minimum search.
+// Per pair the group-minimum search costs 0.34 ps (d <= 8) to 0.43 ps (d <=
+// 16) whatever k; the ALU kernel's cost grows with d and with the list
+// capacity (500,000-row self-searches, ps per pair: f32 k <= 8: d = 3 0.09,
+// d = 8 0.24, d = 16 0.44; k <= 16: d = 3 0.16, d = 6 0.22, d = 8 0.33; f64
+// k <= 8: d = 3 0.18, d = 8 0.50; k <= 16: d = 3 0.25, d = 6 0.44; k <= 32:
+// 0.46 and more).  It also needs many queries to fill its lanes: 30,000 x
+// 30,000 points at d = 3, k = 8 take it 0.54 ms against 0.34, 100,000 x
+// 100,000 1.7 against 3.3, and 1,000 x 1,000,000 1.1 against 0.36.
+static bool lowd_faster(int64_t nq, int64_t nt, int64_t d, int64_t k, size_t elem) {
+    if (nq < 4096 || (double)nq * (double)nt < 4e9) return false;
+    if (elem == 4) return k <= 8 ? d <= 8 : (k <= 16 && d <= 6);
+    return k <= 8 ? d <= 4 : (k <= 16 && d <= 3);
 }
 
 // Process-wide kernel-family override (mlrs_force_path); a family that does
@@ -737,6 +740,178 @@ int32_t knn_gram64(const double* xq, int64_t nq, const double* xt, int64_t nt, i
     return ok();
 }
 
+// The group-minimum search (knn_groupmin.hpp).  T: the arm's arithmetic and
+// the results; TS: the rows' element type (float rows are widened for T =
+// double).
+static bool groupmin_serves(int arm, int64_t d, int64_t k) {
+    return (arm == ARM_EUCLID_FMA || arm == ARM_EUCLID_MULADD || arm == ARM_COS_FOLD || arm == ARM_COS_HOST) &&
+           d <= kGmMaxD && k <= kGmMaxK;
+}
+
+// The allocation-free entry point's limit.  A search this large was always
+// planned with per-segment lists and queues (the k = 1 kernel's split), and
+// callers size their calls by the limit that follows from them, so it stays:
+// the group-minimum search itself fits any scratch by taking fewer queries at
+// a time.
+int32_t noalloc_admits(int64_t nq, int64_t nt, int64_t d, int64_t k, bool vec4, hipStream_t s) {
+    char* ws;
+    int cus;
+    int32_t rc = workspace(256, s, &ws, &cus);
+    if (rc) return rc;
+    int64_t grid_wgs = 1;
+    int nslots = 1;
+    gram_f32_split(nq, nt, d, (int)k, cus, vec4, &grid_wgs, &nslots);
+    const size_t parts = (size_t)nslots * nq * gram_list_cap((int)k);
+    return workspace(2 * aligned_bytes(sizeof(float) * nq) + 3 * aligned_bytes(sizeof(float) * nt) +
+                         2 * aligned_bytes(parts * sizeof(float)) +
+                         (k > 1 ? aligned_bytes(gram_f32_qval_elems(grid_wgs, (int)k) * sizeof(float)) +
+                                      aligned_bytes((size_t)nslots * nq * sizeof(float4))
+                                : 0) +
+                         aligned_bytes(sizeof(unsigned int) * nq) + aligned_bytes(sizeof(NormStats)) + 1024,
+                     s, &ws, &cus);
+}
+
+template <typename T, typename TS>
+int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t d, int k, int arm, int mode,
+                     T* out_v, uint32_t* out_i, hipStream_t s) {
+    const bool cos = (arm == ARM_COS_FOLD || arm == ARM_COS_HOST);
+    // The scan reads an f32 copy of the index (centred or unit rows).  The
+    // allocation-free entry point has no room for one: it scans aligned f32
+    // rows in place, and copies others a part at a time.
+    const bool copy = sizeof(TS) == 8 || !g_noalloc || d % 4 != 0 || (reinterpret_cast<uintptr_t>(xt) & 15) != 0;
+    const int64_t ldx = (d + 3) / 4 * 4;
+    const int64_t dp = 8 * (int64_t)gm_chunks(d);
+    const int64_t ntp = gm_tiles(nt);
+    constexpr int64_t kPart = kGmRows * kGmQuad;  // index parts are whole stores of the scan
+    // Copied rows at a time: 4 GiB holds any index but the largest whole; a
+    // larger one is copied and scanned part by part for each set of queries.
+    const size_t limit = workspace_limit();
+    const size_t fixed = aligned_bytes(sizeof(float) * (size_t)ntp * kGmRows) + aligned_bytes(sizeof(GmStats)) +
+                         aligned_bytes(sizeof(uint32_t) * kGmForced) + sizeof(float) * (size_t)dp * kGmQpb + 4096;
+    size_t room = limit == SIZE_MAX ? (size_t)5 << 30 : (limit > fixed ? limit - fixed : 0);
+    int64_t xrows = 0;
+    if (copy) {
+        const size_t most = limit == SIZE_MAX ? (size_t)4 << 30 : room / 8 * 3;
+        const int64_t fit = (int64_t)(most / (sizeof(float) * (size_t)ldx)) / kPart * kPart;
+        xrows = std::min<int64_t>(ntp * kGmRows, std::max<int64_t>(fit, kPart));
+        room -= std::min(room, sizeof(float) * (size_t)(xrows * ldx) + 256);
+    }
+    const bool whole = !copy || xrows >= nt;
+    // The minima of as many queries as the budget holds: 1 GiB keeps the scan
+    // launches long (the tail of one costs about one unit of the split) and
+    // the memory modest.
+    const size_t per_q = 2 * sizeof(float) * (size_t)ntp + sizeof(float) * (size_t)(dp + 1);
+    int64_t qc = std::max<int64_t>(1, std::min<int64_t>(nq, (int64_t)(std::min(room, (size_t)1 << 30) / per_q)));
+    if (qc < nq && qc > kGmQpb) {
+        const int64_t parts = (nq + qc / kGmQpb * kGmQpb - 1) / (qc / kGmQpb * kGmQpb);
+        qc = ((nq + parts - 1) / parts + kGmQpb - 1) / kGmQpb * kGmQpb;
+    }
+    const int64_t qpad = (qc + kGmQpb - 1) / kGmQpb * kGmQpb;
+    char* ws;
+    int cus;
+    int32_t rc = workspace(fixed + sizeof(float) * (size_t)(xrows * ldx) + 2 * sizeof(float) * (size_t)(ntp * qc) +
+                               sizeof(float) * (size_t)(dp * qc + qc),
+                           s, &ws, &cus);
+    if (rc) return rc;
+    Carver cv(ws);
+    float* bias = cv.take<float>((size_t)ntp * kGmRows);
+    GmStats* stats = cv.take<GmStats>(1);
+    uint32_t* forced = cv.take<uint32_t>(kGmForced);
+    float* xcopy = copy ? cv.take<float>((size_t)(xrows * ldx)) : nullptr;
+    float* qop = cv.take<float>((size_t)(qpad * dp));
+    float* qnorm = cv.take<float>((size_t)qc);
+    float* gmin = cv.take<float>(2 * (size_t)ntp * (size_t)qc);
+
+    GmPrepArgs pq{};
+    pq.d = d;
+    pq.centre = (copy && !cos) ? xt : nullptr;
+    pq.centre_n = nt;
+    pq.out = qop;
+    pq.ldo = dp;
+    pq.norm = qnorm;
+    pq.scale = cos ? -1.0f : -2.0f;
+    pq.queries = 1;
+    pq.cosine = cos;
+    pq.stats = stats;
+    pq.forced = forced;
+    GmPrepArgs px = pq;
+    px.out = xcopy;
+    px.ldo = ldx;
+    px.scale = 1.0f;
+    px.queries = 0;
+    px.unit = copy;
+
+    GmScanArgs sc{};
+    sc.q = qop;
+    sc.ldx = ldx;
+    sc.d = ldx;
+    sc.ntp = ntp;
+    sc.grid_wgs = cus;
+
+    GmSelectArgs<TS> se{};
+    se.x = xt;
+    se.nt = nt;
+    se.d = d;
+    se.k = k;
+    se.mode = mode;
+    se.gmin = gmin;
+    se.ntp = ntp;
+    se.bias = bias;
+    se.qnorm = qnorm;
+    se.stats = stats;
+    se.forced = forced;
+    se.bias_nan = cos && !copy;
+    // |screen - exact| <= eps, with u = 2^-23 and N = ||q||^2 + ||x||^2.
+    // Euclidean: the contraction's d roundings are of partial sums up to 2 N,
+    // in any rounding mode of the matrix core: 2 d u N; the arms' d + 2
+    // roundings to nearest of a value up to 2 N: (d + 2) u N; the norms (sums
+    // of four, then a tree): 6 u N; the copy's rounding moves a distance by at
+    // most 2^-24 (||q|| + ||x||), its square by 2.02 u N.  Cosine, of unit
+    // vectors: d u, the arms' dot product and norms (d + 3) u, the unit rows'
+    // own rounding 12 u.  The absolute term covers flushed subnormals.
+    const double u = std::ldexp(1.0, -23);
+    se.eps_rel = cos ? 0.0 : (3.0 * (double)d + 24.0) * u;
+    se.eps_abs = cos ? (2.0 * (double)d + 32.0) * u : (double)(d + 4) * std::ldexp(1.0, sizeof(TS) == 8 ? -100 : -120);
+    for (int64_t q0 = 0; q0 < nq; q0 += qc) {
+        const int64_t n = std::min<int64_t>(qc, nq - q0);
+        pq.rows = xq + q0 * d;
+        pq.n = n;
+        pq.n_out = (n + kGmQpb - 1) / kGmQpb * kGmQpb;
+        pq.n_norm = n;
+        pq.reset = q0 == 0 || !whole;
+        hipError_t e = launch_gm_prep<TS>(pq, s);
+        sc.nq = n;
+        const int64_t step = whole ? ntp * kGmRows : xrows;
+        for (int64_t x0 = 0; e == hipSuccess && x0 < nt; x0 += step) {
+            const int64_t rows = std::min<int64_t>(step, nt - x0);
+            if (q0 == 0 || !whole) {
+                px.rows = xt + x0 * d;
+                px.row0 = x0;
+                px.n = px.n_out = rows;
+                px.norm = bias + x0;
+                px.n_norm = gm_tiles(rows) * kGmRows;
+                e = launch_gm_prep<TS>(px, s);
+            }
+            sc.x = copy ? xcopy : reinterpret_cast<const float*>(xt) + x0 * d;
+            sc.bias = bias + x0;
+            sc.nt = rows;
+            sc.tiles = gm_tiles(rows);
+            sc.gmin = gmin + x0 / kGmRows;
+            if (e == hipSuccess) {
+                KernelTimer timer(s, "knn_groupmin_kernel");
+                e = cos && !copy ? launch_gm_scan_cosine(sc, s) : launch_gm_scan_euclid(sc, s);
+            }
+        }
+        se.q = xq + q0 * d;
+        se.nq = n;
+        se.out_val = out_v + q0 * k;
+        se.out_idx = out_i + q0 * k;
+        if (e == hipSuccess) e = launch_gm_select<T, TS>(se, arm, s);
+        if (e != hipSuccess) return hip_err(e, "knn_groupmin");
+    }
+    return ok();
+}
+
 // The low-d ALU path (knn_lowd.hip), f32 and f64.
 static hipError_t launch_lowd_t(const LowdArgs32& a, int arm, hipStream_t s) { return launch_lowd_f32(a, arm, s); }
 static hipError_t launch_lowd_t(const LowdArgs64& a, int arm, hipStream_t s) { return launch_lowd_f64(a, arm, s); }
@@ -877,21 +1052,29 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
     const int mode = (metric == MLRS_METRIC_EUCLIDEAN) ? EMIT_SQRT : EMIT_IDENTITY;
     const bool lowd_ok = (metric == MLRS_METRIC_EUCLIDEAN || (metric == MLRS_METRIC_COSINE && arm == ARM_COS_FOLD)) &&
                          n_features <= lowd_max_d() && k <= lowd_max_k();
-    // the knn_host cosine arm on the matrix cores in the wide shape only (it
-    // serves d > 128, where the wide shape runs)
-    const bool gram_ok = (arm == ARM_EUCLID_FMA || arm == ARM_EUCLID_MULADD || arm == ARM_COS_FOLD ||
-                          (arm == ARM_COS_HOST && n_features > 128)) &&
-                         n_features <= gram_f32_max_d() && k <= gram_f32_max_k();
+    const bool gm_ok = groupmin_serves(arm, n_features, k);
     const bool small = small_search(n_query, n_train, n_features);
-    int path = pick_path(lowd_ok, gram_ok);
+    const bool forced = pick_path(lowd_ok, gm_ok) == MLRS_PATH_FUSED;
+    int path = pick_path(lowd_ok, gm_ok);
     if (path == MLRS_PATH_AUTO)
-        path = (lowd_ok && (small || !gram_ok || lowd_f32_faster(n_features, k, metric == MLRS_METRIC_COSINE))) ? MLRS_PATH_LOWD
-               : (gram_ok && !small)                                             ? MLRS_PATH_FUSED
-                                                                                 : MLRS_PATH_GENERIC;
+        path = lowd_ok && lowd_faster(n_query, n_train, n_features, k, sizeof(float)) ? MLRS_PATH_LOWD
+               : gm_ok                                                                ? MLRS_PATH_FUSED
+                                                                                      : MLRS_PATH_GENERIC;
     if (path == MLRS_PATH_LOWD)
         return knn_lowd<float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
-    if (path == MLRS_PATH_FUSED)
-        return knn_gram32(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
+    if (path == MLRS_PATH_FUSED) {
+        const bool vec4 = (n_features % 4 == 0) && ((reinterpret_cast<uintptr_t>(xq) & 15) == 0) &&
+                          ((reinterpret_cast<uintptr_t>(x_train) & 15) == 0);
+        // k = 1 over an index that fits a few workgroups' LDS: resident there
+        if ((forced || !small) && gram_f32_k1_resident_chunks(n_query, n_train, n_features, k, arm, vec4) > 0)
+            return knn_gram32(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
+        if (g_noalloc && (forced || !small)) {
+            const int32_t rc = noalloc_admits(n_query, n_train, n_features, k, vec4, s);
+            if (rc) return rc;
+        }
+        return knn_groupmin<float, float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
+                                          s);
+    }
     return knn_generic<float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s, p);
 }
 
@@ -997,15 +1180,17 @@ int32_t mlrs_knn_topk_f64(const double* xq, int64_t xq_len, int64_t n_query, int
     const int mode = (metric == MLRS_METRIC_EUCLIDEAN) ? EMIT_SQRT : EMIT_IDENTITY;
     const bool lowd_ok = (metric == MLRS_METRIC_EUCLIDEAN || (metric == MLRS_METRIC_COSINE && arm == ARM_COS_FOLD)) &&
                          n_features <= lowd_max_d() && k <= lowd_max_k();
-    const bool gram_ok = arm <= ARM_COS_HOST && n_features <= gram_f64_max_d() && k <= gram_f64_max_k();
-    int path = pick_path(lowd_ok, gram_ok);
+    const bool gm_ok = groupmin_serves(arm, n_features, k);
+    int path = pick_path(lowd_ok, gm_ok);
     if (path == MLRS_PATH_AUTO)
-        path = lowd_ok ? MLRS_PATH_LOWD
-                       : (gram_ok && !small_search(n_query, n_train, n_features)) ? MLRS_PATH_FUSED : MLRS_PATH_GENERIC;
+        path = lowd_ok && lowd_faster(n_query, n_train, n_features, k, sizeof(double)) ? MLRS_PATH_LOWD
+               : gm_ok                                                                 ? MLRS_PATH_FUSED
+                                                                                       : MLRS_PATH_GENERIC;
     if (path == MLRS_PATH_LOWD)
         return knn_lowd<double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
     if (path == MLRS_PATH_FUSED)
-        return knn_gram64(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
+        return knn_groupmin<double, double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
+                                            s);
     return knn_generic<double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s, p);
 }
 
@@ -1740,20 +1925,25 @@ static int32_t pinned_staging(size_t bytes, char** out) {
     return MLRS_OK;
 }
 
-// The f64 search under an explicit arm: the low-d ALU kernel for Euclidean
-// arms ranked by the aggregate (d <= 16, k <= 32), the Gram-MFMA kernel where
-// it serves the arm and shape, else exact tiles + selection.
-static int32_t search_f64(const double* xq, int64_t nq, const double* xt, int64_t nt, int64_t d, int k, int arm,
-                          int mode, double p, double* ov, uint32_t* oi, hipStream_t s) {
-    const bool lowd_ok = (arm == ARM_EUCLID_FMA || arm == ARM_EUCLID_MULADD || arm == ARM_COS_FOLD) &&
+// The graph's search over rows of TS in f64 arithmetic, under an explicit arm.
+template <typename TS>
+static int32_t search_f64(const TS* x, int64_t n, int64_t d, int k, int arm, int mode, double p, double* ov,
+                          uint32_t* oi, hipStream_t s) {
+    const bool lowd_ok = sizeof(TS) == 8 && (arm == ARM_EUCLID_FMA || arm == ARM_EUCLID_MULADD || arm == ARM_COS_FOLD) &&
                          mode != EMIT_ROOT_RANKED && d <= lowd_max_d() && k <= lowd_max_k();
-    const bool gram_ok = arm <= ARM_COS_HOST && d <= gram_f64_max_d() && k <= gram_f64_max_k();
-    int path = pick_path(lowd_ok, gram_ok);
+    const bool gm_ok = groupmin_serves(arm, d, k);
+    int path = pick_path(lowd_ok, gm_ok);
     if (path == MLRS_PATH_AUTO)
-        path = lowd_ok ? MLRS_PATH_LOWD : (gram_ok && !small_search(nq, nt, d)) ? MLRS_PATH_FUSED : MLRS_PATH_GENERIC;
-    if (path == MLRS_PATH_LOWD) return knn_lowd<double>(xq, nq, xt, nt, d, k, arm, mode, ov, oi, s);
-    if (path == MLRS_PATH_FUSED) return knn_gram64(xq, nq, xt, nt, d, k, arm, mode, ov, oi, s);
-    return knn_generic<double>(xq, nq, xt, nt, d, k, arm, mode, ov, oi, s, p);
+        path = lowd_ok && lowd_faster(n, n, d, k, sizeof(double)) ? MLRS_PATH_LOWD
+               : gm_ok                                            ? MLRS_PATH_FUSED
+                                                                  : MLRS_PATH_GENERIC;
+    if (path == MLRS_PATH_FUSED) return knn_groupmin<double, TS>(x, n, x, n, d, k, arm, mode, ov, oi, s);
+    if constexpr (sizeof(TS) == 8) {
+        if (path == MLRS_PATH_LOWD) return knn_lowd<double>(x, n, x, n, d, k, arm, mode, ov, oi, s);
+        return knn_generic<double>(x, n, x, n, d, k, arm, mode, ov, oi, s, p);
+    } else {
+        return set_err(MLRS_ERR_UNSUPPORTED, "x", n, d, 0, 0, "the exact tiles take f64 rows");
+    }
 }
 
 // knn_graph's validate_geometry (crates/mlrs-backend/src/prims/knn_graph.rs:475-539).
@@ -1795,10 +1985,17 @@ static void graph_arm(int32_t metric, int* arm, int* mode) {
 template <typename TIn>
 static int32_t graph_search(const TIn* x, int64_t n, int64_t d, int kk, int32_t metric, double p, hipStream_t s,
                             double** val, uint32_t** idx) {
-    const bool widen = sizeof(TIn) == 4;
     const bool cos = metric == MLRS_METRIC_COSINE;
+    int arm, mode;
+    graph_arm(metric, &arm, &mode);
+    // The group-minimum search widens f32 rows as it evaluates them; cosine
+    // (normalised rows) and the other kernels work on rows widened first.
+    const bool direct = sizeof(TIn) == 4 && !cos && groupmin_serves(arm, d, kk) &&
+                        pick_path(false, true) != MLRS_PATH_GENERIC;
+    const bool widen = sizeof(TIn) == 4 && !direct;
     size_t bytes = aligned_bytes(sizeof(double) * (size_t)n * kk) + aligned_bytes(sizeof(uint32_t) * (size_t)n * kk) +
-                   2 * aligned_bytes(sizeof(double) * (size_t)n * d) + 2 * aligned_bytes(sizeof(double) * (size_t)n) +
+                   (widen ? aligned_bytes(sizeof(double) * (size_t)n * d) : 0) +
+                   (cos ? aligned_bytes(sizeof(double) * (size_t)n * d) : 0) + 2 * aligned_bytes(sizeof(double) * (size_t)n) +
                    1024;
     char* aux;
     int32_t rc = aux_workspace(bytes, s, &aux);
@@ -1806,6 +2003,7 @@ static int32_t graph_search(const TIn* x, int64_t n, int64_t d, int kk, int32_t 
     Carver cv(aux);
     *val = cv.take<double>((size_t)n * kk);
     *idx = cv.take<uint32_t>((size_t)n * kk);
+    if (direct) return search_f64<TIn>(x, n, d, kk, arm, mode, p, *val, *idx, s);
     const double* xd = reinterpret_cast<const double*>(x);
     hipError_t e = hipSuccess;
     if (widen) {
@@ -1822,9 +2020,7 @@ static int32_t graph_search(const TIn* x, int64_t n, int64_t d, int kk, int32_t 
         xd = xn;
     }
     if (e != hipSuccess) return hip_err(e, "graph operand");
-    int arm, mode;
-    graph_arm(metric, &arm, &mode);
-    return search_f64(xd, n, xd, n, d, kk, arm, mode, p, *val, *idx, s);
+    return search_f64<double>(xd, n, d, kk, arm, mode, p, *val, *idx, s);
 }
 
 template <typename TIn>

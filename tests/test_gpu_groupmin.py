@@ -1,0 +1,126 @@
+"""GPU parity of the group-minimum search (knn_groupmin.hip) with the CPU
+oracle, bit for bit, where it can go wrong: index sizes around a 16-row group,
+a 32-row tile and the 128 rows of one store; row widths around the 8-column
+steps; both selection kernels (a workgroup per query below 1,000 queries, a
+wave per query from there) and both list lengths; rows the screen is not
+trusted with (norms past the f32 range, infinities, NaN) singly and more than
+are listed; ties past the candidate lists; clusters and offsets the screen
+does not resolve; the parts of an index too large for the allocation-free
+entry point's scratch."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from mlrs_amd import _lib, prims
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+@pytest.fixture(autouse=True)
+def _family():
+    prims.force_path("fused")
+    yield
+    prims.force_path("auto")
+
+
+def _check(xq, xt, k, metric="euclidean"):
+    wd, wi = oracle.knn_topk(xq, xt, k, metric)
+    gd, gi = prims.knn_topk(torch.from_numpy(xq).to(DEV), torch.from_numpy(xt).to(DEV), k, metric)
+    gd, gi = gd.cpu().numpy(), gi.cpu().numpy()
+    bits = np.int32 if gd.dtype == np.float32 else np.int64
+    assert np.array_equal(gi, wi.astype(np.int64)), np.argwhere(gi != wi)[:3].tolist()
+    assert np.array_equal(gd.view(bits), wd.view(bits)), np.argwhere(gd.view(bits) != wd.view(bits))[:3].tolist()
+
+
+def _rows(seed, n, d, dtype):
+    return np.random.default_rng(seed).standard_normal((n, d)).astype(dtype)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nt,d,k,nq", [
+    (2, 1, 2, 1), (16, 3, 5, 3), (31, 8, 31, 4), (32, 9, 32, 31), (33, 7, 33, 33), (127, 16, 64, 5), (128, 17, 65, 127),
+    (129, 24, 128, 128), (4097, 50, 16, 129), (1000, 63, 17, 999), (1000, 64, 17, 1000), (5000, 65, 64, 1003),
+    (2049, 120, 1, 1001), (700, 127, 10, 64), (700, 128, 10, 64), (700, 129, 10, 64), (300, 192, 100, 20),
+    (300, 193, 3, 20), (300, 255, 7, 20), (300, 256, 7, 1000)])
+def test_edges(dtype, nt, d, k, nq):
+    xt, xq = _rows(nt + d, nt, d, dtype), _rows(nq + k, nq, d, dtype)
+    xt[nt // 2] = xt[nt - 1]  # a tie
+    for metric in ("euclidean", "cosine"):
+        _check(xq, xt, k, metric)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("metric", ["euclidean", "cosine"])
+@pytest.mark.parametrize("d,k,nq", [(6, 12, 60), (50, 100, 60), (50, 12, 1040)])
+def test_rows_the_screen_is_not_trusted_with(dtype, metric, d, k, nq):
+    """A few such rows go to every query from a list; more than it holds, and
+    queries of the kind, have every row evaluated."""
+    xt, xq = _rows(3, 1500, d, dtype), _rows(4, nq, d, dtype)
+    xt[[10, 11]] = 0.0
+    xt[20, 0] = np.nan
+    xt[30, 0], xt[31, d - 1] = np.inf, -np.inf
+    for r, scale in ((40, 1e18), (41, 1e30), (42, 1e-25), (43, 1e-35)):
+        xt[r] *= dtype(scale)
+    xq[:20] = xt[[10, 11, 12, 20, 21, 30, 31, 32, 40, 41, 42, 43, 44, 5, 6, 7, 8, 9, 1, 2]]
+    xq[21] *= dtype(1e30)
+    _check(xq, xt, k, metric)
+    xt[100:500] *= dtype(1e25)
+    _check(xq, xt, k, metric)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("metric", ["euclidean", "cosine"])
+@pytest.mark.parametrize("nq", [40, 1000])
+def test_ties_past_the_candidate_lists(dtype, metric, nq):
+    """Far more groups than a query lists stand at its k-th minimum."""
+    rng = np.random.default_rng(9)
+    xt = rng.integers(0, 2, (20_000, 4)).astype(dtype)
+    _check(xt[:nq].copy(), xt, 25, metric)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nq", [30, 1000])
+def test_distances_the_screen_does_not_resolve(dtype, nq):
+    """Clusters a thousandth of their spacing wide, and a common offset."""
+    rng = np.random.default_rng(11)
+    centres = rng.uniform(-10, 10, (8, 20))
+    xt = (centres[rng.integers(0, 8, 6000)] + 1e-3 * rng.standard_normal((6000, 20))).astype(dtype)
+    _check(xt[:nq].copy(), xt, 20)
+    _check((xt[:nq] + dtype(500)), (xt + dtype(500)), 20)
+
+
+@pytest.mark.parametrize("n,d,k,metric", [(2500, 5, 15, "euclidean"), (1300, 50, 100, "euclidean"),
+                                          (1100, 33, 9, "cosine")])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_graph(dtype, n, d, k, metric):
+    x = _rows(n, n, d, dtype)
+    x[100:140] = x[3]
+    wi, wd = oracle.knn_graph(x, k, metric)
+    gi, gd = prims.knn_graph(torch.from_numpy(x).to(DEV), k, metric)
+    assert np.array_equal(gi.cpu().numpy(), wi.astype(np.int64))
+    assert np.array_equal(gd.cpu().numpy().view(np.int64), wd.view(np.int64))
+
+
+@pytest.mark.parametrize("nt,d,metric", [(300_000, 50, 0), (300_000, 50, 1), (260_000, 64, 0)])
+def test_noalloc_index_parts(nt, d, metric):
+    """Rows that are not 16-byte aligned are copied a part at a time there."""
+    g = torch.Generator(device="cpu").manual_seed(nt + d)
+    xt = torch.randn((nt, d), generator=g).to(DEV)
+    xt[nt - 3] = xt[1]
+    xt[nt - 5] *= 1e25  # a row for the forced list, in the last part
+    xq = torch.randn((300, d), generator=g).to(DEV)
+    xq[0] = xt[1]
+    out = []
+    for name in ("mlrs_knn_topk_f32", "mlrs_knn_topk_f32_noalloc"):
+        dist = torch.empty((300, 12), dtype=torch.float32, device=DEV)
+        idx = torch.empty((300, 12), dtype=torch.int32, device=DEV)
+        _lib.check(getattr(_lib.load(), name)(
+            xq.data_ptr(), xq.numel(), 300, d, xt.data_ptr(), xt.numel(), nt, 12, metric, ctypes.c_double(2.0),
+            dist.data_ptr(), idx.data_ptr(), dist.numel(), torch.cuda.current_stream(DEV).cuda_stream))
+        out.append((dist.view(torch.int32), idx))
+    torch.cuda.synchronize()
+    assert torch.equal(out[0][1], out[1][1]) and torch.equal(out[0][0], out[1][0])
