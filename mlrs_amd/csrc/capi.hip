@@ -517,19 +517,20 @@ static bool small_search(int64_t nq, int64_t nt, int64_t d) {
     return (double)nq * (double)nt * (double)d <= 4294967296.0;
 }
 
-// Searches the low-d ALU kernel serves faster than the group-minimum search.
-// Per pair the group-minimum search costs 0.34 ps (d <= 8) to 0.43 ps (d <=
-// 16) whatever k; the ALU kernel's cost grows with d and with the list
-// capacity (500,000-row self-searches, ps per pair: f32 k <= 8: d = 3 0.09,
-// d = 8 0.24, d = 16 0.44; k <= 16: d = 3 0.16, d = 6 0.22, d = 8 0.33; f64
-// k <= 8: d = 3 0.18, d = 8 0.50; k <= 16: d = 3 0.25, d = 6 0.44; k <= 32:
-// 0.46 and more).  It also needs many queries to fill its lanes: 30,000 x
-// 30,000 points at d = 3, k = 8 take it 0.54 ms against 0.34, 100,000 x
-// 100,000 1.7 against 3.3, and 1,000 x 1,000,000 1.1 against 0.36.
+// Searches the low-d ALU kernel serves faster than the group-minimum search,
+// whose cost is about 0.335 ps per pair whatever k (d <= 8; 0.43 up to 16).  The
+// ALU kernel needs thousands of queries to fill its lanes, pays for its list
+// merges, and its cost per pair grows with d and k; fitted to self-searches of
+// 30,000 and 100,000 rows (us, ALU against group minima): f32 d = 2, k = 2: 298
+// / 314 and 1373 / 3335; d = 3, k = 8: 538 / 344 and 1722 / 3329; d = 8, k = 8:
+// 833 / 338 and 3475 / 3391; f64 d = 2, k = 2: 360 / 321 and 1632 / 3313; d = 3,
+// k = 8: 709 / 354 and 2961 / 3347; d = 4, k = 8: 834 / 353 and 3649 / 3355.  500,000
+// rows, d = 3, k = 8, f32: 23 ms against 93.
 static bool lowd_faster(int64_t nq, int64_t nt, int64_t d, int64_t k, size_t elem) {
-    if (nq < 4096 || (double)nq * (double)nt < 4e9) return false;
-    if (elem == 4) return k <= 8 ? d <= 8 : (k <= 16 && d <= 6);
-    return k <= 8 ? d <= 4 : (k <= 16 && d <= 3);
+    if (nq < 4096 || k > 16) return false;
+    const double pairs = (double)nq * (double)nt;
+    const double ps = elem == 4 ? 0.04 + 0.027 * (double)d + 0.004 * (double)k : 0.02 + 0.06 * (double)d + 0.006 * (double)k;
+    return 150.0 + 35.0 * (double)k + ps * 1e-6 * pairs < (d <= 8 ? 0.335e-6 : 0.43e-6) * pairs;
 }
 
 // Process-wide kernel-family override (mlrs_force_path); a family that does
@@ -912,6 +913,63 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     return ok();
 }
 
+// The Manhattan, Chebyshev and Minkowski searches: the exact tiles' group
+// minima, then the same selection.
+static bool groupmin_metric_serves(int arm, int64_t d, int64_t k) {
+    return (arm == ARM_MANHATTAN || arm == ARM_CHEBYSHEV || arm == ARM_MINKOWSKI_INT || arm == ARM_MINKOWSKI_POW) &&
+           d <= kGmMaxD && k <= kGmMaxK;
+}
+
+template <typename T>
+int32_t knn_groupmin_metric(const T* xq, int64_t nq, const T* xt, int64_t nt, int64_t d, int k, int arm, int mode,
+                            T* out_v, uint32_t* out_i, hipStream_t s, double p) {
+    const int64_t ntp = gm_tiles(nt);
+    const size_t per_q = 2 * sizeof(float) * (size_t)ntp;
+    const size_t limit = workspace_limit();
+    const size_t budget = std::min<size_t>((size_t)1 << 30, limit == SIZE_MAX ? limit : limit - 256);
+    // at most 65535 tiles of 64 queries in a launch's grid
+    const int64_t qc = std::min<int64_t>(std::min<int64_t>(nq, 4000000),
+                                         std::max<int64_t>(1, (int64_t)(budget / per_q)));
+    char* ws;
+    int cus;
+    int32_t rc = workspace(per_q * (size_t)qc + 256, s, &ws, &cus);
+    if (rc) return rc;
+    GmSelectArgs<T> se{};
+    se.x = xt;
+    se.nt = nt;
+    se.d = d;
+    se.k = k;
+    se.mode = mode;
+    se.gmin = reinterpret_cast<const float*>(ws);
+    se.ntp = ntp;
+    se.eps_t = std::ldexp(1.0, -21);  // the minima's rounding to f32 (2^-24) on both sides of a comparison, and a root's
+    se.pexp = p;
+    se.pint = minkowski_powi(p);
+    se.root_exp = 1.0 / p;
+    for (int64_t q0 = 0; q0 < nq; q0 += qc) {
+        const int64_t n = std::min<int64_t>(qc, nq - q0);
+        hipError_t e;
+        {
+            KernelTimer timer(s, "groupmin_tile_kernel");
+            e = launch_groupmin_tile<T>(xq + q0 * d, n, xt, nt, d, arm, (T)p, minkowski_powi(p),
+                                        reinterpret_cast<float*>(ws), ntp, s);
+        }
+        se.q = xq + q0 * d;
+        se.nq = n;
+        se.out_val = out_v + q0 * k;
+        se.out_idx = out_i + q0 * k;
+        if (e == hipSuccess) e = launch_gm_select_metric<T>(se, arm, s);
+        if (e != hipSuccess) return hip_err(e, "knn_groupmin_metric");
+    }
+    // Minkowski's boundary root over the emitted values, exponent
+    // f64_to_host(1/p) (prims/knn.rs:882-888)
+    if ((arm == ARM_MINKOWSKI_INT || arm == ARM_MINKOWSKI_POW) && mode != EMIT_ROOT_RANKED) {
+        hipError_t e = launch_pow_inplace<T>(out_v, nq * k, (T)(1.0 / p), s);
+        if (e != hipSuccess) return hip_err(e, "minkowski root");
+    }
+    return ok();
+}
+
 // The low-d ALU path (knn_lowd.hip), f32 and f64.
 static hipError_t launch_lowd_t(const LowdArgs32& a, int arm, hipStream_t s) { return launch_lowd_f32(a, arm, s); }
 static hipError_t launch_lowd_t(const LowdArgs64& a, int arm, hipStream_t s) { return launch_lowd_f64(a, arm, s); }
@@ -1059,7 +1117,7 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
     if (path == MLRS_PATH_AUTO)
         path = lowd_ok && lowd_faster(n_query, n_train, n_features, k, sizeof(float)) ? MLRS_PATH_LOWD
                : gm_ok                                                                ? MLRS_PATH_FUSED
-                                                                                      : MLRS_PATH_GENERIC;
+                                                                                      : MLRS_PATH_AUTO;
     if (path == MLRS_PATH_LOWD)
         return knn_lowd<float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
     if (path == MLRS_PATH_FUSED) {
@@ -1075,6 +1133,9 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
         return knn_groupmin<float, float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
                                           s);
     }
+    if (path == MLRS_PATH_AUTO && groupmin_metric_serves(arm, n_features, k))
+        return knn_groupmin_metric<float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s,
+                                          p);
     return knn_generic<float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s, p);
 }
 
@@ -1185,12 +1246,15 @@ int32_t mlrs_knn_topk_f64(const double* xq, int64_t xq_len, int64_t n_query, int
     if (path == MLRS_PATH_AUTO)
         path = lowd_ok && lowd_faster(n_query, n_train, n_features, k, sizeof(double)) ? MLRS_PATH_LOWD
                : gm_ok                                                                 ? MLRS_PATH_FUSED
-                                                                                       : MLRS_PATH_GENERIC;
+                                                                                       : MLRS_PATH_AUTO;
     if (path == MLRS_PATH_LOWD)
         return knn_lowd<double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
     if (path == MLRS_PATH_FUSED)
         return knn_groupmin<double, double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
                                             s);
+    if (path == MLRS_PATH_AUTO && groupmin_metric_serves(arm, n_features, k))
+        return knn_groupmin_metric<double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
+                                           s, p);
     return knn_generic<double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s, p);
 }
 
@@ -1936,10 +2000,12 @@ static int32_t search_f64(const TS* x, int64_t n, int64_t d, int k, int arm, int
     if (path == MLRS_PATH_AUTO)
         path = lowd_ok && lowd_faster(n, n, d, k, sizeof(double)) ? MLRS_PATH_LOWD
                : gm_ok                                            ? MLRS_PATH_FUSED
-                                                                  : MLRS_PATH_GENERIC;
+                                                                  : MLRS_PATH_AUTO;
     if (path == MLRS_PATH_FUSED) return knn_groupmin<double, TS>(x, n, x, n, d, k, arm, mode, ov, oi, s);
     if constexpr (sizeof(TS) == 8) {
         if (path == MLRS_PATH_LOWD) return knn_lowd<double>(x, n, x, n, d, k, arm, mode, ov, oi, s);
+        if (path == MLRS_PATH_AUTO && groupmin_metric_serves(arm, d, k))
+            return knn_groupmin_metric<double>(x, n, x, n, d, k, arm, mode, ov, oi, s, p);
         return knn_generic<double>(x, n, x, n, d, k, arm, mode, ov, oi, s, p);
     } else {
         return set_err(MLRS_ERR_UNSUPPORTED, "x", n, d, 0, 0, "the exact tiles take f64 rows");

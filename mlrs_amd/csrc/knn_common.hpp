@@ -136,6 +136,34 @@ __device__ __forceinline__ T exact_pair(const T* __restrict__ q, const T* __rest
     }
 }
 
+// Parameters of the Minkowski arms: the pow arm's exponent, the multiply
+// chain's integer exponent and the exponent of the boundary root.
+template <typename T>
+struct MetricParams {
+    T pexp;
+    int pint;
+    T root;
+};
+
+// One column of the arms that are not a contraction of squares or products.
+template <typename T, int ARM>
+__device__ __forceinline__ T metric_step(T acc, T x, T y, const MetricParams<T>& mp) {
+    using F = FloatTraits<T>;
+    if (ARM == ARM_MANHATTAN) {
+        return acc + F::abs_(x - y);
+    } else if (ARM == ARM_CHEBYSHEV) {
+        const T v = F::abs_(x - y);
+        return (v > acc) ? v : acc;
+    } else if (ARM == ARM_MINKOWSKI_INT) {
+        const T ad = F::abs_(x - y);
+        T r = ad;
+        for (int i = 1; i < mp.pint; ++i) r = r * ad;
+        return acc + r;
+    } else {
+        return acc + F::pow_(F::abs_(x - y), mp.pexp);
+    }
+}
+
 // Smallest float >= t (screen thresholds are rounded up, never down).
 __device__ __forceinline__ float round_up_f(double t) {
     float f = (float)t;

@@ -110,11 +110,13 @@ struct GmSelectArgs {
     int64_t ntp;
     const float* bias;
     const float* qnorm;  // [nq], NaN: evaluate every row
-    const GmStats* stats;
+    const GmStats* stats;  // null: the minima are of the arm's own values (launch_groupmin_tile), no row is left out
     const uint32_t* forced;
     double eps_rel, eps_abs;  // eps = eps_rel (||q||^2 + max ||x||^2) + eps_abs
+    double eps_t;        // relative error of a minimum (values rounded to f32)
     int bias_nan;        // rows left out carry NaN (cosine in place) instead of +inf
-    int cosine;
+    double pexp, root_exp;  // Minkowski: the exponent and (EMIT_ROOT_RANKED) its root's
+    int pint;               // its integer exponent
     void* out_val;       // [nq][k] of T
     uint32_t* out_idx;
 };
@@ -122,5 +124,9 @@ struct GmSelectArgs {
 // widened for T = double).
 template <typename T, typename TS>
 hipError_t launch_gm_select(const GmSelectArgs<TS>& a, int arm, hipStream_t s);
+
+// The Manhattan, Chebyshev and Minkowski arms (knn_groupmin_metric.hip); T = TS.
+template <typename T>
+hipError_t launch_gm_select_metric(const GmSelectArgs<T>& a, int arm, hipStream_t s);
 
 }  // namespace mlrs

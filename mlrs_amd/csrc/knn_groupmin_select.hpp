@@ -1,0 +1,565 @@
+// The selection pass of the group-minimum search (knn_groupmin.hpp).  Included
+// by the sources that instantiate it, so that the arms compile side by side.
+#pragma once
+
+#include "knn_common.hpp"
+#include "knn_groupmin.hpp"
+
+namespace mlrs {
+
+namespace {
+
+// ---------------------------------------------------------------------------
+// Selection: one workgroup per query.
+// ---------------------------------------------------------------------------
+constexpr int kSelCap = 1024;    // candidate groups listed before the query falls back to a pass over all of them
+constexpr int kSelRefine = 512;  // lists up to this long have their k-th minimum found exactly
+
+// Orders this wave's LDS writes before its later LDS reads by other lanes: the
+// LDS serves a wave's accesses in order, so the compiler's order is all.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// 16 bytes of a row that is aligned to its elements only.
+template <typename TS> struct RowVec;
+template <> struct RowVec<float> {
+    static constexpr int V = 4;
+    typedef float type __attribute__((ext_vector_type(4), aligned(4)));
+};
+template <> struct RowVec<double> {
+    static constexpr int V = 2;
+    typedef double type __attribute__((ext_vector_type(2), aligned(8)));
+};
+
+template <typename T, int ARM>
+__device__ __forceinline__ void gm_step(T& acc, T& ya, T x, T y, const MetricParams<T>& mp) {
+    using F = FloatTraits<T>;
+    if (ARM == ARM_EUCLID_FMA) {
+        const T diff = x - y;
+        acc = F::fma_(diff, diff, acc);
+    } else if (ARM == ARM_EUCLID_MULADD) {
+        const T diff = x - y;
+        acc = acc + diff * diff;
+    } else if (ARM == ARM_COS_FOLD) {
+        acc = F::fma_(x, y, acc);
+        ya = ya + y * y;
+    } else if (ARM == ARM_COS_HOST) {
+        acc = acc + x * y;
+        ya = ya + y * y;
+    } else {
+        acc = metric_step<T, ARM>(acc, x, y, mp);
+    }
+}
+
+// The exact value of (query sq, row X[r]), accumulated over ascending columns
+// in the arm's order; for cosine ya is the row's row_sumsq.  A lane reads its
+// own row, 128 bytes of it in flight: the 64 rows of a wave lie in four runs
+// of neighbours, and a line's eight pieces are requested together, so the
+// cache serves seven of them.  (Staging the rows through LDS with coalesced
+// loads, two barriers per 128 bytes, took three to ten times as long.)
+template <typename T, typename TS, int ARM>
+__device__ __forceinline__ T gm_exact(const T* __restrict__ sq, const TS* __restrict__ row, int d, T& ya,
+                                      const MetricParams<T>& mp) {
+    constexpr int V = RowVec<TS>::V;
+    constexpr int U = 8;
+    typedef typename RowVec<TS>::type vec;
+    typedef const __attribute__((address_space(1))) vec* vptr;
+    typedef const __attribute__((address_space(1))) TS* sptr;
+    T acc = T(0);
+    ya = T(0);
+    int c = 0;
+    for (; c + U * V <= d; c += U * V) {
+        vec p[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) p[u] = *(vptr)(row + c + u * V);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < V; ++e) gm_step<T, ARM>(acc, ya, sq[c + u * V + e], (T)p[u][e], mp);
+    }
+    if (c < d) {
+        vec p[U];
+        TS tail[V];
+        const int nv = (d - c) / V, rest = (d - c) % V;  // uniform
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < nv) p[u] = *(vptr)(row + c + u * V);
+#pragma unroll
+        for (int e = 0; e + 1 < V; ++e)
+            if (e < rest) tail[e] = *(sptr)(row + c + nv * V + e);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (u < nv) {
+#pragma unroll
+                for (int e = 0; e < V; ++e) gm_step<T, ARM>(acc, ya, sq[c + u * V + e], (T)p[u][e], mp);
+            }
+#pragma unroll
+        for (int e = 0; e + 1 < V; ++e)
+            if (e < rest) gm_step<T, ARM>(acc, ya, sq[c + nv * V + e], (T)tail[e], mp);
+    }
+    return acc;
+}
+
+// A wave's answer so far: the 64 KL smallest (value, row) pairs it has seen.
+template <typename T, typename TS, int ARM, int KL>
+struct GmList {
+    using F = FloatTraits<T>;
+    static constexpr bool COS = ARM == ARM_COS_FOLD || ARM == ARM_COS_HOST;
+    static constexpr bool MINK = ARM == ARM_MINKOWSKI_INT || ARM == ARM_MINKOWSKI_POW;
+    T lv[KL];
+    uint32_t li[KL];
+    T qa = T(0);  // cosine: the query's row_sumsq (fold) or its reciprocal norm (host)
+    bool qzero = false;
+    MetricParams<T> mp;
+
+    __device__ __forceinline__ GmList(const GmSelectArgs<TS>& a) : mp{(T)a.pexp, a.pint, (T)a.root_exp} {
+#pragma unroll
+        for (int b = 0; b < KL; ++b) {
+            lv[b] = F::inf();
+            li[b] = kSentinelIdx;
+        }
+    }
+    __device__ __forceinline__ void set_query(const T* __restrict__ sq, int d) {
+        if (!COS) return;
+        for (int c = 0; c < d; ++c) qa = qa + sq[c] * sq[c];
+        qzero = qa == T(0);
+        if (ARM == ARM_COS_HOST) qa = (qa > T(0)) ? T(1) / F::sqrt_(qa) : T(0);
+    }
+    __device__ __forceinline__ T kth(int k) const { return list_value_at<T, KL>(lv, k - 1); }
+    __device__ __forceinline__ void merge(T v, uint32_t ix, int lane) {
+        if constexpr (KL == 1) wave_merge64<T>(lv[0], li[0], v, ix, lane);
+        else wave_merge_blocks<T, KL>(lv, li, v, ix, lane);
+    }
+    // 64 rows (kSentinelIdx: none) evaluated exactly and merged in
+    __device__ __forceinline__ void evaluate(uint32_t mine, const T* __restrict__ sq, const TS* __restrict__ X, int d,
+                                             int k, int mode, int lane) {
+        if (__builtin_amdgcn_ballot_w64(mine != kSentinelIdx) == 0ull) return;
+        T ya;
+        T v = gm_exact<T, TS, ARM>(sq, X + (mine != kSentinelIdx ? (int64_t)mine : 0) * d, d, ya, mp);
+        if (ARM == ARM_COS_FOLD) {
+            const T denom = F::sqrt_(qa * ya);
+            const T sim = (denom > T(0)) ? v / denom : T(0);
+            v = clamp02<T>(T(1) - sim);
+        } else if (ARM == ARM_COS_HOST) {
+            const T iy = (ya > T(0)) ? T(1) / F::sqrt_(ya) : T(0);
+            v = clamp02<T>(T(1) - v * qa * iy);
+        }
+        if (mode == EMIT_ROOT_RANKED) v = MINK ? F::pow_(v, mp.root) : F::sqrt_(v);
+        const bool on = mine != kSentinelIdx && v == v;  // NaN is never admitted
+        v = on ? v : F::inf();
+        uint32_t ix = on ? mine : kSentinelIdx;
+        // a batch with nothing at or below the list's k-th value leaves it as it is
+        if (__builtin_amdgcn_ballot_w64(on && !(kth(k) < v)) == 0ull) return;
+        wave_sort64<T>(v, ix, lane);
+        merge(v, ix, lane);
+    }
+    // A screen value no row of the answer exceeds, from the k-th exact value:
+    // exact <= R means screen <= R in screen units + eps.
+    __device__ __forceinline__ float screen_bound(int k, int mode, float qn, double eps, double eps_t) const {
+        if (MINK && mode == EMIT_ROOT_RANKED) return __builtin_huge_valf();
+        double R = (double)kth(k);
+        if (mode == EMIT_ROOT_RANKED) R = R * R * (1.0 + 0x1p-40);
+        return R < (double)__builtin_huge_valf() ? round_up_f(R - (COS ? 1.0 : (double)qn) + eps + eps_t * R)
+                                                 : __builtin_huge_valf();
+    }
+    // A query every row of which is evaluated: a zero query's values are all
+    // exactly 1 (or NaN, never admitted), so the first k rows are its answer.
+    __device__ __forceinline__ bool settled(int k) const { return COS && qzero && kth(k) < F::inf(); }
+    __device__ __forceinline__ void emit(T* __restrict__ ov, uint32_t* __restrict__ oi, int k, int mode, int lane) const {
+#pragma unroll
+        for (int b = 0; b < KL; ++b) {
+            const int s = 64 * b + lane;
+            if (s < k) {
+                ov[s] = mode == EMIT_SQRT ? F::sqrt_(lv[b]) : lv[b];
+                oi[s] = li[b] == kSentinelIdx ? 0u : li[b];
+            }
+        }
+    }
+};
+
+// What both selection kernels read of a query.
+template <typename TS>
+struct GmQuery {
+    const float* G;   // its group minima, [2][ntp]
+    int n, ntp;
+    uint32_t nt;
+    float qn;
+    uint32_t nforced;
+    bool all_rows;
+    double eps, eps_t;
+    const float* bias;
+    int bias_nan;
+    __device__ __forceinline__ GmQuery(const GmSelectArgs<TS>& a, int64_t q) {
+        G = a.gmin + q * 2 * a.ntp;
+        ntp = (int)a.ntp;
+        n = 2 * ntp;  // a multiple of 8
+        nt = (uint32_t)a.nt;
+        eps_t = a.eps_t;
+        if (!a.stats) {  // minima of the arm's own values
+            qn = 0.0f;
+            nforced = 0u;
+            all_rows = false;
+            eps = 0.0;
+        } else {
+            qn = a.qnorm[q];
+            nforced = a.stats->nforced;
+            all_rows = !(qn == qn) || nforced > (uint32_t)kGmForced;
+            eps = a.eps_rel * ((double)qn + (double)__uint_as_float(a.stats->xmax_bits)) + a.eps_abs;
+        }
+        bias = a.bias;
+        bias_nan = a.bias_nan;
+    }
+    // row j of group f; rows left out by the scan are evaluated from their list
+    __device__ __forceinline__ uint32_t row(int f, int j) const {
+        const int half = f >= ntp ? 1 : 0;
+        const uint32_t r = (uint32_t)(f - (half ? ntp : 0)) * kGmRows + (uint32_t)gm_group_row(half, j);
+        bool on = r < nt;
+        if (nforced) {
+            const float b = bias[r];
+            on = on && (bias_nan ? b == b : b < __builtin_huge_valf());
+        }
+        return on ? r : kSentinelIdx;
+    }
+    // every row of the answer lies in a group whose minimum is at or below this
+    __device__ __forceinline__ float bound(float t) const {
+        return t < __builtin_huge_valf() ? round_up_f((double)t + 2.0 * eps + eps_t * (double)t) : __builtin_huge_valf();
+    }
+};
+
+// A workgroup per query: few queries, long indexes.
+template <typename T, typename TS, int ARM, int KL>
+__global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
+    __shared__ __attribute__((aligned(16))) T sq[kGmMaxD];
+    __shared__ __attribute__((aligned(16))) float cm[kSelCap];
+    __shared__ uint32_t cg[kSelCap];
+    __shared__ T mv[3 * 64 * KL];
+    __shared__ uint32_t s_cnt;
+    __shared__ float s_kth;
+    __shared__ float s_wthr[4];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t q = blockIdx.x;
+    const int d = (int)a.d, k = a.k, mode = a.mode;
+    const TS* __restrict__ X = a.x;
+    const float inf = __builtin_huge_valf();
+    const GmQuery<TS> Q(a, q);
+    const int n = Q.n;
+    GmList<T, TS, ARM, KL> L(a);
+    if (tid < d) sq[tid] = (T)a.q[q * d + tid];
+    if (tid == 0) {
+        s_cnt = 0u;
+        s_kth = inf;
+    }
+
+    // ---- the group minima: up to 4096 of them stay in registers ----
+    const bool held = n <= 4096;
+    float4 g[4];
+    float m = inf;
+    auto load_minima = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int at = i + 1024 * j;
+            g[j] = at < n ? gload4(Q.G + at) : make_float4(inf, inf, inf, inf);
+        }
+    };
+    if (!Q.all_rows) {
+        for (int i = 4 * tid; i < n; i += 4096) {
+            load_minima(i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) m = fminf(m, fminf(fminf(g[j].x, g[j].y), fminf(g[j].z, g[j].w)));
+        }
+    }
+    cm[tid] = m;
+    __syncthreads();
+    L.set_query(sq, d);
+
+    if (Q.all_rows) {
+        for (uint32_t r0 = 0; r0 < Q.nt; r0 += 256) {
+            L.evaluate(r0 + tid < Q.nt ? r0 + tid : kSentinelIdx, sq, X, d, k, mode, lane);
+            if (L.settled(k)) break;  // this wave's rows; the others' end alike
+        }
+    } else {
+        if (Q.nforced) L.evaluate(tid < (int)Q.nforced ? a.forced[tid] : kSentinelIdx, sq, X, d, k, mode, lane);
+        // ---- a first bound: the k-th smallest of the 256 threads' minima ----
+        auto rank_of = [&](float v, int at, int count) -> int {
+            int less = 0;
+            int j = 0;
+            for (; j + 4 <= count; j += 4) {
+                const float4 o = *reinterpret_cast<const float4*>(cm + j);
+                less += (o.x < v || (o.x == v && j < at)) ? 1 : 0;
+                less += (o.y < v || (o.y == v && j + 1 < at)) ? 1 : 0;
+                less += (o.z < v || (o.z == v && j + 2 < at)) ? 1 : 0;
+                less += (o.w < v || (o.w == v && j + 3 < at)) ? 1 : 0;
+            }
+            for (; j < count; ++j) {
+                const float o = cm[j];
+                less += (o < v || (o == v && j < at)) ? 1 : 0;
+            }
+            return less;
+        };
+        if (rank_of(m, tid, 256) == k - 1) s_kth = m;
+        __syncthreads();
+        float thr = Q.bound(s_kth);
+        // ---- the groups at or below it ----
+        for (int i = 4 * tid; i < n; i += 4096) {
+            if (!held) load_minima(i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float e[4] = {g[j].x, g[j].y, g[j].z, g[j].w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (e[c] <= thr && e[c] < inf) {
+                        const uint32_t at = atomicAdd(&s_cnt, 1u);
+                        if (at < (uint32_t)kSelCap) {
+                            cm[at] = e[c];
+                            cg[at] = (uint32_t)(i + 1024 * j + c);
+                        }
+                    }
+            }
+        }
+        __syncthreads();
+        int count = (int)s_cnt;
+        if (count <= kSelCap) {
+            // ---- the exact k-th smallest minimum, and the list cut to it.
+            //      (All groups at or below the first bound are listed, the k
+            //      smallest among them.) ----
+            if (count > k && count <= kSelRefine) {
+                float v[2];
+                uint32_t gi[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int at = tid + 256 * j;
+                    v[j] = at < count ? cm[at] : inf;
+                    gi[j] = at < count ? cg[at] : 0u;
+                    if (at < count && rank_of(v[j], at, count) == k - 1) s_kth = v[j];
+                }
+                __syncthreads();
+                thr = Q.bound(s_kth);
+                if (tid == 0) s_cnt = 0u;
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    if (tid + 256 * j < count && v[j] <= thr) cg[atomicAdd(&s_cnt, 1u)] = gi[j];
+                __syncthreads();
+                count = (int)s_cnt;
+            }
+            for (int g0 = 4 * wv; g0 < count; g0 += 16) {
+                const int at = g0 + (lane >> 4);
+                L.evaluate(at < count ? Q.row((int)cg[at], lane & 15) : kSentinelIdx, sq, X, d, k, mode, lane);
+            }
+        } else {
+            // ---- too many to list (ties, or distances the screen does not
+            //      resolve): every group at or below the bound, 16 at a time,
+            //      the bound following the waves' k-th exact values ----
+            for (int f0 = 0; f0 < n; f0 += 16) {
+                const int f = f0 + (tid >> 4);
+                const float gm = f < n ? Q.G[f] : inf;
+                const uint32_t mine = (gm <= thr && gm < inf) ? Q.row(f, tid & 15) : kSentinelIdx;
+                if (!__syncthreads_or(mine != kSentinelIdx)) continue;
+                L.evaluate(mine, sq, X, d, k, mode, lane);
+                const float t = L.screen_bound(k, mode, Q.qn, Q.eps, Q.eps_t);
+                if (lane == 0) s_wthr[wv] = t;
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < 4; ++i) thr = fminf(thr, s_wthr[i]);
+            }
+        }
+    }
+
+    // ---- the four waves' lists into wave 0's, and out ----
+    uint32_t* mi = cg;
+    __syncthreads();
+    if (wv > 0) {
+#pragma unroll
+        for (int b = 0; b < KL; ++b) {
+            mv[(wv - 1) * 64 * KL + 64 * b + lane] = L.lv[b];
+            mi[(wv - 1) * 64 * KL + 64 * b + lane] = L.li[b];
+        }
+    }
+    __syncthreads();
+    if (wv > 0) return;
+#pragma unroll
+    for (int b = 0; b < 3 * KL; ++b) L.merge(mv[64 * b + lane], mi[64 * b + lane], lane);
+    L.emit(static_cast<T*>(a.out_val) + q * k, a.out_idx + q * k, k, mode, lane);
+}
+
+// A wave per query: many queries.  No barrier, no atomic: the bound is the
+// k-th smallest of the lanes' two smallest minima, the groups below it are
+// compacted with ballots, and the wave's own list is the answer.
+constexpr int kSelWaveCap = 256;
+template <typename T, typename TS, int ARM, int KL>
+__global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS> a) {
+    __shared__ __attribute__((aligned(16))) T sq_[4][kGmMaxD];
+    __shared__ float cm_[4][kSelWaveCap];
+    __shared__ uint32_t cg_[4][kSelWaveCap];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t q = (int64_t)blockIdx.x * 4 + wv;
+    if (q >= a.nq) return;
+    T* __restrict__ sq = sq_[wv];
+    float* __restrict__ cm = cm_[wv];
+    uint32_t* __restrict__ cg = cg_[wv];
+    const int d = (int)a.d, k = a.k, mode = a.mode;
+    const TS* __restrict__ X = a.x;
+    const float inf = __builtin_huge_valf();
+    const uint64_t below = (1ull << lane) - 1ull;
+    const GmQuery<TS> Q(a, q);
+    const int n = Q.n;
+    GmList<T, TS, ARM, KL> L(a);
+    for (int c = lane; c < d; c += 64) sq[c] = (T)a.q[q * d + c];
+    wave_lds_fence();
+    L.set_query(sq, d);
+
+    if (Q.all_rows) {
+        for (uint32_t r0 = 0; r0 < Q.nt; r0 += 64) {
+            L.evaluate(r0 + lane < Q.nt ? r0 + lane : kSentinelIdx, sq, X, d, k, mode, lane);
+            if (L.settled(k)) break;
+        }
+        L.emit(static_cast<T*>(a.out_val) + q * k, a.out_idx + q * k, k, mode, lane);
+        return;
+    }
+    for (uint32_t f0 = 0; f0 < Q.nforced; f0 += 64)
+        L.evaluate(f0 + lane < Q.nforced ? a.forced[f0 + lane] : kSentinelIdx, sq, X, d, k, mode, lane);
+
+    // ---- the minima (up to 1024 stay in registers) and the first bound ----
+    const bool held = n <= 1024;
+    float4 g[4];
+    auto load_minima = [&](int i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int at = i + 256 * j;
+            g[j] = at < n ? gload4(Q.G + at) : make_float4(inf, inf, inf, inf);
+        }
+    };
+    float m1 = inf, m2 = inf;
+    for (int i0 = 0; i0 < n; i0 += 1024) {
+        load_minima(i0 + 4 * lane);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float e[4] = {g[j].x, g[j].y, g[j].z, g[j].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                m2 = fminf(m2, fmaxf(m1, e[c]));
+                m1 = fminf(m1, e[c]);
+            }
+        }
+    }
+    float bv[KL];
+    uint32_t bi[KL];
+#pragma unroll
+    for (int b = 0; b < KL; ++b) {
+        bv[b] = inf;
+        bi[b] = kSentinelIdx;
+    }
+    {
+        uint32_t i1 = (uint32_t)lane, i2 = 64u + (uint32_t)lane;
+        wave_sort64<float>(m1, i1, lane);
+        bv[0] = m1;
+        bi[0] = i1;
+        if (KL > 1 || k > 16) {
+            wave_sort64<float>(m2, i2, lane);
+            if constexpr (KL == 1) wave_merge64<float>(bv[0], bi[0], m2, i2, lane);
+            else wave_merge_blocks<float, KL>(bv, bi, m2, i2, lane);
+        }
+    }
+    float thr = Q.bound(list_value_at<float, KL>(bv, k - 1));
+
+    // ---- the groups at or below it ----
+    uint32_t cnt = 0;
+    for (int i0 = 0; i0 < n; i0 += 1024) {
+        if (!held) load_minima(i0 + 4 * lane);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float e[4] = {g[j].x, g[j].y, g[j].z, g[j].w};
+            const float lo = fminf(fminf(e[0], e[1]), fminf(e[2], e[3]));
+            if (__builtin_amdgcn_ballot_w64(lo <= thr && lo < inf) == 0ull) continue;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const bool in = e[c] <= thr && e[c] < inf;
+                const uint64_t bal = __builtin_amdgcn_ballot_w64(in);
+                const uint32_t at = cnt + (uint32_t)__builtin_popcountll(bal & below);
+                if (in && at < (uint32_t)kSelWaveCap) {
+                    cm[at] = e[c];
+                    cg[at] = (uint32_t)(i0 + 256 * j + 4 * lane + c);
+                }
+                cnt += (uint32_t)__builtin_popcountll(bal);
+            }
+        }
+    }
+    wave_lds_fence();
+    if (cnt <= (uint32_t)kSelWaveCap) {
+        // ---- the exact k-th smallest minimum, and the list cut to it ----
+        if (cnt > (uint32_t)k) {
+#pragma unroll
+            for (int b = 0; b < KL; ++b) {
+                bv[b] = inf;
+                bi[b] = kSentinelIdx;
+            }
+            for (uint32_t b0 = 0; b0 < cnt; b0 += 64) {
+                float v = b0 + lane < cnt ? cm[b0 + lane] : inf;
+                uint32_t ix = b0 + lane;
+                wave_sort64<float>(v, ix, lane);
+                if constexpr (KL == 1) wave_merge64<float>(bv[0], bi[0], v, ix, lane);
+                else wave_merge_blocks<float, KL>(bv, bi, v, ix, lane);
+            }
+            thr = Q.bound(list_value_at<float, KL>(bv, k - 1));
+            uint32_t kept = 0;
+            for (uint32_t b0 = 0; b0 < cnt; b0 += 64) {
+                const bool in = b0 + lane < cnt && cm[b0 + lane] <= thr;
+                const uint32_t gi = b0 + lane < cnt ? cg[b0 + lane] : 0u;
+                const uint64_t bal = __builtin_amdgcn_ballot_w64(in);
+                wave_lds_fence();
+                if (in) cg[kept + (uint32_t)__builtin_popcountll(bal & below)] = gi;
+                wave_lds_fence();
+                kept += (uint32_t)__builtin_popcountll(bal);
+            }
+            cnt = kept;
+        }
+        for (uint32_t g0 = 0; g0 < cnt; g0 += 4) {
+            const uint32_t at = g0 + (lane >> 4);
+            L.evaluate(at < cnt ? Q.row((int)cg[at], lane & 15) : kSentinelIdx, sq, X, d, k, mode, lane);
+        }
+    } else {
+        // ---- too many to list: the groups at or below the bound, four at a
+        //      time, the bound following the k-th exact value ----
+        for (int f0 = 0; f0 < n; f0 += 64) {
+            const float gm = f0 + lane < n ? Q.G[f0 + lane] : inf;
+            uint64_t todo = __builtin_amdgcn_ballot_w64(gm <= thr && gm < inf);
+            while (todo) {
+                int f = -1;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int bit = todo ? __builtin_ctzll(todo) : -1;
+                    if ((lane >> 4) == i) f = bit;
+                    todo &= todo - 1;  // 0 stays 0
+                }
+                L.evaluate(f >= 0 ? Q.row(f0 + f, lane & 15) : kSentinelIdx, sq, X, d, k, mode, lane);
+                thr = fminf(thr, L.screen_bound(k, mode, Q.qn, Q.eps, Q.eps_t));
+                todo &= __builtin_amdgcn_ballot_w64(gm <= thr);
+            }
+        }
+    }
+    L.emit(static_cast<T*>(a.out_val) + q * k, a.out_idx + q * k, k, mode, lane);
+}
+
+template <typename T, typename TS, int ARM, int KL>
+void gm_select_launch(const GmSelectArgs<TS>& a, hipStream_t s) {
+    if (KL == 1 && a.nq >= 1000 && 2 * a.ntp <= 16384)
+        hipLaunchKernelGGL((gm_select_wave_kernel<T, TS, ARM, KL>), dim3((unsigned)((a.nq + 3) / 4)), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((gm_select_kernel<T, TS, ARM, KL>), dim3((unsigned)a.nq), dim3(256), 0, s, a);
+}
+
+template <typename T, typename TS, int ARM>
+void gm_select_k(const GmSelectArgs<TS>& a, hipStream_t s) {
+    if (a.k <= 64) gm_select_launch<T, TS, ARM, 1>(a, s);
+    else gm_select_launch<T, TS, ARM, 2>(a, s);
+}
+
+}  // namespace
+
+}  // namespace mlrs

@@ -243,6 +243,12 @@ template <typename T>
 hipError_t launch_pairwise_tile(const T* x, int64_t nx, const T* y, int64_t ny, int64_t d, int arm,
                                 const T* xa, const T* ya, T* out, int64_t ldo, int root,
                                 hipStream_t s, T pexp = T(0), int pint = 0, T root_exp = T(0));
+// The minima over each group of 16 y rows of the Manhattan, Chebyshev and
+// Minkowski arms' exact values, rounded to f32: gmin [nx][2][ntp] as the
+// group-minimum scan lays it out (ntp a multiple of 4).
+template <typename T>
+hipError_t launch_groupmin_tile(const T* x, int64_t nx, const T* y, int64_t ny, int64_t d, int arm, T pexp, int pint,
+                                float* gmin, int64_t ntp, hipStream_t s);
 template <typename T>
 hipError_t launch_pow_inplace(T* v, int64_t n, T e, hipStream_t s);
 // dst[0..n) = src[0..n) (the fit-time ownership copy).

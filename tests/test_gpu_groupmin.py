@@ -124,3 +124,36 @@ def test_noalloc_index_parts(nt, d, metric):
         out.append((dist.view(torch.int32), idx))
     torch.cuda.synchronize()
     assert torch.equal(out[0][1], out[1][1]) and torch.equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("metric", ["manhattan", "chebyshev"])
+@pytest.mark.parametrize("nt,d,k,nq", [(5, 1, 5, 1), (33, 7, 33, 65), (129, 16, 100, 63), (4100, 17, 10, 1000),
+                                       (2000, 40, 65, 200), (700, 256, 3, 64), (20_000, 3, 12, 30)])
+def test_metric_arms(dtype, metric, nt, d, k, nq):
+    """The exact tiles' minima: edges of the 64 x 128 tile, values past the f32
+    range, infinities, NaN, ties."""
+    prims.force_path("auto")
+    xt, xq = _rows(nt + d, nt, d, dtype), _rows(nq, nq, d, dtype)
+    xt[nt // 2] = xt[nt - 1]
+    if nt > 100:
+        xt[3, 0], xt[4, d - 1], xt[5, 0] = np.nan, np.inf, -np.inf
+        xt[6] *= dtype(1e30)
+        if dtype is np.float64:
+            xt[7] *= 1e200
+        xq[0] = xt[nt - 1]
+        xq[nq - 1, 0] = np.inf
+        if nq > 60:
+            xq[nq - 2, 0] = np.nan
+    _check(xq, xt, k, metric)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("metric", ["euclidean", "cosine", "manhattan", "chebyshev"])
+@pytest.mark.parametrize("nx,ny,d", [(1, 1, 1), (63, 129, 15), (64, 128, 16), (65, 127, 17), (130, 300, 50)])
+def test_pairwise_tile_edges(dtype, metric, nx, ny, d):
+    x, y = _rows(nx, nx, d, dtype), _rows(ny + 1, ny, d, dtype)
+    want = oracle.pairwise(x, y, metric, sqrt=True)
+    got = prims.pairwise_distance(torch.from_numpy(x).to(DEV), torch.from_numpy(y).to(DEV), metric, sqrt=True)
+    bits = np.int32 if dtype == np.float32 else np.int64
+    assert np.array_equal(got.cpu().numpy().view(bits), want.view(bits))
