@@ -776,61 +776,59 @@ template <typename T, typename TS>
 int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t d, int k, int arm, int mode,
                      T* out_v, uint32_t* out_i, hipStream_t s) {
     const bool cos = (arm == ARM_COS_FOLD || arm == ARM_COS_HOST);
-    // The scan reads an f32 copy of the index (centred or unit rows).  The
-    // allocation-free entry point has no room for one: it scans aligned f32
-    // rows in place, and copies others a part at a time.
-    const bool copy = sizeof(TS) == 8 || !g_noalloc || d % 4 != 0 || (reinterpret_cast<uintptr_t>(xt) & 15) != 0;
-    const int64_t ldx = (d + 3) / 4 * 4;
+    // The scan reads a copy of the index (centred or unit rows, two f16 halves
+    // per element); what does not fit the scratch is copied a part at a time.
+    const int64_t ldx = (d + 15) / 16 * 16;
     const int64_t dp = 8 * (int64_t)gm_chunks(d);
     const int64_t ntp = gm_tiles(nt);
     constexpr int64_t kPart = kGmRows * kGmQuad;  // index parts are whole stores of the scan
     // Copied rows at a time: 4 GiB holds any index but the largest whole; a
     // larger one is copied and scanned part by part for each set of queries.
     const size_t limit = workspace_limit();
-    const size_t fixed = aligned_bytes(sizeof(float) * (size_t)ntp * kGmRows) + aligned_bytes(sizeof(GmStats)) +
-                         aligned_bytes(sizeof(uint32_t) * kGmForced) + sizeof(float) * (size_t)dp * kGmQpb + 4096;
+    const size_t fixed = 2 * aligned_bytes(sizeof(float) * (size_t)ntp * kGmRows) + aligned_bytes(sizeof(GmStats)) +
+                         aligned_bytes(sizeof(uint32_t) * kGmForced) + sizeof(float) * (size_t)dp * 2 * kGmQpb + 4096;
     size_t room = limit == SIZE_MAX ? (size_t)5 << 30 : (limit > fixed ? limit - fixed : 0);
-    int64_t xrows = 0;
-    if (copy) {
-        const size_t most = limit == SIZE_MAX ? (size_t)4 << 30 : room / 8 * 3;
-        const int64_t fit = (int64_t)(most / (sizeof(float) * (size_t)ldx)) / kPart * kPart;
-        xrows = std::min<int64_t>(ntp * kGmRows, std::max<int64_t>(fit, kPart));
-        room -= std::min(room, sizeof(float) * (size_t)(xrows * ldx) + 256);
-    }
-    const bool whole = !copy || xrows >= nt;
+    const size_t most = limit == SIZE_MAX ? (size_t)4 << 30 : room / 8 * 3;
+    const int64_t fit = (int64_t)(most / (sizeof(float) * (size_t)ldx)) / kPart * kPart;
+    const int64_t xrows = std::min<int64_t>(ntp * kGmRows, std::max<int64_t>(fit, kPart));
+    room -= std::min(room, sizeof(float) * (size_t)(xrows * ldx) + 256);
+    const bool whole = xrows >= nt;
     // The minima of as many queries as the budget holds: 1 GiB keeps the scan
     // launches long (the tail of one costs about one unit of the split) and
     // the memory modest.
-    const size_t per_q = 2 * sizeof(float) * (size_t)ntp + sizeof(float) * (size_t)(dp + 1);
+    const size_t per_q = 2 * sizeof(float) * (size_t)ntp + sizeof(float) * (size_t)(dp + 2);
     int64_t qc = std::max<int64_t>(1, std::min<int64_t>(nq, (int64_t)(std::min(room, (size_t)1 << 30) / per_q)));
-    if (qc < nq && qc > kGmQpb) {
-        const int64_t parts = (nq + qc / kGmQpb * kGmQpb - 1) / (qc / kGmQpb * kGmQpb);
-        qc = ((nq + parts - 1) / parts + kGmQpb - 1) / kGmQpb * kGmQpb;
+    if (qc < nq && qc > 2 * kGmQpb) {
+        constexpr int64_t kSet = 2 * kGmQpb;
+        const int64_t parts = (nq + qc / kSet * kSet - 1) / (qc / kSet * kSet);
+        qc = ((nq + parts - 1) / parts + kSet - 1) / kSet * kSet;
     }
-    const int64_t qpad = (qc + kGmQpb - 1) / kGmQpb * kGmQpb;
+    const int64_t qpad = (qc + 2 * kGmQpb - 1) / (2 * kGmQpb) * (2 * kGmQpb);
     char* ws;
     int cus;
     int32_t rc = workspace(fixed + sizeof(float) * (size_t)(xrows * ldx) + 2 * sizeof(float) * (size_t)(ntp * qc) +
-                               sizeof(float) * (size_t)(dp * qc + qc),
+                               sizeof(float) * (size_t)(dp * qc + 2 * qc),
                            s, &ws, &cus);
     if (rc) return rc;
     Carver cv(ws);
     float* bias = cv.take<float>((size_t)ntp * kGmRows);
     GmStats* stats = cv.take<GmStats>(1);
     uint32_t* forced = cv.take<uint32_t>(kGmForced);
-    float* xcopy = copy ? cv.take<float>((size_t)(xrows * ldx)) : nullptr;
+    float* xinv = cv.take<float>((size_t)ntp * kGmRows);
+    float* xcopy = cv.take<float>((size_t)(xrows * ldx));
     float* qop = cv.take<float>((size_t)(qpad * dp));
     float* qnorm = cv.take<float>((size_t)qc);
+    float* qinv = cv.take<float>((size_t)qc);
     float* gmin = cv.take<float>(2 * (size_t)ntp * (size_t)qc);
 
     GmPrepArgs pq{};
     pq.d = d;
-    pq.centre = (copy && !cos) ? xt : nullptr;
+    pq.centre = cos ? nullptr : xt;
     pq.centre_n = nt;
     pq.out = qop;
     pq.ldo = dp;
     pq.norm = qnorm;
-    pq.scale = cos ? -1.0f : -2.0f;
+    pq.inv = qinv;
     pq.queries = 1;
     pq.cosine = cos;
     pq.stats = stats;
@@ -838,12 +836,12 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     GmPrepArgs px = pq;
     px.out = xcopy;
     px.ldo = ldx;
-    px.scale = 1.0f;
     px.queries = 0;
-    px.unit = copy;
 
     GmScanArgs sc{};
     sc.q = qop;
+    sc.x = xcopy;
+    sc.qinv = qinv;
     sc.ldx = ldx;
     sc.d = ldx;
     sc.ntp = ntp;
@@ -861,23 +859,29 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     se.qnorm = qnorm;
     se.stats = stats;
     se.forced = forced;
-    se.bias_nan = cos && !copy;
     // |screen - exact| <= eps, with u = 2^-23 and N = ||q||^2 + ||x||^2.
-    // Euclidean: the contraction's d roundings are of partial sums up to 2 N,
-    // in any rounding mode of the matrix core: 2 d u N; the arms' d + 2
-    // roundings to nearest of a value up to 2 N: (d + 2) u N; the norms (sums
-    // of four, then a tree): 6 u N; the copy's rounding moves a distance by at
-    // most 2^-24 (||q|| + ||x||), its square by 2.02 u N.  Cosine, of unit
-    // vectors: d u, the arms' dot product and norms (d + 3) u, the unit rows'
-    // own rounding 12 u.  The absolute term covers flushed subnormals.
+    // Euclidean: the contraction's 3 dp additions round partial sums of 2 x.q,
+    // which stay below 1.01 N, in any rounding mode of the matrix core: 3.1 dp
+    // u N.  The halves: each element is kept to 2^-22 of itself, and lo times
+    // lo is left out, 3 * 2^-22 * 2 ||q|| ||x|| <= 6 u N; halves below f16's
+    // normal range, if flushed, lose 2^-27.5 of the row's norm per half, times
+    // sqrt(d) <= 16 over the row: 6 u N for both operands.  The sum with the
+    // norm 2 u N; the arms' d + 2 roundings to nearest of a value up to 2 N:
+    // (d + 2) u N; the norms (sums of four, then a tree): 6 u N; the copy's
+    // rounding moves a distance by at most 2^-24 (||q|| + ||x||), its square by
+    // 2.02 u N.  Cosine, of unit vectors (N = 1 for 2 x.q <= N): 3.1 dp u / 2
+    // and the same allowances, the arms' dot product and norms (d + 3) u, the
+    // unit rows' own rounding 12 u.  The absolute term covers flushed
+    // subnormals and rows below 2^-50, which share a scale.
     const double u = std::ldexp(1.0, -23);
-    se.eps_rel = cos ? 0.0 : (3.0 * (double)d + 24.0) * u;
-    se.eps_abs = cos ? (2.0 * (double)d + 32.0) * u : (double)(d + 4) * std::ldexp(1.0, sizeof(TS) == 8 ? -100 : -120);
+    se.eps_rel = cos ? 0.0 : (3.1 * (double)dp + (double)d + 32.0) * u;
+    se.eps_abs = cos ? (3.1 * (double)dp + (double)d + 40.0) * u
+                     : (double)(d + 16) * std::ldexp(1.0, sizeof(TS) == 8 ? -100 : -120);
     for (int64_t q0 = 0; q0 < nq; q0 += qc) {
         const int64_t n = std::min<int64_t>(qc, nq - q0);
         pq.rows = xq + q0 * d;
         pq.n = n;
-        pq.n_out = (n + kGmQpb - 1) / kGmQpb * kGmQpb;
+        pq.n_out = (n + 2 * kGmQpb - 1) / (2 * kGmQpb) * (2 * kGmQpb);
         pq.n_norm = n;
         pq.reset = q0 == 0 || !whole;
         hipError_t e = launch_gm_prep<TS>(pq, s);
@@ -890,17 +894,18 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
                 px.row0 = x0;
                 px.n = px.n_out = rows;
                 px.norm = bias + x0;
+                px.inv = xinv + x0;
                 px.n_norm = gm_tiles(rows) * kGmRows;
                 e = launch_gm_prep<TS>(px, s);
             }
-            sc.x = copy ? xcopy : reinterpret_cast<const float*>(xt) + x0 * d;
             sc.bias = bias + x0;
+            sc.xinv = xinv + x0;
             sc.nt = rows;
             sc.tiles = gm_tiles(rows);
             sc.gmin = gmin + x0 / kGmRows;
             if (e == hipSuccess) {
                 KernelTimer timer(s, "knn_groupmin_kernel");
-                e = cos && !copy ? launch_gm_scan_cosine(sc, s) : launch_gm_scan_euclid(sc, s);
+                e = launch_gm_scan(sc, s);
             }
         }
         se.q = xq + q0 * d;

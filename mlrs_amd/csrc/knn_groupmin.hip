@@ -7,8 +7,8 @@ namespace mlrs {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Preparation: norms, the rows the screen cannot be trusted with, and where
-// wanted the f32 copy.  LPR lanes share a row, four consecutive columns each.
+// Preparation: norms, the rows the screen cannot be trusted with, and the
+// scaled copy of two halves per element.  LPR lanes share a row, four consecutive columns each.
 // Bound by the read of the rows.
 // ---------------------------------------------------------------------------
 template <typename T> struct GmRange;
@@ -22,6 +22,8 @@ template <> struct GmRange<double> {
     static __device__ __forceinline__ bool euclid(double s) { return s <= 0x1p120; }
     static __device__ __forceinline__ bool cosine(double s) { return s >= 0x1p-500 && s <= 0x1p500; }
 };
+
+typedef _Float16 gm_f16x4 __attribute__((ext_vector_type(4)));
 
 template <typename T, int LPR>
 __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
@@ -52,7 +54,7 @@ __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
                 ctr[e] = (m - m == T(0)) ? m : T(0);
             }
     }
-    const int64_t n = a.n, n_out = a.out ? a.n_out : 0;
+    const int64_t n = a.n, n_out = a.n_out;
     const int64_t n_all = n_out > a.n_norm ? n_out : a.n_norm;
     const bool vec = (d % 4 == 0) && ((reinterpret_cast<uintptr_t>(X) & 15) == 0);
     float xmax = 0.0f;
@@ -120,13 +122,30 @@ __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) f[e] = (float)(v[u][e] * inv);
             }
-            if (a.out && r < n_out && c0 < a.ldo) {
-                float4 o = make_float4(a.scale * f[0], a.scale * f[1], a.scale * f[2], a.scale * f[3]);
-                if (!on || !trusted) o = make_float4(0.f, 0.f, 0.f, 0.f);
-                *reinterpret_cast<float4*>(a.out + r * a.ldo + c0) = o;
+            // The row's scale: the power of two that takes its norm to at most
+            // 2^15, so that no element leaves f16's range and what f16 cannot
+            // resolve (2^-14 and less) is below 2^-27 of the norm.  Norms below
+            // 2^-50 share one scale; what they lose is in eps_abs.
+            int ex = 14;
+            if (!a.cosine) ex = 15 - ((__builtin_amdgcn_frexp_expf(fmaxf((float)s, 0x1p-100f)) + 1) >> 1);
+            if (!on || !trusted) ex = 0;
+            if (r < n_out && c0 < a.ldo) {
+                gm_f16x4 hi, lo;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float v_ = __builtin_ldexpf((on && trusted) ? (a.queries ? -f[e] : f[e]) : 0.0f, ex);
+                    hi[e] = (_Float16)v_;
+                    lo[e] = (_Float16)(v_ - (float)hi[e]);
+                }
+                // 16 columns are four 16-byte chunks: high halves of the first
+                // and the last eight, then the low halves
+                char* o = reinterpret_cast<char*>(a.out + r * a.ldo) + 4 * (c0 & ~15) + 2 * (c0 & 15);
+                *reinterpret_cast<gm_f16x4*>(o) = hi;
+                *reinterpret_cast<gm_f16x4*>(o + 32) = lo;
             }
             if (sub != 0 || r >= a.n_norm) continue;
             const float nan = __builtin_nanf(""), inf = __builtin_huge_valf();
+            a.inv[r] = __builtin_ldexpf(1.0f, (a.queries && !a.cosine ? 1 : 0) - ex);
             if (a.queries) {
                 a.norm[r] = trusted ? (a.cosine ? 0.0f : (float)s) : nan;
                 continue;
@@ -135,8 +154,7 @@ __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
             // Euclidean: a row with a NaN scores NaN against every query and
             // is never admitted; cosine's fold arm scores it 1
             const bool force = on && !trusted && (a.cosine || s == s);
-            if (a.cosine && !a.unit) a.norm[r] = keep ? (float)inv : nan;
-            else a.norm[r] = keep ? (a.cosine ? 0.0f : (float)s) : inf;
+            a.norm[r] = keep ? (a.cosine ? 0.0f : (float)s) : inf;
             if (keep && !a.cosine) xmax = fmaxf(xmax, (float)s);
             if (force) {
                 const unsigned int at = atomicAdd(&a.stats->nforced, 1u);
@@ -169,9 +187,8 @@ void gm_prep_lpr(const GmPrepArgs& a, int64_t n_all, hipStream_t s) {
 
 template <typename T>
 hipError_t launch_gm_prep(const GmPrepArgs& a, hipStream_t s) {
-    const int64_t n_out = a.out ? a.n_out : 0;
-    const int64_t n_all = n_out > a.n_norm ? n_out : a.n_norm;
-    const int64_t cols = a.out && a.ldo > a.d ? a.ldo : a.d;
+    const int64_t n_all = a.n_out > a.n_norm ? a.n_out : a.n_norm;
+    const int64_t cols = a.ldo > a.d ? a.ldo : a.d;
     if (cols <= 16) gm_prep_lpr<T, 4>(a, n_all, s);
     else if (cols <= 32) gm_prep_lpr<T, 8>(a, n_all, s);
     else if (cols <= 64) gm_prep_lpr<T, 16>(a, n_all, s);

@@ -2,7 +2,7 @@
 // and cosine arms (d <= 256, k <= 128), f32 and f64, in two passes.
 //
 //  scan    (knn_groupmin_scan.hpp) every (query, row) pair gets a screen value
-//          on v_mfma_f32_32x32x2f32, and only the minimum over each group of
+//          on the f16 matrix cores from operands of two halves, and only the minimum over each group of
 //          16 index rows is written: 4 bytes for 16 pairs.
 //  select  (knn_groupmin.hip) per query: T, the k-th smallest group minimum,
 //          bounds the k-th screen value (k groups hold k distinct rows at or
@@ -11,18 +11,20 @@
 //          those groups (about k of them) are evaluated exactly, in the
 //          reference arm's operation order, and ranked by (value, index).
 //
-// The screen is f32 whatever the element type: it only decides which pairs are
-// evaluated, never a result.  It works on an f32 copy of the index, made per
-// search: rows around a centre (Euclidean; a common shift leaves distances
+// The screen is the same whatever the element type: it only decides which pairs
+// are evaluated, never a result.  It works on a copy of the index, made per
+// search: f32 rows around a centre (Euclidean; a common shift leaves distances
 // alone, and the screen's error grows with the norms) or unit rows (cosine),
-// 16-byte aligned.  eps carries the rounding.
+// each scaled by a power of two and split into two f16 halves per element, 22
+// bits.  eps carries the rounding.
 //
-// Against the searches this one replaced (per-row admission into per-segment
-// lists behind f32 or f64 MFMA tiles; exact tiles and a selection for small
-// searches), ms per call: 1M x 10k, d = 128, k = 32, f32: 20.8 -> 19.1 (the
-// scan 17.5, 93% of the f32 MFMA peak); 200k x 5k, d = 256, k = 16, f64 cosine:
-// 9.40 -> 4.18; 60k-row f32 graph, d = 50, k = 15: 14.2 -> 3.76; 50k x 5k, d =
-// 50, k = 15, f32: 1.33 -> 0.32; 10k x 1k, d = 64, k = 10, f32: 0.090 -> 0.056.
+// ms per call of the searches this one replaced (per-row admission into
+// per-segment lists behind f32 or f64 MFMA tiles; exact tiles and a selection
+// for small searches), of this one with an f32 MFMA scan at 93% of that peak, and
+// now: 1M x 10k, d = 128, k = 32, f32: 20.8, 19.0, 8.1 (scan 6.3, selection 1.3);
+// 200k x 5k, d = 256, k = 16, f64 cosine: 9.41, 4.17, 1.84; 60k-row f32 graph, d =
+// 50, k = 15: 14.1, 3.69, 2.13; 50k x 5k, d = 50, k = 15, f32: 1.33, 0.32, 0.19; 10k
+// x 1k, d = 64, k = 10, f32: 0.090, 0.056, 0.049.
 // What it is bad at: points whose neighbours the screen cannot tell apart
 // (clusters a hundredth of their spacing wide and less, where every row of a
 // query's cluster is evaluated): 200k x 5k, d = 128 in 100 such clusters take
@@ -40,7 +42,7 @@ namespace mlrs {
 
 constexpr int kGmRows = 32;        // index rows per MFMA tile
 constexpr int kGmQuad = 4;         // tiles between stores of the minima
-constexpr int kGmQpb = 128;        // queries per workgroup: 4 waves of 32
+constexpr int kGmQpb = 128;        // queries of one block: 4 waves of 32; a workgroup takes one block or two
 constexpr int kGmMaxD = 256;
 constexpr int kGmMaxK = 128;
 constexpr int kGmForced = 256;     // forced rows listed before every query evaluates all rows
@@ -52,11 +54,14 @@ struct GmStats {
 };
 
 struct GmScanArgs {
-    const float* q;     // [nqb * 128][DP] query operand: -2 q (Euclidean) or -q / ||q||; zeros past nq
-    const float* x;     // index rows, 16-byte aligned, row stride ldx (a multiple of 4)
-    const float* bias;  // [tiles * 32] Euclidean ||x||^2, cosine in place 1 / ||x||, unit rows 0;
-                        // +inf (cosine in place: NaN) for rows left out
-    int64_t ldx, d;     // d: columns read per row (<= DP, a multiple of 4)
+    // Operand rows hold, per 16 columns, the high halves of the first and the
+    // last eight, then the low halves: 64 bytes, counted as 16 floats.
+    const float* q;     // [queries, rounded up to the launch's 128 or 256][DP] query operand: -q or -q / ||q||, scaled and split; zeros past nq
+    const float* x;     // index rows, scaled and split, row stride ldx (a multiple of 16)
+    const float* bias;  // [tiles * 32] Euclidean ||x||^2, cosine 0; +inf for rows left out
+    const float* xinv;  // [tiles * 32] what undoes the row's scale
+    const float* qinv;  // [nq] the same for the queries, times 2 (Euclidean)
+    int64_t ldx, d;     // d: columns read per row (<= DP, a multiple of 16)
     int64_t nq, nt;     // queries and index rows of this launch
     int64_t tiles;      // ceil(nt / 32), rounded up to kGmQuad
     int64_t ntp;        // tiles of the whole index: stride of gmin
@@ -65,31 +70,38 @@ struct GmScanArgs {
 };
 
 // Padded row width of the query operand: the 8-column steps the scan is
-// compiled for (every multiple of 8 up to 128, of 32 up to 256).
+// compiled for (every multiple of 16 columns up to 128, of 32 up to 256).
 inline int gm_chunks(int64_t d) {
     const int c = (int)((d + 7) / 8);
-    return c <= 16 ? c : (c + 3) / 4 * 4;
+    return c <= 16 ? (c + 1) / 2 * 2 : (c + 3) / 4 * 4;
+}
+// Two query blocks per workgroup read every LDS tile for twice the products
+// (one block keeps the LDS at about 80% of its rate), but leave half the
+// workgroups.  One block / two, us per search: 1M x 10k, d = 128: 8649 / 8091;
+// 60k x 60k, d = 50: 2338 / 2127; 50k x 5k, d = 50: 197 / 192; 10k x 1k, d = 64:
+// 49 / 51.  Past 128 columns two blocks' operands do not fit the registers.
+inline bool gm_two_blocks(int nk, int64_t nq, int64_t nt) {
+    return nk <= 16 && nq > kGmQpb && (double)nq * (double)nt >= 0x1p26;
 }
 inline int64_t gm_tiles(int64_t nt) { return ((nt + kGmRows - 1) / kGmRows + kGmQuad - 1) / kGmQuad * kGmQuad; }
 // Index rows of group (tile, half): row 8 (j / 4) + 4 half + j % 4 of the tile, j < 16.
 __host__ __device__ inline int gm_group_row(int half, int j) { return 8 * (j >> 2) + 4 * half + (j & 3); }
 
-// Rows of one kind, as given (T) to the scan's f32 operands.
+// Rows of one kind, as given (T) to the scan's operands.
 struct GmPrepArgs {
     const void* rows;    // [n][d] of T
     int64_t n, d;
     const void* centre;  // Euclidean copies: the index, whose first, middle and last rows give the centre
     int64_t centre_n;
     int64_t row0;        // index: number of the first row here (the forced list holds row numbers)
-    float* out;          // the f32 copy, row stride ldo (zeros past d), or null
+    float* out;          // the split copy, row stride ldo (a multiple of 16; zeros past d)
     int64_t ldo;
     int64_t n_out;       // rows of out (zeros past n)
     float* norm;         // index: bias; queries: ||q||^2 (0 for cosine), NaN where the screen is not trusted
-    int64_t n_norm;      // entries of norm (index: ntp * 32, +inf / NaN past n; queries: n)
-    float scale;         // queries: -2 (Euclidean) or -1 (cosine); index: 1
+    float* inv;          // undoes the rows' scales (queries, Euclidean: times 2)
+    int64_t n_norm;      // entries of norm and inv (index: ntp * 32, +inf past n; queries: n)
     int queries;         // 1: query operand; 0: index rows
     int cosine;
-    int unit;            // cosine: out holds unit rows and bias is 0; else bias is 1 / ||x|| (rows in place)
     GmStats* stats;      // filled from the index rows
     int reset;           // zero stats (the launch before the index's)
     uint32_t* forced;    // [kGmForced]
@@ -97,8 +109,7 @@ struct GmPrepArgs {
 template <typename T>
 hipError_t launch_gm_prep(const GmPrepArgs& a, hipStream_t s);
 
-hipError_t launch_gm_scan_euclid(const GmScanArgs& a, hipStream_t s);
-hipError_t launch_gm_scan_cosine(const GmScanArgs& a, hipStream_t s);
+hipError_t launch_gm_scan(const GmScanArgs& a, hipStream_t s);
 
 template <typename TS>
 struct GmSelectArgs {
@@ -114,7 +125,6 @@ struct GmSelectArgs {
     const uint32_t* forced;
     double eps_rel, eps_abs;  // eps = eps_rel (||q||^2 + max ||x||^2) + eps_abs
     double eps_t;        // relative error of a minimum (values rounded to f32)
-    int bias_nan;        // rows left out carry NaN (cosine in place) instead of +inf
     double pexp, root_exp;  // Minkowski: the exponent and (EMIT_ROOT_RANKED) its root's
     int pint;               // its integer exponent
     void* out_val;       // [nq][k] of T

@@ -1,9 +1,14 @@
 // The scan of the group-minimum search (knn_groupmin.hpp): screen values on
-// the f32 matrix cores, one minimum per (query, 16 index rows).  Included once
-// per arm family so that they compile side by side.
+// the f16 matrix cores, one minimum per (query, 16 index rows).
 //
-// Bound by the f32 MFMA rate.  A workgroup is 4 waves of 32 queries; each wave
-// holds its queries in VGPRs as the B operand (d / 2 registers), and the index
+// A screen value is the f32 norm plus a contraction whose operands are split
+// into two f16 halves each (gm_prep): x q = xh qh + xh ql + xl qh, three
+// v_mfma_f32_32x32x16_f16 per 16 columns where eight v_mfma_f32_32x32x2f32 of
+// twice the cycles stood, 96 cycles for 512.  Every row is scaled by its own
+// power of two before the split, so that the halves lie within f16's range and
+// hold 22 bits of every element that counts; the products accumulate in f32,
+// about half as many roundings as the f32 chain made.  A workgroup is 4 waves of 32 queries; each wave
+// holds its queries in VGPRs as the B operand (d / 2 registers: two halves of 16 bits per column), and the index
 // is walked in 32-row tiles through two LDS buffers with one barrier per tile.
 // A lane ends a tile with 16 values of one query (its half of the tile's rows)
 // and keeps their minimum: eight v_min3 for up to 128 MFMAs, where a screen
@@ -22,40 +27,45 @@ namespace mlrs {
 namespace {
 
 // A tile reaches LDS one tile ahead of its use, straight from global memory
-// (global_load_lds_dwordx4; the rows are 16-byte aligned, gm_prep makes them so
-// where the caller's are not).  The rows lie back to back there, and chunk c
+// (global_load_lds_dwordx4).  The rows lie back to back there, and chunk c
 // of row r is kept at chunk c ^ gm_swizzle(r), so that the 16-byte A-operand
 // reads of eight rows fall on distinct banks.
 //
-// Rows are 2 NK chunks apart: with NK a multiple of 4 all rows share a bank
-// group and three bits of the row number spread them, else two bits or one.
+// Rows are 2 NK chunks apart (NK is even): with NK a multiple of 4 all rows
+// share a bank group and three bits of the row number spread them, else two.
 template <int NK>
 __device__ __forceinline__ int gm_swizzle(int r) {
-    return NK % 4 == 0 ? (r & 7) : NK % 2 == 0 ? ((r >> 1) & 3) : ((r >> 2) & 1);
+    return NK % 4 == 0 ? (r & 7) : ((r >> 1) & 3);
 }
 
-// Waves per SIMD (workgroups per CU) the kernel is compiled for: the query
-// operand is 4 NK registers beside 16 accumulators and about 48 others.
-constexpr int gm_waves(int nk) { return nk <= 4 ? 6 : nk <= 8 ? 5 : nk <= 16 ? 4 : nk <= 24 ? 3 : 2; }
+// Waves per SIMD (workgroups per CU) the kernel is compiled for: a wave's 32 QB
+// queries take 4 NK QB registers beside 16 QB accumulators and about 60 others.
+constexpr int gm_waves(int nk, int qb) {
+    return 4 * nk * qb + 16 * qb + 60 <= 96    ? 5
+           : 4 * nk * qb + 16 * qb + 60 <= 128 ? 4
+           : 4 * nk * qb + 16 * qb + 60 <= 168 ? 3
+                                               : 2;
+}
 
 typedef float gm_f32x16 __attribute__((ext_vector_type(16)));
+typedef _Float16 gm_f16x8 __attribute__((ext_vector_type(8)));
 
-template <int NK, bool COS>
-__global__ __launch_bounds__(256, gm_waves(NK)) void knn_groupmin_kernel(GmScanArgs a) {
+template <int NK, int QB>
+__global__ __launch_bounds__(256, gm_waves(NK, QB)) void knn_groupmin_kernel(GmScanArgs a) {
     constexpr int DP = NK * 8;
     constexpr int CPR = DP / 4;           // 16-byte chunks per tile row
     constexpr int PF = (NK + 3) / 4;      // loads per wave: NK a tile, 64 chunks each
     __shared__ __attribute__((aligned(16))) float tileA[kGmRows * DP];
     __shared__ __attribute__((aligned(16))) float tileB[kGmRows * DP];
-    __shared__ __attribute__((aligned(16))) float tnA[kGmRows];
-    __shared__ __attribute__((aligned(16))) float tnB[kGmRows];
+    __shared__ __attribute__((aligned(16))) float tnA[2 * kGmRows];  // the rows' norms, then their scales
+    __shared__ __attribute__((aligned(16))) float tnB[2 * kGmRows];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = lane >> 5, jl = lane & 31;
     const float* __restrict__ X = a.x;
-    const float* __restrict__ BIAS = a.bias;
+    const float* __restrict__ NORM = tid < kGmRows ? a.bias : a.xinv;
     const int d = (int)a.d;
     const uint32_t row_bytes = 4u * (uint32_t)a.ldx;
     // rows past the index: their bias leaves them out, so their loads only
@@ -65,8 +75,7 @@ __global__ __launch_bounds__(256, gm_waves(NK)) void knn_groupmin_kernel(GmScanA
     const uint32_t last_bytes = (uint32_t)(a.nt - (int64_t)last_tile * kGmRows) * row_bytes;
 
     // The lane's chunks of a tile, as byte offsets.  Chunks past d repeat the
-    // row's first one: the operand is zero there, and a NaN or infinity in it
-    // is in the row anyway.
+    // row's first one: the query operand is zero there and the copy is finite.
     float pfn = 0.0f;
     uint32_t src[PF];
 #pragma unroll
@@ -78,9 +87,8 @@ __global__ __launch_bounds__(256, gm_waves(NK)) void knn_groupmin_kernel(GmScanA
         src[p] = (uint32_t)r * row_bytes + 16u * (uint32_t)c;
     }
     auto load_tile = [&](float* buf, int t) {
-        if (tid < kGmRows)
-            pfn = *(const __attribute__((address_space(1))) float*)(reinterpret_cast<const char*>(BIAS + (int64_t)t * kGmRows) +
-                                                                   4u * (uint32_t)tid);
+        if (tid < 2 * kGmRows)
+            pfn = *(const __attribute__((address_space(1))) float*)(NORM + ((int64_t)t * kGmRows + (tid & (kGmRows - 1))));
         const int tc = t < last_tile ? t : last_tile;
         const char* base = reinterpret_cast<const char*>(X) + (int64_t)tc * kGmRows * row_bytes;
         const uint32_t lim = (tc < last_tile ? kGmRows * row_bytes : last_bytes) - 16u;
@@ -93,7 +101,7 @@ __global__ __launch_bounds__(256, gm_waves(NK)) void knn_groupmin_kernel(GmScanA
     };
     auto publish = [&](float* tn) {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the tile's loads have landed
-        if (tid < kGmRows) tn[tid] = pfn;
+        if (tid < 2 * kGmRows) tn[tid] = pfn;
         __syncthreads();
     };
 
@@ -102,11 +110,11 @@ __global__ __launch_bounds__(256, gm_waves(NK)) void knn_groupmin_kernel(GmScanA
     int aoff[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) aoff[j] = jl * DP + 4 * (((2 * j) | h) ^ gm_swizzle<NK>(jl));
-    auto a_chunk = [&](const float* buf, int g) -> float4 {
-        return *reinterpret_cast<const float4*>(buf + aoff[g & 3] + 32 * (g >> 2));
+    auto a_chunk = [&](const float* buf, int g) -> gm_f16x8 {
+        return *reinterpret_cast<const gm_f16x8*>(buf + aoff[g & 3] + 32 * (g >> 2));
     };
 
-    const StreamSplit sp(a.nq, a.tiles * kGmRows, kGmQpb, kGmRows * kGmQuad, a.grid_wgs);
+    const StreamSplit sp(a.nq, a.tiles * kGmRows, kGmQpb * QB, kGmRows * kGmQuad, a.grid_wgs);
     const int64_t wg = xcd_grouped_wg(blockIdx.x, gridDim.x);
     const int64_t u_hi = ((wg + 1) * sp.P < sp.T) ? (wg + 1) * sp.P : sp.T;
     for (int64_t u = wg * sp.P; u < u_hi;) {
@@ -116,102 +124,127 @@ __global__ __launch_bounds__(256, gm_waves(NK)) void knn_groupmin_kernel(GmScanA
         u += quads;
         const int t0 = (int)quad0 * kGmQuad, t_end = (int)(quad0 + quads) * kGmQuad;
         load_tile(tileA, t0);
-        const int64_t q = qblock * kGmQpb + w * 32 + jl;
-        float4 qreg[NK];
-        {
-            const float* qp = a.q + q * DP + 4 * h;
+        // the wave's query blocks lie 128 queries apart
+        const int64_t q = qblock * (kGmQpb * QB) + w * 32 + jl;
+        gm_f16x8 qreg[QB][NK];  // of 16-column step g: high halves at 2 g, low halves at 2 g + 1
+        float qi[QB];
 #pragma unroll
-            for (int g = 0; g < NK; ++g) qreg[g] = gload4(qp + 8 * g);
+        for (int b = 0; b < QB; ++b) {
+            const float* qp = a.q + (q + b * kGmQpb) * DP + 4 * h;
+#pragma unroll
+            for (int g = 0; g < NK; ++g) qreg[b][g] = __builtin_bit_cast(gm_f16x8, gload4(qp + 8 * g));
+            qi[b] = a.qinv[q + b * kGmQpb < a.nq ? q + b * kGmQpb : 0];
         }
         float* __restrict__ out = a.gmin + (q * 2 + h) * a.ntp;
-        const bool qvalid = q < a.nq;
         for (int t = t0; t < t_end; t += kGmQuad) {
-            float m[kGmQuad];
+            float m[QB][kGmQuad];
 #pragma unroll
             for (int i = 0; i < kGmQuad; ++i) {
                 float* cur = (i & 1) ? tileB : tileA;
                 float* tn = (i & 1) ? tnB : tnA;
                 publish(tn);
                 if (i + 1 < kGmQuad || t + kGmQuad < t_end) load_tile((i & 1) ? tileA : tileB, t + i + 1);
-                gm_f32x16 acc;
+                gm_f32x16 acc[QB] = {};
+                gm_f16x8 hi = a_chunk(cur, 0), lo = a_chunk(cur, 1);
+#pragma unroll
+                for (int g = 0; g < NK; g += 2) {
+                    gm_f16x8 hn = hi, ln = lo;
+                    if (g + 2 < NK) {
+                        hn = a_chunk(cur, g + 2);
+                        ln = a_chunk(cur, g + 3);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int b = 0; b < QB; ++b)
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, qreg[b][g], acc[b], 0, 0, 0);
+#pragma unroll
+                    for (int b = 0; b < QB; ++b)
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, qreg[b][g + 1], acc[b], 0, 0, 0);
+#pragma unroll
+                    for (int b = 0; b < QB; ++b)
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, qreg[b][g], acc[b], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    hi = hn;
+                    lo = ln;
+                }
+                // rows left out have norm +inf; no value is NaN
+                float v[QB];
+#pragma unroll
+                for (int b = 0; b < QB; ++b) v[b] = __builtin_huge_valf();
 #pragma unroll
                 for (int g4 = 0; g4 < 4; ++g4) {
                     const float4 n4 = *reinterpret_cast<const float4*>(tn + 8 * g4 + 4 * h);
-                    acc[4 * g4 + 0] = COS ? 0.0f : n4.x;
-                    acc[4 * g4 + 1] = COS ? 0.0f : n4.y;
-                    acc[4 * g4 + 2] = COS ? 0.0f : n4.z;
-                    acc[4 * g4 + 3] = COS ? 0.0f : n4.w;
-                }
-                float4 av = a_chunk(cur, 0);
+                    const float4 s4 = *reinterpret_cast<const float4*>(tn + kGmRows + 8 * g4 + 4 * h);
 #pragma unroll
-                for (int g = 0; g < NK; ++g) {
-                    float4 an = av;
-                    if (g + 1 < NK) an = a_chunk(cur, g + 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.x, qreg[g].x, acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.y, qreg[g].y, acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.z, qreg[g].z, acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.w, qreg[g].w, acc, 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                    av = an;
-                }
-                if (COS) {
-#pragma unroll
-                    for (int g4 = 0; g4 < 4; ++g4) {
-                        const float4 s4 = *reinterpret_cast<const float4*>(tn + 8 * g4 + 4 * h);
-                        acc[4 * g4 + 0] *= s4.x;
-                        acc[4 * g4 + 1] *= s4.y;
-                        acc[4 * g4 + 2] *= s4.z;
-                        acc[4 * g4 + 3] *= s4.w;
+                    for (int b = 0; b < QB; ++b) {
+                        v[b] = fminf(v[b], __builtin_fmaf(acc[b][4 * g4 + 0] * s4.x, qi[b], n4.x));
+                        v[b] = fminf(v[b], __builtin_fmaf(acc[b][4 * g4 + 1] * s4.y, qi[b], n4.y));
+                        v[b] = fminf(v[b], __builtin_fmaf(acc[b][4 * g4 + 2] * s4.z, qi[b], n4.z));
+                        v[b] = fminf(v[b], __builtin_fmaf(acc[b][4 * g4 + 3] * s4.w, qi[b], n4.w));
                     }
                 }
-                // NaN (rows left out) is ignored by the minimum
-                float v = __builtin_huge_valf();
 #pragma unroll
-                for (int r = 0; r < 16; ++r) v = fminf(v, acc[r]);
-                // an empty statement that reads and returns v: without it the
-                // compiler sinks the minimum to the store and keeps all four
-                // tiles' accumulators (48 registers) until then
-                asm volatile("" : "+v"(v));
-                m[i] = v;
+                for (int b = 0; b < QB; ++b) {
+                    // an empty statement that reads and returns v: without it the
+                    // compiler sinks the minimum to the store and keeps all four
+                    // tiles' accumulators until then
+                    asm volatile("" : "+v"(v[b]));
+                    m[b][i] = v[b];
+                }
             }
-            if (qvalid) *reinterpret_cast<float4*>(out + t) = make_float4(m[0], m[1], m[2], m[3]);
+#pragma unroll
+            for (int b = 0; b < QB; ++b)
+                if (q + b * kGmQpb < a.nq)
+                    *reinterpret_cast<float4*>(out + b * (2 * kGmQpb) * a.ntp + t) =
+                        make_float4(m[b][0], m[b][1], m[b][2], m[b][3]);
         }
     }
 }
 
+template <int NK, int QB>
+void gm_launch_nk(GmScanArgs a, hipStream_t s) {
+    a.grid_wgs *= gm_waves(NK, QB);
+    const StreamSplit sp(a.nq, a.tiles * kGmRows, kGmQpb * QB, kGmRows * kGmQuad, a.grid_wgs);
+    hipLaunchKernelGGL((knn_groupmin_kernel<NK, QB>), dim3((unsigned)sp.G), dim3(256), 0, s, a);
+}
+
 // a.grid_wgs: the CU count; one resident round of workgroups is launched.
-template <bool COS>
-hipError_t gm_launch(GmScanArgs a, hipStream_t s) {
+hipError_t gm_launch(const GmScanArgs& a, hipStream_t s) {
     const int nk = gm_chunks(a.d);
-    a.grid_wgs *= gm_waves(nk);
-    const StreamSplit sp(a.nq, a.tiles * kGmRows, kGmQpb, kGmRows * kGmQuad, a.grid_wgs);
-    const dim3 grid((unsigned)sp.G);
-    switch (nk) {
+    if (gm_two_blocks(nk, a.nq, a.nt)) {
+        switch (nk) {
 #define MLRS_GM_CASE(N) \
-    case N: hipLaunchKernelGGL((knn_groupmin_kernel<N, COS>), grid, dim3(256), 0, s, a); break;
-        MLRS_GM_CASE(1)
+    case N: gm_launch_nk<N, 2>(a, s); break;
         MLRS_GM_CASE(2)
-        MLRS_GM_CASE(3)
         MLRS_GM_CASE(4)
-        MLRS_GM_CASE(5)
         MLRS_GM_CASE(6)
-        MLRS_GM_CASE(7)
         MLRS_GM_CASE(8)
-        MLRS_GM_CASE(9)
         MLRS_GM_CASE(10)
-        MLRS_GM_CASE(11)
         MLRS_GM_CASE(12)
-        MLRS_GM_CASE(13)
         MLRS_GM_CASE(14)
-        MLRS_GM_CASE(15)
+        MLRS_GM_CASE(16)
+#undef MLRS_GM_CASE
+        default: return hipErrorInvalidValue;
+        }
+    } else {
+        switch (nk) {
+#define MLRS_GM_CASE(N) \
+    case N: gm_launch_nk<N, 1>(a, s); break;
+        MLRS_GM_CASE(2)
+        MLRS_GM_CASE(4)
+        MLRS_GM_CASE(6)
+        MLRS_GM_CASE(8)
+        MLRS_GM_CASE(10)
+        MLRS_GM_CASE(12)
+        MLRS_GM_CASE(14)
         MLRS_GM_CASE(16)
         MLRS_GM_CASE(20)
         MLRS_GM_CASE(24)
         MLRS_GM_CASE(28)
         MLRS_GM_CASE(32)
 #undef MLRS_GM_CASE
-    default: return hipErrorInvalidValue;
+        default: return hipErrorInvalidValue;
+        }
     }
     return hipGetLastError();
 }

@@ -190,7 +190,6 @@ struct GmQuery {
     bool all_rows;
     double eps, eps_t;
     const float* bias;
-    int bias_nan;
     __device__ __forceinline__ GmQuery(const GmSelectArgs<TS>& a, int64_t q) {
         G = a.gmin + q * 2 * a.ntp;
         ntp = (int)a.ntp;
@@ -209,7 +208,6 @@ struct GmQuery {
             eps = a.eps_rel * ((double)qn + (double)__uint_as_float(a.stats->xmax_bits)) + a.eps_abs;
         }
         bias = a.bias;
-        bias_nan = a.bias_nan;
     }
     // row j of group f; rows left out by the scan are evaluated from their list
     __device__ __forceinline__ uint32_t row(int f, int j) const {
@@ -217,8 +215,7 @@ struct GmQuery {
         const uint32_t r = (uint32_t)(f - (half ? ntp : 0)) * kGmRows + (uint32_t)gm_group_row(half, j);
         bool on = r < nt;
         if (nforced) {
-            const float b = bias[r];
-            on = on && (bias_nan ? b == b : b < __builtin_huge_valf());
+            on = on && bias[r] < __builtin_huge_valf();
         }
         return on ? r : kSentinelIdx;
     }

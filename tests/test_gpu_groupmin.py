@@ -157,3 +157,17 @@ def test_pairwise_tile_edges(dtype, metric, nx, ny, d):
     got = prims.pairwise_distance(torch.from_numpy(x).to(DEV), torch.from_numpy(y).to(DEV), metric, sqrt=True)
     bits = np.int32 if dtype == np.float32 else np.int64
     assert np.array_equal(got.cpu().numpy().view(bits), want.view(bits))
+
+
+@pytest.mark.parametrize("d", [5, 16, 17, 100, 128])
+def test_two_query_blocks(d):
+    """Searches of 2^26 pairs and more, up to 128 columns: two query blocks per
+    workgroup, the last of them partly and wholly empty; rows of every scale,
+    down to where they share one."""
+    xt, xq = _rows(d, 9001, d, np.float32), _rows(d + 1, 7500 if d % 2 else 7700, d, np.float32)
+    rng = np.random.default_rng(d)
+    for x in (xt, xq):
+        rows = rng.choice(len(x), 2000, replace=False)
+        x[rows] *= np.exp2(rng.integers(-60, 12, 2000)).astype(np.float32)[:, None]
+    xt[17] = xt[9000]
+    _check(xq, xt, 7)
