@@ -518,19 +518,21 @@ static bool small_search(int64_t nq, int64_t nt, int64_t d) {
 }
 
 // Searches the low-d ALU kernel serves faster than the group-minimum search,
-// whose cost is about 0.335 ps per pair whatever k (d <= 8; 0.43 up to 16).  The
+// whose cost is about 0.335 ps per pair whatever k and d (most of it the minima's way
+// through memory).  The
 // ALU kernel needs thousands of queries to fill its lanes, pays for its list
 // merges, and its cost per pair grows with d and k; fitted to self-searches of
 // 30,000 and 100,000 rows (us, ALU against group minima): f32 d = 2, k = 2: 298
 // / 314 and 1373 / 3335; d = 3, k = 8: 538 / 344 and 1722 / 3329; d = 8, k = 8:
 // 833 / 338 and 3475 / 3391; f64 d = 2, k = 2: 360 / 321 and 1632 / 3313; d = 3,
-// k = 8: 709 / 354 and 2961 / 3347; d = 4, k = 8: 834 / 353 and 3649 / 3355.  500,000
+// k = 8: 709 / 354 and 2961 / 3347; d = 4, k = 8: 834 / 353 and 3649 / 3355; d = 16, k =
+// 8, f32: 1048 / 337 and 5522 / 3378.  500,000
 // rows, d = 3, k = 8, f32: 23 ms against 93.
 static bool lowd_faster(int64_t nq, int64_t nt, int64_t d, int64_t k, size_t elem) {
     if (nq < 4096 || k > 16) return false;
     const double pairs = (double)nq * (double)nt;
     const double ps = elem == 4 ? 0.04 + 0.027 * (double)d + 0.004 * (double)k : 0.02 + 0.06 * (double)d + 0.006 * (double)k;
-    return 150.0 + 35.0 * (double)k + ps * 1e-6 * pairs < (d <= 8 ? 0.335e-6 : 0.43e-6) * pairs;
+    return 150.0 + 35.0 * (double)k + ps * 1e-6 * pairs < 0.335e-6 * pairs;
 }
 
 // Process-wide kernel-family override (mlrs_force_path); a family that does
@@ -636,6 +638,13 @@ int32_t knn_gram32(const float* xq, int64_t nq, const float* xt, int64_t nt, int
     a.out_val = out_v;
     a.out_idx = out_i;
     if (res_chunks) {
+        // The resident search's screen is made of f16 halves: with dp the
+        // columns rounded up to 32, the contraction's 3 dp additions, the
+        // halves' own error and the arm stay below (3.1 dp + d + 40) u N, as
+        // bounded in knn_groupmin (the rows' common scale loses a share of the
+        // largest row's norm, which N holds); dp u more is slack.
+        a.eps_rel = (4.1 * (double)(d <= 32 ? 32 : 64) + (double)d + 40.0) * u;
+        a.eps_abs = (double)(d + 16) * std::ldexp(1.0, -120);
         {
             KernelTimer timer(s, "knn_k1_resident_f32_kernel");
             e = launch_gram_f32_k1_resident(a, arm, cus, res_qsq ? qsq : nullptr, s);

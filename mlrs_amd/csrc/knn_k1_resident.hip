@@ -6,13 +6,16 @@
 // nearest.rs:1058-1343) when the index is small: its rows are cut into
 // chunks that fit one workgroup's LDS, and each workgroup loads one chunk
 // once and keeps it for the whole launch.
-//  * One workgroup of 12 waves per CU (three per SIMD).  Every wave works on
+//  * One workgroup of 16 waves per CU (four per SIMD).  Every wave works on
 //    its own blocks of 32 queries against the resident chunk: the query block
-//    is the MFMA B operand in VGPRs (pre-scaled by -2), the chunk's 32-row
-//    tiles the A operand read from LDS, as in the fused kernel's narrow shape
-//    (v_mfma_f32_32x32x2f32; the accumulator starts at ||x_t||^2).  Nothing
-//    is written to LDS in the loop, so the waves never wait for each other:
-//    no tile barrier, no tile loads.
+//    is the MFMA B operand in VGPRs, the chunk's 32-row tiles the A operand
+//    read from LDS.  Both are held as two f16 halves per element (22 bits),
+//    scaled by powers of two -- the rows by one for the whole index, a query
+//    by its own -- and x q = xh qh + xh ql + xl qh: three
+//    v_mfma_f32_32x32x16_f16 per 16 columns, 96 cycles where the f32 matrix
+//    cores took 512.  The screen value is that contraction, unscaled, plus
+//    ||x_t||^2.  Nothing is written to LDS in the loop, so the waves never wait
+//    for each other: no tile barrier, no tile loads.
 //  * Per tile, the k = 1 steps of the fused kernel: the threshold tightened
 //    with the tile's smallest expansion value + 2 eps, the screen (the sign
 //    of threshold - value where the wave's screen sums cannot overflow, the
@@ -22,12 +25,15 @@
 //    emptied before the tile's rows join it.
 //  * The queued rows are evaluated exactly, in the reference arm's operation
 //    order, with the query row from global memory and the index row from the
-//    resident chunk; the best (value, index) per query is kept with a 64-bit
+//    index in global memory; the best (value, index) per query is kept with a 64-bit
 //    LDS atomicMin, and written as the (chunk, query) list.
 //  * knn_merge1_chunks_f32_kernel takes each query's best over the chunks
 //    (value, then index) and applies the output transform.
-// The results are the fused kernel's, bit for bit: the same screen, error
-// bound and exact rescoring.
+// The results are the fused kernel's, bit for bit: a screen with a bounded
+// error and the same exact rescoring.
+// Bound by the vector instructions of a tile (the unscaling, the minimum and the
+// screen, about 70) beside its 24 MFMAs per 64 columns.  5M x 1024, d = 64: 5.54 ms
+// with f32 MFMA (74% of that peak), 2.63 ms.
 #include "knn_common.hpp"
 #include "knn_kernels.hpp"
 
@@ -41,6 +47,15 @@ constexpr int kResQpw = 32;               // queries per wave block
 constexpr int kResBn = 32;                // rows per tile
 constexpr int kResQcap = 48;              // queued rows per query (flushed above 16)
 constexpr int kResLdsBytes = 163840;      // gfx950's LDS per workgroup
+
+typedef _Float16 res_f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 res_f16x4 __attribute__((ext_vector_type(4)));
+
+// The exponent that takes a vector of squared norm s to a norm of at most
+// 2^15, so that no element leaves f16's range; norms below 2^-50 share one.
+__device__ __forceinline__ int res_exponent(float s) {
+    return 15 - ((__builtin_amdgcn_frexp_expf(fmaxf(s, 0x1p-100f)) + 1) >> 1);
+}
 
 struct ResWave {
     float thr[kResQpw];
@@ -95,11 +110,23 @@ __global__ __launch_bounds__(kResThreads) void knn_k1_resident_f32_kernel(GramAr
     const int64_t row0 = (int64_t)cidx * chunk_rows;
     const int rows = (int)((nt - row0) < chunk_rows ? (nt - row0) : chunk_rows);
     const int tiles = (rows + kResBn - 1) / kResBn;
+    const int xex = res_exponent(a.stats->xsq_max);
     for (int e = tid; e < tiles * kResBn * (DP / 4); e += kResThreads) {
         const int r = e / (DP / 4), c4 = e % (DP / 4);
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (r < rows && 4 * c4 < d) v = *reinterpret_cast<const float4*>(X + (row0 + r) * d + 4 * c4);
-        *reinterpret_cast<float4*>(&chunk[r * STRIDE + 4 * c4]) = v;
+        const float f[4] = {v.x, v.y, v.z, v.w};
+        res_f16x4 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float f_ = __builtin_ldexpf(f[i], xex);
+            hi[i] = (_Float16)f_;
+            lo[i] = (_Float16)(f_ - (float)hi[i]);
+        }
+        // 16 columns: the high halves of the first and the last eight, then the low halves
+        char* o = reinterpret_cast<char*>(&chunk[r * STRIDE]) + 64 * (c4 >> 2) + 8 * (c4 & 3);
+        *reinterpret_cast<res_f16x4*>(o) = hi;
+        *reinterpret_cast<res_f16x4*>(o + 32) = lo;
     }
     for (int r = tid; r < tiles * kResBn; r += kResThreads) cnorm[r] = r < rows ? XSQ[row0 + r] : inf;
     __syncthreads();  // the chunk is read-only from here on
@@ -114,32 +141,43 @@ __global__ __launch_bounds__(kResThreads) void knn_k1_resident_f32_kernel(GramAr
         const int64_t qrow = qvalid ? qmine : nq - 1;
 
         // ---- per-query state (lanes 0..31 of the wave) ----
-        float4 qreg[NG];
+        float4 qf[NG];  // step g / 2's columns 8 h to 8 h + 7
         {
             const float* qp = Q + qrow * d;
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
-                const int64_t c = (int64_t)8 * g + 4 * h;
+                const int64_t c = (int64_t)16 * (g >> 1) + 8 * h + 4 * (g & 1);
                 const float4 v = *reinterpret_cast<const float4*>(qp + (c < d ? c : d - 4));
-                qreg[g] = (qvalid && c < d) ? make_float4(-2.0f * v.x, -2.0f * v.y, -2.0f * v.z, -2.0f * v.w)
-                                            : make_float4(0.f, 0.f, 0.f, 0.f);
+                qf[g] = (qvalid && c < d) ? v : make_float4(0.f, 0.f, 0.f, 0.f);
             }
         }
         float qsq_l;
         if (qsq_out) {
-            // ||q||^2 from the operand: qreg = -2 q exactly, so the sum of its
-            // squares is 4 ||q||^2 in some order (within the screen bound's
-            // allowance for the norm's rounding, as a sum in any order is);
-            // chunk 0 keeps it for the merge's k-means rule
+            // ||q||^2 from the operand, in some order (within the screen
+            // bound's allowance for the norm's rounding, as a sum in any order
+            // is); chunk 0 keeps it for the merge's k-means rule
             float s2 = 0.0f;
 #pragma unroll
             for (int g = 0; g < NG; ++g)
-                s2 = s2 + qreg[g].x * qreg[g].x + qreg[g].y * qreg[g].y + qreg[g].z * qreg[g].z +
-                     qreg[g].w * qreg[g].w;
-            qsq_l = (s2 + shfl_xor_f(s2, 32)) * 0.25f;
+                s2 = s2 + qf[g].x * qf[g].x + qf[g].y * qf[g].y + qf[g].z * qf[g].z + qf[g].w * qf[g].w;
+            qsq_l = s2 + shfl_xor_f(s2, 32);
             if (cidx == 0 && h == 0 && qvalid) qsq_out[qmine] = qsq_l;
         } else {
             qsq_l = QSQ[qrow];
+        }
+        const int qex = res_exponent(qsq_l);
+        const float unscale = __builtin_ldexpf(-2.0f, -qex - xex);
+        res_f16x8 qhi[NG / 2], qlo16[NG / 2];
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const float f[4] = {qf[g].x, qf[g].y, qf[g].z, qf[g].w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float f_ = __builtin_ldexpf(f[i], qex);
+                const _Float16 t_ = (_Float16)f_;
+                qhi[g >> 1][4 * (g & 1) + i] = t_;
+                qlo16[g >> 1][4 * (g & 1) + i] = (_Float16)(f_ - (float)t_);
+            }
         }
         if (lane < kResQpw) {
             const float qsq = qvalid ? qsq_l : 0.0f;
@@ -186,7 +224,7 @@ __global__ __launch_bounds__(kResThreads) void knn_k1_resident_f32_kernel(GramAr
                         if (L.off[j_ + m_] <= e_) j_ += m_;
                     const uint32_t t_ = QI[j_ * kResQcap + (e_ - L.off[j_])];
                     const float* qp = Q + (qwave + j_) * d;
-                    const float* yp = &chunk[(int)t_ * STRIDE];
+                    const float* yp = X + (row0 + (int64_t)t_) * d;
                     float acc = 0.0f;
                     for (int c4 = 0; c4 < (int)(d >> 2); ++c4) {
                         const float4 qv = *reinterpret_cast<const float4*>(qp + 4 * c4);
@@ -222,33 +260,36 @@ __global__ __launch_bounds__(kResThreads) void knn_k1_resident_f32_kernel(GramAr
 
         for (int t = 0; t < tiles; ++t) {
             // A operands from the resident chunk: lane (h, jl) reads row jl's
-            // chunk 2g + h; the next group's read issued before this group's
-            // four MFMAs
-            f32x16_t acc;
+            // chunks 4 g + h (high halves) and 4 g + 2 + h (low); the next
+            // step's read issued before this step's three MFMAs
+            f32x16_t acc = {};
+            const float* arow = &chunk[(t * kResBn + jl) * STRIDE + 4 * h];
+            res_f16x8 hi = *reinterpret_cast<const res_f16x8*>(arow), lo = *reinterpret_cast<const res_f16x8*>(arow + 8);
+#pragma unroll
+            for (int g = 0; g < NG / 2; ++g) {
+                res_f16x8 hn = hi, ln = lo;
+                if (g + 1 < NG / 2) {
+                    hn = *reinterpret_cast<const res_f16x8*>(arow + 16 * (g + 1));
+                    ln = *reinterpret_cast<const res_f16x8*>(arow + 16 * (g + 1) + 8);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, qhi[g], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, qlo16[g], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(hi, qhi[g], acc, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                hi = hn;
+                lo = ln;
+            }
             {
                 const float* nrm = &cnorm[t * kResBn];
 #pragma unroll
                 for (int g4 = 0; g4 < 4; ++g4) {
                     const float4 n4 = *reinterpret_cast<const float4*>(nrm + 8 * g4 + 4 * h);
-                    acc[4 * g4 + 0] = n4.x;
-                    acc[4 * g4 + 1] = n4.y;
-                    acc[4 * g4 + 2] = n4.z;
-                    acc[4 * g4 + 3] = n4.w;
+                    acc[4 * g4 + 0] = __builtin_fmaf(acc[4 * g4 + 0], unscale, n4.x);
+                    acc[4 * g4 + 1] = __builtin_fmaf(acc[4 * g4 + 1], unscale, n4.y);
+                    acc[4 * g4 + 2] = __builtin_fmaf(acc[4 * g4 + 2], unscale, n4.z);
+                    acc[4 * g4 + 3] = __builtin_fmaf(acc[4 * g4 + 3], unscale, n4.w);
                 }
-            }
-            const float* arow = &chunk[(t * kResBn + jl) * STRIDE + 4 * h];
-            float4 av = *reinterpret_cast<const float4*>(arow);
-#pragma unroll
-            for (int g = 0; g < NG; ++g) {
-                float4 an = av;
-                if (g + 1 < NG) an = *reinterpret_cast<const float4*>(arow + 8 * (g + 1));
-                __builtin_amdgcn_sched_barrier(0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.x, qreg[g].x, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.y, qreg[g].y, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.z, qreg[g].z, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.w, qreg[g].w, acc, 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                av = an;
             }
 
             // ---- tighten with this tile's smallest expansion value ----

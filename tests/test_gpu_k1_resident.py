@@ -141,3 +141,17 @@ def test_knn_k1(d):
     np.testing.assert_array_equal(gi.cpu().numpy(), wi.astype(np.int64))
     np.testing.assert_array_equal(gd.cpu().numpy(), wd)
     assert (gi.cpu().numpy()[:5, 0] == 50).all()
+
+
+@pytest.mark.parametrize("d", [4, 16, 20, 32, 64])
+def test_assign_rows_of_every_scale(d):
+    """The screen's halves share one scale for all centres and take a power of
+    two per point: centres and points of every magnitude, down to where f16
+    resolves nothing of a centre and the points share a scale."""
+    rng = np.random.default_rng(70 + d)
+    x, c = _blobs(60 + d, 5003, 777, d)
+    x *= np.exp2(rng.integers(-58, 20, len(x))).astype(np.float32)[:, None]
+    c *= np.exp2(rng.integers(-58, 20, len(c))).astype(np.float32)[:, None]
+    _, _, kern = _assign(x, c)
+    assert kern == "knn_k1_resident_f32_kernel"
+    _assign(x * np.float32(2.0 ** -30), c * np.float32(2.0 ** -40))
