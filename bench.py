@@ -3,8 +3,8 @@
 Default workload (c2): 1,000,000 x 128 index, 10,000 x 128 queries from a
 100-component Gaussian mixture, f32, Euclidean, k=32 -- the configuration the
 headline metric is quoted on.  One step = one full kneighbors search of all
-queries against the index (row norms, the fused Gram-MFMA + exact top-k kernel
-and the strip merge), inputs already resident in HBM.
+queries against the index (row norms, the group-minimum scan on the matrix cores and
+the exact selection), inputs already resident in HBM.
 
 Prints ONE JSON line.  `roofline` is for the dominant kernel, timed with HIP
 events recorded by the engine around that kernel's launch on the stream it runs
@@ -45,7 +45,9 @@ PEAKS = {  # MI355X published dense peaks (TFLOP/s, GB/s)
     # packed FP32 ops, so its own ceiling is the non-packed rate, 78.6 TFLOP/s
     # (FP64's figure, one FMA per lane per cycle); `bench.py --probe-peak`
     # measures what register-only FMA/MFMA chains reach on the card.
-    "mfma_f32": 157.3, "mfma_f64": 78.6, "valu_f32": 157.3, "valu_f64": 78.6, "hbm": 8000.0,
+    "mfma_f32": 157.3, "mfma_f64": 78.6,
+    # screens of two f16 halves per element: three f16 products per multiply-add
+    "mfma_f16_halves": 2500.0 / 3.0, "valu_f32": 157.3, "valu_f64": 78.6, "hbm": 8000.0,
 }
 VALU_F32_NONPACKED = 78.6
 METRIC = "kNN dist-evals/s, 1M×10k d=128 k=32 f32; % of MFMA/HBM roofline"
@@ -268,7 +270,9 @@ def main():
         bound, peak, unit = "valu", PEAKS["valu_f64" if f64 else "valu_f32"], "TFLOP/s"
     elif kname.startswith("knn_gram_f64"):
         bound, peak, unit = "mfma", PEAKS["mfma_f64"], "TFLOP/s"
-    elif kname.startswith("knn_gram_f32") or kname.startswith("knn_k1_resident_f32"):
+    elif kname.startswith("knn_groupmin_kernel") or kname.startswith("knn_k1_resident_f32"):
+        bound, peak, unit = "mfma", PEAKS["mfma_f16_halves"], "TFLOP/s"
+    elif kname.startswith("knn_gram_f32"):
         bound, peak, unit = "mfma", PEAKS["mfma_f32"], "TFLOP/s"
     else:
         # the low-d ALU kernel and the exact tiles of small searches: vector
@@ -283,7 +287,9 @@ def main():
     tfile = os.path.join(ROOT, "profiles", "traffic_%s%s%s.json" % ("radius_" if radius is not None else "",
                                                                      args.config, "_" + args.dtype if retyped else ""))
     if os.path.exists(tfile):
-        traffic = json.load(open(tfile)).get("hbm_bytes_per_launch")
+        measured = json.load(open(tfile))
+        if measured.get("kernel", kname) == kname:  # of the kernel that ran
+            traffic = measured.get("hbm_bytes_per_launch")
 
     cpu = None
     if not args.no_cpu:
@@ -381,7 +387,8 @@ def main():
                      "kernel_launches_per_step": launches.value / args.steps, "kernel_ms_per_step": kern_ms_step,
                      "frac_nonpacked": (achieved / VALU_F32_NONPACKED
                                         if bound == "valu" and not f64 and achieved is not None else None),
-                     "basis": {"mfma": "dense MFMA peak, 2*d flops per distance evaluation",
+                     "basis": {"mfma": "dense MFMA peak (screens of f16 halves: a third of the f16 peak), 2*d flops per "
+                                       "distance evaluation",
                                "valu": ("published vector FP64 peak 78.6 TFLOP/s; 2*d flops per distance "
                                         "evaluation" if f64 else
                                         "published vector FP32 peak 157.3 TFLOP/s, which counts packed FP32 "
