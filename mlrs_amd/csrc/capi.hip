@@ -519,9 +519,8 @@ static bool small_search(int64_t nq, int64_t nt, int64_t d) {
 
 // Searches the low-d ALU kernel serves faster than the group-minimum search,
 // whose cost is about 0.335 ps per pair whatever k and d (most of it the minima's way
-// through memory).  The
-// ALU kernel needs thousands of queries to fill its lanes, pays for its list
-// merges, and its cost per pair grows with d and k; fitted to self-searches of
+// through memory).  The ALU kernel needs thousands of queries to fill its lanes,
+// pays for its list merges, and its cost per pair grows with d and k; fitted to self-searches of
 // 30,000 and 100,000 rows (us, ALU against group minima): f32 d = 2, k = 2: 298
 // / 314 and 1373 / 3335; d = 3, k = 8: 538 / 344 and 1722 / 3329; d = 8, k = 8:
 // 833 / 338 and 3475 / 3391; f64 d = 2, k = 2: 360 / 321 and 1632 / 3313; d = 3,
@@ -568,17 +567,9 @@ int32_t knn_gram32(const float* xq, int64_t nq, const float* xt, int64_t nt, int
     const int res_chunks = gram_f32_k1_resident_chunks(nq, nt, d, k, arm, vec4);
     // per-(segment slot, query) lists: the kernel's top-k state, merged at the end
     size_t parts = (size_t)std::max<int64_t>(nslots, res_chunks) * nq * gram_list_cap(k);
-    size_t qvals = (k > 1) ? gram_f32_qval_elems(grid_wgs, k)
-                 : res_chunks ? (gram_f32_k1_resident_queue_bytes(cus) + sizeof(float) - 1) / sizeof(float) : 0;
-    size_t summs = (k > 1) ? (size_t)nslots * nq : 0;
+    size_t qvals = res_chunks ? (gram_f32_k1_resident_queue_bytes(cus) + sizeof(float) - 1) / sizeof(float) : 0;
     size_t bytes = fixed + aligned_bytes(parts * sizeof(float)) + aligned_bytes(parts * sizeof(uint32_t)) +
-                   aligned_bytes(qvals * sizeof(float)) + aligned_bytes(summs * sizeof(float4)) +
-                   aligned_bytes(sizeof(unsigned int) * nq);
-    // the seed's screen values on the matrix cores, where served and where
-    // the workspace allows (otherwise the exact seed, which needs none)
-    size_t seed_bytes = gram_f32_seed_screen_bytes(nq, nt, d, k, arm, vec4);
-    if (seed_bytes && bytes + aligned_bytes(seed_bytes) > workspace_limit()) seed_bytes = 0;
-    if (seed_bytes) bytes += aligned_bytes(seed_bytes);
+                   aligned_bytes(qvals * sizeof(float)) + aligned_bytes(sizeof(unsigned int) * nq);
     rc = workspace(bytes, s, &ws, &cus);
     if (rc) return rc;
     Carver cv(ws);
@@ -632,9 +623,7 @@ int32_t knn_gram32(const float* xq, int64_t nq, const float* xt, int64_t nt, int
     a.part_val = cv.take<float>(parts);
     a.part_idx = cv.take<uint32_t>(parts);
     if (qvals) a.qval = cv.take<float>(qvals);
-    if (summs) a.summ = cv.take<float4>(summs);
-    if (nslots > 1 || k > 1) a.shared_r = cv.take<unsigned int>(nq);
-    void* seed_buf = seed_bytes ? static_cast<void*>(cv.take<char>(seed_bytes)) : nullptr;
+    if (nslots > 1) a.shared_r = cv.take<unsigned int>(nq);
     a.out_val = out_v;
     a.out_idx = out_i;
     if (res_chunks) {
@@ -653,12 +642,12 @@ int32_t knn_gram32(const float* xq, int64_t nq, const float* xt, int64_t nt, int
         if (e != hipSuccess) return hip_err(e, "knn_k1_resident_f32");
         return ok();
     }
-    e = launch_gram_f32_prep(a, arm, s, seed_buf);
+    e = launch_gram_f32_prep(a, s);
     if (e == hipSuccess) {
         KernelTimer timer(s, "knn_gram_f32_kernel");
         e = launch_gram_f32(a, arm, s);
     }
-    if (e == hipSuccess) e = launch_gram_f32_merge(a, arm, s);
+    if (e == hipSuccess) e = launch_gram_f32_merge(a, s);
     if (e != hipSuccess) return hip_err(e, "knn_gram_f32");
     return ok();
 }
@@ -677,16 +666,8 @@ int32_t knn_gram64(const double* xq, int64_t nq, const double* xt, int64_t nt, i
     gram_f64_split(nq, nt, cus, &grid_wgs, &nslots);
     size_t parts = (size_t)nslots * nq * gram_list_cap(k);
     size_t qvals = gram_f64_qval_elems(grid_wgs);
-    const bool ranked = mode == EMIT_ROOT_RANKED;
     size_t bytes = fixed + aligned_bytes(parts * sizeof(double)) + aligned_bytes(parts * sizeof(uint32_t)) +
-                   aligned_bytes(qvals * sizeof(double)) + aligned_bytes(sizeof(unsigned long long) * nq) +
-                   (ranked ? aligned_bytes(sizeof(uint32_t) * nq) : 0);
-    // the seed's screen values on the matrix cores where the workspace allows
-    const bool vec2 = (d % 2 == 0) && ((reinterpret_cast<uintptr_t>(xq) & 15) == 0) &&
-                      ((reinterpret_cast<uintptr_t>(xt) & 15) == 0);
-    size_t seed_bytes = gram_f64_seed_screen_bytes(nq, nt, d, k, vec2);
-    if (seed_bytes && bytes + aligned_bytes(seed_bytes) > workspace_limit()) seed_bytes = 0;
-    if (seed_bytes) bytes += aligned_bytes(seed_bytes);
+                   aligned_bytes(qvals * sizeof(double)) + aligned_bytes(sizeof(unsigned long long) * nq);
     rc = workspace(bytes, s, &ws, &cus);
     if (rc) return rc;
     Carver cv(ws);
@@ -735,17 +716,14 @@ int32_t knn_gram64(const double* xq, int64_t nq, const double* xt, int64_t nt, i
     a.part_idx = cv.take<uint32_t>(parts);
     a.qval = cv.take<double>(qvals);
     a.shared_r = cv.take<unsigned long long>(nq);
-    a.root_flag = ranked ? cv.take<unsigned int>(nq) : nullptr;
-    void* seed_buf = seed_bytes ? static_cast<void*>(cv.take<char>(seed_bytes)) : nullptr;
     a.out_val = out_v;
     a.out_idx = out_i;
-    e = launch_gram_f64_prep(a, arm, s, seed_buf);
+    e = launch_gram_f64_prep(a, s);
     if (e == hipSuccess) {
         KernelTimer timer(s, "knn_gram_f64_kernel");
         e = launch_gram_f64(a, arm, s);
     }
-    if (e == hipSuccess) e = launch_gram_f64_merge(a, arm, s);
-    if (e == hipSuccess && ranked) e = launch_gram_f64_root_fill(a, arm, s);
+    if (e == hipSuccess) e = launch_gram_f64_merge(a, s);
     if (e != hipSuccess) return hip_err(e, "knn_gram_f64");
     return ok();
 }

@@ -5,6 +5,10 @@
 // distance_direct -> top_k fallback (crates/mlrs-algos/src/neighbors/
 // nearest.rs:1058-1343) for f32, d <= 256, k <= 128, Euclidean and cosine.
 //
+// Launched for the k-means assignment only (k = 1, ARM_EUCLID_MULADD), where the
+// centres do not fit knn_k1_resident.hip; the searches of k > 1 and of the
+// other arms that the text below also describes are knn_groupmin's.
+//
 // Two register shapes (GramShape below): d <= 128, 4 waves x 32 queries =
 // 128 queries per workgroup on v_mfma_f32_32x32x2f32; 128 < d <= 256, 4 waves
 // x 16 queries = 64 per workgroup on v_mfma_f32_16x16x4f32.  Either walks one
@@ -104,7 +108,6 @@ struct GramShape {
 };
 constexpr int kQpbNarrow = GramShape<false>::qpb;
 constexpr int kQpbWide = GramShape<true>::qpb;
-constexpr int kQvalPerWave = 32 * 128;            // pairs a wave may queue (any shape), k > 1
 // Per wave in a.qval: the kernel's QPW x QCAP screen values, then as many
 // index-row numbers, both [queue position][query] (gram_f32_qval_elems sizes
 // the buffer for the launch's list length).
@@ -1173,199 +1176,8 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
     }
 }
 
-// Initial per-query bound: the k-th smallest exact value over an evenly
-// spaced sample of index rows (seed_kth_block).  Any k distinct rows bound the
-// final k-th value from above, so the screen starts tight instead of at +inf.
-// SB: 64-entry blocks of the running sample list (k <= 64 SB).
-template <int ARM, int SB>
-__global__ __launch_bounds__(256) void knn_seed_f32_kernel(GramArgs32 a, int64_t nsamp) {
-    const float* qop = (ARM == ARM_COS_FOLD) ? a.qsq : a.qinv;
-    const float* yop = (ARM == ARM_COS_FOLD) ? a.xsq : a.xinv;
-    seed_kth_block<float, ARM, unsigned int, SB>(a.q, a.x, a.nq, a.nt, a.d, a.k, nsamp, qop, yop, a.shared_r);
-}
-
-// Merge the per-segment lists of one query per wave and emit the output
-// transform (the strip merge of select_k_onepass_indexed,
-// crates/mlrs-kernels/src/topk.rs:612-758, here over sorted lists).  Every
-// list entry's value lies within eps of its pair's exact value (exact-mode
-// entries equal it), and the segments hold disjoint index rows.  So with V
-// the k-th smallest value over all lists, k distinct pairs are exactly <=
-// V + eps, and a pair can be among the k best only if its value is
-// <= V + 2 eps: exactly those pairs are evaluated in the reference arm's
-// operation order and ranked by (exact value, index), NaN never admitted.
-template <int ARM, bool VEC4>
-__global__ __launch_bounds__(256) void knn_merge_f32_kernel(GramArgs32 a) {
-    __shared__ uint32_t cand[4][128];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    const int64_t qg = (int64_t)blockIdx.x * 4 + wv;
-    if (qg >= a.nq) return;
-    const int k = a.k;
-    const int K2 = gram_list_cap(k);
-    const int64_t d = a.d;
-    const float inf = __builtin_huge_valf();
-    const StreamSplit sp(a.nq, a.nt, a.qpb, kBn, a.grid_wgs);
-    const int64_t nsl = sp.slots_of(qg / a.qpb);
-    // the k-th smallest value over the union of the lists
-    float uv = inf;
-    uint32_t ui = kSentinelIdx;
-    for (int64_t s = 0; s < nsl; ++s) {
-        float v = inf;
-        uint32_t ix = kSentinelIdx;
-        if (lane < K2) {
-            const int64_t o = (s * a.nq + qg) * K2 + lane;
-            v = a.part_val[o];
-            ix = a.part_idx[o];
-        }
-        wave_merge64<float>(uv, ui, v, ix, lane);
-    }
-    const float qsq = a.qsq[qg];
-    const float eps = (ARM == ARM_COS_FOLD || ARM == ARM_COS_HOST)
-                          ? (float)a.eps_abs
-                          : (float)(a.eps_rel * ((double)qsq + (double)a.stats->xsq_max) + a.eps_abs);
-    double W = (double)bcast_f(uv, k - 1) + 2.0 * (double)eps;
-    W += __builtin_fabs(W) * 0x1p-40;
-    // exact evaluation of the window's pairs, compacted 64 at a time
-    float lv = inf;
-    uint32_t li = kSentinelIdx;
-    uint32_t nc = 0;
-    auto evaluate = [&](uint32_t count) {
-        float e = inf;
-        uint32_t t = kSentinelIdx;
-        if ((uint32_t)lane < count) {
-            t = cand[wv][lane];
-            e = exact_f32<ARM, VEC4, 8>(a.q + qg * d, a.x + (int64_t)t * d, d, query_operand<ARM>(a, qg),
-                                        row_operand<ARM>(a, t));
-            if (e != e) {
-                e = inf;
-                t = kSentinelIdx;
-            }
-        }
-        wave_sort64<float>(e, t, lane);
-        wave_merge64<float>(lv, li, e, t, lane);
-    };
-    for (int64_t s = 0; s < nsl; ++s) {
-        bool in = false;
-        uint32_t ix = kSentinelIdx;
-        if (lane < K2) {
-            const int64_t o = (s * a.nq + qg) * K2 + lane;
-            ix = a.part_idx[o];
-            in = (ix != kSentinelIdx) && !((double)a.part_val[o] > W);
-        }
-        const uint64_t bal = __builtin_amdgcn_ballot_w64(in);
-        const uint32_t pre = (uint32_t)__builtin_popcountll(bal & ((1ull << lane) - 1ull));
-        if (in) cand[wv][nc + pre] = ix;
-        nc += (uint32_t)__builtin_popcountll(bal);
-        if (nc >= 64) {
-            evaluate(64);
-            const uint32_t rest = nc - 64;
-            const uint32_t mv = ((uint32_t)lane < rest) ? cand[wv][64 + lane] : 0u;
-            if ((uint32_t)lane < rest) cand[wv][lane] = mv;
-            nc = rest;
-        }
-    }
-    if (nc > 0) evaluate(nc);
-    if (lane < k) emit_pair(a.mode, a.q, a.x, a.qsq, a.xsq, a.d, k, qg, lane, lv, li, a.out_val, a.out_idx);
-}
-
-// 64 < k <= 128: the same merge over lists of up to three 64-entry blocks
-// (k + 32 entries).  The union and the result are kept as two-block lists
-// (the k smallest fit in 128 entries), merged block by block on 64-bit
-// (value bits, index) keys.
-template <int ARM, bool VEC4>
-__global__ __launch_bounds__(256) void knn_merge_blocks_f32_kernel(GramArgs32 a) {
-    constexpr int SLB = 3;  // blocks of a segment list
-    constexpr int UB = 2;   // blocks of the union and of the result
-    __shared__ uint32_t cand[4][128];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    const int64_t qg = (int64_t)blockIdx.x * 4 + wv;
-    if (qg >= a.nq) return;
-    const int k = a.k;
-    const int K2 = gram_list_cap(k);
-    const int64_t d = a.d;
-    const StreamSplit sp(a.nq, a.nt, a.qpb, kBn, a.grid_wgs);
-    const int64_t nsl = sp.slots_of(qg / a.qpb);
-    // the k-th smallest value over the union of the lists
-    unsigned long long u[UB];
-#pragma unroll
-    for (int r = 0; r < UB; ++r) u[r] = kKeyEmpty;
-    for (int64_t s = 0; s < nsl; ++s) {
-#pragma unroll
-        for (int r = 0; r < SLB; ++r) {
-            if (64 * r >= K2) break;
-            const int p = 64 * r + lane;
-            unsigned long long key = kKeyEmpty;
-            if (p < K2) {
-                const int64_t o = (s * a.nq + qg) * K2 + p;
-                key = pair_key(a.part_val[o], a.part_idx[o]);
-            }
-            (void)wave_merge_blocks_key_drop<UB>(u, key, lane);
-        }
-    }
-    const float qsq = a.qsq[qg];
-    const float eps = (ARM == ARM_COS_FOLD || ARM == ARM_COS_HOST)
-                          ? (float)a.eps_abs
-                          : (float)(a.eps_rel * ((double)qsq + (double)a.stats->xsq_max) + a.eps_abs);
-    double W = (double)f32_from_order_bits(list_hi_at<UB>(u, k - 1)) + 2.0 * (double)eps;
-    W += __builtin_fabs(W) * 0x1p-40;
-    // exact evaluation of the window's pairs, compacted 64 at a time
-    unsigned long long res[UB];
-#pragma unroll
-    for (int r = 0; r < UB; ++r) res[r] = kKeyEmpty;
-    uint32_t nc = 0;
-    auto evaluate = [&](uint32_t count) {
-        float e = __builtin_huge_valf();
-        uint32_t t = kSentinelIdx;
-        if ((uint32_t)lane < count) {
-            t = cand[wv][lane];
-            e = exact_f32<ARM, VEC4, 8>(a.q + qg * d, a.x + (int64_t)t * d, d, query_operand<ARM>(a, qg),
-                                        row_operand<ARM>(a, t));
-            if (e != e) {
-                e = __builtin_huge_valf();
-                t = kSentinelIdx;
-            }
-        }
-        unsigned long long ek = pair_key(e, t);
-        wave_sort64_key(ek, lane);
-        (void)wave_merge_blocks_key_drop<UB>(res, ek, lane);
-    };
-    for (int64_t s = 0; s < nsl; ++s) {
-        for (int r = 0; r < SLB; ++r) {
-            if (64 * r >= K2) break;
-            const int p = 64 * r + lane;
-            bool in = false;
-            uint32_t ix = kSentinelIdx;
-            if (p < K2) {
-                const int64_t o = (s * a.nq + qg) * K2 + p;
-                ix = a.part_idx[o];
-                in = (ix != kSentinelIdx) && !((double)a.part_val[o] > W);
-            }
-            const uint64_t bal = __builtin_amdgcn_ballot_w64(in);
-            const uint32_t pre = (uint32_t)__builtin_popcountll(bal & ((1ull << lane) - 1ull));
-            if (in) cand[wv][nc + pre] = ix;
-            nc += (uint32_t)__builtin_popcountll(bal);
-            if (nc >= 64) {
-                evaluate(64);
-                const uint32_t rest = nc - 64;
-                const uint32_t mv = ((uint32_t)lane < rest) ? cand[wv][64 + lane] : 0u;
-                if ((uint32_t)lane < rest) cand[wv][lane] = mv;
-                nc = rest;
-            }
-        }
-    }
-    if (nc > 0) evaluate(nc);
-#pragma unroll
-    for (int r = 0; r < UB; ++r) {
-        const int slot = 64 * r + lane;
-        if (slot < k)
-            emit_pair(a.mode, a.q, a.x, a.qsq, a.xsq, a.d, k, qg, slot, key_value(res[r]), key_index(res[r]),
-                      a.out_val, a.out_idx);
-    }
-}
-
-// k = 1: the same merge with one lane per query (the segment lists are one
-// pair each, so the merge is a (value, index) minimum).
+// The strip merge, one lane per query: the segment lists are one pair each, so
+// the merge is a (value, index) minimum.
 __global__ __launch_bounds__(256) void knn_merge1_f32_kernel(GramArgs32 a) {
     const int64_t qg = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (qg >= a.nq) return;
@@ -1384,216 +1196,32 @@ __global__ __launch_bounds__(256) void knn_merge1_f32_kernel(GramArgs32 a) {
     emit_pair(a.mode, a.q, a.x, a.qsq, a.xsq, a.d, 1, qg, 0, lv, li, a.out_val, a.out_idx);
 }
 
-// Seed on the matrix cores (d <= 256, 16-byte rows): the screen value of
-// every (query, sampled row) pair, formed as the narrow main kernel forms it
-// (Euclidean: acc = ||x||^2, then v_mfma_f32_32x32x2f32 over -2 q; cosine:
-// the contraction over q scaled by -1/||x|| afterwards; above d = 128 too,
-// where the main kernel contracts on 16x16x4 tiles: the screen bound holds
-// for any summation order), turned into the distance it stands for, rounded
-// up -- u = max(acc + ||q||^2, 0) or clamp(1 + acc/||q||, 0, 2) -- and
-// written to S[q][s] (NaN for a NaN screen value, which the selection never
-// admits).  The k-th smallest u then bounds the query's k-th exact value
-// once eps is added (k sampled rows have exact <= u + eps <= u_k + eps).  A
-// workgroup takes 128 queries and one contiguous range of the sample's
-// 32-row tiles (blockIdx.y: the tiles are split so that the launch fills the
-// chip); sampled row s is index row s * n / m.  The next tile's rows are
-// loaded into registers while the current tile's MFMA chain runs.
-template <int NG, bool COS>
-__global__ __launch_bounds__(256, 2) void knn_seed_screen_f32_kernel(GramArgs32 a, int64_t nsamp,
-                                                                     float* __restrict__ S, int64_t ld) {
-    constexpr int DP = NG * 8;
-    constexpr int STRIDE = DP + 4;
-    __shared__ __attribute__((aligned(16))) float tile[kBn * STRIDE];
-    __shared__ __attribute__((aligned(16))) float tn[kBn];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int h = lane >> 5, jl = lane & 31;
-    const int64_t nq = a.nq, nt = a.nt, d = a.d;
-    const float inf = __builtin_huge_valf();
-    const int64_t q = (int64_t)blockIdx.x * kQpbNarrow + (int64_t)w * 32 + jl;
-    const bool qvalid = q < nq;
-    const int64_t qrow = qvalid ? q : nq - 1;
-    const float qsq = a.qsq[qrow];
-    const float qs = COS ? __builtin_sqrtf(qsq) : qsq;  // the main kernel's screen operand
-    const float scale = COS ? 1.0f : -2.0f;
-    float4 qreg[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-        const int64_t c = 8 * g + 4 * h;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (c < d) v = *reinterpret_cast<const float4*>(a.q + qrow * d + c);
-        qreg[g] = make_float4(scale * v.x, scale * v.y, scale * v.z, scale * v.w);
-    }
-    const int64_t ntiles = (nsamp + kBn - 1) / kBn;
-    const int64_t per = (ntiles + gridDim.y - 1) / gridDim.y;
-    const int64_t s_lo = (int64_t)blockIdx.y * per * kBn;
-    int64_t s_hi = s_lo + per * kBn;
-    if (s_hi > nsamp) s_hi = nsamp;
-    // staging: chunk f = tid + 256 p is column chunk f % (DP / 4) of tile row
-    // f / (DP / 4); the next tile is loaded into registers under the chain
-    constexpr int PF = (kBn * DP / 4 + 255) / 256;
-    float4 pf[PF];
-    float pfn = 0.0f;
-    auto load_tile = [&](int64_t s0) {
-#pragma unroll
-        for (int p = 0; p < PF; ++p) {
-            const int f = tid + 256 * p;
-            const int r = f / (DP / 4), c4 = f % (DP / 4);
-            const int64_t sr = s0 + r;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (f < kBn * DP / 4 && sr < nsamp && 4 * c4 < d)
-                v = *reinterpret_cast<const float4*>(a.x + ((sr * nt) / nsamp) * d + 4 * c4);
-            pf[p] = v;
-        }
-        if (tid < kBn) {
-            const int64_t sr = s0 + tid;
-            const int64_t t = (sr < nsamp) ? (sr * nt) / nsamp : 0;
-            pfn = (sr < nsamp) ? (COS ? a.xscale[t] : a.xsq[t]) : (COS ? 0.0f : inf);
-        }
-    };
-    if (s_lo < s_hi) load_tile(s_lo);
-    for (int64_t s0 = s_lo; s0 < s_hi; s0 += kBn) {
-        __syncthreads();  // the previous tile is no longer read
-#pragma unroll
-        for (int p = 0; p < PF; ++p) {
-            const int f = tid + 256 * p;
-            if (f < kBn * DP / 4)
-                *reinterpret_cast<float4*>(&tile[(f / (DP / 4)) * STRIDE + 4 * (f % (DP / 4))]) = pf[p];
-        }
-        if (tid < kBn) tn[tid] = pfn;
-        __syncthreads();
-        if (s0 + kBn < s_hi) load_tile(s0 + kBn);  // in flight under the chain
-        f32x16 acc;
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-            const float4 n4 = *reinterpret_cast<const float4*>(&tn[8 * g4 + 4 * h]);
-            acc[4 * g4 + 0] = COS ? 0.0f : n4.x;
-            acc[4 * g4 + 1] = COS ? 0.0f : n4.y;
-            acc[4 * g4 + 2] = COS ? 0.0f : n4.z;
-            acc[4 * g4 + 3] = COS ? 0.0f : n4.w;
-        }
-        const float* arow = &tile[jl * STRIDE + 4 * h];
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-            const float4 av = *reinterpret_cast<const float4*>(arow + 8 * g);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.x, qreg[g].x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.y, qreg[g].y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.z, qreg[g].z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av.w, qreg[g].w, acc, 0, 0, 0);
-        }
-        if (qvalid) {
-            // values r = 4 g4 .. 4 g4 + 3 are four consecutive sampled rows:
-            // one 16-byte store (ld and s0 are multiples of 4)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                float u4[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int r = 4 * g4 + e;
-                    // cosine: the contraction scaled by -1/||x|| afterwards, as
-                    // in the main kernel
-                    const float v = COS ? acc[r] * tn[8 * g4 + 4 * h + e] : acc[r];
-                    float u = __builtin_nanf("");
-                    if (v == v) {
-                        if (COS) {
-                            u = round_up_f(1.0 + (double)v / (double)qs);
-                            u = u < 0.0f ? 0.0f : (u > 2.0f ? 2.0f : u);
-                        } else {
-                            u = round_up_f((double)v + (double)qs);
-                            u = u < 0.0f ? 0.0f : u;
-                        }
-                    }
-                    u4[e] = u;
-                }
-                const int64_t sr0 = s0 + 8 * g4 + 4 * h;
-                if (sr0 + 3 < nsamp) {
-                    *reinterpret_cast<float4*>(S + q * ld + sr0) = make_float4(u4[0], u4[1], u4[2], u4[3]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (sr0 + e < nsamp) S[q * ld + sr0 + e] = u4[e];
-                }
-            }
-        }
-    }
-}
-
-// The seed bound from each query's k-th smallest u (out_val[q][k - 1]):
-// round_up(u_k + eps), for queries in screen-value mode (norms well inside
-// the float range); +inf otherwise.
-__global__ void seed_screen_finalize_kernel(GramArgs32 a, const float* __restrict__ kv, int k, int cos) {
-    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (q >= a.nq) return;
-    const float inf = __builtin_huge_valf();
-    const double qsq = (double)a.qsq[q], xmax = (double)a.stats->xsq_max;
-    const double eps = cos ? a.eps_abs : a.eps_rel * (qsq + xmax) + a.eps_abs;
-    const float vk = kv[q * k + (k - 1)];
-    float R = inf;
-    // cosine: a zero query ties every row and is never screened
-    if (qsq + xmax <= 0x1p124 && eps < 0x1p120 && vk < inf && (!cos || qsq > 0.0))
-        R = round_up_f((double)vk + eps);
-    a.shared_r[q] = __float_as_uint(R);
-}
-
 // The shared per-query threshold words start at +inf (as float bits).
 __global__ void fill_inf_bits_kernel(unsigned int* p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0x7F800000u;
 }
 
-template <int NG, int ARM, bool COS, bool VEC4>
-hipError_t launch_ng(const GramArgs32& a, int64_t nblocks, hipStream_t s) {
+template <int NG, bool VEC4>
+hipError_t launch_ng(const GramArgs32& a, hipStream_t s) {
     dim3 grid((unsigned)StreamSplit(a.nq, a.nt, a.qpb, kBn, a.grid_wgs).G);
     const dim3 block(GramShape<(NG > 16)>::threads);
-    (void)nblocks;
-    // rows exactly 128 floats wide take the paired-row kernels' fixed-stride
-    // instance (k > 1: the k = 1 kernel stages its tiles)
-    constexpr bool kPairs = NG == 16 && VEC4;
-    const bool fullw = kPairs && a.d == 8 * NG;
-    if (a.k == 1)
-        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM, COS, VEC4, true, 1>), grid, block, 0, s, a);
-    else if (a.k <= 64 && fullw)
-        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM, COS, VEC4, false, 1, kPairs>), grid, block, 0, s, a);
-    else if (a.k <= 64)
-        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM, COS, VEC4, false, 1>), grid, block, 0, s, a);
-    else if (fullw)
-        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM, COS, VEC4, false, 3, kPairs>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM, COS, VEC4, false, 3>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM_EUCLID_MULADD, false, VEC4, true, 1>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
-template <int ARM, bool COS, bool VEC4>
-hipError_t launch_arm(const GramArgs32& a, int64_t nblocks, hipStream_t s) {
+template <bool VEC4>
+hipError_t launch_d(const GramArgs32& a, hipStream_t s) {
     const int ng = (int)((a.d + 7) / 8);
     // the split and the merge must see the query-block size of the shape
     if (a.qpb != (ng > 16 ? kQpbWide : kQpbNarrow)) return hipErrorInvalidValue;
-    if (ng <= 2) return launch_ng<2, ARM, COS, VEC4>(a, nblocks, s);
-    if (ng <= 4) return launch_ng<4, ARM, COS, VEC4>(a, nblocks, s);
-    if (ng <= 8) return launch_ng<8, ARM, COS, VEC4>(a, nblocks, s);
-    if (ng <= 12) return launch_ng<12, ARM, COS, VEC4>(a, nblocks, s);
-    if (ng <= 16) return launch_ng<16, ARM, COS, VEC4>(a, nblocks, s);
-    if (ng <= 24) return launch_ng<24, ARM, COS, VEC4>(a, nblocks, s);
-    return launch_ng<32, ARM, COS, VEC4>(a, nblocks, s);
-}
-
-template <int ARM, bool COS, bool VEC4>
-hipError_t launch_wide(const GramArgs32& a, int64_t nblocks, hipStream_t s) {
-    const int ng = (int)((a.d + 7) / 8);
-    if (ng <= 16 || a.qpb != kQpbWide) return hipErrorInvalidValue;
-    if (ng <= 24) return launch_ng<24, ARM, COS, VEC4>(a, nblocks, s);
-    return launch_ng<32, ARM, COS, VEC4>(a, nblocks, s);
-}
-
-template <int ARM>
-hipError_t launch_seed(const GramArgs32& a, int64_t nsamp, hipStream_t s) {
-    const dim3 grid((unsigned)((a.nq + kSeedQpb - 1) / kSeedQpb));
-    if (a.k <= 64)
-        hipLaunchKernelGGL((knn_seed_f32_kernel<ARM, 1>), grid, dim3(256), 0, s, a, nsamp);
-    else
-        hipLaunchKernelGGL((knn_seed_f32_kernel<ARM, 2>), grid, dim3(256), 0, s, a, nsamp);
-    return hipGetLastError();
+    if (ng <= 2) return launch_ng<2, VEC4>(a, s);
+    if (ng <= 4) return launch_ng<4, VEC4>(a, s);
+    if (ng <= 8) return launch_ng<8, VEC4>(a, s);
+    if (ng <= 12) return launch_ng<12, VEC4>(a, s);
+    if (ng <= 16) return launch_ng<16, VEC4>(a, s);
+    if (ng <= 24) return launch_ng<24, VEC4>(a, s);
+    return launch_ng<32, VEC4>(a, s);
 }
 
 }  // namespace
@@ -1618,144 +1246,22 @@ int gram_f32_max_k() { return kKcap; }
 int gram_f32_max_d() { return 256; }
 int gram_f32_rows_per_tile() { return kBn; }
 
-// Rows the matrix-core seed samples: 128 k, at most 8192 and nt / 128, at
-// least 512 -- more than the exact seed's cap, since a sampled pair costs a
-// few MFMA cycles here instead of a d-long FMA chain.  c2 with k = 128: 7812
-// rows, step 27.2 -> 26.6 ms against the exact seed's 1953 (kernel 26.3 ->
-// 25.2 ms); k = 32 takes 4096: kernel 20.76 -> 20.68 ms against 2048 at the
-// same step (8192 rows at k = 32: kernel 20.59 ms, step +0.1 ms).
-static int64_t seed_screen_rows(int64_t nt, int k) {
-    int64_t n = 128 * (int64_t)k;
-    if (n > 8192) n = 8192;
-    if (n > nt / 128) n = nt / 128;
-    if (n < 512) n = 512;
-    return nt < n ? nt : n;
-}
-
-template <bool COS>
-static void launch_seed_screen_ng(const GramArgs32& a, int64_t nsamp, float* S, int64_t ld, dim3 grid, int ng,
-                                  hipStream_t s) {
-    if (ng <= 4)
-        hipLaunchKernelGGL((knn_seed_screen_f32_kernel<4, COS>), grid, dim3(256), 0, s, a, nsamp, S, ld);
-    else if (ng <= 8)
-        hipLaunchKernelGGL((knn_seed_screen_f32_kernel<8, COS>), grid, dim3(256), 0, s, a, nsamp, S, ld);
-    else if (ng <= 12)
-        hipLaunchKernelGGL((knn_seed_screen_f32_kernel<12, COS>), grid, dim3(256), 0, s, a, nsamp, S, ld);
-    else if (ng <= 16)
-        hipLaunchKernelGGL((knn_seed_screen_f32_kernel<16, COS>), grid, dim3(256), 0, s, a, nsamp, S, ld);
-    else if (ng <= 24)
-        hipLaunchKernelGGL((knn_seed_screen_f32_kernel<24, COS>), grid, dim3(256), 0, s, a, nsamp, S, ld);
-    else
-        hipLaunchKernelGGL((knn_seed_screen_f32_kernel<32, COS>), grid, dim3(256), 0, s, a, nsamp, S, ld);
-}
-
-size_t gram_f32_seed_screen_bytes(int64_t nq, int64_t nt, int64_t d, int k, int arm, bool vec4) {
-    if (k <= 1 || k > kKcap || d > 256 || !vec4) return 0;
-    const int64_t nsamp = seed_screen_rows(nt, k);
-    if (nsamp < k) return 0;
-    const int64_t ld = (nsamp + 3) / 4 * 4;
-    const size_t bytes = (size_t)nq * (size_t)ld * 4 + 2 * (((size_t)nq * (size_t)k * 4 + 255) & ~(size_t)255) + 512;
-    return bytes <= ((size_t)512 << 20) ? bytes : 0;  // larger searches keep the exact seed
-}
-
-hipError_t launch_gram_f32_prep(const GramArgs32& a, int arm, hipStream_t s, void* seed_buf) {
+hipError_t launch_gram_f32_prep(const GramArgs32& a, hipStream_t s) {
     if (!a.shared_r) return hipSuccess;
-    if (a.summ) {
-        const int64_t n = (int64_t)a.nslots * a.nq * 4;
-        hipLaunchKernelGGL(fill_inf_bits_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           reinterpret_cast<unsigned int*>(a.summ), n);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    if (a.k > 1) {
-        const int64_t nsamp = seed_buf ? seed_screen_rows(a.nt, a.k) : gram_seed_rows(a.nt, a.k);
-        if (seed_buf) {
-            const int64_t ld = (nsamp + 3) / 4 * 4;
-            float* S = static_cast<float*>(seed_buf);
-            char* p = reinterpret_cast<char*>(S + (size_t)a.nq * (size_t)ld);
-            p = reinterpret_cast<char*>(((uintptr_t)p + 255) & ~(uintptr_t)255);
-            float* kv = reinterpret_cast<float*>(p);
-            p += ((size_t)a.nq * (size_t)a.k * 4 + 255) & ~(size_t)255;
-            uint32_t* ki = reinterpret_cast<uint32_t*>(p);
-            // about four workgroups per CU: the sample's tiles split over blockIdx.y
-            const int64_t nqb = (a.nq + kQpbNarrow - 1) / kQpbNarrow;
-            const int64_t ntiles = (nsamp + kBn - 1) / kBn;
-            int64_t ys = (1024 + nqb - 1) / nqb;
-            if (ys > ntiles) ys = ntiles;
-            if (ys > 65535) ys = 65535;
-            if (ys < 1) ys = 1;
-            const dim3 grid((unsigned)nqb, (unsigned)ys);
-            const int ng = (int)((a.d + 7) / 8);
-            const bool cos = (arm == ARM_COS_FOLD || arm == ARM_COS_HOST);
-            if (cos)
-                launch_seed_screen_ng<true>(a, nsamp, S, ld, grid, ng, s);
-            else
-                launch_seed_screen_ng<false>(a, nsamp, S, ld, grid, ng, s);
-            hipError_t e = hipGetLastError();
-            if (e == hipSuccess) e = launch_select_rows<float>(S, a.nq, nsamp, ld, a.k, EMIT_IDENTITY, kv, ki, nullptr, s);
-            if (e != hipSuccess) return e;
-            hipLaunchKernelGGL(seed_screen_finalize_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a,
-                               kv, a.k, cos ? 1 : 0);
-            return hipGetLastError();
-        }
-        if (arm == ARM_EUCLID_FMA) return launch_seed<ARM_EUCLID_FMA>(a, nsamp, s);
-        if (arm == ARM_EUCLID_MULADD) return launch_seed<ARM_EUCLID_MULADD>(a, nsamp, s);
-        if (arm == ARM_COS_FOLD) return launch_seed<ARM_COS_FOLD>(a, nsamp, s);
-        if (arm == ARM_COS_HOST) return launch_seed<ARM_COS_HOST>(a, nsamp, s);
-        return hipErrorInvalidValue;
-    }
     hipLaunchKernelGGL(fill_inf_bits_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a.shared_r, a.nq);
     return hipGetLastError();
 }
 
-template <int ARM, bool VEC4>
-hipError_t launch_merge(const GramArgs32& a, hipStream_t s) {
-    const dim3 grid((unsigned)((a.nq + 3) / 4));
-    if (a.k <= 64)
-        hipLaunchKernelGGL((knn_merge_f32_kernel<ARM, VEC4>), grid, dim3(256), 0, s, a);
-    else
-        hipLaunchKernelGGL((knn_merge_blocks_f32_kernel<ARM, VEC4>), grid, dim3(256), 0, s, a);
+hipError_t launch_gram_f32_merge(const GramArgs32& a, hipStream_t s) {
+    hipLaunchKernelGGL(knn_merge1_f32_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_gram_f32_merge(const GramArgs32& a, int arm, hipStream_t s) {
-    if (a.k == 1) {
-        hipLaunchKernelGGL(knn_merge1_f32_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a);
-        return hipGetLastError();
-    }
-    const bool vec4 = (a.d % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.q) & 15) == 0) &&
-                      ((reinterpret_cast<uintptr_t>(a.x) & 15) == 0);
-    if (arm == ARM_EUCLID_FMA)
-        return vec4 ? launch_merge<ARM_EUCLID_FMA, true>(a, s) : launch_merge<ARM_EUCLID_FMA, false>(a, s);
-    if (arm == ARM_EUCLID_MULADD)
-        return vec4 ? launch_merge<ARM_EUCLID_MULADD, true>(a, s) : launch_merge<ARM_EUCLID_MULADD, false>(a, s);
-    if (arm == ARM_COS_FOLD)
-        return vec4 ? launch_merge<ARM_COS_FOLD, true>(a, s) : launch_merge<ARM_COS_FOLD, false>(a, s);
-    if (arm == ARM_COS_HOST)
-        return vec4 ? launch_merge<ARM_COS_HOST, true>(a, s) : launch_merge<ARM_COS_HOST, false>(a, s);
-    return hipErrorInvalidValue;
-}
-
 hipError_t launch_gram_f32(const GramArgs32& a, int arm, hipStream_t s) {
-    const int64_t nblocks = (a.nq + a.qpb - 1) / a.qpb;
+    if (a.k != 1 || arm != ARM_EUCLID_MULADD) return hipErrorInvalidValue;
     const bool vec4 = (a.d % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.q) & 15) == 0) &&
                       ((reinterpret_cast<uintptr_t>(a.x) & 15) == 0);
-    hipError_t e;
-    if (arm == ARM_EUCLID_FMA)
-        e = vec4 ? launch_arm<ARM_EUCLID_FMA, false, true>(a, nblocks, s)
-                 : launch_arm<ARM_EUCLID_FMA, false, false>(a, nblocks, s);
-    else if (arm == ARM_EUCLID_MULADD)
-        e = vec4 ? launch_arm<ARM_EUCLID_MULADD, false, true>(a, nblocks, s)
-                 : launch_arm<ARM_EUCLID_MULADD, false, false>(a, nblocks, s);
-    else if (arm == ARM_COS_FOLD)
-        e = vec4 ? launch_arm<ARM_COS_FOLD, true, true>(a, nblocks, s)
-                 : launch_arm<ARM_COS_FOLD, true, false>(a, nblocks, s);
-    else if (arm == ARM_COS_HOST)  // the knn_host arm serves cosine above d = 128 only: wide shapes
-        e = vec4 ? launch_wide<ARM_COS_HOST, true, true>(a, nblocks, s)
-                 : launch_wide<ARM_COS_HOST, true, false>(a, nblocks, s);
-    else
-        return hipErrorInvalidValue;
-    return e;
+    return vec4 ? launch_d<true>(a, s) : launch_d<false>(a, s);
 }
 
 }  // namespace mlrs

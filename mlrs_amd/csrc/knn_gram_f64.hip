@@ -7,6 +7,9 @@
 // 1058-1512) and the host scan of knn_host_topk (crates/mlrs-backend/src/
 // prims/knn_host.rs:418-851) for f64.
 //
+// Launched for the k-means assignment only (k = 1, ARM_EUCLID_MULADD); searches
+// are knn_groupmin's.
+//
 // Shape of one workgroup: 4 waves x 16 queries = 64 queries, walking one
 // segment of index rows 16 at a time with v_mfma_f64_16x16x4f64.
 //  * Lane l of a wave owns query l%16 and lane group g = l/16.  The K
@@ -708,156 +711,6 @@ __global__ __launch_bounds__(256) void knn_merge_f64_kernel(GramArgs64 a) {
     }
 }
 
-// 64 < k <= 128: the same merge over lists of up to three 64-entry blocks
-// (k + 32 entries); the union and the result are two-block lists (the k
-// smallest fit in 128 entries), merged block by block.  k-means assignment
-// (k = 1) never comes here, so the output transform is the root or identity.
-template <int ARM, bool VEC2>
-__global__ __launch_bounds__(256) void knn_merge_blocks_f64_kernel(GramArgs64 a) {
-    constexpr int SLB = 3;  // blocks of a segment list
-    constexpr int UB = 2;   // blocks of the union and of the result
-    __shared__ uint32_t cand[4][128];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    const int64_t qg = (int64_t)blockIdx.x * 4 + wv;
-    if (qg >= a.nq) return;
-    const int k = a.k;
-    const int K2 = gram_list_cap(k);
-    const int64_t d = a.d;
-    const double inf = __builtin_huge_val();
-    const StreamSplit sp(a.nq, a.nt, kQpb, kBn, a.grid_wgs);
-    const int64_t nsl = sp.slots_of(qg / kQpb);
-    double uv[UB];
-    uint32_t ui[UB];
-#pragma unroll
-    for (int r = 0; r < UB; ++r) {
-        uv[r] = inf;
-        ui[r] = kSentinelIdx;
-    }
-    for (int64_t s = 0; s < nsl; ++s) {
-#pragma unroll
-        for (int r = 0; r < SLB; ++r) {
-            if (64 * r >= K2) break;
-            const int p = 64 * r + lane;
-            double v = inf;
-            uint32_t ix = kSentinelIdx;
-            if (p < K2) {
-                const int64_t o = (s * a.nq + qg) * K2 + p;
-                v = a.part_val[o];
-                ix = a.part_idx[o];
-            }
-            wave_merge_blocks<double, UB>(uv, ui, v, ix, lane);
-        }
-    }
-    const double qsq = a.qsq[qg];
-    const bool cos = (ARM == ARM_COS_FOLD || ARM == ARM_COS_HOST);
-    const double eps = cos ? a.eps_abs : a.eps_rel * (qsq + a.stats->xsq_max64) + a.eps_abs;
-    double W = list_value_at<double, UB>(uv, k - 1) + 2.0 * eps;
-    W += __builtin_fabs(W) * 0x1p-40;
-    const double qa = (ARM == ARM_COS_HOST) ? a.qinv[qg] : qsq;
-    double lv[UB];
-    uint32_t li[UB];
-#pragma unroll
-    for (int r = 0; r < UB; ++r) {
-        lv[r] = inf;
-        li[r] = kSentinelIdx;
-    }
-    uint32_t nc = 0;
-    auto evaluate = [&](uint32_t count) {
-        double e = inf;
-        uint32_t t = kSentinelIdx;
-        if ((uint32_t)lane < count) {
-            t = cand[wv][lane];
-            const double ya = (ARM == ARM_COS_FOLD) ? a.xsq[t] : (ARM == ARM_COS_HOST) ? a.xinv[t] : 0.0;
-            e = exact_f64<ARM, VEC2, 8>(a.q + qg * d, a.x + (int64_t)t * d, d, qa, ya);
-            if (e != e) {
-                e = inf;
-                t = kSentinelIdx;
-            } else if (a.mode == EMIT_ROOT_RANKED) {
-                e = __builtin_sqrt(e);  // ranked by (root, index)
-            }
-        }
-        wave_sort64<double>(e, t, lane);
-        wave_merge_blocks<double, UB>(lv, li, e, t, lane);
-    };
-    for (int64_t s = 0; s < nsl; ++s) {
-        for (int r = 0; r < SLB; ++r) {
-            if (64 * r >= K2) break;
-            const int p = 64 * r + lane;
-            bool in = false;
-            uint32_t ix = kSentinelIdx;
-            if (p < K2) {
-                const int64_t o = (s * a.nq + qg) * K2 + p;
-                ix = a.part_idx[o];
-                in = (ix != kSentinelIdx) && !(a.part_val[o] > W);
-            }
-            const uint64_t bal = __builtin_amdgcn_ballot_w64(in);
-            const uint32_t pre = (uint32_t)__builtin_popcountll(bal & ((1ull << lane) - 1ull));
-            if (in) cand[wv][nc + pre] = ix;
-            nc += (uint32_t)__builtin_popcountll(bal);
-            if (nc >= 64) {
-                evaluate(64);
-                const uint32_t rest = nc - 64;
-                const uint32_t mv = ((uint32_t)lane < rest) ? cand[wv][64 + lane] : 0u;
-                if ((uint32_t)lane < rest) cand[wv][lane] = mv;
-                nc = rest;
-            }
-        }
-    }
-    if (nc > 0) evaluate(nc);
-#pragma unroll
-    for (int r = 0; r < UB; ++r) {
-        const int slot = 64 * r + lane;
-        if (slot < k) {
-            const int64_t o = qg * k + slot;
-            a.out_val[o] = (a.mode == EMIT_SQRT) ? __builtin_sqrt(lv[r]) : lv[r];
-            a.out_idx[o] = (li[r] == kSentinelIdx) ? 0u : li[r];
-        }
-    }
-}
-
-// EMIT_ROOT_RANKED, queries with root_flag set (an exact list dropped a pair
-// whose root may equal the k-th root, so ties of that root may be missing
-// from the merge): the emitted row keeps its m entries below the k-th root
-// r (all pairs with a smaller root: their aggregates are below the k-th, so
-// the merge saw them) and slots m..k-1 get r with the lowest-index rows whose
-// root is r, found by evaluating every index row in ascending order, 64 at a
-// time (one wave per query; unflagged queries return at once).  This is the
-// host scan's KNearest order (crates/mlrs-algos/src/manifold/
-// umap_host_knn.rs:171-198): (root, index).
-template <int ARM, bool VEC2>
-__global__ __launch_bounds__(256) void knn_root_fill_f64_kernel(GramArgs64 a) {
-    const int lane = threadIdx.x & 63;
-    const int64_t qg = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (qg >= a.nq || a.root_flag[qg] == 0u) return;
-    const int k = a.k;
-    double* ov = a.out_val + qg * k;
-    uint32_t* oi = a.out_idx + qg * k;
-    const double r = ov[k - 1];
-    if (!(r < __builtin_huge_val())) return;
-    uint32_t m = 0;
-    for (int j0 = 0; j0 < k; j0 += 64)
-        m += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(j0 + lane < k && ov[j0 + lane] < r));
-    const uint32_t need = (uint32_t)k - m;
-    const int64_t d = a.d;
-    uint32_t found = 0;
-    for (int64_t t0 = 0; t0 < a.nt && found < need; t0 += 64) {
-        const int64_t t = t0 + lane;
-        bool hit = false;
-        if (t < a.nt) {
-            const double e = exact_f64<ARM, VEC2, 8>(a.q + qg * d, a.x + t * d, d, 0.0, 0.0);
-            hit = (e == e) && __builtin_sqrt(e) == r;
-        }
-        const uint64_t bal = __builtin_amdgcn_ballot_w64(hit);
-        const uint32_t pos = found + (uint32_t)__builtin_popcountll(bal & ((1ull << lane) - 1ull));
-        if (hit && pos < need) {
-            ov[m + pos] = r;
-            oi[m + pos] = (uint32_t)t;
-        }
-        found += (uint32_t)__builtin_popcountll(bal);
-    }
-}
-
 // Initial per-query bound: the k-th smallest exact value over an evenly
 // spaced sample of index rows (seed_kth_block): any k distinct rows bound the
 // final k-th value from above, so each segment's screen starts tight instead
@@ -876,32 +729,19 @@ __global__ void fill_u64_kernel(unsigned long long* p, int64_t n, unsigned long 
     if (i < n) p[i] = v;
 }
 
-template <int NS, int ARM, bool COS>
+template <int NS>
 hipError_t launch_ns(const GramArgs64& a, bool vec2, hipStream_t s) {
     dim3 grid((unsigned)StreamSplit(a.nq, a.nt, kQpb, kBn, a.grid_wgs).G);
-    if (a.k <= 64) {
-        if (vec2)
-            hipLaunchKernelGGL((knn_gram_f64_kernel<NS, ARM, COS, true, 1>), grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((knn_gram_f64_kernel<NS, ARM, COS, false, 1>), grid, dim3(256), 0, s, a);
-    } else {
-        if (vec2)
-            hipLaunchKernelGGL((knn_gram_f64_kernel<NS, ARM, COS, true, 3>), grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((knn_gram_f64_kernel<NS, ARM, COS, false, 3>), grid, dim3(256), 0, s, a);
-    }
+    if (vec2)
+        hipLaunchKernelGGL((knn_gram_f64_kernel<NS, ARM_EUCLID_MULADD, false, true, 1>), grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((knn_gram_f64_kernel<NS, ARM_EUCLID_MULADD, false, false, 1>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-template <int ARM, bool COS>
-hipError_t launch_arm64(const GramArgs64& a, bool vec2, hipStream_t s) {
-    // k-steps per lane group, even (one 16-byte LDS read feeds two)
-    const int64_t ns = ((a.d + 3) / 4 + 1) / 2 * 2;
-    if (ns <= 8) return launch_ns<8, ARM, COS>(a, vec2, s);
-    if (ns <= 16) return launch_ns<16, ARM, COS>(a, vec2, s);
-    if (ns <= 32) return launch_ns<32, ARM, COS>(a, vec2, s);
-    if (ns <= 48) return launch_ns<48, ARM, COS>(a, vec2, s);
-    return launch_ns<64, ARM, COS>(a, vec2, s);
+bool rows_vec2(const GramArgs64& a) {
+    return (a.d % 2 == 0) && ((reinterpret_cast<uintptr_t>(a.q) & 15) == 0) &&
+           ((reinterpret_cast<uintptr_t>(a.x) & 15) == 0);
 }
 
 }  // namespace
@@ -919,289 +759,36 @@ void gram_f64_split(int64_t nq, int64_t nt, int cus, int64_t* grid_wgs, int* nsl
 int gram_f64_max_k() { return kKcap; }
 int gram_f64_max_d() { return kMaxD; }
 
-// Seed on the matrix cores (16-byte rows): the screen value of every
-// (query, sampled row) pair on v_mfma_f64_16x16x4f64 (Euclidean: acc =
-// ||x||^2 - 2 x.q; cosine: acc = -(x.q)/||x||), turned into the distance it
-// stands for, u = max(acc + ||q||^2, 0) or clamp(1 + acc/||q||, 0, 2) (NaN
-// kept), written to S[q][s].  The screen bound eps holds for any summation
-// order, so k sampled rows have exact <= u + eps <= u_k + eps.  A wave takes
-// 16 queries (lane l: query l % 16; k-slot g = l / 16 supplies feature
-// g KS + s at k-step s, so each lane's query operand and tile reads are
-// contiguous runs, loaded 16 bytes at a time), a workgroup 64 queries and a
-// slice of the sample's 16-row tiles (blockIdx.y); sampled row s is index row
-// s * n / m.  The next tile's rows are loaded into registers while the
-// current tile's MFMA chain runs (two accumulator chains: the even and odd
-// k-steps), and stored into the one LDS tile between two barriers.
-template <int KS, bool COS>
-__global__ __launch_bounds__(256, 2) void knn_seed_screen_f64_kernel(GramArgs64 a, int64_t nsamp,
-                                                                     double* __restrict__ S, int64_t ld) {
-    static_assert(KS % 2 == 0, "k-steps come in 16-byte pairs");
-    constexpr int DP = 4 * KS;
-    constexpr int STR = DP + 2;               // rows 16 bytes apart in the banks
-    constexpr int CPR = DP / 2;               // 16-byte chunks per tile row
-    constexpr int PF = kBn * CPR / 256;       // chunks each thread stages per tile
-    static_assert(kBn * CPR % 256 == 0, "whole chunks per thread");
-    __shared__ __attribute__((aligned(16))) double tile[kBn * STR];
-    __shared__ double tn[kBn];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int g = lane >> 4, j = lane & 15;
-    const int64_t nq = a.nq, nt = a.nt, d = a.d;
-    const double inf = __builtin_huge_val();
-    const int64_t q = (int64_t)blockIdx.x * kQpb + (int64_t)w * kQpw + j;
-    const bool qvalid = q < nq;
-    const int64_t qrow = qvalid ? q : nq - 1;
-    const double qsq = a.qsq[qrow];
-    const double qs = COS ? __builtin_sqrt(qsq) : qsq;
-    double qreg[KS];
-#pragma unroll
-    for (int st = 0; st < KS; st += 2) {
-        const int64_t c = (int64_t)g * KS + st;  // c and d even: c < d covers c + 1
-        double2 v = make_double2(0.0, 0.0);
-        if (c < d) v = *reinterpret_cast<const double2*>(a.q + qrow * d + c);
-        qreg[st] = v.x * (COS ? 1.0 : -2.0);
-        qreg[st + 1] = v.y * (COS ? 1.0 : -2.0);
-    }
-    const int64_t ntiles = (nsamp + kBn - 1) / kBn;
-    const int64_t per = (ntiles + gridDim.y - 1) / gridDim.y;
-    const int64_t s_lo = (int64_t)blockIdx.y * per * kBn;
-    int64_t s_hi = s_lo + per * kBn;
-    if (s_hi > nsamp) s_hi = nsamp;
-    // staging: chunk f = tid + 256 p is column pair f % CPR of tile row f / CPR
-    double2 pf[PF];
-    double pfn = 0.0;
-    auto load_tile = [&](int64_t s0) {
-#pragma unroll
-        for (int p = 0; p < PF; ++p) {
-            const int f = tid + 256 * p;
-            const int r = f / CPR, c2 = f % CPR;
-            const int64_t sr = s0 + r;
-            double2 v = make_double2(0.0, 0.0);
-            if (sr < nsamp && 2 * c2 < d)
-                v = *reinterpret_cast<const double2*>(a.x + ((sr * nt) / nsamp) * d + 2 * c2);
-            pf[p] = v;
-        }
-        if (tid < kBn) {
-            const int64_t sr = s0 + tid;
-            const int64_t t = (sr < nsamp) ? (sr * nt) / nsamp : 0;
-            pfn = (sr < nsamp) ? (COS ? a.xscale[t] : a.xsq[t]) : (COS ? 0.0 : inf);
-        }
-    };
-    if (s_lo < s_hi) load_tile(s_lo);
-    for (int64_t s0 = s_lo; s0 < s_hi; s0 += kBn) {
-        __syncthreads();  // the previous tile is no longer read
-#pragma unroll
-        for (int p = 0; p < PF; ++p) {
-            const int f = tid + 256 * p;
-            *reinterpret_cast<double2*>(&tile[(f / CPR) * STR + 2 * (f % CPR)]) = pf[p];
-        }
-        if (tid < kBn) tn[tid] = pfn;
-        __syncthreads();
-        if (s0 + kBn < s_hi) load_tile(s0 + kBn);  // in flight under the chain
-        f64x4 acc0, acc1;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            acc0[r] = COS ? 0.0 : tn[g + 4 * r];
-            acc1[r] = 0.0;
-        }
-        const double* arow = &tile[j * STR + g * KS];
-#pragma unroll
-        for (int st = 0; st < KS; st += 2) {
-            const double2 av = *reinterpret_cast<const double2*>(arow + st);
-            acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, qreg[st], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, qreg[st + 1], acc1, 0, 0, 0);
-        }
-        if (qvalid) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t sr = s0 + g + 4 * r;
-                if (sr < nsamp) {
-                    const double acc = acc0[r] + acc1[r];
-                    const double v = COS ? acc * tn[g + 4 * r] : acc;
-                    double u = __builtin_nan("");
-                    if (v == v) {
-                        if (COS) {
-                            u = 1.0 + v / qs;
-                            u = u < 0.0 ? 0.0 : (u > 2.0 ? 2.0 : u);
-                        } else {
-                            u = v + qsq;
-                            u = u < 0.0 ? 0.0 : u;
-                        }
-                    }
-                    S[q * ld + sr] = u;
-                }
-            }
-        }
-    }
-}
-
-// The seed bound from each query's k-th smallest u: (u_k + eps) rounded
-// up by a relative 2^-50, for queries in screen-value mode; +inf otherwise.
-__global__ void seed_screen_finalize64_kernel(GramArgs64 a, const double* __restrict__ kv, int k, int cos) {
-    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (q >= a.nq) return;
-    const double inf = __builtin_huge_val();
-    const double qsq = a.qsq[q], xmax = a.stats->xsq_max64;
-    const double eps = cos ? a.eps_abs : a.eps_rel * (qsq + xmax) + a.eps_abs;
-    const bool sv = (qsq + xmax <= 0x1p1020) && (eps < inf) && (!cos || qsq > 0.0);
-    const double vk = kv[q * k + (k - 1)];
-    double R = inf;
-    if (sv && vk < inf) R = (vk + eps) * (1.0 + 0x1p-50);
-    a.shared_r[q] = (unsigned long long)__double_as_longlong(R);
-}
-
-// Rows the matrix-core seed samples: 128 k, at most 8192 and nt / 64, at
-// least 512.  With the tile loads under the MFMA chain the launch is cheap
-// enough for four times the exact seed's sample at c3 (k = 16, 2048 rows):
-// kernel 9.15 -> 9.01 ms and step 9.43 -> 9.41 ms against 512 rows (A/B of
-// two builds on one box; 4096 rows: kernel 8.96 ms, step 9.53 ms).
-static int64_t seed_screen_rows64(int64_t nt, int k) {
-    int64_t n = 128 * (int64_t)k;
-    if (n > 8192) n = 8192;
-    if (n > nt / 64) n = nt / 64;
-    if (n < 512) n = 512;
-    return nt < n ? nt : n;
-}
-
-size_t gram_f64_seed_screen_bytes(int64_t nq, int64_t nt, int64_t d, int k, bool vec2) {
-    if (k <= 1 || k > kKcap || d > kMaxD || !vec2) return 0;
-    const int64_t nsamp = seed_screen_rows64(nt, k);
-    if (nsamp < k) return 0;
-    const int64_t ld = (nsamp + 1) / 2 * 2;
-    const size_t bytes = (size_t)nq * (size_t)ld * 8 + (((size_t)nq * (size_t)k * 8 + 255) & ~(size_t)255) +
-                         (((size_t)nq * (size_t)k * 4 + 255) & ~(size_t)255) + 512;
-    return bytes <= ((size_t)512 << 20) ? bytes : 0;
-}
-
-template <int KS, bool COS>
-static void launch_seed_screen64_ks(const GramArgs64& a, int64_t nsamp, double* S, int64_t ld, dim3 grid,
-                                    hipStream_t s) {
-    hipLaunchKernelGGL((knn_seed_screen_f64_kernel<KS, COS>), grid, dim3(256), 0, s, a, nsamp, S, ld);
-}
-
-template <int ARM>
-hipError_t launch_seed64(const GramArgs64& a, int64_t nsamp, hipStream_t s) {
-    const dim3 grid((unsigned)((a.nq + kSeedQpb - 1) / kSeedQpb));
-    if (a.k <= 64)
-        hipLaunchKernelGGL((knn_seed_f64_kernel<ARM, 1>), grid, dim3(256), 0, s, a, nsamp);
-    else
-        hipLaunchKernelGGL((knn_seed_f64_kernel<ARM, 2>), grid, dim3(256), 0, s, a, nsamp);
-    return hipGetLastError();
-}
-
-hipError_t launch_gram_f64_prep(const GramArgs64& a, int arm, hipStream_t s, void* seed_buf) {
-    if (a.root_flag) {
-        const hipError_t e = launch_fill_u32(a.root_flag, a.nq, 0u, s);
-        if (e != hipSuccess) return e;
-    }
-    if (!a.shared_r) return hipSuccess;
-    if (seed_buf && a.k > 1) {
-        const bool cos = (arm == ARM_COS_FOLD || arm == ARM_COS_HOST);
-        const int64_t nsamp = seed_screen_rows64(a.nt, a.k);
-        const int64_t ld = (nsamp + 1) / 2 * 2;
-        double* S = static_cast<double*>(seed_buf);
-        char* p = reinterpret_cast<char*>(S + (size_t)a.nq * (size_t)ld);
-        p = reinterpret_cast<char*>(((uintptr_t)p + 255) & ~(uintptr_t)255);
-        double* kv = reinterpret_cast<double*>(p);
-        p += ((size_t)a.nq * (size_t)a.k * 8 + 255) & ~(size_t)255;
-        uint32_t* ki = reinterpret_cast<uint32_t*>(p);
-        // about four workgroups per CU: the sample's tiles split over blockIdx.y
-        const int64_t nqb = (a.nq + kQpb - 1) / kQpb;
-        const int64_t ntiles = (nsamp + kBn - 1) / kBn;
-        int64_t ys = (1024 + nqb - 1) / nqb;
-        if (ys > ntiles) ys = ntiles;
-        if (ys > 65535) ys = 65535;
-        if (ys < 1) ys = 1;
-        const dim3 grid((unsigned)nqb, (unsigned)ys);
-        const int64_t ks = (a.d + 3) / 4;
-        if (cos) {
-            if (ks <= 16) launch_seed_screen64_ks<16, true>(a, nsamp, S, ld, grid, s);
-            else if (ks <= 32) launch_seed_screen64_ks<32, true>(a, nsamp, S, ld, grid, s);
-            else if (ks <= 48) launch_seed_screen64_ks<48, true>(a, nsamp, S, ld, grid, s);
-            else launch_seed_screen64_ks<64, true>(a, nsamp, S, ld, grid, s);
-        } else {
-            if (ks <= 16) launch_seed_screen64_ks<16, false>(a, nsamp, S, ld, grid, s);
-            else if (ks <= 32) launch_seed_screen64_ks<32, false>(a, nsamp, S, ld, grid, s);
-            else if (ks <= 48) launch_seed_screen64_ks<48, false>(a, nsamp, S, ld, grid, s);
-            else launch_seed_screen64_ks<64, false>(a, nsamp, S, ld, grid, s);
-        }
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess) e = launch_select_rows<double>(S, a.nq, nsamp, ld, a.k, EMIT_IDENTITY, kv, ki, nullptr, s);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(seed_screen_finalize64_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a,
-                           kv, a.k, cos ? 1 : 0);
-        return hipGetLastError();
-    }
+hipError_t launch_gram_f64_prep(const GramArgs64& a, hipStream_t s) {
     const int64_t nsamp = gram_seed_rows(a.nt, a.k);
-    if (nsamp >= a.k) {
-        if (arm == ARM_EUCLID_FMA) return launch_seed64<ARM_EUCLID_FMA>(a, nsamp, s);
-        if (arm == ARM_EUCLID_MULADD) return launch_seed64<ARM_EUCLID_MULADD>(a, nsamp, s);
-        if (arm == ARM_COS_FOLD) return launch_seed64<ARM_COS_FOLD>(a, nsamp, s);
-        if (arm == ARM_COS_HOST) return launch_seed64<ARM_COS_HOST>(a, nsamp, s);
-        return hipErrorInvalidValue;
-    }
-    hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a.shared_r, a.nq,
-                       kInfBits64);
+    if (nsamp >= a.k)
+        hipLaunchKernelGGL((knn_seed_f64_kernel<ARM_EUCLID_MULADD, 1>),
+                           dim3((unsigned)((a.nq + kSeedQpb - 1) / kSeedQpb)), dim3(256), 0, s, a, nsamp);
+    else
+        hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a.shared_r, a.nq,
+                           kInfBits64);
     return hipGetLastError();
 }
 
 hipError_t launch_gram_f64(const GramArgs64& a, int arm, hipStream_t s) {
-    const bool vec2 = (a.d % 2 == 0) && ((reinterpret_cast<uintptr_t>(a.q) & 15) == 0) &&
-                      ((reinterpret_cast<uintptr_t>(a.x) & 15) == 0);
-    if (arm == ARM_EUCLID_FMA) return launch_arm64<ARM_EUCLID_FMA, false>(a, vec2, s);
-    if (arm == ARM_EUCLID_MULADD) return launch_arm64<ARM_EUCLID_MULADD, false>(a, vec2, s);
-    if (arm == ARM_COS_FOLD) return launch_arm64<ARM_COS_FOLD, true>(a, vec2, s);
-    if (arm == ARM_COS_HOST) return launch_arm64<ARM_COS_HOST, true>(a, vec2, s);
-    return hipErrorInvalidValue;
+    if (a.k != 1 || arm != ARM_EUCLID_MULADD) return hipErrorInvalidValue;
+    const bool vec2 = rows_vec2(a);
+    // k-steps per lane group, even (one 16-byte LDS read feeds two)
+    const int64_t ns = ((a.d + 3) / 4 + 1) / 2 * 2;
+    if (ns <= 8) return launch_ns<8>(a, vec2, s);
+    if (ns <= 16) return launch_ns<16>(a, vec2, s);
+    if (ns <= 32) return launch_ns<32>(a, vec2, s);
+    if (ns <= 48) return launch_ns<48>(a, vec2, s);
+    return launch_ns<64>(a, vec2, s);
 }
 
-template <int ARM>
-hipError_t launch_merge64(const GramArgs64& a, bool vec2, hipStream_t s) {
+hipError_t launch_gram_f64_merge(const GramArgs64& a, hipStream_t s) {
     const dim3 grid((unsigned)((a.nq + 3) / 4));
-    if (a.k > 64) {
-        if (vec2)
-            hipLaunchKernelGGL((knn_merge_blocks_f64_kernel<ARM, true>), grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((knn_merge_blocks_f64_kernel<ARM, false>), grid, dim3(256), 0, s, a);
-    } else if (vec2) {
-        hipLaunchKernelGGL((knn_merge_f64_kernel<ARM, true>), grid, dim3(256), 0, s, a);
-    } else {
-        hipLaunchKernelGGL((knn_merge_f64_kernel<ARM, false>), grid, dim3(256), 0, s, a);
-    }
+    if (rows_vec2(a))
+        hipLaunchKernelGGL((knn_merge_f64_kernel<ARM_EUCLID_MULADD, true>), grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((knn_merge_f64_kernel<ARM_EUCLID_MULADD, false>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
-}
-
-hipError_t launch_gram_f64_merge(const GramArgs64& a, int arm, hipStream_t s) {
-    const bool vec2 = (a.d % 2 == 0) && ((reinterpret_cast<uintptr_t>(a.q) & 15) == 0) &&
-                      ((reinterpret_cast<uintptr_t>(a.x) & 15) == 0);
-    if (arm == ARM_EUCLID_FMA) return launch_merge64<ARM_EUCLID_FMA>(a, vec2, s);
-    if (arm == ARM_EUCLID_MULADD) return launch_merge64<ARM_EUCLID_MULADD>(a, vec2, s);
-    if (arm == ARM_COS_FOLD) return launch_merge64<ARM_COS_FOLD>(a, vec2, s);
-    if (arm == ARM_COS_HOST) return launch_merge64<ARM_COS_HOST>(a, vec2, s);
-    return hipErrorInvalidValue;
-}
-
-hipError_t launch_gram_f64_root_fill(const GramArgs64& a, int arm, hipStream_t s) {
-    if (!a.root_flag || a.mode != EMIT_ROOT_RANKED) return hipSuccess;
-    const bool vec2 = (a.d % 2 == 0) && ((reinterpret_cast<uintptr_t>(a.q) & 15) == 0) &&
-                      ((reinterpret_cast<uintptr_t>(a.x) & 15) == 0);
-    const dim3 grid((unsigned)((a.nq + 3) / 4));
-    if (arm == ARM_EUCLID_MULADD) {
-        if (vec2)
-            hipLaunchKernelGGL((knn_root_fill_f64_kernel<ARM_EUCLID_MULADD, true>), grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((knn_root_fill_f64_kernel<ARM_EUCLID_MULADD, false>), grid, dim3(256), 0, s, a);
-        return hipGetLastError();
-    }
-    if (arm == ARM_EUCLID_FMA) {
-        if (vec2)
-            hipLaunchKernelGGL((knn_root_fill_f64_kernel<ARM_EUCLID_FMA, true>), grid, dim3(256), 0, s, a);
-        else
-            hipLaunchKernelGGL((knn_root_fill_f64_kernel<ARM_EUCLID_FMA, false>), grid, dim3(256), 0, s, a);
-        return hipGetLastError();
-    }
-    return hipErrorInvalidValue;  // the roots are sqrt: Euclidean arms only
 }
 
 }  // namespace mlrs

@@ -158,13 +158,9 @@ inline int64_t gram_seed_rows(int64_t nt, int k) {
 // which picks the kernel and with it the workgroups per CU the split assumes.
 void gram_f32_split(int64_t nq, int64_t nt, int64_t d, int k, int cus, bool vec4, int64_t* grid_wgs, int* nslots);
 
-// Three launches per search: prep (the shared per-query bound: seeded from a
-// row sample for k > 1, else reset), the Gram kernel, the strip merge +
-// output transform.
-// seed_buf: gram_f32_seed_screen_bytes(...) bytes of workspace when that is
-// nonzero (the seed then runs on the matrix cores), else null.
-hipError_t launch_gram_f32_prep(const GramArgs32& a, int arm, hipStream_t s, void* seed_buf);
-size_t gram_f32_seed_screen_bytes(int64_t nq, int64_t nt, int64_t d, int k, int arm, bool vec4);
+// Three launches per assignment (k = 1, ARM_EUCLID_MULADD): prep (the shared
+// per-query bound reset), the Gram kernel, the strip merge + output transform.
+hipError_t launch_gram_f32_prep(const GramArgs32& a, hipStream_t s);
 hipError_t launch_gram_f32(const GramArgs32& a, int arm, hipStream_t s);
 // k = 1 Euclidean searches whose index fits a few workgroups' LDS
 // (knn_k1_resident.hip): the chunk count the launch uses (each chunk one
@@ -178,7 +174,7 @@ int gram_f32_k1_resident_chunks(int64_t nq, int64_t nt, int64_t d, int k, int ar
 hipError_t launch_gram_f32_k1_resident(const GramArgs32& a, int arm, int cus, float* qsq_out, hipStream_t s);
 size_t gram_f32_k1_resident_queue_bytes(int cus);
 hipError_t launch_gram_f32_k1_resident_merge(const GramArgs32& a, int nchunks, hipStream_t s);
-hipError_t launch_gram_f32_merge(const GramArgs32& a, int arm, hipStream_t s);
+hipError_t launch_gram_f32_merge(const GramArgs32& a, hipStream_t s);
 int gram_f32_max_k();
 int gram_f32_max_d();
 // 128 queries per workgroup for d <= 128 (32 per wave), 64 above (16 per wave)
@@ -211,22 +207,16 @@ struct GramArgs64 {
     unsigned long long* shared_r;  // [nq] best known exact k-th value per query (double bits)
     // EMIT_ROOT_RANKED only, else null: [nq], set to 1 where an exact list
     // dropped a pair whose root may equal the k-th root (the merge cannot
-    // then rank that root's ties by index; launch_gram_f64_root_fill does)
+    // then rank that root's ties by index)
     unsigned int* root_flag;
 };
 
 void gram_f64_split(int64_t nq, int64_t nt, int cus, int64_t* grid_wgs, int* nslots);
-// prep: the shared per-query bound, seeded with the k-th exact value over a
-// row sample (arm: the exact arithmetic)
-// seed_buf: gram_f64_seed_screen_bytes(...) bytes when that is nonzero (the
-// seed then runs on the matrix cores), else null.
-hipError_t launch_gram_f64_prep(const GramArgs64& a, int arm, hipStream_t s, void* seed_buf);
-size_t gram_f64_seed_screen_bytes(int64_t nq, int64_t nt, int64_t d, int k, bool vec2);
+// Assignments only (k = 1, ARM_EUCLID_MULADD).  prep: the shared per-query
+// bound, seeded with the smallest exact value over a row sample.
+hipError_t launch_gram_f64_prep(const GramArgs64& a, hipStream_t s);
 hipError_t launch_gram_f64(const GramArgs64& a, int arm, hipStream_t s);
-hipError_t launch_gram_f64_merge(const GramArgs64& a, int arm, hipStream_t s);
-// EMIT_ROOT_RANKED (Euclidean arms): the queries root_flag marks get the
-// rows whose root equals their k-th root in ascending index order
-hipError_t launch_gram_f64_root_fill(const GramArgs64& a, int arm, hipStream_t s);
+hipError_t launch_gram_f64_merge(const GramArgs64& a, hipStream_t s);
 int gram_f64_max_k();
 int gram_f64_max_d();
 
