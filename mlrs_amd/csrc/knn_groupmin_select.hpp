@@ -150,8 +150,11 @@ struct GmList {
         const bool on = mine != kSentinelIdx && v == v;  // NaN is never admitted
         v = on ? v : F::inf();
         uint32_t ix = on ? mine : kSentinelIdx;
-        // a batch with nothing at or below the list's k-th value leaves it as it is
-        if (__builtin_amdgcn_ballot_w64(on && !(kth(k) < v)) == 0ull) return;
+        // a batch with nothing at or below the list's k-th value leaves it as it
+        // is (the k-th value is taken with all lanes: behind `on &&` its lane
+        // need not be running, and a list of two blocks is selected from first)
+        const T last = kth(k);
+        if (__builtin_amdgcn_ballot_w64(on && !(last < v)) == 0ull) return;
         wave_sort64<T>(v, ix, lane);
         merge(v, ix, lane);
     }
@@ -166,7 +169,11 @@ struct GmList {
     }
     // A query every row of which is evaluated: a zero query's values are all
     // exactly 1 (or NaN, never admitted), so the first k rows are its answer.
-    __device__ __forceinline__ bool settled(int k) const { return COS && qzero && kth(k) < F::inf(); }
+    __device__ __forceinline__ bool settled(int k) const {
+        if (!COS) return false;
+        const T last = kth(k);
+        return qzero && last < F::inf();
+    }
     __device__ __forceinline__ void emit(T* __restrict__ ov, uint32_t* __restrict__ oi, int k, int mode, int lane) const {
 #pragma unroll
         for (int b = 0; b < KL; ++b) {

@@ -171,3 +171,23 @@ def test_two_query_blocks(d):
         x[rows] *= np.exp2(rng.integers(-60, 12, 2000)).astype(np.float32)[:, None]
     xt[17] = xt[9000]
     _check(xq, xt, 7)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("metric", ["euclidean", "cosine", "manhattan"])
+@pytest.mark.parametrize("nt,k", [(135, 100), (300, 100), (333, 128), (1300, 70)])
+@pytest.mark.parametrize("d", [5, 50, 140])
+def test_last_batch_of_rows(dtype, metric, nt, k, d):
+    """Lists of two blocks where the last, partly filled batch of 64 rows holds
+    the nearest: for queries that evaluate every row (untrusted themselves, or
+    more untrusted rows than are listed) and for the others."""
+    prims.force_path("auto" if metric == "manhattan" else "fused")
+    rng = np.random.default_rng(nt + k + d)
+    xt, xq = (rng.standard_normal((n, d)) for n in (nt, 64))
+    xt = xt[np.argsort(-((xt - xq[0]) ** 2).sum(1))]
+    xt, xq = np.ascontiguousarray(xt.astype(dtype)), xq.astype(dtype)
+    xq[10:20] *= dtype(1e25)
+    _check(xq, xt, k, metric)
+    far = max(nt // 4, min(nt - k, 300))
+    xt[:far] *= dtype(1e25)
+    _check(xq, xt, k, metric)
