@@ -759,54 +759,77 @@ int32_t noalloc_admits(int64_t nq, int64_t nt, int64_t d, int64_t k, bool vec4, 
                      s, &ws, &cus);
 }
 
+// How a search is cut.  An index whose copy fits is prepared once and searched
+// with one set of queries after another, as many as the budget for the minima
+// holds.  A larger one is cut into parts of rows, each copied, scanned and
+// searched for all queries of a set, the lists waiting in the outputs from part
+// to part; norms and scales are kept for one part only, so that any index fits
+// any scratch.  Every set copies the whole index again, so the parts shrink (a
+// query's minima take 1/4 byte per row) until one set holds all queries, down
+// to kPartRows (against 10,000 queries 55 us of scan beside four launches).
+struct GmPlan {
+    int64_t ldx, dp;       // row widths of the index's and the queries' copies
+    int64_t rows, qc;      // index rows of a part, queries of a set
+    int64_t ntp, qpad;     // the part's tiles, the set's padded queries
+    size_t bytes;
+};
+static GmPlan gm_plan(int64_t nq, int64_t nt, int64_t d) {
+    constexpr int64_t kStore = kGmRows * kGmQuad;  // parts are whole stores of the scan
+    constexpr int64_t kPartRows = 16384;
+    constexpr int64_t kSet = 2 * kGmQpb;
+    GmPlan P;
+    P.ldx = (d + 15) / 16 * 16;
+    P.dp = 8 * (int64_t)gm_chunks(d);
+    const size_t limit = workspace_limit();
+    // copied rows (split elements, bias, scale); a query beside its minima (split
+    // elements, norm, scale)
+    const size_t per_row = sizeof(float) * (size_t)(P.ldx + 2), per_q = sizeof(float) * (size_t)(P.dp + 2);
+    const size_t fixed = sizeof(GmStats) + sizeof(uint32_t) * kGmForced + per_q * kSet + per_row * kStore + 4096;
+    // Without a limit 4 GiB of copied rows hold any index but the largest
+    // whole, and 1 GiB of minima keeps the scan launches long (the tail of one
+    // costs about one unit of the split) and the memory modest.
+    const size_t room = limit == SIZE_MAX ? (size_t)5 << 30 : (limit > fixed ? limit - fixed : 0);
+    const size_t copy = limit == SIZE_MAX ? (size_t)4 << 30 : room / 8 * 3;
+    P.rows = nt;
+    size_t left = (size_t)1 << 30;
+    if (limit != SIZE_MAX) left = std::min(left, room - std::min(room, per_row * (size_t)(gm_tiles(nt) * kGmRows)));
+    if (per_row * (size_t)nt > copy) {
+        const double r = ((double)room - (double)per_q * (double)nq) / ((double)per_row + 0.25 * (double)nq);
+        P.rows = std::min<int64_t>(nt, std::max<int64_t>((int64_t)std::max(r, 0.0) / kStore * kStore, kPartRows));
+        left = room - std::min(room, per_row * (size_t)P.rows);
+    }
+    P.ntp = gm_tiles(P.rows);
+    P.qc = std::max<int64_t>(1, std::min<int64_t>(nq, (int64_t)(left / (2 * sizeof(float) * (size_t)P.ntp + per_q))));
+    if (P.qc < nq && P.qc > kSet) {
+        const int64_t sets = (nq + P.qc / kSet * kSet - 1) / (P.qc / kSet * kSet);
+        P.qc = ((nq + sets - 1) / sets + kSet - 1) / kSet * kSet;
+    }
+    P.qpad = (P.qc + kSet - 1) / kSet * kSet;
+    P.bytes = fixed + per_row * (size_t)(P.ntp * kGmRows) + (2 * sizeof(float) * (size_t)P.ntp + per_q) * (size_t)P.qc;
+    return P;
+}
+
 template <typename T, typename TS>
 int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t d, int k, int arm, int mode,
                      T* out_v, uint32_t* out_i, hipStream_t s) {
     const bool cos = (arm == ARM_COS_FOLD || arm == ARM_COS_HOST);
-    // The scan reads a copy of the index (centred or unit rows, two f16 halves
-    // per element); what does not fit the scratch is copied a part at a time.
-    const int64_t ldx = (d + 15) / 16 * 16;
-    const int64_t dp = 8 * (int64_t)gm_chunks(d);
-    const int64_t ntp = gm_tiles(nt);
-    constexpr int64_t kPart = kGmRows * kGmQuad;  // index parts are whole stores of the scan
-    // Copied rows at a time: 4 GiB holds any index but the largest whole; a
-    // larger one is copied and scanned part by part for each set of queries.
-    const size_t limit = workspace_limit();
-    const size_t fixed = 2 * aligned_bytes(sizeof(float) * (size_t)ntp * kGmRows) + aligned_bytes(sizeof(GmStats)) +
-                         aligned_bytes(sizeof(uint32_t) * kGmForced) + sizeof(float) * (size_t)dp * 2 * kGmQpb + 4096;
-    size_t room = limit == SIZE_MAX ? (size_t)5 << 30 : (limit > fixed ? limit - fixed : 0);
-    const size_t most = limit == SIZE_MAX ? (size_t)4 << 30 : room / 8 * 3;
-    const int64_t fit = (int64_t)(most / (sizeof(float) * (size_t)ldx)) / kPart * kPart;
-    const int64_t xrows = std::min<int64_t>(ntp * kGmRows, std::max<int64_t>(fit, kPart));
-    room -= std::min(room, sizeof(float) * (size_t)(xrows * ldx) + 256);
-    const bool whole = xrows >= nt;
-    // The minima of as many queries as the budget holds: 1 GiB keeps the scan
-    // launches long (the tail of one costs about one unit of the split) and
-    // the memory modest.
-    const size_t per_q = 2 * sizeof(float) * (size_t)ntp + sizeof(float) * (size_t)(dp + 2);
-    int64_t qc = std::max<int64_t>(1, std::min<int64_t>(nq, (int64_t)(std::min(room, (size_t)1 << 30) / per_q)));
-    if (qc < nq && qc > 2 * kGmQpb) {
-        constexpr int64_t kSet = 2 * kGmQpb;
-        const int64_t parts = (nq + qc / kSet * kSet - 1) / (qc / kSet * kSet);
-        qc = ((nq + parts - 1) / parts + kSet - 1) / kSet * kSet;
-    }
-    const int64_t qpad = (qc + 2 * kGmQpb - 1) / (2 * kGmQpb) * (2 * kGmQpb);
+    const GmPlan P = gm_plan(nq, nt, d);
+    const int64_t ldx = P.ldx, dp = P.dp, ntp = P.ntp;
+    const bool whole = P.rows >= nt;
     char* ws;
     int cus;
-    int32_t rc = workspace(fixed + sizeof(float) * (size_t)(xrows * ldx) + 2 * sizeof(float) * (size_t)(ntp * qc) +
-                               sizeof(float) * (size_t)(dp * qc + 2 * qc),
-                           s, &ws, &cus);
+    int32_t rc = workspace(P.bytes, s, &ws, &cus);
     if (rc) return rc;
     Carver cv(ws);
-    float* bias = cv.take<float>((size_t)ntp * kGmRows);
+    float* bias = cv.take<float>((size_t)(ntp * kGmRows));
     GmStats* stats = cv.take<GmStats>(1);
     uint32_t* forced = cv.take<uint32_t>(kGmForced);
-    float* xinv = cv.take<float>((size_t)ntp * kGmRows);
-    float* xcopy = cv.take<float>((size_t)(xrows * ldx));
-    float* qop = cv.take<float>((size_t)(qpad * dp));
-    float* qnorm = cv.take<float>((size_t)qc);
-    float* qinv = cv.take<float>((size_t)qc);
-    float* gmin = cv.take<float>(2 * (size_t)ntp * (size_t)qc);
+    float* xinv = cv.take<float>((size_t)(ntp * kGmRows));
+    float* xcopy = cv.take<float>((size_t)(ntp * kGmRows * ldx));
+    float* qop = cv.take<float>((size_t)(P.qpad * dp));
+    float* qnorm = cv.take<float>((size_t)P.qc);
+    float* qinv = cv.take<float>((size_t)P.qc);
+    float* gmin = cv.take<float>(2 * (size_t)ntp * (size_t)P.qc);
 
     GmPrepArgs pq{};
     pq.d = d;
@@ -823,25 +846,26 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     GmPrepArgs px = pq;
     px.out = xcopy;
     px.ldo = ldx;
+    px.norm = bias;
+    px.inv = xinv;
     px.queries = 0;
 
     GmScanArgs sc{};
     sc.q = qop;
     sc.x = xcopy;
+    sc.bias = bias;
+    sc.xinv = xinv;
     sc.qinv = qinv;
     sc.ldx = ldx;
     sc.d = ldx;
-    sc.ntp = ntp;
+    sc.gmin = gmin;
     sc.grid_wgs = cus;
 
     GmSelectArgs<TS> se{};
-    se.x = xt;
-    se.nt = nt;
     se.d = d;
     se.k = k;
     se.mode = mode;
     se.gmin = gmin;
-    se.ntp = ntp;
     se.bias = bias;
     se.qnorm = qnorm;
     se.stats = stats;
@@ -864,45 +888,46 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     se.eps_rel = cos ? 0.0 : (3.1 * (double)dp + (double)d + 32.0) * u;
     se.eps_abs = cos ? (3.1 * (double)dp + (double)d + 40.0) * u
                      : (double)(d + 16) * std::ldexp(1.0, sizeof(TS) == 8 ? -100 : -120);
-    for (int64_t q0 = 0; q0 < nq; q0 += qc) {
-        const int64_t n = std::min<int64_t>(qc, nq - q0);
+    hipError_t e = hipSuccess;
+    for (int64_t q0 = 0; q0 < nq && e == hipSuccess; q0 += P.qc) {
+        const int64_t n = std::min<int64_t>(P.qc, nq - q0);
         pq.rows = xq + q0 * d;
         pq.n = n;
         pq.n_out = (n + 2 * kGmQpb - 1) / (2 * kGmQpb) * (2 * kGmQpb);
         pq.n_norm = n;
-        pq.reset = q0 == 0 || !whole;
-        hipError_t e = launch_gm_prep<TS>(pq, s);
         sc.nq = n;
-        const int64_t step = whole ? ntp * kGmRows : xrows;
-        for (int64_t x0 = 0; e == hipSuccess && x0 < nt; x0 += step) {
-            const int64_t rows = std::min<int64_t>(step, nt - x0);
-            if (q0 == 0 || !whole) {
-                px.rows = xt + x0 * d;
-                px.row0 = x0;
-                px.n = px.n_out = rows;
-                px.norm = bias + x0;
-                px.inv = xinv + x0;
-                px.n_norm = gm_tiles(rows) * kGmRows;
-                e = launch_gm_prep<TS>(px, s);
-            }
-            sc.bias = bias + x0;
-            sc.xinv = xinv + x0;
-            sc.nt = rows;
-            sc.tiles = gm_tiles(rows);
-            sc.gmin = gmin + x0 / kGmRows;
-            if (e == hipSuccess) {
-                KernelTimer timer(s, "knn_groupmin_kernel");
-                e = launch_gm_scan(sc, s);
-            }
-        }
         se.q = xq + q0 * d;
         se.nq = n;
         se.out_val = out_v + q0 * k;
         se.out_idx = out_i + q0 * k;
-        if (e == hipSuccess) e = launch_gm_select<T, TS>(se, arm, s);
-        if (e != hipSuccess) return hip_err(e, "knn_groupmin");
+        for (int64_t x0 = 0; x0 < nt && e == hipSuccess; x0 += P.rows) {
+            const int64_t rows = std::min<int64_t>(P.rows, nt - x0);
+            const bool prepare = q0 == 0 || !whole;
+            // the queries' launch also clears what the index's counts
+            pq.reset = prepare;
+            e = launch_gm_prep<TS>(pq, s);
+            if (e == hipSuccess && prepare) {
+                px.rows = xt + x0 * d;
+                px.n = px.n_out = rows;
+                px.n_norm = gm_tiles(rows) * kGmRows;
+                e = launch_gm_prep<TS>(px, s);
+            }
+            sc.nt = rows;
+            sc.tiles = sc.ntp = gm_tiles(rows);
+            if (e == hipSuccess) {
+                KernelTimer timer(s, "knn_groupmin_kernel");
+                e = launch_gm_scan(sc, s);
+            }
+            se.x = xt + x0 * d;
+            se.nt = rows;
+            se.ntp = sc.ntp;
+            se.row0 = x0;
+            se.first = x0 == 0;
+            se.last = x0 + rows == nt;
+            if (e == hipSuccess) e = launch_gm_select<T, TS>(se, arm, s);
+        }
     }
-    return ok();
+    return e == hipSuccess ? ok() : hip_err(e, "knn_groupmin");
 }
 
 // The Manhattan, Chebyshev and Minkowski searches: the exact tiles' group
@@ -934,6 +959,7 @@ int32_t knn_groupmin_metric(const T* xq, int64_t nq, const T* xt, int64_t nt, in
     se.mode = mode;
     se.gmin = reinterpret_cast<const float*>(ws);
     se.ntp = ntp;
+    se.first = se.last = 1;
     se.eps_t = std::ldexp(1.0, -21);  // the minima's rounding to f32 (2^-24) on both sides of a comparison, and a root's
     se.pexp = p;
     se.pint = minkowski_powi(p);

@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
             if (keep && !a.cosine) xmax = fmaxf(xmax, (float)s);
             if (force) {
                 const unsigned int at = atomicAdd(&a.stats->nforced, 1u);
-                if (at < (unsigned int)kGmForced) a.forced[at] = (uint32_t)(a.row0 + r);
+                if (at < (unsigned int)kGmForced) a.forced[at] = (uint32_t)r;
             }
         }
     }

@@ -64,8 +64,8 @@ struct GmScanArgs {
     int64_t ldx, d;     // d: columns read per row (<= DP, a multiple of 16)
     int64_t nq, nt;     // queries and index rows of this launch
     int64_t tiles;      // ceil(nt / 32), rounded up to kGmQuad
-    int64_t ntp;        // tiles of the whole index: stride of gmin
-    float* gmin;        // [nq][2][ntp]: minima of group (tile, half), from this launch's first tile
+    int64_t ntp;        // the same: stride of gmin
+    float* gmin;        // [nq][2][ntp]: minima of group (tile, half)
     int64_t grid_wgs;   // launch: the CU count; kernel: workgroups of one resident round
 };
 
@@ -93,7 +93,6 @@ struct GmPrepArgs {
     int64_t n, d;
     const void* centre;  // Euclidean copies: the index, whose first, middle and last rows give the centre
     int64_t centre_n;
-    int64_t row0;        // index: number of the first row here (the forced list holds row numbers)
     float* out;          // the split copy, row stride ldo (a multiple of 16; zeros past d)
     int64_t ldo;
     int64_t n_out;       // rows of out (zeros past n)
@@ -114,8 +113,10 @@ hipError_t launch_gm_scan(const GmScanArgs& a, hipStream_t s);
 template <typename TS>
 struct GmSelectArgs {
     const TS* q;         // [nq][d] queries as given
-    const TS* x;         // [nt][d] index rows as given
+    const TS* x;         // [nt][d] index rows of this part, as given
     int64_t nq, nt, d;
+    int64_t row0;        // the part's first row in the index
+    int first, last;     // the index's first / last part: between them the lists wait in the outputs, untransformed
     int k, mode;
     const float* gmin;   // [nq][2][ntp]
     int64_t ntp;

@@ -109,12 +109,14 @@ struct GmList {
     static constexpr bool COS = ARM == ARM_COS_FOLD || ARM == ARM_COS_HOST;
     static constexpr bool MINK = ARM == ARM_MINKOWSKI_INT || ARM == ARM_MINKOWSKI_POW;
     T lv[KL];
-    uint32_t li[KL];
+    uint32_t li[KL];      // rows of the whole index
+    uint32_t row0;
     T qa = T(0);  // cosine: the query's row_sumsq (fold) or its reciprocal norm (host)
     bool qzero = false;
     MetricParams<T> mp;
 
-    __device__ __forceinline__ GmList(const GmSelectArgs<TS>& a) : mp{(T)a.pexp, a.pint, (T)a.root_exp} {
+    __device__ __forceinline__ GmList(const GmSelectArgs<TS>& a)
+        : row0((uint32_t)a.row0), mp{(T)a.pexp, a.pint, (T)a.root_exp} {
 #pragma unroll
         for (int b = 0; b < KL; ++b) {
             lv[b] = F::inf();
@@ -132,7 +134,18 @@ struct GmList {
         if constexpr (KL == 1) wave_merge64<T>(lv[0], li[0], v, ix, lane);
         else wave_merge_blocks<T, KL>(lv, li, v, ix, lane);
     }
-    // 64 rows (kSentinelIdx: none) evaluated exactly and merged in
+    // The list the parts before this one left in the outputs.
+    __device__ __forceinline__ void resume(const T* __restrict__ ov, const uint32_t* __restrict__ oi, int k, int lane) {
+#pragma unroll
+        for (int b = 0; b < KL; ++b) {
+            const int s = 64 * b + lane;
+            if (s < k) {
+                lv[b] = ov[s];
+                li[b] = oi[s];
+            }
+        }
+    }
+    // 64 rows of the part (kSentinelIdx: none) evaluated exactly and merged in
     __device__ __forceinline__ void evaluate(uint32_t mine, const T* __restrict__ sq, const TS* __restrict__ X, int d,
                                              int k, int mode, int lane) {
         if (__builtin_amdgcn_ballot_w64(mine != kSentinelIdx) == 0ull) return;
@@ -149,7 +162,7 @@ struct GmList {
         if (mode == EMIT_ROOT_RANKED) v = MINK ? F::pow_(v, mp.root) : F::sqrt_(v);
         const bool on = mine != kSentinelIdx && v == v;  // NaN is never admitted
         v = on ? v : F::inf();
-        uint32_t ix = on ? mine : kSentinelIdx;
+        uint32_t ix = on ? row0 + mine : kSentinelIdx;
         // a batch with nothing at or below the list's k-th value leaves it as it
         // is (the k-th value is taken with all lanes: behind `on &&` its lane
         // need not be running, and a list of two blocks is selected from first)
@@ -174,13 +187,14 @@ struct GmList {
         const T last = kth(k);
         return qzero && last < F::inf();
     }
-    __device__ __forceinline__ void emit(T* __restrict__ ov, uint32_t* __restrict__ oi, int k, int mode, int lane) const {
+    __device__ __forceinline__ void emit(T* __restrict__ ov, uint32_t* __restrict__ oi, int k, int mode, int last,
+                                         int lane) const {
 #pragma unroll
         for (int b = 0; b < KL; ++b) {
             const int s = 64 * b + lane;
             if (s < k) {
-                ov[s] = mode == EMIT_SQRT ? F::sqrt_(lv[b]) : lv[b];
-                oi[s] = li[b] == kSentinelIdx ? 0u : li[b];
+                ov[s] = last && mode == EMIT_SQRT ? F::sqrt_(lv[b]) : lv[b];
+                oi[s] = last && li[b] == kSentinelIdx ? 0u : li[b];
             }
         }
     }
@@ -253,6 +267,15 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
     const GmQuery<TS> Q(a, q);
     const int n = Q.n;
     GmList<T, TS, ARM, KL> L(a);
+    T* const ov = static_cast<T*>(a.out_val) + q * k;
+    uint32_t* const oi = a.out_idx + q * k;
+    // earlier parts' list: wave 0 goes on with it, and its k-th value bounds all
+    float carried = inf;
+    if (!a.first) {
+        L.resume(ov, oi, k, lane);
+        carried = L.screen_bound(k, mode, Q.qn, Q.eps, Q.eps_t);
+        if (wv > 0) L = GmList<T, TS, ARM, KL>(a);
+    }
     if (tid < d) sq[tid] = (T)a.q[q * d + tid];
     if (tid == 0) {
         s_cnt = 0u;
@@ -307,7 +330,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
         };
         if (rank_of(m, tid, 256) == k - 1) s_kth = m;
         __syncthreads();
-        float thr = Q.bound(s_kth);
+        float thr = fminf(Q.bound(s_kth), carried);
         // ---- the groups at or below it ----
         for (int i = 4 * tid; i < n; i += 4096) {
             if (!held) load_minima(i);
@@ -342,7 +365,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
                     if (at < count && rank_of(v[j], at, count) == k - 1) s_kth = v[j];
                 }
                 __syncthreads();
-                thr = Q.bound(s_kth);
+                thr = fminf(Q.bound(s_kth), carried);
                 if (tid == 0) s_cnt = 0u;
                 __syncthreads();
 #pragma unroll
@@ -388,7 +411,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
     if (wv > 0) return;
 #pragma unroll
     for (int b = 0; b < 3 * KL; ++b) L.merge(mv[64 * b + lane], mi[64 * b + lane], lane);
-    L.emit(static_cast<T*>(a.out_val) + q * k, a.out_idx + q * k, k, mode, lane);
+    L.emit(ov, oi, k, mode, a.last, lane);
 }
 
 // A wave per query: many queries.  No barrier, no atomic: the bound is the
@@ -414,6 +437,13 @@ __global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS>
     const GmQuery<TS> Q(a, q);
     const int n = Q.n;
     GmList<T, TS, ARM, KL> L(a);
+    T* const ov = static_cast<T*>(a.out_val) + q * k;
+    uint32_t* const oi = a.out_idx + q * k;
+    float carried = inf;  // what the earlier parts' list bounds
+    if (!a.first) {
+        L.resume(ov, oi, k, lane);
+        carried = L.screen_bound(k, mode, Q.qn, Q.eps, Q.eps_t);
+    }
     for (int c = lane; c < d; c += 64) sq[c] = (T)a.q[q * d + c];
     wave_lds_fence();
     L.set_query(sq, d);
@@ -423,7 +453,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS>
             L.evaluate(r0 + lane < Q.nt ? r0 + lane : kSentinelIdx, sq, X, d, k, mode, lane);
             if (L.settled(k)) break;
         }
-        L.emit(static_cast<T*>(a.out_val) + q * k, a.out_idx + q * k, k, mode, lane);
+        L.emit(ov, oi, k, mode, a.last, lane);
         return;
     }
     for (uint32_t f0 = 0; f0 < Q.nforced; f0 += 64)
@@ -470,7 +500,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS>
             else wave_merge_blocks<float, KL>(bv, bi, m2, i2, lane);
         }
     }
-    float thr = Q.bound(list_value_at<float, KL>(bv, k - 1));
+    float thr = fminf(Q.bound(list_value_at<float, KL>(bv, k - 1)), carried);
 
     // ---- the groups at or below it ----
     uint32_t cnt = 0;
@@ -510,7 +540,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS>
                 if constexpr (KL == 1) wave_merge64<float>(bv[0], bi[0], v, ix, lane);
                 else wave_merge_blocks<float, KL>(bv, bi, v, ix, lane);
             }
-            thr = Q.bound(list_value_at<float, KL>(bv, k - 1));
+            thr = fminf(Q.bound(list_value_at<float, KL>(bv, k - 1)), carried);
             uint32_t kept = 0;
             for (uint32_t b0 = 0; b0 < cnt; b0 += 64) {
                 const bool in = b0 + lane < cnt && cm[b0 + lane] <= thr;
@@ -547,7 +577,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS>
             }
         }
     }
-    L.emit(static_cast<T*>(a.out_val) + q * k, a.out_idx + q * k, k, mode, lane);
+    L.emit(ov, oi, k, mode, a.last, lane);
 }
 
 template <typename T, typename TS, int ARM, int KL>

@@ -1,0 +1,74 @@
+"""The group-minimum search where it works under limits: an index searched in
+parts, several sets of queries, and what either may cost.  Bits are compared
+with the call that has no limit (held to the CPU oracle elsewhere); times with
+one another on the same box, with room for noise."""
+import ctypes
+
+import pytest
+import torch
+
+from mlrs_amd import _lib, prims
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _rows(seed, n, d, dtype=torch.float32):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn((n, d), generator=g, device=DEV, dtype=dtype)
+
+
+def _search(name, xq, xt, k, metric=0):
+    nq, d = xq.shape
+    dist = torch.empty((nq, k), dtype=xq.dtype, device=DEV)
+    idx = torch.empty((nq, k), dtype=torch.int32, device=DEV)
+
+    def call():
+        _lib.check(getattr(_lib.load(), name)(
+            xq.data_ptr(), xq.numel(), nq, d, xt.data_ptr(), xt.numel(), xt.shape[0], k, metric, ctypes.c_double(2.0),
+            dist.data_ptr(), idx.data_ptr(), dist.numel(), torch.cuda.current_stream(DEV).cuda_stream))
+        return dist, idx
+    return call
+
+
+def _ms(call, reps=3):
+    """The fastest of a few passes after one to warm up."""
+    call()
+    best = float("inf")
+    for _ in range(reps):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        call()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+# two parts; four; two sets of queries by sixteen parts
+@pytest.mark.parametrize("nt,nq,d,k", [(600_000, 300, 50, 12), (600_000, 2_500, 50, 12), (250_000, 40_000, 50, 5),
+                                       (600_000, 60, 50, 100), (400_000, 1_000, 96, 40)])
+@pytest.mark.parametrize("metric", [0, 1])
+def test_parts_and_sets(nt, nq, d, k, metric):
+    xt, xq = _rows(nt + d, nt, d), _rows(nq, nq, d)
+    xt[nt - 3] = xt[1]  # ties between the first part and the last
+    xt[nt // 2] = xt[1]
+    for r in (0, nt // 2 + 1, nt - 5):  # rows for the forced list, in several parts
+        xt[r] *= 1e25
+    xt[7, 0] = float("nan")
+    xq[0] = xq[nq - 1] = xt[1]
+    xq[1] = xq[nq - 2] = 0.0
+    xq[2] *= 1e25  # every row is evaluated for these
+    xq[nq - 3, 0] = float("nan")
+    free, bound = (_search(n, xq, xt, k, metric)() for n in ("mlrs_knn_topk_f32", "mlrs_knn_topk_f32_noalloc"))
+    torch.cuda.synchronize()
+    assert torch.equal(free[1], bound[1])
+    assert torch.equal(free[0].view(torch.int32), bound[0].view(torch.int32))
+
+
+def test_a_limit_on_the_scratch_costs_no_multiple():
+    """1M rows against 10,000 queries in 128 MiB: the index is copied once, not
+    once per few hundred queries."""
+    xt, xq = _rows(1, 1_000_000, 128), _rows(2, 10_000, 128)
+    free, bound = (_ms(_search(n, xq, xt, 32)) for n in ("mlrs_knn_topk_f32", "mlrs_knn_topk_f32_noalloc"))
+    assert bound < 2.2 * free, (bound, free)
