@@ -123,7 +123,7 @@ int32_t mlrs_knn_max_k(int32_t dtype_bytes, int64_t n_features, int32_t metric);
  * under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  Same arguments, validation,
  * kernels and bits as mlrs_knn_topk_f32; the only difference is where the
- * kernels' scratch (norms, per-segment lists, queued screen values, exact
+ * kernels' scratch (the copied operands, norms, group minima, lists, exact
  * tiles) lives: in a static device array of MLRS_NOALLOC_SCRATCH_BYTES per
  * GPU, held until the process ends, instead of the library's cached
  * workspace.  The call makes no hipMalloc / hipFree / allocating library
@@ -131,12 +131,16 @@ int32_t mlrs_knn_max_k(int32_t dtype_bytes, int64_t n_features, int32_t metric);
  * (hipGetSymbolAddress) and the CU count up once: make that first call, which
  * may have n_query = 0, outside a graph capture.  After it, calls can be
  * captured into a HIP graph (every step is a kernel launch: no memset, no
- * copy, no event) and replayed with new data in the same buffers.  A search
- * whose scratch would exceed the array
- * returns MLRS_ERR_UNSUPPORTED, operand "scratch" {rows = bytes needed,
- * len = MLRS_NOALLOC_SCRATCH_BYTES}, before any launch (the exact-tile path
- * sizes its tiles to fit; the Gram path at n_train = 1M, d = 128, k = 32
- * needs ~64 MiB for 10k queries).  Every call on a GPU shares that GPU's
+ * copy, no event) and replayed with new data in the same buffers.  The
+ * searches for d <= 256 and k <= 128 cut the index and the queries to fit the
+ * array; what cannot be cut (the low-d kernel's lists, a row of the exact
+ * tiles for every query) and exceeds it, and searches of more than 2^32
+ * n_query * n_train * n_features whose d or k is past the low-d kernel's range
+ * and for which 12 bytes per row, a list per query and index segment and
+ * their queues would exceed it (about 100,000 queries at n_train = 1M, d =
+ * 128, k = 32), return MLRS_ERR_UNSUPPORTED, operand "scratch" {rows = bytes
+ * needed, len = MLRS_NOALLOC_SCRATCH_BYTES}, before any launch.  Every call on
+ * a GPU shares that GPU's
  * array: calls that overlap on one GPU (two streams, no ordering between
  * them) RACE -- order them yourself.  Not ordered against the other entry
  * points' calls (they use other memory), and no timing events are recorded.

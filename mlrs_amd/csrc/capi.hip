@@ -736,11 +736,12 @@ static bool groupmin_serves(int arm, int64_t d, int64_t k) {
            d <= kGmMaxD && k <= kGmMaxK;
 }
 
-// The allocation-free entry point's limit.  A search this large was always
-// planned with per-segment lists and queues (the k = 1 kernel's split), and
-// callers size their calls by the limit that follows from them, so it stays:
-// the group-minimum search itself fits any scratch by taking fewer queries at
-// a time.
+// The allocation-free entry point's limit where it always was one of lists and
+// queues: searches past small_search's size with more columns or neighbours
+// than the low-d kernel was given are refused by the scratch that per-segment
+// lists, their queues and three norms a row would take.  Callers size their
+// calls by it, so it stays for these; the search itself fits any scratch
+// (gm_plan), and no other call is bound by it.
 int32_t noalloc_admits(int64_t nq, int64_t nt, int64_t d, int64_t k, bool vec4, hipStream_t s) {
     char* ws;
     int cus;
@@ -1144,7 +1145,9 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
         // k = 1 over an index that fits a few workgroups' LDS: resident there
         if ((forced || !small) && gram_f32_k1_resident_chunks(n_query, n_train, n_features, k, arm, vec4) > 0)
             return knn_gram32(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
-        if (g_noalloc && (forced || !small)) {
+        const bool few_columns = lowd_ok && (k <= 8 || (k <= 16 && n_features <= 11) ||
+                                             (n_features <= 3 && metric == MLRS_METRIC_EUCLIDEAN));
+        if (g_noalloc && (forced || !(small || few_columns))) {
             const int32_t rc = noalloc_admits(n_query, n_train, n_features, k, vec4, s);
             if (rc) return rc;
         }

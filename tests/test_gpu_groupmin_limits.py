@@ -72,3 +72,18 @@ def test_a_limit_on_the_scratch_costs_no_multiple():
     xt, xq = _rows(1, 1_000_000, 128), _rows(2, 10_000, 128)
     free, bound = (_ms(_search(n, xq, xt, 32)) for n in ("mlrs_knn_topk_f32", "mlrs_knn_topk_f32_noalloc"))
     assert bound < 2.2 * free, (bound, free)
+
+
+@pytest.mark.parametrize("nt,nq,d,k,metric", [(5_000_000, 1_000, 3, 8, 0), (5_000_000, 4_000, 3, 8, 0),
+                                              (8_000_000, 3_000, 2, 5, 0), (4_000_000, 2_000, 11, 16, 1),
+                                              (20_000_000, 64, 3, 8, 0)])
+def test_few_columns_against_long_indexes_fit(nt, nq, d, k, metric):
+    """Searches the allocation-free entry point always took: few columns, few
+    thousand queries, millions of rows."""
+    xt, xq = _rows(nt + d, nt, d), _rows(nq, nq, d)
+    xt[nt - 3] = xt[1]
+    xq[0] = xt[1]
+    free, bound = (_search(n, xq, xt, k, metric)() for n in ("mlrs_knn_topk_f32", "mlrs_knn_topk_f32_noalloc"))
+    torch.cuda.synchronize()
+    assert torch.equal(free[1], bound[1])
+    assert torch.equal(free[0].view(torch.int32), bound[0].view(torch.int32))
