@@ -851,6 +851,26 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     px.inv = xinv;
     px.queries = 0;
 
+    // |screen - exact| <= eps_rel N + eps_abs, with u = 2^-23 and N = ||q||^2 + ||x||^2.
+    // Euclidean: the contraction's 3 dp additions round partial sums of 2 x.q,
+    // which stay below 1.01 N, in any rounding mode of the matrix core: 3.1 dp
+    // u N.  The halves: each element is kept to 2^-22 of itself, and lo times
+    // lo is left out, 3 * 2^-22 * 2 ||q|| ||x|| <= 6 u N; halves below f16's
+    // normal range, if flushed, lose 2^-27.5 of the row's norm per half, times
+    // sqrt(d) <= 16 over the row: 6 u N for both operands.  The sum with the
+    // norm 2 u N; the arms' d + 2 roundings to nearest of a value up to 2 N:
+    // (d + 2) u N; the norms (sums of four, then a tree): 6 u N; the copy's
+    // rounding moves a distance by at most 2^-24 (||q|| + ||x||), its square by
+    // 2.02 u N; the bias lowered by its share of the error, one more rounding
+    // and multiplication, 2 u N.  Cosine, of unit vectors (N = 1 for 2 x.q <= N): 3.1 dp u / 2
+    // and the same allowances, the arms' dot product and norms (d + 3) u, the
+    // unit rows' own rounding 12 u.  The absolute term covers flushed
+    // subnormals and rows below 2^-50, which share a scale.
+    const double u = std::ldexp(1.0, -23);
+    const double eps_rel = cos ? 0.0 : (3.1 * (double)dp + (double)d + 32.0) * u;
+    const double eps_abs = cos ? (3.1 * (double)dp + (double)d + 40.0) * u
+                               : (double)(d + 16) * std::ldexp(1.0, sizeof(TS) == 8 ? -100 : -120);
+    px.eps_rel = (float)eps_rel;
     GmScanArgs sc{};
     sc.q = qop;
     sc.x = xcopy;
@@ -871,24 +891,8 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     se.qnorm = qnorm;
     se.stats = stats;
     se.forced = forced;
-    // |screen - exact| <= eps, with u = 2^-23 and N = ||q||^2 + ||x||^2.
-    // Euclidean: the contraction's 3 dp additions round partial sums of 2 x.q,
-    // which stay below 1.01 N, in any rounding mode of the matrix core: 3.1 dp
-    // u N.  The halves: each element is kept to 2^-22 of itself, and lo times
-    // lo is left out, 3 * 2^-22 * 2 ||q|| ||x|| <= 6 u N; halves below f16's
-    // normal range, if flushed, lose 2^-27.5 of the row's norm per half, times
-    // sqrt(d) <= 16 over the row: 6 u N for both operands.  The sum with the
-    // norm 2 u N; the arms' d + 2 roundings to nearest of a value up to 2 N:
-    // (d + 2) u N; the norms (sums of four, then a tree): 6 u N; the copy's
-    // rounding moves a distance by at most 2^-24 (||q|| + ||x||), its square by
-    // 2.02 u N.  Cosine, of unit vectors (N = 1 for 2 x.q <= N): 3.1 dp u / 2
-    // and the same allowances, the arms' dot product and norms (d + 3) u, the
-    // unit rows' own rounding 12 u.  The absolute term covers flushed
-    // subnormals and rows below 2^-50, which share a scale.
-    const double u = std::ldexp(1.0, -23);
-    se.eps_rel = cos ? 0.0 : (3.1 * (double)dp + (double)d + 32.0) * u;
-    se.eps_abs = cos ? (3.1 * (double)dp + (double)d + 40.0) * u
-                     : (double)(d + 16) * std::ldexp(1.0, sizeof(TS) == 8 ? -100 : -120);
+    se.eps_rel = eps_rel;
+    se.eps_abs = eps_abs;
     hipError_t e = hipSuccess;
     for (int64_t q0 = 0; q0 < nq && e == hipSuccess; q0 += P.qc) {
         const int64_t n = std::min<int64_t>(P.qc, nq - q0);

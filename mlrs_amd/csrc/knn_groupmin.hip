@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
             // Euclidean: a row with a NaN scores NaN against every query and
             // is never admitted; cosine's fold arm scores it 1
             const bool force = on && !trusted && (a.cosine || s == s);
-            a.norm[r] = keep ? (a.cosine ? 0.0f : (float)s) : inf;
+            a.norm[r] = keep ? (a.cosine ? 0.0f : (float)s - a.eps_rel * (float)s) : inf;
             if (keep && !a.cosine) xmax = fmaxf(xmax, (float)s);
             if (force) {
                 const unsigned int at = atomicAdd(&a.stats->nforced, 1u);

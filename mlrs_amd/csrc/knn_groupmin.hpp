@@ -6,8 +6,8 @@
 //          16 index rows is written: 4 bytes for 16 pairs.
 //  select  (knn_groupmin.hip) per query: T, the k-th smallest group minimum,
 //          bounds the k-th screen value (k groups hold k distinct rows at or
-//          below it), so with |screen - exact| <= eps every row of the answer
-//          lies in a group whose minimum is at most T + 2 eps.  The rows of
+//          below it), so with the screen's error bounded (gm_bound) every row
+//          of the answer lies in a group whose minimum is not far above T.  The rows of
 //          those groups (about k of them) are evaluated exactly, in the
 //          reference arm's operation order, and ranked by (value, index).
 //
@@ -58,7 +58,7 @@ struct GmScanArgs {
     // last eight, then the low halves: 64 bytes, counted as 16 floats.
     const float* q;     // [queries, rounded up to the launch's 128 or 256][DP] query operand: -q or -q / ||q||, scaled and split; zeros past nq
     const float* x;     // index rows, scaled and split, row stride ldx (a multiple of 16)
-    const float* bias;  // [tiles * 32] Euclidean ||x||^2, cosine 0; +inf for rows left out
+    const float* bias;  // [tiles * 32] Euclidean ||x||^2 less its share of the error, cosine 0; +inf for rows left out
     const float* xinv;  // [tiles * 32] what undoes the row's scale
     const float* qinv;  // [nq] the same for the queries, times 2 (Euclidean)
     int64_t ldx, d;     // d: columns read per row (<= DP, a multiple of 16)
@@ -101,6 +101,7 @@ struct GmPrepArgs {
     int64_t n_norm;      // entries of norm and inv (index: ntp * 32, +inf past n; queries: n)
     int queries;         // 1: query operand; 0: index rows
     int cosine;
+    float eps_rel;       // index: the share of ||x||^2 the bias is lowered by
     GmStats* stats;      // filled from the index rows
     int reset;           // zero stats (the launch before the index's)
     uint32_t* forced;    // [kGmForced]
@@ -124,7 +125,7 @@ struct GmSelectArgs {
     const float* qnorm;  // [nq], NaN: evaluate every row
     const GmStats* stats;  // null: the minima are of the arm's own values (launch_groupmin_tile), no row is left out
     const uint32_t* forced;
-    double eps_rel, eps_abs;  // eps = eps_rel (||q||^2 + max ||x||^2) + eps_abs
+    double eps_rel, eps_abs;  // |screen - exact| <= eps_rel (||q||^2 + ||x||^2) + eps_abs (gm_bound)
     double eps_t;        // relative error of a minimum (values rounded to f32)
     double pexp, root_exp;  // Minkowski: the exponent and (EMIT_ROOT_RANKED) its root's
     int pint;               // its integer exponent

@@ -102,6 +102,29 @@ __device__ __forceinline__ T gm_exact(const T* __restrict__ sq, const TS* __rest
     return acc;
 }
 
+// The largest minimum a group with a row of the answer can have, from the k-th
+// smallest minimum t.  A pair's screen value and exact value (less ||q||^2)
+// differ by at most e (||q||^2 + ||x||^2) + e_abs, e = eps_rel.  The bias is
+// lowered by e ||x||^2, so a minimum m is at most its row's exact value plus
+// eq = e ||q||^2 + e_abs, and the exact value is at most m + eq + 2 e ||x||^2.
+// That norm is at most the index's largest, xmax, and, since the row is near,
+// at most (||q|| + its distance)^2: one outlier in the index does not widen the
+// bound of the others (200k x 5k, d = 128, k = 16, f64, one row a thousand times
+// the others' norm: 109 ms with xmax alone, 0.97 with both, as without the row).
+// Two estimates of the distance's square D (the exact value's rounding is below
+// 2^-12 of it): from ||x||^2 <= 2 (||q||^2 + D) follows D <= (||q||^2 + t + eq +
+// 4.01 e ||q||^2) / (1 - 4.01 e), which then gives the norm.
+__device__ __forceinline__ float gm_bound(float t, float qn, float xmax, double e, float eq) {
+    if (!(t < __builtin_huge_valf())) return __builtin_huge_valf();
+    double b = (double)t + 2.0 * (double)eq;
+    if (e != 0.0) {
+        const double D = fmax(((double)t + (double)qn + (double)eq + 4.01 * e * (double)qn) * (1.0 + 4.1 * e), 0.0);
+        const float r = __builtin_sqrtf(qn) + __builtin_sqrtf((float)D);
+        b += 2.0 * e * (double)fminf(xmax, 1.002f * r * r);
+    }
+    return round_up_f(b);
+}
+
 // A wave's answer so far: the 64 KL smallest (value, row) pairs it has seen.
 template <typename T, typename TS, int ARM, int KL>
 struct GmList {
@@ -173,11 +196,11 @@ struct GmList {
     }
     // A screen value no row of the answer exceeds, from the k-th exact value:
     // exact <= R means screen <= R in screen units + eps.
-    __device__ __forceinline__ float screen_bound(int k, int mode, float qn, double eps, double eps_t) const {
+    __device__ __forceinline__ float screen_bound(int k, int mode, float qn, float eps, double eps_t) const {
         if (MINK && mode == EMIT_ROOT_RANKED) return __builtin_huge_valf();
         double R = (double)kth(k);
         if (mode == EMIT_ROOT_RANKED) R = R * R * (1.0 + 0x1p-40);
-        return R < (double)__builtin_huge_valf() ? round_up_f(R - (COS ? 1.0 : (double)qn) + eps + eps_t * R)
+        return R < (double)__builtin_huge_valf() ? round_up_f(R - (COS ? 1.0 : (double)qn) + (double)eps + eps_t * R)
                                                  : __builtin_huge_valf();
     }
     // A query every row of which is evaluated: a zero query's values are all
@@ -209,24 +232,26 @@ struct GmQuery {
     float qn;
     uint32_t nforced;
     bool all_rows;
-    double eps, eps_t;
+    float eps;      // the part of the error that does not depend on the row
+    float xmax;
+    const GmSelectArgs<TS>& a;
     const float* bias;
-    __device__ __forceinline__ GmQuery(const GmSelectArgs<TS>& a, int64_t q) {
+    __device__ __forceinline__ GmQuery(const GmSelectArgs<TS>& args, int64_t q) : a(args) {
         G = a.gmin + q * 2 * a.ntp;
         ntp = (int)a.ntp;
         n = 2 * ntp;  // a multiple of 8
         nt = (uint32_t)a.nt;
-        eps_t = a.eps_t;
         if (!a.stats) {  // minima of the arm's own values
             qn = 0.0f;
             nforced = 0u;
             all_rows = false;
-            eps = 0.0;
+            eps = xmax = 0.0f;
         } else {
             qn = a.qnorm[q];
             nforced = a.stats->nforced;
             all_rows = !(qn == qn) || nforced > (uint32_t)kGmForced;
-            eps = a.eps_rel * ((double)qn + (double)__uint_as_float(a.stats->xmax_bits)) + a.eps_abs;
+            xmax = __uint_as_float(a.stats->xmax_bits);
+            eps = round_up_f(a.eps_rel * (double)qn + a.eps_abs);
         }
         bias = a.bias;
     }
@@ -242,7 +267,9 @@ struct GmQuery {
     }
     // every row of the answer lies in a group whose minimum is at or below this
     __device__ __forceinline__ float bound(float t) const {
-        return t < __builtin_huge_valf() ? round_up_f((double)t + 2.0 * eps + eps_t * (double)t) : __builtin_huge_valf();
+        if (!a.stats)
+            return t < __builtin_huge_valf() ? round_up_f((double)t + a.eps_t * (double)t) : __builtin_huge_valf();
+        return gm_bound(t, qn, xmax, a.eps_rel, eps);
     }
 };
 
@@ -273,7 +300,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
     float carried = inf;
     if (!a.first) {
         L.resume(ov, oi, k, lane);
-        carried = L.screen_bound(k, mode, Q.qn, Q.eps, Q.eps_t);
+        carried = L.screen_bound(k, mode, Q.qn, Q.eps, a.eps_t);
         if (wv > 0) L = GmList<T, TS, ARM, KL>(a);
     }
     if (tid < d) sq[tid] = (T)a.q[q * d + tid];
@@ -388,7 +415,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
                 const uint32_t mine = (gm <= thr && gm < inf) ? Q.row(f, tid & 15) : kSentinelIdx;
                 if (!__syncthreads_or(mine != kSentinelIdx)) continue;
                 L.evaluate(mine, sq, X, d, k, mode, lane);
-                const float t = L.screen_bound(k, mode, Q.qn, Q.eps, Q.eps_t);
+                const float t = L.screen_bound(k, mode, Q.qn, Q.eps, a.eps_t);
                 if (lane == 0) s_wthr[wv] = t;
                 __syncthreads();
 #pragma unroll
@@ -418,8 +445,13 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
 // k-th smallest of the lanes' two smallest minima, the groups below it are
 // compacted with ballots, and the wave's own list is the answer.
 constexpr int kSelWaveCap = 256;
+// Five waves per SIMD where the arm's state fits 96 registers (200k x 5k, d = 256,
+// k = 16, f64 cosine: 1.90 ms with 102 registers, 1.84 with 96).
+constexpr int gm_select_waves(int arm, int kl) {
+    return kl == 1 && arm != ARM_COS_FOLD && arm != ARM_MINKOWSKI_INT && arm != ARM_MINKOWSKI_POW ? 5 : 4;
+}
 template <typename T, typename TS, int ARM, int KL>
-__global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS> a) {
+__global__ __launch_bounds__(256, gm_select_waves(ARM, KL)) void gm_select_wave_kernel(GmSelectArgs<TS> a) {
     __shared__ __attribute__((aligned(16))) T sq_[4][kGmMaxD];
     __shared__ float cm_[4][kSelWaveCap];
     __shared__ uint32_t cg_[4][kSelWaveCap];
@@ -442,7 +474,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS>
     float carried = inf;  // what the earlier parts' list bounds
     if (!a.first) {
         L.resume(ov, oi, k, lane);
-        carried = L.screen_bound(k, mode, Q.qn, Q.eps, Q.eps_t);
+        carried = L.screen_bound(k, mode, Q.qn, Q.eps, a.eps_t);
     }
     for (int c = lane; c < d; c += 64) sq[c] = (T)a.q[q * d + c];
     wave_lds_fence();
@@ -572,7 +604,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_wave_kernel(GmSelectArgs<TS>
                     todo &= todo - 1;  // 0 stays 0
                 }
                 L.evaluate(f >= 0 ? Q.row(f0 + f, lane & 15) : kSentinelIdx, sq, X, d, k, mode, lane);
-                thr = fminf(thr, L.screen_bound(k, mode, Q.qn, Q.eps, Q.eps_t));
+                thr = fminf(thr, L.screen_bound(k, mode, Q.qn, Q.eps, a.eps_t));
                 todo &= __builtin_amdgcn_ballot_w64(gm <= thr);
             }
         }

@@ -191,3 +191,17 @@ def test_last_batch_of_rows(dtype, metric, nt, k, d):
     far = max(nt // 4, min(nt - k, 300))
     xt[:far] *= dtype(1e25)
     _check(xq, xt, k, metric)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("nq", [40, 1000])
+@pytest.mark.parametrize("scale", [30.0, 1e3, 1e8])
+def test_outliers(dtype, nq, scale):
+    """Rows and queries far from the rest, near one another among them."""
+    xt, xq = _rows(5, 3000, 20, dtype), _rows(6, nq, 20, dtype)
+    xt[100:130] *= dtype(scale)
+    xt[200:240] += dtype(scale)
+    xq[:30] = xt[100:130] + dtype(0.5) * xq[:30]
+    xq[30:38] = xt[200:208]
+    _check(xq, xt, 20)
+    _check(xq, np.ascontiguousarray(xt[90:260]), 100)

@@ -87,3 +87,14 @@ def test_few_columns_against_long_indexes_fit(nt, nq, d, k, metric):
     torch.cuda.synchronize()
     assert torch.equal(free[1], bound[1])
     assert torch.equal(free[0].view(torch.int32), bound[0].view(torch.int32))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_an_outlier_costs_the_others_nothing(dtype):
+    """The error bound of a pair follows its own norms: one far row does not
+    make every query evaluate the index."""
+    xt, xq = _rows(3, 100_000, 64, dtype), _rows(4, 2_000, 64, dtype)
+    name = "mlrs_knn_topk_" + ("f32" if dtype is torch.float32 else "f64")
+    plain = _ms(_search(name, xq, xt, 10))
+    xt[777] *= 1e4
+    assert _ms(_search(name, xq, xt, 10)) < 3.0 * plain
