@@ -888,6 +888,7 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     se.mode = mode;
     se.gmin = gmin;
     se.bias = bias;
+    se.xinv = xinv;
     se.qnorm = qnorm;
     se.stats = stats;
     se.forced = forced;

@@ -145,15 +145,15 @@ __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
             }
             if (sub != 0 || r >= a.n_norm) continue;
             const float nan = __builtin_nanf(""), inf = __builtin_huge_valf();
-            a.inv[r] = __builtin_ldexpf(1.0f, (a.queries && !a.cosine ? 1 : 0) - ex);
+            // Euclidean: a row with a NaN scores NaN against every query and
+            // is never admitted; cosine's fold arm scores it 1
+            const bool force = on && !trusted && !a.queries && (a.cosine || s == s);
+            a.inv[r] = force ? -1.0f : __builtin_ldexpf(1.0f, (a.queries && !a.cosine ? 1 : 0) - ex);
             if (a.queries) {
                 a.norm[r] = trusted ? (a.cosine ? 0.0f : (float)s) : nan;
                 continue;
             }
             const bool keep = on && trusted;
-            // Euclidean: a row with a NaN scores NaN against every query and
-            // is never admitted; cosine's fold arm scores it 1
-            const bool force = on && !trusted && (a.cosine || s == s);
             a.norm[r] = keep ? (a.cosine ? 0.0f : (float)s - a.eps_rel * (float)s) : inf;
             if (keep && !a.cosine) xmax = fmaxf(xmax, (float)s);
             if (force) {

@@ -32,8 +32,8 @@
 //
 // Rows whose screen value cannot be trusted (norms near the ends of the f32
 // range, NaN under the fold arm) are "forced": their screen value is +inf and
-// a short list hands them to every query.  Queries of that kind, and every
-// query when the list overflows, evaluate all rows.
+// a short list hands them to every query.  More rows than it holds are found by
+// a mark in the rows' scales.  Queries of that kind evaluate all rows.
 #pragma once
 
 #include "knn_kernels.hpp"
@@ -45,12 +45,12 @@ constexpr int kGmQuad = 4;         // tiles between stores of the minima
 constexpr int kGmQpb = 128;        // queries of one block: 4 waves of 32; a workgroup takes one block or two
 constexpr int kGmMaxD = 256;
 constexpr int kGmMaxK = 128;
-constexpr int kGmForced = 256;     // forced rows listed before every query evaluates all rows
+constexpr int kGmForced = 256;     // forced rows listed; more are found by their mark
 
 // Written by the preparation launches.
 struct GmStats {
     unsigned int xmax_bits;  // largest trusted ||x||^2 (f32 bits, non-negative)
-    unsigned int nforced;    // rows not trusted (kGmForced of them are listed)
+    unsigned int nforced;    // forced rows (kGmForced of them are listed)
 };
 
 struct GmScanArgs {
@@ -97,7 +97,7 @@ struct GmPrepArgs {
     int64_t ldo;
     int64_t n_out;       // rows of out (zeros past n)
     float* norm;         // index: bias; queries: ||q||^2 (0 for cosine), NaN where the screen is not trusted
-    float* inv;          // undoes the rows' scales (queries, Euclidean: times 2)
+    float* inv;          // undoes the rows' scales (queries, Euclidean: times 2); -1: a forced row (its operand is zero)
     int64_t n_norm;      // entries of norm and inv (index: ntp * 32, +inf past n; queries: n)
     int queries;         // 1: query operand; 0: index rows
     int cosine;
@@ -122,6 +122,7 @@ struct GmSelectArgs {
     const float* gmin;   // [nq][2][ntp]
     int64_t ntp;
     const float* bias;
+    const float* xinv;   // below 0: a forced row
     const float* qnorm;  // [nq], NaN: evaluate every row
     const GmStats* stats;  // null: the minima are of the arm's own values (launch_groupmin_tile), no row is left out
     const uint32_t* forced;

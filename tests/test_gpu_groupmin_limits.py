@@ -98,3 +98,15 @@ def test_an_outlier_costs_the_others_nothing(dtype):
     plain = _ms(_search(name, xq, xt, 10))
     xt[777] *= 1e4
     assert _ms(_search(name, xq, xt, 10)) < 3.0 * plain
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("metric", [0, 1])
+def test_rows_the_screen_is_not_trusted_with_cost_their_share(dtype, metric):
+    """300 infinite (Euclidean) or NaN (cosine) rows, more than are listed: they
+    are evaluated for every query, and not the whole index."""
+    xt, xq = _rows(5, 100_000, 100, dtype), _rows(6, 2_000, 100, dtype)
+    name = "mlrs_knn_topk_" + ("f32" if dtype is torch.float32 else "f64")
+    plain = _ms(_search(name, xq, xt, 10, metric))
+    xt[1_000:1_300, 3] = float("nan") if metric else float("inf")
+    assert _ms(_search(name, xq, xt, 10, metric)) < 5.0 * plain
