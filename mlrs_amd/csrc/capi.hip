@@ -517,21 +517,58 @@ static bool small_search(int64_t nq, int64_t nt, int64_t d) {
     return (double)nq * (double)nt * (double)d <= 4294967296.0;
 }
 
-// Searches the low-d ALU kernel serves faster than the group-minimum search,
-// whose cost is about 0.335 ps per pair whatever k and d (most of it the minima's way
-// through memory).  The ALU kernel needs thousands of queries to fill its lanes,
-// pays for its list merges, and its cost per pair grows with d and k; fitted to self-searches of
-// 30,000 and 100,000 rows (us, ALU against group minima): f32 d = 2, k = 2: 298
-// / 314 and 1373 / 3335; d = 3, k = 8: 538 / 344 and 1722 / 3329; d = 8, k = 8:
-// 833 / 338 and 3475 / 3391; f64 d = 2, k = 2: 360 / 321 and 1632 / 3313; d = 3,
-// k = 8: 709 / 354 and 2961 / 3347; d = 4, k = 8: 834 / 353 and 3649 / 3355; d = 16, k =
-// 8, f32: 1048 / 337 and 5522 / 3378.  500,000
-// rows, d = 3, k = 8, f32: 23 ms against 93.
-static bool lowd_faster(int64_t nq, int64_t nt, int64_t d, int64_t k, size_t elem) {
-    if (nq < 4096 || k > 16) return false;
-    const double pairs = (double)nq * (double)nt;
-    const double ps = elem == 4 ? 0.04 + 0.027 * (double)d + 0.004 * (double)k : 0.02 + 0.06 * (double)d + 0.006 * (double)k;
-    return 150.0 + 35.0 * (double)k + ps * 1e-6 * pairs < 0.335e-6 * pairs;
+// Which kernels serve a search: the cheapest by the costs below, in us, fitted
+// to calls of this library.  What the terms stand for:
+//  exact   launches; one wave walks a row of values (2.4 ns a value) and a row
+//          costs 1.5 ns among many; a value's tile work grows with d.  It wins
+//          where the index is a few hundred rows, or a few thousand and the
+//          queries few.
+//  groups  launches; a query's selection, in batches of 64 rows evaluated (its
+//          k + 1 nearest groups of 16); 0.3 ps a pair for the scan whatever d and
+//          k, the tile work for the metric arms.
+//  low-d   launches; a walk through a strip of rows at the pace of its list
+//          merges, which become rarer along it; pairs at a pace that grows with
+//          d and k, less where 64 strips do not give the CUs their workgroups.
+// us measured, exact / groups / low-d:
+//   f32 Euclidean, k = 5: 100 x 300,000, d = 50: 510 / 1037; 300 x 20,000, d = 50:
+//   67 / 108; 1000 x 20,000, d = 200: 272 / 183; 3000 x 1,000, d = 50: 42 / 43;
+//   3000 x 16, d = 50: 30 / 40; 300 x 300,000, d = 8: 546 / 971 / 267; 3000 x
+//   20,000, d = 8: 135 / 100 / 694
+//   f64 Euclidean, k = 5: 300 x 20,000, d = 50: 83 / 129; 3000 x 20,000, d = 50:
+//   417 / 138; 100 x 300,000, d = 200: 1248 / 3220
+//   f32 Manhattan, k = 5: 300 x 300,000, d = 50: 693 / 1214; 3000 x 300,000, d = 8:
+//   2037 / 1260
+//   low-d against groups, Euclidean: 1M x 4,000, d = 3, k = 8, f32: 1176 / 1387; d =
+//   2, k = 2, f64: 892 / 1479; 30,000 against itself, d = 2, k = 2, f32: 287 / 326;
+//   100,000 against itself, d = 8, k = 8, f32: 3352 / 3391, d = 16: 5507 / 3378;
+//   500,000 against itself, d = 3, k = 8, f32: 23,000 / 93,000.
+// exact: k <= 64 only (longer lists go through a radix selection).
+enum class SearchKind { Exact, Groups, Lowd };
+static SearchKind cheapest_search(int64_t nq, int64_t nt, int64_t d, int64_t k, int arm, size_t elem, bool lowd_ok) {
+    const bool f64 = elem == 8;
+    const bool cos = arm == ARM_COS_FOLD || arm == ARM_COS_HOST;
+    const bool gram = cos || arm == ARM_EUCLID_FMA || arm == ARM_EUCLID_MULADD;
+    const double q = (double)nq, D = (double)d, mpairs = 1e-6 * q * (double)nt;
+    const double batches = std::ceil((double)std::min<int64_t>(nt, 16 * (k + 1)) / 64.0);
+    const double groups =
+        (gram ? 34.5 + 0.05 * D + 0.3 * mpairs : 28.0 + (f64 ? 0.22 : 0.17) * D + (f64 ? 0.066 : 0.033) * D * mpairs) +
+        1e-3 * q * (0.3 + batches * (f64 ? 1.5 + 0.019 * D : 1.25 + 0.008 * D));
+    double exact = HUGE_VAL;
+    if (k <= 64)
+        exact = (cos ? 33.0 + (f64 ? 0.002 : 0.006) * std::min(q, 1000.0) : 27.0) + std::max(0.0, D - 60.0) * (gram ? 0.12 : 0.08) * (f64 ? 1.5 : 1.0) + 2.4e-3 * (double)nt + 1e-3 * q * (f64 ? 1.8 : 1.5) +
+                mpairs * (gram ? (f64 ? 2.2 + 0.1 * D : 0.9 + 0.045 * D) : (f64 ? 2.6 + 0.066 * D : 0.9 + 0.036 * D));
+    double lowd = HUGE_VAL;
+    if (lowd_ok && k <= 16) {
+        const double blocks = std::ceil(q / (double)lowd_queries_per_block((int)k, d, (int)elem));
+        const double strips = std::max(1.0, std::min(64.0, std::ceil((double)nt / 4096.0)));
+        const double fill = std::min(1.0, blocks * strips / 640.0);
+        const double strip = std::min(1.0, std::pow((double)nt / 4096.0, 0.4));
+        const double ps = (f64 ? 0.02 + 0.06 * D + 0.006 * (double)k : 0.04 + 0.027 * D + 0.004 * (double)k) +
+                          (cos ? 0.05 : 0.0) + (k > 8 ? (f64 ? 0.35 : 0.15) : 0.0);
+        lowd = 30.0 + (120.0 + 35.0 * (double)k) * strip + ps * mpairs / fill;
+    }
+    if (lowd < exact && lowd < groups) return SearchKind::Lowd;
+    return exact < groups ? SearchKind::Exact : SearchKind::Groups;
 }
 
 // Process-wide kernel-family override (mlrs_force_path); a family that does
@@ -943,6 +980,18 @@ static bool groupmin_metric_serves(int arm, int64_t d, int64_t k) {
            d <= kGmMaxD && k <= kGmMaxK;
 }
 
+// The automatic choice as a family: AUTO stands for the group minima of the
+// metric arms, where they serve, GENERIC for the exact tiles.
+static int automatic_path(int64_t nq, int64_t nt, int64_t d, int64_t k, int arm, size_t elem, bool lowd_ok,
+                          bool gm_ok) {
+    const SearchKind kind = cheapest_search(nq, nt, d, k, arm, elem, lowd_ok);
+    if (kind == SearchKind::Lowd) return MLRS_PATH_LOWD;
+    // in a bounded scratch the exact tiles keep norms of every query there
+    const bool exact = kind == SearchKind::Exact && !(g_noalloc && nq > 1000000);
+    if (gm_ok) return exact ? MLRS_PATH_GENERIC : MLRS_PATH_FUSED;
+    return exact || !groupmin_metric_serves(arm, d, k) ? MLRS_PATH_GENERIC : MLRS_PATH_AUTO;
+}
+
 template <typename T>
 int32_t knn_groupmin_metric(const T* xq, int64_t nq, const T* xt, int64_t nt, int64_t d, int k, int arm, int mode,
                             T* out_v, uint32_t* out_i, hipStream_t s, double p) {
@@ -1139,9 +1188,7 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
     const bool forced = pick_path(lowd_ok, gm_ok) == MLRS_PATH_FUSED;
     int path = pick_path(lowd_ok, gm_ok);
     if (path == MLRS_PATH_AUTO)
-        path = lowd_ok && lowd_faster(n_query, n_train, n_features, k, sizeof(float)) ? MLRS_PATH_LOWD
-               : gm_ok                                                                ? MLRS_PATH_FUSED
-                                                                                      : MLRS_PATH_AUTO;
+        path = automatic_path(n_query, n_train, n_features, k, arm, sizeof(float), lowd_ok, gm_ok);
     if (path == MLRS_PATH_LOWD)
         return knn_lowd<float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
     if (path == MLRS_PATH_FUSED) {
@@ -1159,7 +1206,7 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
         return knn_groupmin<float, float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
                                           s);
     }
-    if (path == MLRS_PATH_AUTO && groupmin_metric_serves(arm, n_features, k))
+    if (path == MLRS_PATH_AUTO)
         return knn_groupmin_metric<float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s,
                                           p);
     return knn_generic<float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s, p);
@@ -1270,15 +1317,13 @@ int32_t mlrs_knn_topk_f64(const double* xq, int64_t xq_len, int64_t n_query, int
     const bool gm_ok = groupmin_serves(arm, n_features, k);
     int path = pick_path(lowd_ok, gm_ok);
     if (path == MLRS_PATH_AUTO)
-        path = lowd_ok && lowd_faster(n_query, n_train, n_features, k, sizeof(double)) ? MLRS_PATH_LOWD
-               : gm_ok                                                                 ? MLRS_PATH_FUSED
-                                                                                       : MLRS_PATH_AUTO;
+        path = automatic_path(n_query, n_train, n_features, k, arm, sizeof(double), lowd_ok, gm_ok);
     if (path == MLRS_PATH_LOWD)
         return knn_lowd<double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
     if (path == MLRS_PATH_FUSED)
         return knn_groupmin<double, double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
                                             s);
-    if (path == MLRS_PATH_AUTO && groupmin_metric_serves(arm, n_features, k))
+    if (path == MLRS_PATH_AUTO)
         return knn_groupmin_metric<double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
                                            s, p);
     return knn_generic<double>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s, p);
@@ -2023,14 +2068,11 @@ static int32_t search_f64(const TS* x, int64_t n, int64_t d, int k, int arm, int
                          mode != EMIT_ROOT_RANKED && d <= lowd_max_d() && k <= lowd_max_k();
     const bool gm_ok = groupmin_serves(arm, d, k);
     int path = pick_path(lowd_ok, gm_ok);
-    if (path == MLRS_PATH_AUTO)
-        path = lowd_ok && lowd_faster(n, n, d, k, sizeof(double)) ? MLRS_PATH_LOWD
-               : gm_ok                                            ? MLRS_PATH_FUSED
-                                                                  : MLRS_PATH_AUTO;
+    if (path == MLRS_PATH_AUTO) path = automatic_path(n, n, d, k, arm, sizeof(double), lowd_ok, gm_ok);
     if (path == MLRS_PATH_FUSED) return knn_groupmin<double, TS>(x, n, x, n, d, k, arm, mode, ov, oi, s);
     if constexpr (sizeof(TS) == 8) {
         if (path == MLRS_PATH_LOWD) return knn_lowd<double>(x, n, x, n, d, k, arm, mode, ov, oi, s);
-        if (path == MLRS_PATH_AUTO && groupmin_metric_serves(arm, d, k))
+        if (path == MLRS_PATH_AUTO)
             return knn_groupmin_metric<double>(x, n, x, n, d, k, arm, mode, ov, oi, s, p);
         return knn_generic<double>(x, n, x, n, d, k, arm, mode, ov, oi, s, p);
     } else {
@@ -2082,8 +2124,12 @@ static int32_t graph_search(const TIn* x, int64_t n, int64_t d, int kk, int32_t 
     graph_arm(metric, &arm, &mode);
     // The group-minimum search widens f32 rows as it evaluates them; cosine
     // (normalised rows) and the other kernels work on rows widened first.
-    const bool direct = sizeof(TIn) == 4 && !cos && groupmin_serves(arm, d, kk) &&
-                        pick_path(false, true) != MLRS_PATH_GENERIC;
+    bool direct = sizeof(TIn) == 4 && !cos && groupmin_serves(arm, d, kk);
+    if (direct) {
+        int path = pick_path(false, true);
+        if (path == MLRS_PATH_AUTO) path = automatic_path(n, n, d, kk, arm, sizeof(double), false, true);
+        direct = path == MLRS_PATH_FUSED;
+    }
     const bool widen = sizeof(TIn) == 4 && !direct;
     size_t bytes = aligned_bytes(sizeof(double) * (size_t)n * kk) + aligned_bytes(sizeof(uint32_t) * (size_t)n * kk) +
                    (widen ? aligned_bytes(sizeof(double) * (size_t)n * d) : 0) +

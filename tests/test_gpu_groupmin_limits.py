@@ -110,3 +110,38 @@ def test_rows_the_screen_is_not_trusted_with_cost_their_share(dtype, metric):
     plain = _ms(_search(name, xq, xt, 10, metric))
     xt[1_000:1_300, 3] = float("nan") if metric else float("inf")
     assert _ms(_search(name, xq, xt, 10, metric)) < 5.0 * plain
+
+
+@pytest.mark.parametrize("nt,nq,d,k,metric,dtype,kernel", [
+    (100, 20_000, 50, 5, "euclidean", torch.float32, "pairwise_tile_kernel"),
+    (300, 20_000, 20, 5, "cosine", torch.float64, "pairwise_tile_kernel"),
+    (300, 20_000, 50, 5, "manhattan", torch.float32, "pairwise_tile_kernel"),
+    (3_000, 16, 50, 1, "euclidean", torch.float64, "pairwise_tile_kernel"),
+    (32, 300_000, 8, 5, "euclidean", torch.float32, "knn_lowd_kernel"),
+    (1_000_000, 4_000, 2, 2, "euclidean", torch.float32, "knn_lowd_kernel"),
+    (1_000_000, 4_000, 2, 2, "euclidean", torch.float64, "knn_lowd_kernel"),
+    (1_000_000, 1_000, 3, 8, "euclidean", torch.float32, "knn_groupmin_kernel"),
+    (1_000_000, 4_000, 8, 8, "cosine", torch.float64, "knn_groupmin_kernel"),
+    (10_000, 1_000, 64, 10, "euclidean", torch.float32, "knn_groupmin_kernel"),
+    (3_000, 20_000, 50, 5, "euclidean", torch.float32, "knn_groupmin_kernel"),
+    (60_000, 2_000, 40, 10, "manhattan", torch.float64, "groupmin_tile_kernel")])
+def test_family_chosen(nt, nq, d, k, metric, dtype, kernel):
+    """Small indexes and few columns go where they were measured fastest, and
+    with the same answer as the group minima."""
+    xt, xq = _rows(nt, nt, d, dtype), _rows(nq, nq, d, dtype)
+    lib = _lib.load()
+    _lib.check(lib.mlrs_timing_enable(1))
+    try:
+        dist, idx = prims.knn_topk(xq, xt, k, metric)
+        ms, launches, name = ctypes.c_double(), ctypes.c_int64(), ctypes.create_string_buffer(64)
+        _lib.check(lib.mlrs_timing_read(ctypes.byref(ms), ctypes.byref(launches), name, 64))
+    finally:
+        _lib.check(lib.mlrs_timing_enable(0))
+    assert name.value.decode() == kernel
+    if metric != "manhattan":
+        prims.force_path("fused")
+        try:
+            d2, i2 = prims.knn_topk(xq, xt, k, metric)
+        finally:
+            prims.force_path("auto")
+        assert torch.equal(idx, i2) and torch.equal(dist, d2)
