@@ -1012,9 +1012,12 @@ hipError_t launch_pairwise_tile(const T* x, int64_t nx, const T* y, int64_t ny, 
                                 T pexp, int pint, T root_exp) {
     if (nx == 0 || ny == 0) return hipSuccess;
     // 8 y rows per thread reuse operands best (8,009 x 8,209 at d = 100, f32:
-    // 0.41 ms against 0.45), 4 fill the chip where there are few tiles
+    // 0.41 ms against 0.45), 4 fill the chip where there are few tiles, and
+    // where they leave less of the last tile empty (300,000 x 32, d = 200, k = 5
+    // search by these tiles, f64: 1.22 ms with 8, 0.88 with 4)
     const unsigned gx = (unsigned)((nx + PTX - 1) / PTX);
-    const bool wide = (int64_t)gx * ((ny + 127) / 128) >= 2048;
+    const int64_t n4 = (ny + 63) / 64, n8 = (ny + 127) / 128;
+    const bool wide = (int64_t)gx * n8 >= 2048 && 20 * n8 <= 11 * n4;
     const dim3 grid((unsigned)((ny + (wide ? 127 : 63)) / (wide ? 128 : 64)), gx);
     const MetricParams<T> mp{pexp, pint, root_exp};
 #define MLRS_PT_CASE(A)                                                                                        \

@@ -145,3 +145,11 @@ def test_family_chosen(nt, nq, d, k, metric, dtype, kernel):
         finally:
             prims.force_path("auto")
         assert torch.equal(idx, i2) and torch.equal(dist, d2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_few_rows_take_narrow_tiles(dtype):
+    """A matrix of 64 columns costs about half of one of 128, not as much."""
+    x, y = _rows(1, 200_000, 200, dtype), _rows(2, 128, 200, dtype)
+    half = y[:64].contiguous()
+    assert _ms(lambda: prims.pairwise_distance(x, half)) < 0.75 * _ms(lambda: prims.pairwise_distance(x, y))
