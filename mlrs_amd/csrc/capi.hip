@@ -1015,7 +1015,7 @@ int32_t knn_groupmin_metric(const T* xq, int64_t nq, const T* xt, int64_t nt, in
     se.gmin = reinterpret_cast<const float*>(ws);
     se.ntp = ntp;
     se.first = se.last = 1;
-    se.eps_t = std::ldexp(1.0, -21);  // the minima's rounding to f32 (2^-24) on both sides of a comparison, and a root's
+    se.eps_t = std::ldexp(1.0, -21);  // the minima's rounding down to f32 (2^-23) and a root's ties
     se.pexp = p;
     se.pint = minkowski_powi(p);
     se.root_exp = 1.0 / p;

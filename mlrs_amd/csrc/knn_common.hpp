@@ -177,6 +177,13 @@ __device__ __forceinline__ float round_up_f(double t) {
     return f;
 }
 
+// t >= 0 (or a quiet NaN) rounded down to f32 by cutting its mantissa: one
+// instruction beside the conversion.  Below 2^-126 the conversion itself rounds.
+__device__ __forceinline__ float round_down_f(float t) { return t; }
+__device__ __forceinline__ float round_down_f(double t) {
+    return (float)__longlong_as_double(__double_as_longlong(t) & ~0x1FFFFFFFll);
+}
+
 // ---------------------------------------------------------------------------
 // Wave64 bitonic machinery over (value, index) pairs, one pair per lane.
 // ---------------------------------------------------------------------------

@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256) void pairwise_tile_kernel(const T* __restrict_
     }
 }
 
-// Only the minima, rounded to f32, of each 16 y rows (knn_groupmin.hpp's
+// Only the minima, rounded down to f32, of each 16 y rows (knn_groupmin.hpp's
 // groups: the runs of 4 rows 0, 2, 4, 6 and 1, 3, 5, 7 of 32), for the
 // group-minimum selection: no matrix is written and read again, and the
 // selection reads 1/16 of the values (60,013 x 2,001, d = 40, k = 10, f64
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(256) void groupmin_tile_kernel(const T* __restrict_
 #pragma unroll
             for (int i = 0; i < V; ++i) {
                 const T av = acc[a][e * V + i];
-                const float v = fminf((float)av, av == av ? top : __builtin_nanf(""));
+                const float v = fminf(round_down_f(av), av == av ? top : __builtin_nanf(""));
                 m[e] = fminf(m[e], j0 + tile_y<T>(tx, e * V + i) < ny ? v : inf);
             }
             if (V == 4) {

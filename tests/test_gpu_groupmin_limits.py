@@ -153,3 +153,20 @@ def test_few_rows_take_narrow_tiles(dtype):
     x, y = _rows(1, 200_000, 200, dtype), _rows(2, 128, 200, dtype)
     half = y[:64].contiguous()
     assert _ms(lambda: prims.pairwise_distance(x, half)) < 0.75 * _ms(lambda: prims.pairwise_distance(x, y))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("nt,nq,metric", [(100_000, 2_000, 3), (100_000, 400, 3), (30_000, 3_000, 0)])
+def test_ties_cost_no_pass_over_the_index(dtype, nt, nq, metric):
+    """Rows of three values in thirty columns at one Chebyshev distance nearly
+    all, and rows that are all the same: of equal distances the first rows are
+    the answer, and no later one is evaluated."""
+    g = torch.Generator(device="cuda").manual_seed(nt)
+    name = "mlrs_knn_topk_" + ("f32" if dtype is torch.float32 else "f64")
+    xt, xq = _rows(7, nt, 30, dtype), _rows(8, nq, 30, dtype)
+    plain = _ms(_search(name, xq, xt, 10, metric))
+    if metric:
+        xt, xq = (torch.randint(0, 3, x.shape, generator=g, device=DEV).to(dtype) for x in (xt, xq))
+    else:
+        xt, xq = torch.ones_like(xt), torch.ones_like(xq)
+    assert _ms(_search(name, xq, xt, 10, metric)) < 3.0 * plain
