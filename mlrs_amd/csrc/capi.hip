@@ -926,6 +926,11 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     se.gmin = gmin;
     se.bias = bias;
     se.xinv = xinv;
+    se.xcopy = xcopy;
+    se.qop = qop;
+    se.qinv = qinv;
+    se.ldx = ldx;
+    se.dp = dp;
     se.qnorm = qnorm;
     se.stats = stats;
     se.forced = forced;

@@ -23,8 +23,6 @@ template <> struct GmRange<double> {
     static __device__ __forceinline__ bool cosine(double s) { return s >= 0x1p-500 && s <= 0x1p500; }
 };
 
-typedef _Float16 gm_f16x4 __attribute__((ext_vector_type(4)));
-
 template <typename T, int LPR>
 __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
     constexpr int RPW = 64 / LPR;      // rows a wave takes at once

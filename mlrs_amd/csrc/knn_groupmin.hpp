@@ -123,6 +123,10 @@ struct GmSelectArgs {
     int64_t ntp;
     const float* bias;
     const float* xinv;   // below 0: a forced row
+    const float* xcopy;  // the part's operand rows, stride ldx
+    const float* qop;    // the queries', stride dp
+    const float* qinv;
+    int64_t ldx, dp;
     const float* qnorm;  // [nq], NaN: evaluate every row
     const GmStats* stats;  // null: the minima are of the arm's own values (launch_groupmin_tile), no row is left out
     const uint32_t* forced;
