@@ -820,8 +820,8 @@ static GmPlan gm_plan(int64_t nq, int64_t nt, int64_t d) {
     P.dp = 8 * (int64_t)gm_chunks(d);
     const size_t limit = workspace_limit();
     // copied rows (split elements, bias, scale); a query beside its minima (split
-    // elements, norm, scale)
-    const size_t per_row = sizeof(float) * (size_t)(P.ldx + 2), per_q = sizeof(float) * (size_t)(P.dp + 2);
+    // elements, norm, scale, place in the precise scan's list)
+    const size_t per_row = sizeof(float) * (size_t)(P.ldx + 2), per_q = sizeof(float) * (size_t)(P.dp + 3);
     const size_t fixed = sizeof(GmStats) + sizeof(uint32_t) * kGmForced + per_q * kSet + per_row * kStore + 4096;
     // Without a limit 4 GiB of copied rows hold any index but the largest
     // whole, and 1 GiB of minima keeps the scan launches long (the tail of one
@@ -867,6 +867,7 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     float* qop = cv.take<float>((size_t)(P.qpad * dp));
     float* qnorm = cv.take<float>((size_t)P.qc);
     float* qinv = cv.take<float>((size_t)P.qc);
+    uint32_t* flag = cv.take<uint32_t>((size_t)P.qc);
     float* gmin = cv.take<float>(2 * (size_t)ntp * (size_t)P.qc);
 
     GmPrepArgs pq{};
@@ -936,6 +937,31 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
     se.forced = forced;
     se.eps_rel = eps_rel;
     se.eps_abs = eps_abs;
+    // Queries whose candidates are too many to evaluate get the precise scan, where
+    // its two launches (7 us, most searches leave them empty) are lost in the
+    // search.  200k x 5k, d = 250, k = 15, f64, in five clusters a thousandth of
+    // their spacing wide: 258 ms evaluating every group, 79.5 with gm_pass's
+    // probe, 12.0 so (9.9 with an f64 scan alone).  In f32 the values' own
+    // rounding is most of what cannot be told apart.
+    const bool precise = sizeof(T) == 8 && ((double)nq * (double)nt >= 1e8 || nt * d >= (1 << 25));
+    se.flag = precise ? flag : nullptr;
+    GmPreciseArgs<TS> pr{};
+    pr.d = d;
+    pr.centre = xt;
+    pr.centre_n = nt;
+    pr.bias = bias;
+    pr.list = flag;
+    pr.stats = stats;
+    pr.gmin = gmin;
+    pr.grid_wgs = cus;
+    // Its values: with v = 2^-52, products and sums of f64 operands round to
+    // (d + 4) v N, the centred operands, the norms and the f64 arms no more each:
+    // 4 (d + 8) v N; cosine of unit vectors likewise.  The minima's rounding to f32
+    // is u of a value; the absolute term covers f32's subnormals.
+    const double v = std::ldexp(1.0, -52);
+    const double pr_rel = cos ? 0.0 : 4.0 * (double)(d + 8) * v;
+    const double pr_abs = cos ? 4.0 * (double)(d + 16) * v : (double)(d + 16) * std::ldexp(1.0, -120);
+    const double pr_t = 2.0 * u;
     hipError_t e = hipSuccess;
     for (int64_t q0 = 0; q0 < nq && e == hipSuccess; q0 += P.qc) {
         const int64_t n = std::min<int64_t>(P.qc, nq - q0);
@@ -972,7 +998,26 @@ int32_t knn_groupmin(const TS* xq, int64_t nq, const TS* xt, int64_t nt, int64_t
             se.row0 = x0;
             se.first = x0 == 0;
             se.last = x0 + rows == nt;
+            // a query's pass over its candidate groups reads 64 + 4 bytes of every row
+            // and one row in full of each, at about 8 TB/s; its share of the precise
+            // scan runs at 50 TFLOP/s
+            se.flag_above = (uint32_t)(0.32 * (double)rows * (double)d / (1088.0 + 1.1 * (double)(sizeof(TS) * d)));
             if (e == hipSuccess) e = launch_gm_select<T, TS>(se, arm, s);
+            if (precise && e == hipSuccess) {
+                pr.q = se.q;
+                pr.x = se.x;
+                pr.nt = rows;
+                pr.tiles = pr.ntp = sc.tiles;
+                e = launch_gm_precise<TS>(pr, cos, s);
+                GmSelectArgs<TS> sp = se;
+                sp.kind = GM_PRECISE;
+                sp.list = flag;
+                sp.flag = nullptr;
+                sp.eps_rel = pr_rel;
+                sp.eps_abs = pr_abs;
+                sp.eps_t = pr_t;
+                if (e == hipSuccess) e = launch_gm_select<T, TS>(sp, arm, s);
+            }
         }
     }
     return e == hipSuccess ? ok() : hip_err(e, "knn_groupmin");
@@ -1019,6 +1064,7 @@ int32_t knn_groupmin_metric(const T* xq, int64_t nq, const T* xt, int64_t nt, in
     se.mode = mode;
     se.gmin = reinterpret_cast<const float*>(ws);
     se.ntp = ntp;
+    se.kind = GM_EXACT;
     se.first = se.last = 1;
     se.eps_t = std::ldexp(1.0, -21);  // the minima's rounding down to f32 (2^-23) and a root's ties
     se.pexp = p;

@@ -177,6 +177,17 @@ __device__ __forceinline__ float round_up_f(double t) {
     return f;
 }
 
+// The centre group-minimum copies are taken around: per column the median of
+// three rows, so that one outlier among them does not become it; 0 where it is
+// not finite.
+template <typename T>
+__device__ __forceinline__ T gm_centre(const T* __restrict__ X, int64_t n, int d, int c) {
+    const T u = X[c], v = X[(n / 2) * d + c], w = X[(n - 1) * d + c];
+    const T lo = u < v ? u : v, hi = u < v ? v : u;
+    const T m = w < lo ? lo : (w > hi ? hi : w);
+    return (m - m == T(0)) ? m : T(0);
+}
+
 // t >= 0 (or a quiet NaN) rounded down to f32 by cutting its mantissa: one
 // instruction beside the conversion.  Below 2^-126 the conversion itself rounds.
 __device__ __forceinline__ float round_down_f(float t) { return t; }

@@ -33,24 +33,20 @@ __global__ __launch_bounds__(256) void gm_prep_kernel(GmPrepArgs a) {
     const T* __restrict__ X = static_cast<const T*>(a.rows);
     const int d = (int)a.d;
     const int c0 = 4 * sub;
-    if (a.reset && blockIdx.x == 0 && threadIdx.x == 0) {
-        // the index launch behind this one fills them
-        a.stats->xmax_bits = 0u;
-        a.stats->nforced = 0u;
+    if (a.queries && blockIdx.x == 0 && threadIdx.x == 0) {
+        a.stats->nflag = 0u;
+        if (a.reset) {
+            // the index launch behind this one fills them
+            a.stats->xmax_bits = 0u;
+            a.stats->nforced = 0u;
+        }
     }
-    // The centre: per column the median of three rows, so that one outlier
-    // among them does not become it; 0 where it is not finite.
     T ctr[4] = {T(0), T(0), T(0), T(0)};
     if (a.centre) {
         const T* C = static_cast<const T*>(a.centre);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            if (c0 + e < d) {
-                const T u = C[c0 + e], v = C[(a.centre_n / 2) * d + c0 + e], w = C[(a.centre_n - 1) * d + c0 + e];
-                const T lo = u < v ? u : v, hi = u < v ? v : u;
-                const T m = w < lo ? lo : (w > hi ? hi : w);
-                ctr[e] = (m - m == T(0)) ? m : T(0);
-            }
+            if (c0 + e < d) ctr[e] = gm_centre(C, a.centre_n, d, c0 + e);
     }
     const int64_t n = a.n, n_out = a.n_out;
     const int64_t n_all = n_out > a.n_norm ? n_out : a.n_norm;

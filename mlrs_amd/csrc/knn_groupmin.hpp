@@ -51,6 +51,7 @@ constexpr int kGmForced = 256;     // forced rows listed; more are found by thei
 struct GmStats {
     unsigned int xmax_bits;  // largest trusted ||x||^2 (f32 bits, non-negative)
     unsigned int nforced;    // forced rows (kGmForced of them are listed)
+    unsigned int nflag;      // queries the selection leaves to the precise scan
 };
 
 struct GmScanArgs {
@@ -103,13 +104,41 @@ struct GmPrepArgs {
     int cosine;
     float eps_rel;       // index: the share of ||x||^2 the bias is lowered by
     GmStats* stats;      // filled from the index rows
-    int reset;           // zero stats (the launch before the index's)
+    int reset;           // zero the index's stats (the launch before the index's; the queries' always zeroes nflag)
     uint32_t* forced;    // [kGmForced]
 };
 template <typename T>
 hipError_t launch_gm_prep(const GmPrepArgs& a, hipStream_t s);
 
 hipError_t launch_gm_scan(const GmScanArgs& a, hipStream_t s);
+
+// The precise scan (knn_groupmin_precise.hip): the same minima on the f64
+// matrix cores, of the rows as given, for the queries whose candidates were too
+// many to evaluate.  How many those are is known on the device only, so the launch
+// is made whenever the search is large enough for it not to show.
+template <typename TS>
+struct GmPreciseArgs {
+    const TS* q;           // [..][d] queries as given
+    const TS* x;           // [nt][d] index rows of this part, as given
+    int64_t nt, d;
+    const TS* centre;      // the index, as the preparation takes its centre
+    int64_t centre_n;
+    const float* bias;     // +inf for rows left out
+    const uint32_t* list;  // [stats->nflag] queries
+    const GmStats* stats;
+    int64_t tiles, ntp;    // as GmScanArgs
+    float* gmin;           // [stats->nflag][2][ntp]: distances (Euclidean: squared), rounded down
+    int64_t grid_wgs;      // the CU count
+};
+template <typename TS>
+hipError_t launch_gm_precise(const GmPreciseArgs<TS>& a, bool cosine, hipStream_t s);
+
+// What the minima are.
+enum GmKind {
+    GM_SCREEN,   // launch_gm_scan's
+    GM_PRECISE,  // launch_gm_precise's
+    GM_EXACT,    // the arm's own values (launch_groupmin_tile): no statistics, no row left out
+};
 
 template <typename TS>
 struct GmSelectArgs {
@@ -118,9 +147,12 @@ struct GmSelectArgs {
     int64_t nq, nt, d;
     int64_t row0;        // the part's first row in the index
     int first, last;     // the index's first / last part: between them the lists wait in the outputs, untransformed
-    int k, mode;
-    const float* gmin;   // [nq][2][ntp]
+    int k, mode, kind;
+    const float* gmin;   // [nq][2][ntp], GM_PRECISE: rows as list
     int64_t ntp;
+    const uint32_t* list;  // GM_PRECISE: the stats->nflag queries to select for (null: all)
+    uint32_t* flag;        // where to list queries for the precise scan, or null
+    uint32_t flag_above;   // at once with more candidate groups than this
     const float* bias;
     const float* xinv;   // below 0: a forced row
     const float* xcopy;  // the part's operand rows, stride ldx
@@ -128,10 +160,10 @@ struct GmSelectArgs {
     const float* qinv;
     int64_t ldx, dp;
     const float* qnorm;  // [nq], NaN: evaluate every row
-    const GmStats* stats;  // null: the minima are of the arm's own values (launch_groupmin_tile), no row is left out
+    GmStats* stats;        // GM_EXACT: null
     const uint32_t* forced;
-    double eps_rel, eps_abs;  // |screen - exact| <= eps_rel (||q||^2 + ||x||^2) + eps_abs (gm_bound)
-    double eps_t;        // relative error of a minimum (values rounded to f32)
+    // |minimum's value - exact| <= eps_rel (||q||^2 + ||x||^2) + eps_abs + eps_t |value|
+    double eps_rel, eps_abs, eps_t;
     double pexp, root_exp;  // Minkowski: the exponent and (EMIT_ROOT_RANKED) its root's
     int pint;               // its integer exponent
     void* out_val;       // [nq][k] of T

@@ -125,6 +125,96 @@ __device__ __forceinline__ float gm_bound(float t, float qn, float xmax, double 
     return round_up_f(b);
 }
 
+// The same for the precise scan's minima, which are distances: |value - exact| <=
+// e (||q||^2 + ||x||^2) + e_abs + e_t value, and ||x|| <= ||q|| + the distance.
+__device__ __forceinline__ float gm_bound_precise(double v, float qn, float xmax, double e, double e_abs, int sides) {
+    double b = v + sides * e_abs;
+    if (e != 0.0) {
+        const float r = __builtin_sqrtf(qn) + __builtin_sqrtf((float)fmax((v + 5.0 * e * (double)qn) * (1.0 + 5.0 * e), 0.0));
+        b += sides * e * ((double)qn + (double)fminf(xmax, 1.002f * r * r));
+    }
+    return round_up_f(b);
+}
+
+// What both selection kernels read of a query.  What an arm's minima cannot be
+// is known when it is compiled: METRIC ones are exact, precise ones come with f64
+// values only.
+template <typename T, typename TS, int ARM>
+struct GmQuery {
+    static constexpr bool COS = ARM == ARM_COS_FOLD || ARM == ARM_COS_HOST;
+    static constexpr bool exact = !COS && ARM != ARM_EUCLID_FMA && ARM != ARM_EUCLID_MULADD;
+    static constexpr bool twice = !exact && sizeof(T) == 8;
+    __device__ __forceinline__ bool precise() const { return twice && a.kind == GM_PRECISE; }
+    const float* G;   // its group minima, [2][ntp]
+    int n, ntp;
+    uint32_t nt;
+    float qn;
+    uint32_t nforced;
+    bool all_rows;  // a query the screen is not trusted with
+    float eps;      // the part of the error that does not depend on the row
+    float xmax;
+    float base;     // a value and its minimum's unit differ by this
+    const GmSelectArgs<TS>& a;
+    const float* bias;
+    double width;   // bound's distance above its argument, which only shrinks with it
+    __device__ __forceinline__ GmQuery(const GmSelectArgs<TS>& args, int64_t q, int64_t i) : a(args), width(0.0) {
+        G = a.gmin + i * 2 * a.ntp;
+        ntp = (int)a.ntp;
+        n = 2 * ntp;  // a multiple of 8
+        nt = (uint32_t)a.nt;
+        if constexpr (exact) {
+            base = 0.0f;
+            qn = 0.0f;
+            nforced = 0u;
+            all_rows = false;
+            eps = xmax = 0.0f;
+        } else {
+            qn = a.qnorm[q];
+            base = precise() ? 0.0f : COS ? 1.0f : qn;
+            nforced = a.stats->nforced;
+            all_rows = !(qn == qn);
+            xmax = __uint_as_float(a.stats->xmax_bits);
+            eps = round_up_f(a.eps_rel * (double)qn + a.eps_abs);
+        }
+        bias = a.bias;
+    }
+    // row j of group f; rows left out by the scan are evaluated from their list
+    __device__ __forceinline__ uint32_t row(int f, int j) const {
+        const int half = f >= ntp ? 1 : 0;
+        const uint32_t r = (uint32_t)(f - (half ? ntp : 0)) * kGmRows + (uint32_t)gm_group_row(half, j);
+        bool on = r < nt;
+        if (nforced) {
+            on = on && bias[r] < __builtin_huge_valf();
+        }
+        return on ? r : kSentinelIdx;
+    }
+    // the group's first row
+    __device__ __forceinline__ uint32_t first_row(int f) const {
+        const int half = f >= ntp ? 1 : 0;
+        return (uint32_t)(f - (half ? ntp : 0)) * kGmRows + (uint32_t)gm_group_row(half, 0);
+    }
+    // no row of a group with this minimum has a smaller exact value (minima near
+    // f32's subnormals are not rounded down)
+    __device__ __forceinline__ float least(float gm, bool ranked) const {
+        return exact && !ranked && gm > 0x1p-100f ? gm : 0.0f;
+    }
+    // every row of the answer lies in a group whose minimum is at or below this
+    __device__ __forceinline__ float bound(float t) {
+        if (!(t < __builtin_huge_valf())) return __builtin_huge_valf();
+        const double v = (double)t + a.eps_t * (double)t;
+        if constexpr (exact) return round_up_f(v);
+        const float b = precise() ? gm_bound_precise(v, qn, xmax, a.eps_rel, a.eps_abs, 2)
+                                  : gm_bound(t, qn, xmax, a.eps_rel, eps);
+        width = (double)b - (double)t;
+        return b;
+    }
+    // bound of a smaller argument than before
+    __device__ __forceinline__ float bound_again(float t) {
+        if (exact || !(width > 0.0)) return bound(t);
+        return round_up_f((double)t + width);
+    }
+};
+
 // A wave's answer so far: the 64 KL smallest (value, row) pairs it has seen.
 template <typename T, typename TS, int ARM, int KL>
 struct GmList {
@@ -201,14 +291,17 @@ struct GmList {
         wave_sort64<T>(v, ix, lane);
         merge(v, ix, lane);
     }
-    // A screen value no row of the answer exceeds, from the k-th exact value:
-    // exact <= R means screen <= R in screen units + eps.
-    __device__ __forceinline__ float screen_bound(int k, int mode, float qn, float eps, double eps_t) const {
+    // A minimum no row of the answer exceeds, from the k-th exact value: exact
+    // <= R means a value of at most R in its units + eps.
+    __device__ __forceinline__ float screen_bound(const GmQuery<T, TS, ARM>& Q) const {
+        const int mode = Q.a.mode;
         if (MINK && mode == EMIT_ROOT_RANKED) return __builtin_huge_valf();
-        double R = (double)kth(k);
+        double R = (double)kth(Q.a.k);
         if (mode == EMIT_ROOT_RANKED) R = R * R * (1.0 + 0x1p-40);
-        return R < (double)__builtin_huge_valf() ? round_up_f(R - (COS ? 1.0 : (double)qn) + (double)eps + eps_t * R)
-                                                 : __builtin_huge_valf();
+        if (!(R < (double)__builtin_huge_valf())) return __builtin_huge_valf();
+        if (!COS && Q.precise())
+            return gm_bound_precise(R + Q.a.eps_t * R, Q.qn, Q.xmax, Q.a.eps_rel, Q.a.eps_abs, 1);
+        return round_up_f(R - (double)Q.base + (double)Q.eps + Q.a.eps_t * R);
     }
     // A query every row of which is evaluated: a zero query's values are all
     // exactly 1 (or NaN, never admitted), so the first k rows are its answer.
@@ -227,68 +320,6 @@ struct GmList {
                 oi[s] = last && li[b] == kSentinelIdx ? 0u : li[b];
             }
         }
-    }
-};
-
-// What both selection kernels read of a query.
-template <typename TS>
-struct GmQuery {
-    const float* G;   // its group minima, [2][ntp]
-    int n, ntp;
-    uint32_t nt;
-    float qn;
-    uint32_t nforced;
-    bool exact;     // minima of the arm's own values
-    bool all_rows;  // a query the screen is not trusted with
-    float eps;      // the part of the error that does not depend on the row
-    float xmax;
-    const GmSelectArgs<TS>& a;
-    const float* bias;
-    __device__ __forceinline__ GmQuery(const GmSelectArgs<TS>& args, int64_t q) : a(args) {
-        G = a.gmin + q * 2 * a.ntp;
-        ntp = (int)a.ntp;
-        n = 2 * ntp;  // a multiple of 8
-        nt = (uint32_t)a.nt;
-        exact = !a.stats;
-        if (exact) {
-            qn = 0.0f;
-            nforced = 0u;
-            all_rows = false;
-            eps = xmax = 0.0f;
-        } else {
-            qn = a.qnorm[q];
-            nforced = a.stats->nforced;
-            all_rows = !(qn == qn);
-            xmax = __uint_as_float(a.stats->xmax_bits);
-            eps = round_up_f(a.eps_rel * (double)qn + a.eps_abs);
-        }
-        bias = a.bias;
-    }
-    // row j of group f; rows left out by the scan are evaluated from their list
-    __device__ __forceinline__ uint32_t row(int f, int j) const {
-        const int half = f >= ntp ? 1 : 0;
-        const uint32_t r = (uint32_t)(f - (half ? ntp : 0)) * kGmRows + (uint32_t)gm_group_row(half, j);
-        bool on = r < nt;
-        if (nforced) {
-            on = on && bias[r] < __builtin_huge_valf();
-        }
-        return on ? r : kSentinelIdx;
-    }
-    // the group's first row
-    __device__ __forceinline__ uint32_t first_row(int f) const {
-        const int half = f >= ntp ? 1 : 0;
-        return (uint32_t)(f - (half ? ntp : 0)) * kGmRows + (uint32_t)gm_group_row(half, 0);
-    }
-    // no row of a group with this minimum has a smaller exact value (minima near
-    // f32's subnormals are not rounded down)
-    __device__ __forceinline__ float least(float gm, bool ranked) const {
-        return exact && !ranked && gm > 0x1p-100f ? gm : 0.0f;
-    }
-    // every row of the answer lies in a group whose minimum is at or below this
-    __device__ __forceinline__ float bound(float t) const {
-        if (!a.stats)
-            return t < __builtin_huge_valf() ? round_up_f((double)t + a.eps_t * (double)t) : __builtin_huge_valf();
-        return gm_bound(t, qn, xmax, a.eps_rel, eps);
     }
 };
 
@@ -348,21 +379,20 @@ struct GmProbe {
         return s;
     }
     // What no row of the answer exceeds, given that none has a minimum above
-    // thr: its exact value is then at most thr + ||q||^2 (cosine: thr + 1), eps
-    // and the factor take the roundings of that sum and of the exact value; the
+    // thr: its exact value is then at most thr + base, eps and the factor take the roundings of that sum and of the exact value; the
     // operands hold 2^-22 of their elements, a distance of at most 2^-20 of
     // (||q|| + ||x||), ||x|| <= ||q|| + the distance.
-    static __device__ __forceinline__ float limit(float thr, float qn, float eps) {
+    static __device__ __forceinline__ float limit(float thr, float base, float qn, float eps) {
         if (!(thr < __builtin_huge_valf())) return __builtin_huge_valf();
-        const float D = COS ? 2.0f * (thr + 1.0f + eps) : thr + qn + eps;
+        const float D = (COS ? 2.0f : 1.0f) * (thr + base + eps);
         const float r = __builtin_sqrtf(fmaxf(1.001f * D, 0.0f));
         const float m = r + 0x1p-18f * ((COS ? 1.0f : __builtin_sqrtf(qn)) + r);
         return m * m * (1.0f + 0x1p-15f) + 0x1p-100f;
     }
 };
 
-// Too many groups to list (ties, or distances the screen does not resolve):
-// every group at or below thr, four at a time, the bound following the k-th
+// Too many groups to list (ties, or distances the screen does not resolve): every
+// group at or below thr, four at a time, the bound following the k-th
 // exact value of the waves that share the query (shared: their bounds).  A
 // group that can at best tie with the k-th value, behind its row, is passed
 // over: of equal values the list has the first rows already (100,000 rows of
@@ -371,20 +401,28 @@ struct GmProbe {
 // clusters a thousandth of their spacing wide, ms, every row of a group and
 // with the probe: f32 9.4 / 3.6, cosine 9.5 / 3.5, f64 18.6 / 4.3); the
 // others gather in buf, 128 entries of the wave's own; cols: 16 floats of it.
+// Where a precise scan may follow (a.flag), a query is left to it, and false
+// returned, once it has evaluated a 32nd of the index: that is what its share
+// of that scan costs (f64, 200k x 5k in clusters as above, ms: 100 of them, d =
+// 128: 4.3 this way, 6.0 by the scan; 5 of them, d = 250: 79.5 and 12.0).
 template <typename T, typename TS, int ARM, int KL>
-__device__ __forceinline__ void gm_pass(GmList<T, TS, ARM, KL>& L, const GmQuery<TS>& Q, const GmSelectArgs<TS>& a,
+__device__ __forceinline__ bool gm_pass(GmList<T, TS, ARM, KL>& L, const GmQuery<T, TS, ARM>& Q, const GmSelectArgs<TS>& a,
                                         int64_t q, const T* __restrict__ sq, float thr, int wv, int nw,
-                                        volatile float* __restrict__ shared, float* __restrict__ cols,
-                                        uint32_t* __restrict__ buf, int lane) {
+                                        volatile float* __restrict__ shared, volatile int* __restrict__ stop,
+                                        float* __restrict__ cols, uint32_t* __restrict__ buf, int lane) {
     using List = GmList<T, TS, ARM, KL>;
-    constexpr bool METRIC = !List::COS && ARM != ARM_EUCLID_FMA && ARM != ARM_EUCLID_MULADD;
+    constexpr bool METRIC = GmQuery<T, TS, ARM>::exact;
     const int d = (int)a.d, k = a.k, mode = a.mode;
     const float inf = __builtin_huge_valf();
     const bool ranked = List::MINK && mode == EMIT_ROOT_RANKED;
     const uint64_t below = (1ull << lane) - 1ull;
     uint32_t held = 0;
-    auto pass = [&](auto rules_out) {
+    // batches of 64 rows left to this wave
+    const bool bounded = GmQuery<T, TS, ARM>::twice && a.flag;
+    int batches = bounded ? ((int)(Q.nt / 2048u) + 16) / nw : 0;
+    auto pass = [&](auto rules_out) -> bool {
         for (int f0 = 64 * wv; f0 < Q.n; f0 += 64 * nw) {
+            if (bounded && *stop) return false;
             const float gm = f0 + lane < Q.n ? Q.G[f0 + lane] : inf;
             const uint32_t row = L.row0 + Q.first_row(f0 + lane);
             const T least = (T)Q.least(gm, ranked);
@@ -414,20 +452,27 @@ __device__ __forceinline__ void gm_pass(GmList<T, TS, ARM, KL>& L, const GmQuery
                     mine = buf[held + lane];
                     wave_lds_fence();
                     L.evaluate(mine, sq, a.x, d, k, mode, lane);
-                    thr = fminf(thr, L.screen_bound(k, mode, Q.qn, Q.eps, a.eps_t));
+                    thr = fminf(thr, L.screen_bound(Q));
                     todo &= open();
+                    if (bounded && --batches < 0) {
+                        *stop = 1;
+                        return false;
+                    }
                 }
             }
             if (lane == 0) shared[wv] = thr;
         }
+        return true;
     };
     if constexpr (METRIC) {
         pass([](uint32_t) { return false; });
     } else {
         const GmProbe<TS, List::COS> probe(a, q, cols, lane);
-        pass([&](uint32_t r) { return probe.share(r, a.xinv[r]) > probe.limit(thr, Q.qn, Q.eps); });
+        if (!pass([&](uint32_t r) { return probe.share(r, a.xinv[r]) > probe.limit(thr, Q.base, Q.qn, Q.eps); }))
+            return false;
     }
     if (held) L.evaluate((uint32_t)lane < held ? buf[lane] : kSentinelIdx, sq, a.x, d, k, mode, lane);
+    return true;
 }
 
 // The forced rows, where there are more than are listed: a wave's share of the
@@ -474,15 +519,19 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
     __shared__ uint32_t s_cnt;
     __shared__ float s_kth;
     __shared__ float s_wthr[4];
+    __shared__ int s_stop;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t q = blockIdx.x;
+    const int64_t at_ = blockIdx.x;  // the query's place among those of the launch
+    const bool listed = GmQuery<T, TS, ARM>::twice && a.list;
+    if (listed && at_ >= (int64_t)a.stats->nflag) return;
+    const int64_t q = listed ? (int64_t)a.list[at_] : at_;
     const int d = (int)a.d, k = a.k, mode = a.mode;
     const TS* __restrict__ X = a.x;
     const float inf = __builtin_huge_valf();
-    const GmQuery<TS> Q(a, q);
+    GmQuery<T, TS, ARM> Q(a, q, at_);
     const int n = Q.n;
     GmList<T, TS, ARM, KL> L(a);
     T* const ov = static_cast<T*>(a.out_val) + q * k;
@@ -491,7 +540,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
     float carried = inf;
     if (!a.first) {
         L.resume(ov, oi, k, lane);
-        carried = L.screen_bound(k, mode, Q.qn, Q.eps, a.eps_t);
+        carried = L.screen_bound(Q);
         if (wv > 0) L = GmList<T, TS, ARM, KL>(a);
     }
     if (tid < d) sq[tid] = (T)a.q[q * d + tid];
@@ -586,7 +635,7 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
                     if (at < count && rank_of(v[j], at, count) == k - 1) s_kth = v[j];
                 }
                 __syncthreads();
-                thr = fminf(Q.bound(s_kth), carried);
+                thr = fminf(Q.bound_again(s_kth), carried);
                 if (tid == 0) s_cnt = 0u;
                 __syncthreads();
 #pragma unroll
@@ -600,9 +649,21 @@ __global__ __launch_bounds__(256, 4) void gm_select_kernel(GmSelectArgs<TS> a) {
                 L.evaluate(at < count ? Q.row((int)cg[at], lane & 15) : kSentinelIdx, sq, X, d, k, mode, lane);
             }
         } else {
+            if (GmQuery<T, TS, ARM>::twice && a.flag && (uint32_t)count > a.flag_above) {
+                if (tid == 0) a.flag[atomicAdd(&a.stats->nflag, 1u)] = (uint32_t)q;
+                return;
+            }
             if (tid < 4) s_wthr[tid] = thr;
+            if (tid == 0) s_stop = 0;
             __syncthreads();
-            gm_pass<T, TS, ARM, KL>(L, Q, a, q, sq, thr, wv, 4, s_wthr, cm + 16 * wv, cg + 320 * wv, lane);
+            gm_pass<T, TS, ARM, KL>(L, Q, a, q, sq, thr, wv, 4, s_wthr, &s_stop, cm + 16 * wv, cg + 320 * wv, lane);
+            if (GmQuery<T, TS, ARM>::twice && a.flag) {
+                __syncthreads();
+                if (s_stop) {
+                    if (tid == 0) a.flag[atomicAdd(&a.stats->nflag, 1u)] = (uint32_t)q;
+                    return;
+                }
+            }
         }
     }
 
@@ -639,8 +700,10 @@ __global__ __launch_bounds__(256, gm_select_waves(ARM, KL)) void gm_select_wave_
     __shared__ uint32_t cg_[4][kSelWaveCap + 64];
     const int lane = threadIdx.x & 63;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t q = (int64_t)blockIdx.x * 4 + wv;
-    if (q >= a.nq) return;
+    const int64_t at_ = (int64_t)blockIdx.x * 4 + wv;  // the query's place among those of the launch
+    const bool listed = GmQuery<T, TS, ARM>::twice && a.list;
+    if (at_ >= (listed ? (int64_t)a.stats->nflag : a.nq)) return;
+    const int64_t q = listed ? (int64_t)a.list[at_] : at_;
     T* __restrict__ sq = sq_[wv];
     float* __restrict__ cm = cm_[wv];
     uint32_t* __restrict__ cg = cg_[wv];
@@ -648,7 +711,7 @@ __global__ __launch_bounds__(256, gm_select_waves(ARM, KL)) void gm_select_wave_
     const TS* __restrict__ X = a.x;
     const float inf = __builtin_huge_valf();
     const uint64_t below = (1ull << lane) - 1ull;
-    const GmQuery<TS> Q(a, q);
+    GmQuery<T, TS, ARM> Q(a, q, at_);
     const int n = Q.n;
     GmList<T, TS, ARM, KL> L(a);
     T* const ov = static_cast<T*>(a.out_val) + q * k;
@@ -656,7 +719,7 @@ __global__ __launch_bounds__(256, gm_select_waves(ARM, KL)) void gm_select_wave_
     float carried = inf;  // what the earlier parts' list bounds
     if (!a.first) {
         L.resume(ov, oi, k, lane);
-        carried = L.screen_bound(k, mode, Q.qn, Q.eps, a.eps_t);
+        carried = L.screen_bound(Q);
     }
     for (int c = lane; c < d; c += 64) sq[c] = (T)a.q[q * d + c];
     wave_lds_fence();
@@ -757,7 +820,7 @@ __global__ __launch_bounds__(256, gm_select_waves(ARM, KL)) void gm_select_wave_
                 if constexpr (KL == 1) wave_merge64<float>(bv[0], bi[0], v, ix, lane);
                 else wave_merge_blocks<float, KL>(bv, bi, v, ix, lane);
             }
-            thr = fminf(Q.bound(list_value_at<float, KL>(bv, k - 1)), carried);
+            thr = fminf(Q.bound_again(list_value_at<float, KL>(bv, k - 1)), carried);
             uint32_t kept = 0;
             for (uint32_t b0 = 0; b0 < cnt; b0 += 64) {
                 const bool in = b0 + lane < cnt && cm[b0 + lane] <= thr;
@@ -775,10 +838,21 @@ __global__ __launch_bounds__(256, gm_select_waves(ARM, KL)) void gm_select_wave_
             L.evaluate(at < cnt ? Q.row((int)cg[at], lane & 15) : kSentinelIdx, sq, X, d, k, mode, lane);
         }
     } else {
+        if (GmQuery<T, TS, ARM>::twice && a.flag && cnt > a.flag_above) {
+            if (lane == 0) a.flag[atomicAdd(&a.stats->nflag, 1u)] = (uint32_t)q;
+            return;
+        }
         // the list of one wave bounds itself
-        if (lane == 0) cm[16] = thr;
+        if (lane == 0) {
+            cm[16] = thr;
+            cm[17] = 0.0f;
+        }
         wave_lds_fence();
-        gm_pass<T, TS, ARM, KL>(L, Q, a, q, sq, thr, 0, 1, cm + 16, cm, cg, lane);
+        if (!gm_pass<T, TS, ARM, KL>(L, Q, a, q, sq, thr, 0, 1, cm + 16, reinterpret_cast<volatile int*>(cm + 17), cm, cg,
+                                     lane)) {
+            if (lane == 0) a.flag[atomicAdd(&a.stats->nflag, 1u)] = (uint32_t)q;
+            return;
+        }
     }
     L.emit(ov, oi, k, mode, a.last, lane);
 }

@@ -205,3 +205,49 @@ def test_outliers(dtype, nq, scale):
     xq[30:38] = xt[200:208]
     _check(xq, xt, 20)
     _check(xq, np.ascontiguousarray(xt[90:260]), 100)
+
+
+def _clusters(seed, nt, nq, d, width, count, dtype):
+    rng = np.random.default_rng(seed)
+    centres = rng.uniform(-10, 10, (count, d))
+    return tuple((centres[rng.integers(0, count, n)] + width * rng.standard_normal((n, d))).astype(dtype) for n in (nt, nq))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("metric", ["euclidean", "cosine"])
+@pytest.mark.parametrize("nt,nq,d,k", [(30_000, 40, 20, 10), (6_000, 1_100, 37, 100), (30_100, 1_003, 5, 24)])
+@pytest.mark.parametrize("width", [1e-2, 1e-5])
+def test_clusters_past_the_lists(dtype, metric, nt, nq, d, k, width):
+    """Clusters of more groups than are listed: the pass over the groups, its
+    probe and its gathered rows, in both selections."""
+    xt, xq = _clusters(nt + d, nt, nq, d, width, 3, dtype)
+    xt[nt - 100:nt - 50] = xt[50:100]
+    _check(xq, xt, k, metric)
+
+
+@pytest.mark.parametrize("dtype,metric", [(np.float64, "euclidean"), (np.float64, "cosine")])
+@pytest.mark.parametrize("d", [3, 31, 33, 64, 100, 150, 193, 256])
+@pytest.mark.parametrize("nt,nq,k", [(100_001, 3_000, 10), (300_000, 1_001, 70)])
+def test_precise_scan(dtype, metric, d, nt, nq, k):
+    """Searches large enough for the second scan: its column counts, partly
+    filled query blocks and tiles, rows left out, flagged queries among others;
+    against the exact tiles."""
+    xt, xq = _clusters(nt + d, nt, nq, d, 1e-3, 4, dtype)
+    rng = np.random.default_rng(d)
+    far = rng.choice(nq, nq // 3, replace=False)
+    xq[far] = rng.uniform(-10, 10, (len(far), d)).astype(dtype)  # not flagged
+    xt[nt - 90:nt - 60] = xt[60:90]
+    xt[17, 0], xt[18, d - 1] = np.nan, np.inf
+    xt[19] *= dtype(1e25)
+    xq[0], xq[1] = xt[19], 0
+    xt, xq = (torch.from_numpy(x).to(DEV) for x in (xt, xq))
+    got = prims.knn_topk(xq, xt, k, metric)
+    prims.force_path("generic")
+    want = prims.knn_topk(xq, xt, k, metric)
+    if metric == "euclidean" and nq == 1_001:  # f32 rows, f64 values
+        x = xt[:20_000].float()
+        wi, wd = prims.knn_graph(x, k, metric)
+        prims.force_path("fused")
+        gi, gd = prims.knn_graph(x, k, metric)
+        assert torch.equal(gi, wi) and torch.equal(gd.view(torch.int64), wd.view(torch.int64))
+    assert torch.equal(got[1], want[1]) and torch.equal(got[0].view(torch.int32), want[0].view(torch.int32))

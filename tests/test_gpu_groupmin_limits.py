@@ -170,3 +170,18 @@ def test_ties_cost_no_pass_over_the_index(dtype, nt, nq, metric):
     else:
         xt, xq = torch.ones_like(xt), torch.ones_like(xq)
     assert _ms(_search(name, xq, xt, 10, metric)) < 3.0 * plain
+
+
+@pytest.mark.parametrize("dtype,metric,limit", [(torch.float32, 0, 30.0), (torch.float32, 1, 30.0),
+                                                (torch.float64, 0, 10.0), (torch.float64, 1, 10.0)])
+def test_clusters_the_screen_does_not_resolve(dtype, metric, limit):
+    """Clusters a thousandth of their spacing wide, where every group has a row of
+    the query's cluster: f64 searches take a second scan in their precision, f32
+    ones evaluate the cluster's rows, neither every row of every group."""
+    name = "mlrs_knn_topk_" + ("f32" if dtype is torch.float32 else "f64")
+    xt, xq = _rows(9, 100_000, 128, dtype), _rows(10, 5_000, 128, dtype)
+    plain = _ms(_search(name, xq, xt, 16, metric))
+    g = torch.Generator(device="cuda").manual_seed(11)
+    centres = 20.0 * torch.rand((20, 128), generator=g, device=DEV, dtype=dtype) - 10.0
+    xt, xq = (centres[torch.randint(0, 20, (x.shape[0],), generator=g, device=DEV)] + 0.01 * x for x in (xt, xq))
+    assert _ms(_search(name, xq, xt, 16, metric)) < limit * plain
