@@ -1066,7 +1066,12 @@ int32_t knn_groupmin_metric(const T* xq, int64_t nq, const T* xt, int64_t nt, in
     se.ntp = ntp;
     se.kind = GM_EXACT;
     se.first = se.last = 1;
-    se.eps_t = std::ldexp(1.0, -21);  // the minima's rounding down to f32 (2^-23) and a root's ties
+    // The minima's rounding down to f32 is 2^-23; a graph ranks by the root, and
+    // values whose roots round to one double (pow's own error taken as 16 ulp)
+    // differ by a factor of up to (1 + 2^-48)^p, or by f32's smallest number.
+    const bool ranked = mode == EMIT_ROOT_RANKED;
+    se.eps_t = std::ldexp(1.0, -21) + (ranked ? std::expm1(std::min(p * std::ldexp(1.0, -46), 700.0)) : 0.0);
+    se.eps_abs = ranked ? std::ldexp(1.0, -148) : 0.0;
     se.pexp = p;
     se.pint = minkowski_powi(p);
     se.root_exp = 1.0 / p;

@@ -202,7 +202,7 @@ struct GmQuery {
     __device__ __forceinline__ float bound(float t) {
         if (!(t < __builtin_huge_valf())) return __builtin_huge_valf();
         const double v = (double)t + a.eps_t * (double)t;
-        if constexpr (exact) return round_up_f(v);
+        if constexpr (exact) return round_up_f(v + a.eps_abs);
         const float b = precise() ? gm_bound_precise(v, qn, xmax, a.eps_rel, a.eps_abs, 2)
                                   : gm_bound(t, qn, xmax, a.eps_rel, eps);
         width = (double)b - (double)t;

@@ -251,3 +251,19 @@ def test_precise_scan(dtype, metric, d, nt, nq, k):
         gi, gd = prims.knn_graph(x, k, metric)
         assert torch.equal(gi, wi) and torch.equal(gd.view(torch.int64), wd.view(torch.int64))
     assert torch.equal(got[1], want[1]) and torch.equal(got[0].view(torch.int32), want[0].view(torch.int32))
+
+
+@pytest.mark.parametrize("p", [3.0, 2.0 ** 36, 2.0 ** 40])
+def test_root_ties_of_large_exponents(p):
+    """Sums that differ by more than the minima's rounding and whose roots are one
+    double: the graph ranks them by index."""
+    rng = np.random.default_rng(3)
+    steps = 0.69 / (p * 2.0 ** -53) if p > 3 else 1e14
+    x = np.stack([np.ones(2000), 1.0 - (np.floor(steps) + rng.integers(0, 31, 2000)) * 2.0 ** -53], 1)
+    x[0] = 0.0
+    x = torch.from_numpy(x).to(DEV)
+    out = []
+    for family in ("auto", "generic"):
+        prims.force_path(family)
+        out.append(prims.knn_graph(x, 15, "minkowski", p=p))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1].view(torch.int64), out[1][1].view(torch.int64))
