@@ -1259,6 +1259,13 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
             const int32_t rc = noalloc_admits(n_query, n_train, n_features, k, vec4, s);
             if (rc) return rc;
         }
+        // k = 1 over a short index of other rows: a pass of the f32 matrix cores
+        // costs less than a selection per query (us, Gram / groups, 300 x 300,000,
+        // d = 50: 301 / 612; 1000 x 200,000, d = 50: 373 / 468; 500,000 x 2,000, d =
+        // 128: 2094 / 857)
+        const bool euclid = arm == ARM_EUCLID_FMA || arm == ARM_EUCLID_MULADD;
+        if (!forced && !small && k == 1 && euclid && n_train * n_features <= 80000)
+            return knn_gram32(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
         return knn_groupmin<float, float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
                                           s);
     }

@@ -1203,25 +1203,28 @@ __global__ void fill_inf_bits_kernel(unsigned int* p, int64_t n) {
 }
 
 template <int NG, bool VEC4>
-hipError_t launch_ng(const GramArgs32& a, hipStream_t s) {
+hipError_t launch_ng(const GramArgs32& a, int arm, hipStream_t s) {
     dim3 grid((unsigned)StreamSplit(a.nq, a.nt, a.qpb, kBn, a.grid_wgs).G);
     const dim3 block(GramShape<(NG > 16)>::threads);
-    hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM_EUCLID_MULADD, false, VEC4, true, 1>), grid, block, 0, s, a);
+    if (arm == ARM_EUCLID_MULADD)
+        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM_EUCLID_MULADD, false, VEC4, true, 1>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM_EUCLID_FMA, false, VEC4, true, 1>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
 template <bool VEC4>
-hipError_t launch_d(const GramArgs32& a, hipStream_t s) {
+hipError_t launch_d(const GramArgs32& a, int arm, hipStream_t s) {
     const int ng = (int)((a.d + 7) / 8);
     // the split and the merge must see the query-block size of the shape
     if (a.qpb != (ng > 16 ? kQpbWide : kQpbNarrow)) return hipErrorInvalidValue;
-    if (ng <= 2) return launch_ng<2, VEC4>(a, s);
-    if (ng <= 4) return launch_ng<4, VEC4>(a, s);
-    if (ng <= 8) return launch_ng<8, VEC4>(a, s);
-    if (ng <= 12) return launch_ng<12, VEC4>(a, s);
-    if (ng <= 16) return launch_ng<16, VEC4>(a, s);
-    if (ng <= 24) return launch_ng<24, VEC4>(a, s);
-    return launch_ng<32, VEC4>(a, s);
+    if (ng <= 2) return launch_ng<2, VEC4>(a, arm, s);
+    if (ng <= 4) return launch_ng<4, VEC4>(a, arm, s);
+    if (ng <= 8) return launch_ng<8, VEC4>(a, arm, s);
+    if (ng <= 12) return launch_ng<12, VEC4>(a, arm, s);
+    if (ng <= 16) return launch_ng<16, VEC4>(a, arm, s);
+    if (ng <= 24) return launch_ng<24, VEC4>(a, arm, s);
+    return launch_ng<32, VEC4>(a, arm, s);
 }
 
 }  // namespace
@@ -1258,10 +1261,10 @@ hipError_t launch_gram_f32_merge(const GramArgs32& a, hipStream_t s) {
 }
 
 hipError_t launch_gram_f32(const GramArgs32& a, int arm, hipStream_t s) {
-    if (a.k != 1 || arm != ARM_EUCLID_MULADD) return hipErrorInvalidValue;
+    if (a.k != 1 || (arm != ARM_EUCLID_MULADD && arm != ARM_EUCLID_FMA)) return hipErrorInvalidValue;
     const bool vec4 = (a.d % 4 == 0) && ((reinterpret_cast<uintptr_t>(a.q) & 15) == 0) &&
                       ((reinterpret_cast<uintptr_t>(a.x) & 15) == 0);
-    return vec4 ? launch_d<true>(a, s) : launch_d<false>(a, s);
+    return vec4 ? launch_d<true>(a, arm, s) : launch_d<false>(a, arm, s);
 }
 
 }  // namespace mlrs

@@ -124,6 +124,9 @@ def test_rows_the_screen_is_not_trusted_with_cost_their_share(dtype, metric):
     (1_000_000, 4_000, 8, 8, "cosine", torch.float64, "knn_groupmin_kernel"),
     (10_000, 1_000, 64, 10, "euclidean", torch.float32, "knn_groupmin_kernel"),
     (3_000, 20_000, 50, 5, "euclidean", torch.float32, "knn_groupmin_kernel"),
+    (300, 300_000, 50, 1, "euclidean", torch.float32, "knn_gram_f32_kernel"),
+    (300, 120_000, 130, 1, "euclidean", torch.float32, "knn_gram_f32_kernel"),
+    (500_000, 2_000, 50, 1, "euclidean", torch.float32, "knn_groupmin_kernel"),
     (60_000, 2_000, 40, 10, "manhattan", torch.float64, "groupmin_tile_kernel")])
 def test_family_chosen(nt, nq, d, k, metric, dtype, kernel):
     """Small indexes and few columns go where they were measured fastest, and
