@@ -581,15 +581,15 @@ static int pick_path(bool lowd_ok, bool gram_ok) {
     return MLRS_PATH_AUTO;
 }
 
-// qsq_pre: the queries' row_sumsq when the caller already holds them (the
-// k-means loop assigns the same rows every iteration); Euclidean arms only.
-int32_t knn_gram32(const float* xq, int64_t nq, const float* xt, int64_t nt, int64_t d, int k, int arm,
-                   int mode, float* out_v, uint32_t* out_i, hipStream_t s, const float* qsq_pre = nullptr) {
-    const bool cos = (arm == ARM_COS_FOLD || arm == ARM_COS_HOST);
-    const bool host_cos = arm == ARM_COS_HOST;
+// The nearest row (k = 1) under a Euclidean arm: the resident search where a few
+// workgroups' LDS holds the index, else the Gram kernel (d <= 256).  qsq_pre: the
+// queries' row_sumsq when the caller already holds them (the k-means loop
+// assigns the same rows every iteration).
+int32_t knn_gram32(const float* xq, int64_t nq, const float* xt, int64_t nt, int64_t d, int arm, int mode,
+                   float* out_v, uint32_t* out_i, hipStream_t s, const float* qsq_pre = nullptr) {
     // sizes that do not depend on the strip count
-    size_t fixed = 2 * aligned_bytes(sizeof(float) * nq) + 3 * aligned_bytes(sizeof(float) * nt) +
-                   aligned_bytes(sizeof(NormStats)) + 1024;
+    const size_t fixed = aligned_bytes(sizeof(float) * nq) + aligned_bytes(sizeof(float) * nt) +
+                         aligned_bytes(sizeof(NormStats)) + 1024;
     char* ws;
     int cus;
     int32_t rc = workspace(fixed, s, &ws, &cus);
@@ -598,62 +598,47 @@ int32_t knn_gram32(const float* xq, int64_t nq, const float* xt, int64_t nt, int
     int nslots = 1;
     const bool vec4 = (d % 4 == 0) && ((reinterpret_cast<uintptr_t>(xq) & 15) == 0) &&
                       ((reinterpret_cast<uintptr_t>(xt) & 15) == 0);
-    gram_f32_split(nq, nt, d, k, cus, vec4, &grid_wgs, &nslots);
-    // k = 1 over an index that a few workgroups' LDS holds: the resident
-    // search (knn_k1_resident.hip), one list slot per chunk
-    const int res_chunks = gram_f32_k1_resident_chunks(nq, nt, d, k, arm, vec4);
-    // per-(segment slot, query) lists: the kernel's top-k state, merged at the end
-    size_t parts = (size_t)std::max<int64_t>(nslots, res_chunks) * nq * gram_list_cap(k);
-    size_t qvals = res_chunks ? (gram_f32_k1_resident_queue_bytes(cus) + sizeof(float) - 1) / sizeof(float) : 0;
-    size_t bytes = fixed + aligned_bytes(parts * sizeof(float)) + aligned_bytes(parts * sizeof(uint32_t)) +
-                   aligned_bytes(qvals * sizeof(float)) + aligned_bytes(sizeof(unsigned int) * nq);
-    rc = workspace(bytes, s, &ws, &cus);
+    gram_f32_split(nq, nt, d, cus, &grid_wgs, &nslots);
+    // one pair per (segment or chunk, query)
+    const int res_chunks = gram_f32_k1_resident_chunks(nq, nt, d, 1, arm, vec4);
+    const size_t parts = (size_t)std::max<int64_t>(nslots, res_chunks) * nq;
+    const size_t qvals = res_chunks ? (gram_f32_k1_resident_queue_bytes(cus) + sizeof(float) - 1) / sizeof(float) : 0;
+    rc = workspace(fixed + aligned_bytes(parts * sizeof(float)) + aligned_bytes(parts * sizeof(uint32_t)) +
+                       aligned_bytes(qvals * sizeof(float)) + aligned_bytes(sizeof(unsigned int) * nq),
+                   s, &ws, &cus);
     if (rc) return rc;
     Carver cv(ws);
     GramArgs32 a;
     std::memset(&a, 0, sizeof(a));
     float* qsq = cv.take<float>(nq);
-    float* qinv = cv.take<float>(nq);
     float* xsq = cv.take<float>(nt);
-    float* xinv = cv.take<float>(nt);
-    float* xscale = cv.take<float>(nt);
     NormStats* stats = cv.take<NormStats>(1);
     hipError_t e = hipSuccess;
-    // the resident k = 1 search forms the query norms from its operand
+    // the resident search forms the query norms from its operand
     const bool res_qsq = res_chunks && !qsq_pre;
-    if (qsq_pre && !cos)
+    if (qsq_pre)
         qsq = const_cast<float*>(qsq_pre);  // only read
     else if (!res_qsq)
-        e = launch_row_norms<float>(xq, nq, d, qsq, host_cos ? qinv : nullptr, nullptr, nullptr, s);
-    if (e == hipSuccess)
-        e = launch_row_norms<float>(xt, nt, d, xsq, host_cos ? xinv : nullptr, cos ? xscale : nullptr, stats, s);
+        e = launch_row_norms<float>(xq, nq, d, qsq, nullptr, nullptr, nullptr, s);
+    if (e == hipSuccess) e = launch_row_norms<float>(xt, nt, d, xsq, nullptr, nullptr, stats, s);
     if (e != hipSuccess) return hip_err(e, "row_norms");
     a.q = xq;
     a.nq = nq;
     a.x = xt;
     a.nt = nt;
     a.d = d;
-    a.k = k;
+    a.k = 1;
     a.mode = mode;
     a.qsq = qsq;
     a.xsq = xsq;
-    a.xscale = xscale;
-    a.qinv = host_cos ? qinv : nullptr;
-    a.xinv = host_cos ? xinv : nullptr;
     a.stats = stats;
     // Screen bounds (see knn_gram_f32.hip): with u = 2^-23 (covers any
     // rounding mode of the matrix core) the expansion's and the reference's
-    // rounding errors together stay below 6(d+3)u(||q||^2 + ||x||^2) for
-    // Euclidean and (4d+11)u for cosine; the bounds used are 8(d+4)u and
-    // (8d+32)u, plus an absolute floor for flushed subnormal products.
+    // rounding errors together stay below 6(d+3)u(||q||^2 + ||x||^2); the bound
+    // used is 8(d+4)u, plus an absolute floor for flushed subnormal products.
     const double u = std::ldexp(1.0, -23);
-    if (!cos) {
-        a.eps_rel = 8.0 * (double)(d + 4) * u;
-        a.eps_abs = (double)(d + 4) * std::ldexp(1.0, -120);
-    } else {
-        a.eps_rel = 0.0;
-        a.eps_abs = (8.0 * (double)d + 32.0) * u;
-    }
+    a.eps_rel = 8.0 * (double)(d + 4) * u;
+    a.eps_abs = (double)(d + 4) * std::ldexp(1.0, -120);
     a.grid_wgs = grid_wgs;
     a.nslots = nslots;
     a.qpb = gram_f32_queries_per_block(d);
@@ -689,11 +674,11 @@ int32_t knn_gram32(const float* xq, int64_t nq, const float* xt, int64_t nt, int
     return ok();
 }
 
-int32_t knn_gram64(const double* xq, int64_t nq, const double* xt, int64_t nt, int64_t d, int k, int arm,
-                   int mode, double* out_v, uint32_t* out_i, hipStream_t s, const double* qsq_pre = nullptr) {
-    const bool cos = (arm == ARM_COS_FOLD || arm == ARM_COS_HOST);
-    size_t fixed = 2 * aligned_bytes(sizeof(double) * nq) + 3 * aligned_bytes(sizeof(double) * nt) +
-                   aligned_bytes(sizeof(NormStats)) + 1024;
+// The k-means assignment's nearest centre in f64 (d <= 256).
+int32_t knn_gram64(const double* xq, int64_t nq, const double* xt, int64_t nt, int64_t d, int mode, double* out_v,
+                   uint32_t* out_i, hipStream_t s, const double* qsq_pre = nullptr) {
+    const size_t fixed = aligned_bytes(sizeof(double) * nq) + aligned_bytes(sizeof(double) * nt) +
+                         aligned_bytes(sizeof(NormStats)) + 1024;
     char* ws;
     int cus;
     int32_t rc = workspace(fixed, s, &ws, &cus);
@@ -701,64 +686,50 @@ int32_t knn_gram64(const double* xq, int64_t nq, const double* xt, int64_t nt, i
     int64_t grid_wgs = 1;
     int nslots = 1;
     gram_f64_split(nq, nt, cus, &grid_wgs, &nslots);
-    size_t parts = (size_t)nslots * nq * gram_list_cap(k);
-    size_t qvals = gram_f64_qval_elems(grid_wgs);
-    size_t bytes = fixed + aligned_bytes(parts * sizeof(double)) + aligned_bytes(parts * sizeof(uint32_t)) +
-                   aligned_bytes(qvals * sizeof(double)) + aligned_bytes(sizeof(unsigned long long) * nq);
-    rc = workspace(bytes, s, &ws, &cus);
+    const size_t parts = (size_t)nslots * nq;
+    rc = workspace(fixed + aligned_bytes(parts * sizeof(double)) + aligned_bytes(parts * sizeof(uint32_t)) +
+                       aligned_bytes(sizeof(unsigned long long) * nq),
+                   s, &ws, &cus);
     if (rc) return rc;
     Carver cv(ws);
     GramArgs64 a;
     std::memset(&a, 0, sizeof(a));
     double* qsq = cv.take<double>(nq);
-    double* qinv = cv.take<double>(nq);
     double* xsq = cv.take<double>(nt);
-    double* xinv = cv.take<double>(nt);
-    double* xscale = cv.take<double>(nt);
     NormStats* stats = cv.take<NormStats>(1);
     hipError_t e = hipSuccess;
-    if (qsq_pre && !cos)
-        qsq = const_cast<double*>(qsq_pre);  // only read; qinv serves cosine only
+    if (qsq_pre)
+        qsq = const_cast<double*>(qsq_pre);  // only read
     else
-        e = launch_row_norms<double>(xq, nq, d, qsq, qinv, nullptr, nullptr, s);
-    if (e == hipSuccess) e = launch_row_norms<double>(xt, nt, d, xsq, xinv, xscale, stats, s);
+        e = launch_row_norms<double>(xq, nq, d, qsq, nullptr, nullptr, nullptr, s);
+    if (e == hipSuccess) e = launch_row_norms<double>(xt, nt, d, xsq, nullptr, nullptr, stats, s);
     if (e != hipSuccess) return hip_err(e, "row_norms");
     a.q = xq;
     a.nq = nq;
     a.x = xt;
     a.nt = nt;
     a.d = d;
-    a.k = k;
     a.mode = mode;
     a.qsq = qsq;
     a.xsq = xsq;
-    a.qinv = qinv;
-    a.xinv = xinv;
-    a.xscale = xscale;
     a.stats = stats;
-    // Screen bounds as for f32 with u = 2^-52, plus 16u (Euclidean, relative)
-    // and 16u (cosine, absolute) for the rounding of the threshold arithmetic
-    // itself, which the f64 kernel does in double.
+    // Screen bounds as for f32 with u = 2^-52, plus 16u (relative) for the
+    // rounding of the threshold arithmetic itself, which the f64 kernel does in
+    // double.
     const double u = std::ldexp(1.0, -52);
-    if (!cos) {
-        a.eps_rel = (8.0 * (double)(d + 4) + 16.0) * u;
-        a.eps_abs = (double)(d + 4) * std::ldexp(1.0, -1000);
-    } else {
-        a.eps_rel = 0.0;
-        a.eps_abs = (8.0 * (double)d + 48.0) * u;
-    }
+    a.eps_rel = (8.0 * (double)(d + 4) + 16.0) * u;
+    a.eps_abs = (double)(d + 4) * std::ldexp(1.0, -1000);
     a.grid_wgs = grid_wgs;
     a.nslots = nslots;
     a.part_val = cv.take<double>(parts);
     a.part_idx = cv.take<uint32_t>(parts);
-    a.qval = cv.take<double>(qvals);
     a.shared_r = cv.take<unsigned long long>(nq);
     a.out_val = out_v;
     a.out_idx = out_i;
     e = launch_gram_f64_prep(a, s);
     if (e == hipSuccess) {
         KernelTimer timer(s, "knn_gram_f64_kernel");
-        e = launch_gram_f64(a, arm, s);
+        e = launch_gram_f64(a, ARM_EUCLID_MULADD, s);
     }
     if (e == hipSuccess) e = launch_gram_f64_merge(a, s);
     if (e != hipSuccess) return hip_err(e, "knn_gram_f64");
@@ -784,14 +755,18 @@ int32_t noalloc_admits(int64_t nq, int64_t nt, int64_t d, int64_t k, bool vec4, 
     int cus;
     int32_t rc = workspace(256, s, &ws, &cus);
     if (rc) return rc;
-    int64_t grid_wgs = 1;
-    int nslots = 1;
-    gram_f32_split(nq, nt, d, (int)k, cus, vec4, &grid_wgs, &nslots);
-    const size_t parts = (size_t)nslots * nq * gram_list_cap((int)k);
+    // one resident round of workgroups, at least 16 tiles of 32 rows each; a
+    // list is one block of 64 pairs, k + 32 of them past k = 64
+    const int64_t qpb = gram_f32_queries_per_block(d), ng = (d + 7) / 8;
+    const int64_t per_cu = (k == 1 ? ng <= 8 : ng <= 16 || vec4) ? 3 : 2;
+    const int64_t wgs =
+        std::max<int64_t>(1, std::min<int64_t>(per_cu * std::max(cus, 1), StreamSplit(nq, nt, qpb, 32, 1).T / 16));
+    const size_t slots = (size_t)StreamSplit(nq, nt, qpb, 32, wgs).nslots();
+    const size_t list = k == 1 ? 1 : k <= 64 ? std::min<size_t>((size_t)k + 32, 64) : (size_t)k + 32;
+    const size_t queue = 2 * 4 * 32 * (size_t)(k > 64 ? 128 : 64);
     return workspace(2 * aligned_bytes(sizeof(float) * nq) + 3 * aligned_bytes(sizeof(float) * nt) +
-                         2 * aligned_bytes(parts * sizeof(float)) +
-                         (k > 1 ? aligned_bytes(gram_f32_qval_elems(grid_wgs, (int)k) * sizeof(float)) +
-                                      aligned_bytes((size_t)nslots * nq * sizeof(float4))
+                         2 * aligned_bytes(slots * nq * list * sizeof(float)) +
+                         (k > 1 ? aligned_bytes(wgs * queue * sizeof(float)) + aligned_bytes(slots * nq * sizeof(float4))
                                 : 0) +
                          aligned_bytes(sizeof(unsigned int) * nq) + aligned_bytes(sizeof(NormStats)) + 1024,
                      s, &ws, &cus);
@@ -1252,7 +1227,7 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
                           ((reinterpret_cast<uintptr_t>(x_train) & 15) == 0);
         // k = 1 over an index that fits a few workgroups' LDS: resident there
         if ((forced || !small) && gram_f32_k1_resident_chunks(n_query, n_train, n_features, k, arm, vec4) > 0)
-            return knn_gram32(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
+            return knn_gram32(xq, n_query, x_train, n_train, n_features, arm, mode, out_dist, out_idx, s);
         const bool few_columns = lowd_ok && (k <= 8 || (k <= 16 && n_features <= 11) ||
                                              (n_features <= 3 && metric == MLRS_METRIC_EUCLIDEAN));
         if (g_noalloc && (forced || !(small || few_columns))) {
@@ -1265,7 +1240,7 @@ int32_t knn_topk_f32_dispatch(const float* xq, int64_t n_query, int64_t n_featur
         // 128: 2094 / 857)
         const bool euclid = arm == ARM_EUCLID_FMA || arm == ARM_EUCLID_MULADD;
         if (!forced && !small && k == 1 && euclid && n_train * n_features <= 80000)
-            return knn_gram32(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx, s);
+            return knn_gram32(xq, n_query, x_train, n_train, n_features, arm, mode, out_dist, out_idx, s);
         return knn_groupmin<float, float>(xq, n_query, x_train, n_train, n_features, k, arm, mode, out_dist, out_idx,
                                           s);
     }
@@ -1420,7 +1395,7 @@ int32_t mlrs_kmeans_assign_f32(const float* x, int64_t x_len, int64_t n, int64_t
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
     if (n_features <= gram_f32_max_d() && pick_path(false, true) != MLRS_PATH_GENERIC)
-        return knn_gram32(x, n, centers, n_centers, n_features, 1, ARM_EUCLID_MULADD, EMIT_KMEANS, sqdist, labels,
+        return knn_gram32(x, n, centers, n_centers, n_features, ARM_EUCLID_MULADD, EMIT_KMEANS, sqdist, labels,
                           s);
     return kmeans_generic<float>(x, n, centers, n_centers, n_features, labels, sqdist, s);
 }
@@ -1433,7 +1408,7 @@ int32_t mlrs_kmeans_assign_f64(const double* x, int64_t x_len, int64_t n, int64_
                                          labels_len, sqdist, dist_len);
     if (rc) return rc;
     if (n_features <= gram_f64_max_d() && pick_path(false, true) != MLRS_PATH_GENERIC)
-        return knn_gram64(x, n, centers, n_centers, n_features, 1, ARM_EUCLID_MULADD, EMIT_KMEANS, sqdist, labels,
+        return knn_gram64(x, n, centers, n_centers, n_features, EMIT_KMEANS, sqdist, labels,
                           (hipStream_t)stream);
     return kmeans_generic<double>(x, n, centers, n_centers, n_features, labels, sqdist, (hipStream_t)stream);
 }
@@ -2303,13 +2278,13 @@ extern "C++" {
 static int32_t km_assign(const float* x, int64_t n, const float* c, int64_t k, int64_t d, uint32_t* labels,
                          float* dist, hipStream_t s, const float* xsq = nullptr) {
     if (d <= gram_f32_max_d() && pick_path(false, true) != MLRS_PATH_GENERIC)
-        return knn_gram32(x, n, c, k, d, 1, ARM_EUCLID_MULADD, EMIT_KMEANS, dist, labels, s, xsq);
+        return knn_gram32(x, n, c, k, d, ARM_EUCLID_MULADD, EMIT_KMEANS, dist, labels, s, xsq);
     return kmeans_generic<float>(x, n, c, k, d, labels, dist, s);
 }
 static int32_t km_assign(const double* x, int64_t n, const double* c, int64_t k, int64_t d, uint32_t* labels,
                          double* dist, hipStream_t s, const double* xsq = nullptr) {
     if (d <= gram_f64_max_d() && pick_path(false, true) != MLRS_PATH_GENERIC)
-        return knn_gram64(x, n, c, k, d, 1, ARM_EUCLID_MULADD, EMIT_KMEANS, dist, labels, s, xsq);
+        return knn_gram64(x, n, c, k, d, EMIT_KMEANS, dist, labels, s, xsq);
     return kmeans_generic<double>(x, n, c, k, d, labels, dist, s);
 }
 

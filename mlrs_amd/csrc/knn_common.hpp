@@ -312,96 +312,6 @@ __device__ __forceinline__ void wave_merge64(T& lv, uint32_t& li, T v, uint32_t 
     for (int m = 32; m > 0; m >>= 1) bitonic_step<T>(lv, li, lane, m, true);
 }
 
-// wave_merge64 that also returns the smallest value it discards (the upper
-// half of the union), +inf when only sentinels are discarded.  Values must
-// not be NaN.
-template <typename T>
-__device__ __forceinline__ T wave_merge64_drop(T& lv, uint32_t& li, T v, uint32_t ix, int lane) {
-    T rv = reverse_f(v);
-    uint32_t ri = reverse_u(ix);
-    const bool take = pair_less<T>(rv, ri, lv, li);
-    const T dv0 = take ? lv : rv;
-    lv = take ? rv : lv;
-    li = take ? ri : li;
-    T dv = dv0;
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) bitonic_step<T>(lv, li, lane, m, true);
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) {
-        const T o = shfl_xor_f(dv, m);
-        dv = (o < dv) ? o : dv;
-    }
-    return dv;
-}
-
-// ---------------------------------------------------------------------------
-// The same machinery on 64-bit keys: for f32 values the (value, index) order
-// is the unsigned order of (orderable value bits << 32 | index), so one
-// 64-bit compare replaces the two-part comparison.
-// ---------------------------------------------------------------------------
-
-// Order-preserving map of float bits to unsigned (negative values flipped).
-__device__ __forceinline__ uint32_t f32_order_bits(float v) {
-    const uint32_t u = __float_as_uint(v + 0.0f);  // -0 -> +0: equal values order by index
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ __forceinline__ float f32_from_order_bits(uint32_t o) {
-    return __uint_as_float((o & 0x80000000u) ? (o & 0x7FFFFFFFu) : ~o);
-}
-__device__ __forceinline__ unsigned long long pair_key(float v, uint32_t ix) {
-    return ((unsigned long long)f32_order_bits(v) << 32) | ix;
-}
-__device__ __forceinline__ float key_value(unsigned long long key) { return f32_from_order_bits((uint32_t)(key >> 32)); }
-__device__ __forceinline__ uint32_t key_index(unsigned long long key) { return (uint32_t)key; }
-constexpr unsigned long long kKeyEmpty = 0xFF800000FFFFFFFFull;  // (+inf, sentinel index)
-
-__device__ __forceinline__ unsigned long long xor_lane_key(unsigned long long v, int m) {
-    return ((unsigned long long)xor_lane_u((uint32_t)(v >> 32), m) << 32) | xor_lane_u((uint32_t)v, m);
-}
-
-// Compare-exchange with lane ^ m.  Equal keys may be exchanged: they are
-// the same pair (or both empty), so the sequence is unchanged.
-__device__ __forceinline__ void bitonic_step_key(unsigned long long& v, int lane, int m, bool up) {
-    const unsigned long long o = xor_lane_key(v, m);
-    const bool first = (((lane & m) == 0) == up);
-    const bool take = (o < v) == first;
-    v = take ? o : v;
-}
-
-__device__ __forceinline__ void wave_sort64_key(unsigned long long& v, int lane) {
-#pragma unroll
-    for (int size = 2; size <= 64; size <<= 1) {
-        const bool up = (lane & size) == 0 || size == 64;
-#pragma unroll
-        for (int m = size >> 1; m > 0; m >>= 1) bitonic_step_key(v, lane, m, up);
-    }
-}
-
-// Merge the ascending sequence v into the ascending list lv (the 64 smallest
-// keys of the union stay in lv) and return the smallest key discarded.
-__device__ __forceinline__ unsigned long long wave_merge64_key_drop(unsigned long long& lv, unsigned long long v,
-                                                                    int lane) {
-    const unsigned long long r =
-        ((unsigned long long)reverse_lane_u((uint32_t)(v >> 32)) << 32) | reverse_lane_u((uint32_t)v);
-    unsigned long long dv = (r < lv) ? lv : r;
-    lv = (r < lv) ? r : lv;
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) bitonic_step_key(lv, lane, m, true);
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) {
-        const unsigned long long o = xor_lane_key(dv, m);
-        dv = (o < dv) ? o : dv;
-    }
-    return dv;
-}
-__device__ __forceinline__ void wave_merge64_key(unsigned long long& lv, unsigned long long v, int lane) {
-    const unsigned long long r =
-        ((unsigned long long)reverse_lane_u((uint32_t)(v >> 32)) << 32) | reverse_lane_u((uint32_t)v);
-    lv = (r < lv) ? r : lv;
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) bitonic_step_key(lv, lane, m, true);
-}
-
 // ---------------------------------------------------------------------------
 // Lists longer than a wave: NB blocks, element 64 r + lane in block r, the
 // whole list ascending.  A sorted 64-lane sequence is merged in block by
@@ -410,75 +320,17 @@ __device__ __forceinline__ void wave_merge64_key(unsigned long long& lv, unsigne
 // of block r, so the smallest 64 of everything from block r on lie in block r
 // or the carry).  Each step is a half-cleaner of the bitonic union.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ unsigned long long reverse_key(unsigned long long v) {
-    return ((unsigned long long)reverse_lane_u((uint32_t)(v >> 32)) << 32) | reverse_lane_u((uint32_t)v);
-}
-__device__ __forceinline__ void bitonic_clean_key(unsigned long long& v, int lane) {
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) bitonic_step_key(v, lane, m, true);
-}
-__device__ __forceinline__ uint32_t key_hi_u(unsigned long long v) { return (uint32_t)(v >> 32); }
-
-// Merge the ascending 64-lane sequence v into the NB-block list lv; the
-// 64 NB smallest keys stay, ascending, and the smallest discarded key is
-// returned (kKeyEmpty-like keys when only empties are discarded).  A block
-// whose largest key is below the carry's smallest is left as it is.
-template <int NB>
-__device__ __forceinline__ unsigned long long wave_merge_blocks_key_drop(unsigned long long (&lv)[NB],
-                                                                         unsigned long long v, int lane) {
-    unsigned long long carry = v;
-#pragma unroll
-    for (int r = 0; r < NB; ++r) {
-        if (NB > 1) {
-            // both keys are wave-uniform after the readlanes: a uniform branch
-            const unsigned long long cmin = ((unsigned long long)bcast_u(key_hi_u(carry), 0) << 32) |
-                                            bcast_u((uint32_t)carry, 0);
-            const unsigned long long bmax = ((unsigned long long)bcast_u(key_hi_u(lv[r]), 63) << 32) |
-                                            bcast_u((uint32_t)lv[r], 63);
-            if (bmax < cmin) continue;
-        }
-        const unsigned long long rc = reverse_key(carry);
-        const bool t = rc < lv[r];
-        const unsigned long long lo = t ? rc : lv[r];
-        carry = t ? lv[r] : rc;
-        lv[r] = lo;
-        bitonic_clean_key(lv[r], lane);
-        if (r + 1 < NB) bitonic_clean_key(carry, lane);
-    }
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) {
-        const unsigned long long o = xor_lane_key(carry, m);
-        carry = (o < carry) ? o : carry;
-    }
-    return carry;
-}
-
-// The order bits of list element `pos` (wave-uniform pos), from its block.
-template <int NB>
-__device__ __forceinline__ uint32_t list_hi_at(const unsigned long long (&lv)[NB], int pos) {
-    const int b = pos >> 6;
-    uint32_t v = key_hi_u(lv[0]);
-#pragma unroll
-    for (int r = 1; r < NB; ++r)
-        if (b == r) v = key_hi_u(lv[r]);
-    return bcast_u(v, pos & 63);
-}
-
-// The same block merge on (value, index) pairs (the seeds' lists, the f64
-// kernel's lists); returns the smallest value discarded.  A block whose
-// largest pair is below the carry's smallest is left as it is (a uniform
-// test, NB > 1 only).
+// A block whose largest pair is below the carry's smallest is left as it is (a
+// uniform test).
 template <typename T, int NB>
-__device__ __forceinline__ T wave_merge_blocks_drop(T (&lv)[NB], uint32_t (&li)[NB], T v, uint32_t ix, int lane) {
+__device__ __forceinline__ void wave_merge_blocks(T (&lv)[NB], uint32_t (&li)[NB], T v, uint32_t ix, int lane) {
     T cv = v;
     uint32_t ci = ix;
 #pragma unroll
     for (int r = 0; r < NB; ++r) {
-        if (NB > 1) {
-            const T cmin = bcast_f(cv, 0), bmax = bcast_f(lv[r], 63);
-            const uint32_t cmi = bcast_u(ci, 0), bmi = bcast_u(li[r], 63);
-            if (pair_less<T>(bmax, bmi, cmin, cmi)) continue;
-        }
+        const T cmin = bcast_f(cv, 0), bmax = bcast_f(lv[r], 63);
+        const uint32_t cmi = bcast_u(ci, 0), bmi = bcast_u(li[r], 63);
+        if (pair_less<T>(bmax, bmi, cmin, cmi)) continue;
         const T rv = reverse_f(cv);
         const uint32_t ri = reverse_u(ci);
         const bool t = pair_less<T>(rv, ri, lv[r], li[r]);
@@ -495,16 +347,6 @@ __device__ __forceinline__ T wave_merge_blocks_drop(T (&lv)[NB], uint32_t (&li)[
             for (int m = 32; m > 0; m >>= 1) bitonic_step<T>(cv, ci, lane, m, true);
         }
     }
-#pragma unroll
-    for (int m = 32; m > 0; m >>= 1) {
-        const T o = shfl_xor_f(cv, m);
-        cv = (o < cv) ? o : cv;
-    }
-    return cv;
-}
-template <typename T, int NB>
-__device__ __forceinline__ void wave_merge_blocks(T (&lv)[NB], uint32_t (&li)[NB], T v, uint32_t ix, int lane) {
-    (void)wave_merge_blocks_drop<T, NB>(lv, li, v, ix, lane);
 }
 
 // Value of list element `pos` (wave-uniform pos), from its block.
@@ -528,29 +370,7 @@ __device__ __forceinline__ float4 gload4(const float* p) {
     return make_float4(v.x, v.y, v.z, v.w);
 }
 
-// Element r of a 16-float accumulator for a lane-varying r: a v_bfi_b32
-// select tree on the bits of r (15 bitfield selects).  Written in asm: as
-// C++ selects the compiler rebuilds a dynamic extract and expands it into a
-// compare chain per element.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ float pick16(const f32x16_t& a, int r) {
-    const uint32_t s0 = 0u - ((uint32_t)r & 1u), s1 = 0u - (((uint32_t)r >> 1) & 1u),
-                   s2 = 0u - (((uint32_t)r >> 2) & 1u), s3 = 0u - (((uint32_t)r >> 3) & 1u);
-    uint32_t l1[8], l2[4], l3[2], v;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(l1[i]) : "v"(s0), "v"(__float_as_uint(a[2 * i + 1])),
-            "v"(__float_as_uint(a[2 * i])));
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(l2[i]) : "v"(s1), "v"(l1[2 * i + 1]), "v"(l1[2 * i]));
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(l3[i]) : "v"(s2), "v"(l2[2 * i + 1]), "v"(l2[2 * i]));
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(v) : "v"(s3), "v"(l3[1]), "v"(l3[0]));
-    return __uint_as_float(v);
-}
-
 // Rotating wave priority for the kernels that run several workgroups per CU.
 // The SIMD's instruction arbiter favours older waves, so with equal
 // priorities the workgroups sharing a CU finish in dispatch order and the
@@ -586,25 +406,6 @@ __device__ __forceinline__ void global_to_lds16(const void* g, void* lds_wave_ba
     (void)g;
     (void)lds_wave_base;
 #endif
-}
-
-// Element r (0..7) of the pair (a0, a1) = (a0[0..3], a1[0..3]), by the same
-// v_bfi_b32 select tree as pick16.
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ float pick8(const f32x4_t& a0, const f32x4_t& a1, int r) {
-    const uint32_t s0 = 0u - ((uint32_t)r & 1u), s1 = 0u - (((uint32_t)r >> 1) & 1u),
-                   s2 = 0u - (((uint32_t)r >> 2) & 1u);
-    const float e[8] = {a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-    uint32_t l1[4], l2[2], v;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(l1[i]) : "v"(s0), "v"(__float_as_uint(e[2 * i + 1])),
-            "v"(__float_as_uint(e[2 * i])));
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-        asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(l2[i]) : "v"(s1), "v"(l1[2 * i + 1]), "v"(l1[2 * i]));
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(v) : "v"(s2), "v"(l2[1]), "v"(l2[0]));
-    return __uint_as_float(v);
 }
 
 // The Gram kernels' seed: for the kSeedQpb queries of one workgroup (four

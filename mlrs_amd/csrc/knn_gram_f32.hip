@@ -1,62 +1,36 @@
-// Fused f32 Gram-MFMA kNN with exact rescoring (gfx950).
-//
-// Replaces the GPU arm euclidean_topk_fused{,_dot,_dot_vec,_dot_vec8}
-// (crates/mlrs-kernels/src/knn.rs:377-2112) and the two-kernel
-// distance_direct -> top_k fallback (crates/mlrs-algos/src/neighbors/
-// nearest.rs:1058-1343) for f32, d <= 256, k <= 128, Euclidean and cosine.
-//
-// Launched for the k-means assignment only (k = 1, ARM_EUCLID_MULADD), where the
-// centres do not fit knn_k1_resident.hip; the searches of k > 1 and of the
-// other arms that the text below also describes are knn_groupmin's.
+// Fused f32 Gram-MFMA nearest row with exact rescoring (gfx950): the k-means
+// assignment (argmin_dist_rows, crates/mlrs-kernels/src/kmeans.rs:284-310)
+// where the centres do not fit knn_k1_resident.hip, and k = 1 Euclidean
+// searches of short indexes.  d <= 256.
 //
 // Two register shapes (GramShape below): d <= 128, 4 waves x 32 queries =
 // 128 queries per workgroup on v_mfma_f32_32x32x2f32; 128 < d <= 256, 4 waves
 // x 16 queries = 64 per workgroup on v_mfma_f32_16x16x4f32.  Either walks one
 // strip of index rows 32 at a time.
 //  * Each wave keeps its query rows in VGPRs as the B operand (pre-scaled by
-//    -2 for Euclidean), loaded once per segment.
+//    -2), loaded once per segment.
 //  * The 32-row index tile is staged in LDS (row stride d_pad + 4 floats, so
 //    16 consecutive rows fall on distinct bank groups; rows of 128 floats in
 //    pairs that share one 1 KB slot), double-buffered in two distinct LDS
-//    objects.  Aligned rows of at least 64 floats are loaded one tile ahead
-//    straight from global memory into LDS (global_load_lds_dwordx4); other
-//    shapes, and k = 1, prefetch into registers.
-//  * Euclidean: the accumulator starts at ||x_t||^2, so after the contraction
-//    acc = ||x_t||^2 - 2 x_t.q_j, the expansion minus the per-query constant.
-//    Cosine: the contraction is scaled by -1/||x_t|| per row afterwards,
-//    acc = -x_t.q_j/||x_t||.
+//    objects, the next tile prefetched into registers.
+//  * The accumulator starts at ||x_t||^2, so after the contraction acc =
+//    ||x_t||^2 - 2 x_t.q_j, the expansion minus the per-query constant.
 //  * Screen: acc is compared against a per-query threshold derived from the
-//    best bound known on the query's k-th exact value (its own list, any
-//    segment's, shared through a per-query word and per-segment list
-//    summaries in global memory) plus a rigorous bound eps on the expansion's
-//    rounding error and the reference's own.  A pair that can still enter the
-//    exact top-k always passes; the comparison is !(acc > thr), so NaN passes
-//    too.  For k = 1 the bound is tightened every tile with the tile's
-//    smallest expansion value.
-//  * For k > 1 the per-query bound starts from a seed launch: the k-th
-//    smallest exact value over evenly spaced index rows (gram_seed_rows).
-//  * Passing (query, row) pairs are queued in a per-wave global array (index
-//    rows and screen values; queue lengths live in registers; the lanes
-//    screening a query append with a popcount prefix, no atomics), which
-//    leaves the LDS small enough for three workgroups per CU at d <= 128.
-//    Before a queue could overflow, the wave sorts it and merges it into the
-//    query's list for this segment (global memory, one per query and
-//    segment): a queued pair enters with its screen value mapped back to a
-//    distance, which is within eps of its exact value, and the list keeps
-//    the k + 32 (at most 64) smallest.  No pair is evaluated exactly during
-//    the scan, except in the rare lists that turn exact (a dropped pair
-//    inside the 2 eps window of the k-th, NaN screen values, norms that could
-//    overflow).  k = 1 queues index rows in LDS and keeps one exact
-//    (value, index) pair per query there.
-//  * The merge kernel takes each query's lists from all segments, finds the
-//    k-th value V of their union and evaluates EXACTLY, in the reference
-//    arm's operation order, every listed pair whose screen value is within
-//    2 eps of V (window rescoring), then ranks by (exact value, index).
+//    best value known for the query (its own, any segment's through a
+//    per-query word in global memory) plus a rigorous bound eps on the
+//    expansion's rounding error and the reference's own, tightened every tile
+//    with the tile's smallest expansion value.  A pair that can still win
+//    always passes; the comparison is !(acc > thr), so NaN passes too.
+//  * Passing rows are queued per query in LDS (queue lengths live in
+//    registers; the lanes screening a query append with a popcount prefix, no
+//    atomics) and evaluated EXACTLY in lane-parallel batches, in the arm's
+//    operation order; one (value, index) pair per query and segment is kept.
+//  * The merge kernel takes the best pair of a query's segments.
 //  * Work split: StreamSplit (knn_kernels.hpp), panel-major, with XCD-grouped
 //    workgroup numbering, so the workgroups on one XCD stream the same index
 //    panel in lockstep.
-// The kept lists are therefore the reference's own top-k: the full distance
-// matrix never reaches HBM and no tolerance is involved.
+// The kept pair is therefore the reference's own: the full distance matrix
+// never reaches HBM and no tolerance is involved.
 #include "knn_common.hpp"
 #include "knn_kernels.hpp"
 
@@ -66,18 +40,9 @@ namespace {
 
 constexpr int kWaves = 4;                // waves per workgroup, narrow shape (the wide shape: 6)
 constexpr int kBn = 32;                  // index rows per tile
-constexpr int kKcap = 128;               // largest k this kernel keeps
-constexpr int kQcapK1 = 48;              // k = 1: the screen tightens every tile, queues stay short
+constexpr int kQcap = 48;                // queued rows per query: the screen tightens every tile, queues stay short
+constexpr int kFlushAt = kQcap - kBn;    // flush when a queue may overflow on the next tile
 constexpr int kShareEvery = 64;          // tiles between reads of the shared thresholds
-// The narrow shape's k <= 64 lists (k > 1) read them every 128 tiles: c2
-// kernel 20.38 -> 20.29 ms; the three-block lists and the wide shape keep 64
-// (at 128: c2k128 +0.1 ms, d256 +0.07 ms; 96, not a power of two, was slower
-// for both narrow kernels; 256: c2 +0.15 ms)
-constexpr int share_every(bool k1, int kl, bool w16) {
-    return (!k1 && kl == 1 && !w16) ? 2 * kShareEvery : kShareEvery;
-}
-constexpr int kSumSlots = 16;            // segment summaries read per refresh (k > 1)
-
 // The two register shapes of a wave's block of (row, query) values.
 //  d <= 128 (W16 = false): 32 queries per wave, v_mfma_f32_32x32x2f32 over
 //    the 32-row tile; lane (h = lane / 32, jl = lane % 32) holds 16 of query
@@ -98,78 +63,41 @@ struct GramShape {
     static constexpr int threads = 64 * waves;
     static constexpr int qpb = waves * qpw;        // queries per workgroup
     static constexpr int vals = W16 ? 8 : 16;      // tile values per lane
-    // queued candidates per query (k > 1): the wide shape 128 (flushed as two
-    // 64-entry blocks: d256 kernel 4.83 -> 4.59 ms against 48; 64: 4.64,
-    // 96: 4.60); the narrow k <= 64 kernel 64 (128 measured slower there)
-    static constexpr int qcap = W16 ? 128 : 64;
-    // three-block lists (k > 64): longer queues, about half as many flushes
-    // (c2k128 kernel 24.5 -> 23.0 ms; 96 entries 24.0, 192 23.4, 256 23.2)
-    static constexpr int qcap3 = 128;
 };
 constexpr int kQpbNarrow = GramShape<false>::qpb;
 constexpr int kQpbWide = GramShape<true>::qpb;
-// Per wave in a.qval: the kernel's QPW x QCAP screen values, then as many
-// index-row numbers, both [queue position][query] (gram_f32_qval_elems sizes
-// the buffer for the launch's list length).
-
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// Per-wave LDS state.  Only k = 1 queues its candidates' indices here (QCAP
-// per query); k > 1 queues them in global memory beside their screen values,
-// which leaves room for a third workgroup per CU.
-template <int QCAP, int QPW>
+// Per-wave LDS state.
+template <int QPW>
 struct WaveLds {
-    uint32_t qidx[QPW][QCAP];
+    uint32_t qidx[QPW][kQcap];
     float thr[QPW];
-    float qa[QPW];   // exact arm's query operand (row_sumsq for the fold arm)
-    float qs[QPW];   // screen operand: ||q||^2 (Euclidean) or ||q|| (cosine)
+    float qs[QPW];   // ||q||^2
     float eps[QPW];  // screen error bound
-    uint32_t off[QPW];                 // k = 1: queue offsets of the batched flush
-    uint32_t mode[QPW];                // 0: screen values lie within eps of exact values (k > 1: screen-value list); 1: not (exact list)
-    unsigned long long best[QPW];      // k = 1: (value bits << 32 | index) of the kept pair
+    uint32_t off[QPW];                 // queue offsets of the batched flush
+    uint32_t mode[QPW];                // 0: screen values lie within eps of exact values; 1: a sum may overflow
+    unsigned long long best[QPW];      // (value bits << 32 | index) of the kept pair
 };
 
 // (value, index) packed so that unsigned order is the (value, index) order
 // for the non-negative values every served arm produces.
 constexpr unsigned long long kBestEmpty = (0x7F800000ull << 32) | 0xFFFFFFFFull;
 
-template <bool COS>
 __device__ __forceinline__ float screen_threshold(float R, float qs, float eps) {
     const float inf = __builtin_huge_valf();
-    if (!(R < inf)) return inf;  // no finite k-th value known yet
-    if (!COS) {
-        // exact <= R  =>  ||x||^2 - 2 x.q <= R - ||q||^2 + eps
-        return round_up_f((double)R - (double)qs + (double)eps);
-    } else {
-        // exact <= R  =>  1 + acc/||q|| <= R + eps  =>  acc <= (R + eps - 1)||q||
-        // A zero query scores exactly 1 against every row: all rows tie, and a
-        // bound published by another segment cannot tell which of them win
-        // (lower indices may lie in a segment that has not run yet), so such a
-        // query is never screened.
-        if (qs == 0.0f) return inf;
-        return round_up_f(((double)R + (double)eps - 1.0) * (double)qs);
-    }
-}
-
-// The arms' per-row and per-query operands of the exact evaluation: the
-// squared norm (cosine fold: sqrt(||q||^2 ||x||^2)), the reciprocal norm
-// (knn_host cosine) or nothing (Euclidean).
-template <int ARM>
-__device__ __forceinline__ float row_operand(const GramArgs32& a, int64_t t) {
-    return (ARM == ARM_COS_FOLD) ? a.xsq[t] : (ARM == ARM_COS_HOST) ? a.xinv[t] : 0.0f;
-}
-template <int ARM>
-__device__ __forceinline__ float query_operand(const GramArgs32& a, int64_t q) {
-    return (ARM == ARM_COS_FOLD) ? a.qsq[q] : (ARM == ARM_COS_HOST) ? a.qinv[q] : 0.0f;
+    if (!(R < inf)) return inf;  // no finite value known yet
+    // exact <= R  =>  ||x||^2 - 2 x.q <= R - ||q||^2 + eps
+    return round_up_f((double)R - (double)qs + (double)eps);
 }
 
 // Exact value of one (query, row) pair in the arm's operation order, loads
 // issued U 16-byte chunks at a time.
 template <int ARM, bool VEC4, int U = 4>
 __device__ __forceinline__ float exact_f32(const float* __restrict__ q, const float* __restrict__ y,
-                                           int64_t d, float qa, float ya) {
-    if (!VEC4) return exact_pair<float, ARM>(q, y, d, qa, ya);
+                                           int64_t d) {
+    if (!VEC4) return exact_pair<float, ARM>(q, y, d, 0.0f, 0.0f);
     const float4* q4 = reinterpret_cast<const float4*>(q);
     const float4* y4 = reinterpret_cast<const float4*>(y);
     const int n4 = (int)(d >> 2);
@@ -190,22 +118,12 @@ __device__ __forceinline__ float exact_f32(const float* __restrict__ q, const fl
                 acc = __builtin_fmaf(d1, d1, acc);
                 acc = __builtin_fmaf(d2, d2, acc);
                 acc = __builtin_fmaf(d3, d3, acc);
-            } else if (ARM == ARM_EUCLID_MULADD) {
+            } else {
                 float d0 = a[u].x - b[u].x, d1 = a[u].y - b[u].y, d2 = a[u].z - b[u].z, d3 = a[u].w - b[u].w;
                 acc = acc + d0 * d0;
                 acc = acc + d1 * d1;
                 acc = acc + d2 * d2;
                 acc = acc + d3 * d3;
-            } else if (ARM == ARM_COS_HOST) {  // mul + add dot
-                acc = acc + a[u].x * b[u].x;
-                acc = acc + a[u].y * b[u].y;
-                acc = acc + a[u].z * b[u].z;
-                acc = acc + a[u].w * b[u].w;
-            } else {  // ARM_COS_FOLD: fma dot
-                acc = __builtin_fmaf(a[u].x, b[u].x, acc);
-                acc = __builtin_fmaf(a[u].y, b[u].y, acc);
-                acc = __builtin_fmaf(a[u].z, b[u].z, acc);
-                acc = __builtin_fmaf(a[u].w, b[u].w, acc);
             }
         }
     }
@@ -217,62 +135,27 @@ __device__ __forceinline__ float exact_f32(const float* __restrict__ q, const fl
             acc = __builtin_fmaf(d1, d1, acc);
             acc = __builtin_fmaf(d2, d2, acc);
             acc = __builtin_fmaf(d3, d3, acc);
-        } else if (ARM == ARM_EUCLID_MULADD) {
+        } else {
             float d0 = a.x - b.x, d1 = a.y - b.y, d2 = a.z - b.z, d3 = a.w - b.w;
             acc = acc + d0 * d0;
             acc = acc + d1 * d1;
             acc = acc + d2 * d2;
             acc = acc + d3 * d3;
-        } else if (ARM == ARM_COS_HOST) {
-            acc = acc + a.x * b.x;
-            acc = acc + a.y * b.y;
-            acc = acc + a.z * b.z;
-            acc = acc + a.w * b.w;
-        } else {
-            acc = __builtin_fmaf(a.x, b.x, acc);
-            acc = __builtin_fmaf(a.y, b.y, acc);
-            acc = __builtin_fmaf(a.z, b.z, acc);
-            acc = __builtin_fmaf(a.w, b.w, acc);
         }
     }
-    if (ARM == ARM_COS_FOLD) {
-        float denom = __builtin_sqrtf(qa * ya);
-        float sim = (denom > 0.0f) ? acc / denom : 0.0f;
-        return clamp02<float>(1.0f - sim);
-    }
-    // knn_host cosine (crates/mlrs-backend/src/prims/knn_host.rs:749-760):
-    // reciprocal norms, 1 - dot * (1/||q||) * (1/||x||), clamped
-    if (ARM == ARM_COS_HOST) return clamp02<float>(1.0f - acc * qa * ya);
     return acc;
 }
 
-// Workgroups per CU.  Three (at most 168 VGPRs, 53 KB LDS) wherever they
-// fit: k = 1 with d <= 64 (its LDS queues allow no more), the narrow shape
-// (d <= 128) with k > 1, whose queues live in global memory (k <= 128: the
-// compiler spills a little of the three-block lists), and the wide shape
-// with k > 1 and 16-byte rows, which then keeps one tile buffer (33 KB at
-// d = 256; two barriers per tile).  A third wave per SIMD keeps the matrix
-// core fed while the other two wait at a tile barrier or merge a queue into
-// a list.
-__host__ __device__ constexpr int gram_f32_wgs_per_cu(int ng, bool k1, int kl, bool vec4) {
-    return (k1 && ng <= 8) || (!k1 && (ng <= 16 || vec4)) ? 3 : 2;
-}
-template <int NG, bool K1, int KL, bool VEC4>
-struct GramOcc {
-    static constexpr int wgs = gram_f32_wgs_per_cu(NG, K1, KL, VEC4);
-};
+// Workgroups per CU: three (at most 168 VGPRs, 53 KB LDS) with d <= 64; the
+// LDS queues allow no more above.  A third wave per SIMD keeps the matrix core
+// fed while the other two wait at a tile barrier.
+__host__ __device__ constexpr int gram_f32_wgs_per_cu(int ng) { return ng <= 8 ? 3 : 2; }
 
-// KL: 64-entry blocks of a (segment, query) list in registers during a flush
-// (1 for k <= 64, 3 for k <= 128: k + 32 entries).
-// FULLW: every row is exactly DP = 8 NG floats wide (d = DP), launched for the
-// paired-row kernels (d = 128) so that their tile loads need no runtime
-// stride.
-template <int NG, int ARM, bool COS, bool VEC4, bool K1, int KL, bool FULLW = false>
 // (__launch_bounds__' second argument is waves per SIMD: workgroups per CU x
 // waves per workgroup / 4.)
-__global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
-                             (GramOcc<NG, K1, KL, VEC4>::wgs * GramShape<(NG > 16)>::waves / 4)) void knn_gram_f32_kernel(
-    GramArgs32 a) {
+template <int NG, int ARM, bool VEC4>
+__global__ __launch_bounds__(GramShape<(NG > 16)>::threads, (gram_f32_wgs_per_cu(NG) * GramShape<(NG > 16)>::waves / 4))
+void knn_gram_f32_kernel(GramArgs32 a) {
     constexpr bool W16 = NG > 16;     // the wide shape (GramShape)
     typedef GramShape<W16> SH;
     constexpr int QPW = SH::qpw;
@@ -293,42 +176,22 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
     constexpr int TILE_FL = PAIRS ? 16 * SLOT : kBn * STRIDE;
     constexpr int TILE_F4 = kBn * DP / 4;
     constexpr int PF = (TILE_F4 + NT - 1) / NT;
-    // 16-byte aligned rows of at least 64 floats go from global memory
-    // straight into LDS (gfx950's global_load_lds_dwordx4, one instruction per
-    // row, or per slot of two rows, with the first CPR (2 CPR) lanes active:
-    // lane i's 16 bytes land 16 i bytes after the row start), so no registers
-    // hold the next tile in flight and no ds_write stores it; other shapes
-    // stage it through registers.  The k = 1 kernel (short segments, three
-    // workgroups per CU already) runs faster staged.
-    constexpr bool DIRECT = VEC4 && NG >= 8 && !K1;
-    // Wide shape, direct loads: one tile buffer, refilled once every wave's
-    // MFMA chain has read it, so that three workgroups fit a CU.
-    constexpr bool SINGLE = W16 && DIRECT;
-    constexpr int RPW = (kBn + WV - 1) / WV;  // tile rows each wave fills (direct): w, w + WV, ...
     constexpr int QQ = DP / 4;        // wide: features per lane-group quarter
     constexpr int NQR = W16 ? QQ / 4 : NG;  // 16-byte query-operand chunks per lane
 
-    // The two tile buffers are distinct objects, so the compiler can tell the
-    // direct loads into one from the reads of the other.
     __shared__ __attribute__((aligned(16))) float tileA[TILE_FL];
-    __shared__ __attribute__((aligned(16))) float tileB[SINGLE ? 4 : TILE_FL];
+    __shared__ __attribute__((aligned(16))) float tileB[TILE_FL];
     __shared__ __attribute__((aligned(16))) float tnA[kBn];
     __shared__ __attribute__((aligned(16))) float tnB[kBn];
-    constexpr int QCAP = K1 ? kQcapK1 : (KL > 1 ? SH::qcap3 : SH::qcap);
-    constexpr int QB = (QCAP + 63) / 64;  // 64-entry blocks of a flushed queue
-    constexpr int kFlushAt = QCAP - kBn;  // flush when a queue may overflow next tile
-    __shared__ WaveLds<K1 ? QCAP : 1, QPW> wl[WV];
+    __shared__ WaveLds<QPW> wl[WV];
 
     // Kernel arguments as locals: they stay in SGPRs.
     const float* __restrict__ Q = a.q;
     const float* __restrict__ X = a.x;
     const float* __restrict__ QSQ = a.qsq;
     const float* __restrict__ XSQ = a.xsq;
-    const float* __restrict__ XSCALE = a.xscale;
     unsigned int* __restrict__ SHARED_R = a.shared_r;
     const int64_t nq = a.nq, nt = a.nt, d = a.d;
-    const int k = a.k;
-    const int K2 = gram_list_cap(k);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
@@ -337,15 +200,8 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
     // feature quarter.  jl: the lane's query within the wave.
     const int h = W16 ? (lane >> 4) : (lane >> 5);
     const int jl = lane & (QPW - 1);
-    WaveLds<K1 ? QCAP : 1, QPW>& L = wl[w];
+    WaveLds<QPW>& L = wl[w];
     const float inf = __builtin_huge_valf();
-    // screen values and index rows of this wave's queued pairs (k > 1),
-    // [queue position][query]
-    constexpr int QVW = QPW * QCAP;  // this kernel's pairs per wave (<= kQvalPerWave)
-    static_assert(QVW <= (KL > 1 ? 32 * 128 : 32 * 64), "gram_f32_qval_elems sizes the queues");
-    float* __restrict__ QVw = K1 ? nullptr : a.qval + ((int64_t)blockIdx.x * WV + w) * (2 * QVW);
-    uint32_t* __restrict__ QIw = K1 ? nullptr : reinterpret_cast<uint32_t*>(QVw + QVW);
-
     // Tile row of value r of this lane.
     auto row_of = [&](int r) -> int {
         return W16 ? 16 * (r >> 2) + 4 * h + (r & 3) : 8 * (r >> 2) + 4 * h + (r & 3);
@@ -354,21 +210,9 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
     auto row_at = [&](int r) -> int { return PAIRS ? (r & 15) * SLOT + (r >> 4) * DP : r * STRIDE; };
     auto chunk_at = [&](int r, int c) -> int { return row_at(r) + 4 * c; };
 
-    // Direct fills never write the columns past d (d < DP): zero them once in
-    // both buffers, as they meet the query operand's zeros and left alone
-    // could hold NaN.
-    if (DIRECT && d < DP) {
-        const int pad = (int)(DP - d);
-        for (int e = tid; e < kBn * pad; e += NT) {
-            tileA[row_at(e / pad) + d + e % pad] = 0.0f;
-            if constexpr (!SINGLE) tileB[row_at(e / pad) + d + e % pad] = 0.0f;
-        }
-    }
-
     // ---- work split (StreamSplit): this workgroup's range of (query block,
     //      tile) units, panel-major; each piece of a job in the range is a
-    //      segment with its own exact lists [slot][nq][k], merged at the end
-    //      by knn_merge_f32_kernel. ----
+    //      segment with its own best pair [slot][nq], merged at the end. ----
     const StreamSplit sp(nq, nt, QPB, kBn, a.grid_wgs);
     const int64_t wg = xcd_grouped_wg(blockIdx.x, gridDim.x);
     const int64_t u_hi = ((wg + 1) * sp.P < sp.T) ? (wg + 1) * sp.P : sp.T;
@@ -377,15 +221,8 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
     sp.decode(u, panel, qblock, tile0, left);
     const int64_t tile1 = tile0 + ((left < u_hi - u) ? left : (u_hi - u));
     const int64_t slot = sp.slot(wg, panel, qblock);
-    float* __restrict__ LV = a.part_val + slot * nq * K2;
-    uint32_t* __restrict__ LI = a.part_idx + slot * nq * K2;
-    // Summaries of the query block's segment lists: segment s holds at least
-    // rank_i pairs whose exact value is <= summ[s][q].i (rank_i = ceil(i k/4));
-    // the union over segments (disjoint rows) bounds the query's k-th value.
-    float4* __restrict__ SUMM = a.summ;
-    const int64_t nsum = SUMM ? (sp.slots_of(qblock) < kSumSlots ? sp.slots_of(qblock) : kSumSlots) : 0;
-    const int rk1 = (k + 3) / 4, rk2 = (k + 1) / 2, rk3 = (3 * k + 3) / 4;
-
+    float* __restrict__ LV = a.part_val + slot * nq;
+    uint32_t* __restrict__ LI = a.part_idx + slot * nq;
     const int64_t qwave = qblock * QPB + w * QPW;  // first query of this wave
     const int64_t qmine = qwave + jl;
     const bool qvalid = qmine < nq;
@@ -417,51 +254,27 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
         }
     }
 
-    // ---- per-query constants, lists, queues ----
+    // ---- per-query constants, queues ----
     uint32_t cntr = 0u;  // queued candidates of query jl
     if (lane < QPW) {
         const float qsq = qvalid ? qsq_l : 0.0f;
         L.thr[lane] = qvalid ? inf : -inf;
-        if (!COS) {
-            L.qs[lane] = qsq;
-            L.qa[lane] = 0.0f;
-            L.eps[lane] = (float)(a.eps_rel * ((double)qsq + (double)a.stats->xsq_max) + a.eps_abs);
-        } else {
-            L.qs[lane] = __builtin_sqrtf(qsq);
-            L.qa[lane] = (ARM == ARM_COS_HOST) ? (qvalid ? a.qinv[qrow] : 0.0f) : qsq;
-            L.eps[lane] = (float)a.eps_abs;
-        }
-        // Screen-value lists need |screen distance - exact| <= eps for every
-        // pair, which the error bound gives while no sum can overflow: norms
-        // well inside the float range (and a nonzero query for cosine).
-        // Other queries keep exact lists.
-        bool sv = qvalid && ((double)qsq + (double)a.stats->xsq_max <= 0x1p124) && (L.eps[lane] < inf);
-        if (COS) sv = sv && (L.qs[lane] > 0.0f);
+        L.qs[lane] = qsq;
+        L.eps[lane] = (float)(a.eps_rel * ((double)qsq + (double)a.stats->xsq_max) + a.eps_abs);
+        // |screen distance - exact| <= eps holds while no sum can overflow:
+        // norms well inside the float range.
+        const bool sv = qvalid && ((double)qsq + (double)a.stats->xsq_max <= 0x1p124) && (L.eps[lane] < inf);
         L.mode[lane] = sv ? 0u : 1u;
     }
-    if (K1) {
-        if (lane < QPW) L.best[lane] = kBestEmpty;
-    } else {
-        for (int j = 0; j < QPW; ++j) {
-            const int64_t qg = qwave + j;
-#pragma unroll
-            for (int r = 0; r < KL; ++r) {
-                const int p = 64 * r + lane;
-                if (qg < nq && p < K2) {
-                    LV[qg * K2 + p] = inf;
-                    LI[qg * K2 + p] = kSentinelIdx;
-                }
-            }
-        }
-    }
+    if (lane < QPW) L.best[lane] = kBestEmpty;
     // Strips that start late begin from the bound earlier strips have reached.
     if (SHARED_R && lane < QPW && qvalid)
-        L.thr[lane] = fminf(L.thr[lane], screen_threshold<COS>(r0_l, L.qs[lane], L.eps[lane]));
+        L.thr[lane] = fminf(L.thr[lane], screen_threshold(r0_l, L.qs[lane], L.eps[lane]));
 
     // ---- query operand: qreg[i] = scale * q[qfeat(i, 0..3)] (aligned rows:
     //      one 16-byte load per chunk) ----
     {
-        const float scale = COS ? 1.0f : -2.0f;
+        const float scale = -2.0f;
         const float* qp = Q + qmine * d;
         if (VEC4) {
             if (!kEarlyQ) {
@@ -547,164 +360,13 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
         _Pragma("unroll") for (int p = 0; p < (PF_ONE_PTR ? 1 : PF); ++p) pf_src[p] += kBn * d; \
         if (tid < kBn) {                                                                     \
             const uint32_t t = t0_ + (uint32_t)tid;                                          \
-            if (COS)                                                                         \
-                pfn = (t < t_end32) ? XSCALE[t] : 0.0f;                                      \
-            else                                                                             \
-                pfn = (t < t_end32) ? XSQ[t] : inf;                                          \
+            pfn = (t < t_end32) ? XSQ[t] : inf;                                              \
         }                                                                                    \
     } while (0)
 
-    // ---- flush (k > 1): one query's queue sorted and merged into its list.
-    //      Screen-value mode: a queued pair enters with its screen value
-    //      mapped back to a distance, within eps of its exact value; the list
-    //      keeps the K2 smallest, and the segment's bound is its k-th + eps.
-    //      A pair whose screen value is NaN, and every pair of an exact-mode
-    //      query, is evaluated exactly in the arm's operation order.  When a
-    //      discarded pair lies within 2 eps of the k-th (it could still be
-    //      among the k best), the old list and the queue are re-evaluated
-    //      exactly and the query's list stays exact from then on. ----
-#define MLRS_EXACT_AT(T_)                                                                    \
-    exact_f32<ARM, VEC4>(Q + qg_ * d, X + (int64_t)(T_) * d, d, L.qa[j_], row_operand<ARM>(a, (T_)))
-#define MLRS_FLUSH(J)                                                                        \
-    do {                                                                                     \
-        const int j_ = (J);                                                                  \
-        const int64_t qg_ = qwave + j_;                                                      \
-        const uint32_t n_ = bcast_u(cntr, j_);                                               \
-        const bool exact_ = L.mode[j_] != 0u;                                                \
-        unsigned long long lk_[KL];                                                          \
-        _Pragma("unroll") for (int r_ = 0; r_ < KL; ++r_) {                                  \
-            const int p_ = 64 * r_ + lane;                                                   \
-            lk_[r_] = kKeyEmpty;                                                             \
-            if (p_ < K2) lk_[r_] = pair_key(LV[qg_ * K2 + p_], LI[qg_ * K2 + p_]);           \
-        }                                                                                    \
-        const unsigned long long ok_ = lk_[0];                                               \
-        unsigned long long dk_ = kKeyEmpty;                                                  \
-        unsigned long long ek_ = kKeyEmpty;                                                  \
-        if constexpr (QB == 1) {                                                             \
-            float e_ = inf;                                                                  \
-            uint32_t t_ = kSentinelIdx;                                                      \
-            if ((uint32_t)lane < n_) {                                                       \
-                t_ = QIw[lane * QPW + j_];                                                   \
-                const float s_ = exact_ ? 0.0f : QVw[lane * QPW + j_];                       \
-                if (exact_ || s_ != s_)                                                      \
-                    e_ = MLRS_EXACT_AT(t_);                                                  \
-                else                                                                         \
-                    e_ = COS ? 1.0f + s_ / L.qs[j_] : s_ + L.qs[j_];                         \
-                if (e_ != e_) { /* NaN is never admitted */                                  \
-                    e_ = inf;                                                                \
-                    t_ = kSentinelIdx;                                                       \
-                }                                                                            \
-            }                                                                                \
-            ek_ = pair_key(e_, t_);                                                          \
-            wave_sort64_key(ek_, lane);                                                      \
-            if constexpr (KL == 1)                                                           \
-                dk_ = wave_merge64_key_drop(lk_[0], ek_, lane);                              \
-            else                                                                             \
-                dk_ = wave_merge_blocks_key_drop<KL>(lk_, ek_, lane);                        \
-        } else {                                                                             \
-          _Pragma("unroll") for (int b_ = 0; b_ < QB; ++b_) {                                \
-            if (b_ == 0 || n_ > 64u * (uint32_t)b_) {                                        \
-              float e_ = inf;                                                                \
-              uint32_t t_ = kSentinelIdx;                                                    \
-              const uint32_t qi_ = 64u * (uint32_t)b_ + (uint32_t)lane;                      \
-              if (qi_ < n_) {                                                                \
-                  t_ = QIw[qi_ * QPW + j_];                                                  \
-                  const float s_ = exact_ ? 0.0f : QVw[qi_ * QPW + j_];                      \
-                  if (exact_ || s_ != s_)                                                    \
-                      e_ = MLRS_EXACT_AT(t_);                                                \
-                  else                                                                       \
-                      e_ = COS ? 1.0f + s_ / L.qs[j_] : s_ + L.qs[j_];                       \
-                  if (e_ != e_) { /* NaN is never admitted */                                \
-                      e_ = inf;                                                              \
-                      t_ = kSentinelIdx;                                                     \
-                  }                                                                          \
-              }                                                                              \
-              ek_ = pair_key(e_, t_);                                                        \
-              wave_sort64_key(ek_, lane);                                                    \
-              const unsigned long long d_ = wave_merge_blocks_key_drop<KL>(lk_, ek_, lane);  \
-              dk_ = (b_ == 0 || d_ < dk_) ? d_ : dk_; /* the smallest dropped */           \
-            }                                                                                \
-          }                                                                                  \
-        }                                                                                    \
-        float R_ = f32_from_order_bits(list_hi_at<KL>(lk_, k - 1));                          \
-        if (!exact_) {                                                                       \
-            const float dr_ = (K2 < 64 * KL) ? f32_from_order_bits(list_hi_at<KL>(lk_, K2))  \
-                                             : key_value(dk_);                               \
-            double w_ = (double)R_ + 2.0 * (double)L.eps[j_];                                \
-            w_ += __builtin_fabs(w_) * 0x1p-40;                                              \
-            if (dr_ < inf && (double)dr_ <= w_) {                                            \
-              if constexpr (KL == 1 && QB == 1) {                                            \
-                /* the old list and the queue, exactly */                                    \
-                float x1_ = inf, x2_ = inf;                                                  \
-                uint32_t i1_ = key_index(ok_), i2_ = key_index(ek_);                         \
-                if (i1_ != kSentinelIdx) x1_ = MLRS_EXACT_AT(i1_);                           \
-                if (i2_ != kSentinelIdx) x2_ = MLRS_EXACT_AT(i2_);                           \
-                if (x1_ != x1_) { x1_ = inf; i1_ = kSentinelIdx; }                           \
-                if (x2_ != x2_) { x2_ = inf; i2_ = kSentinelIdx; }                           \
-                unsigned long long k1_ = pair_key(x1_, i1_), k2_ = pair_key(x2_, i2_);       \
-                wave_sort64_key(k1_, lane);                                                  \
-                wave_sort64_key(k2_, lane);                                                  \
-                wave_merge64_key(k1_, k2_, lane);                                            \
-                lk_[0] = k1_;                                                                \
-              } else {                                                                       \
-                /* the old list (still in memory) and the queue, exactly */                  \
-                _Pragma("unroll") for (int r_ = 0; r_ < KL; ++r_) lk_[r_] = kKeyEmpty;       \
-                _Pragma("unroll") for (int r_ = 0; r_ < KL + QB; ++r_) {                     \
-                    uint32_t i_ = kSentinelIdx;                                              \
-                    if (r_ < KL) {                                                           \
-                        const int p_ = 64 * r_ + lane;                                       \
-                        if (p_ < K2) i_ = LI[qg_ * K2 + p_];                                 \
-                    } else if (64u * (uint32_t)(r_ - KL) + (uint32_t)lane < n_) {            \
-                        i_ = QIw[(64u * (uint32_t)(r_ - KL) + (uint32_t)lane) * QPW + j_];   \
-                    }                                                                        \
-                    float x_ = inf;                                                          \
-                    if (i_ != kSentinelIdx) x_ = MLRS_EXACT_AT(i_);                          \
-                    if (x_ != x_) { x_ = inf; i_ = kSentinelIdx; }                           \
-                    unsigned long long b_ = pair_key(x_, i_);                                \
-                    wave_sort64_key(b_, lane);                                               \
-                    (void)wave_merge_blocks_key_drop<KL>(lk_, b_, lane);                     \
-                }                                                                            \
-              }                                                                              \
-                R_ = f32_from_order_bits(list_hi_at<KL>(lk_, k - 1));                        \
-                if (lane == 0) L.mode[j_] = 1u;                                              \
-            } else if (R_ < inf) {                                                           \
-                R_ = round_up_f((double)R_ + (double)L.eps[j_]);                             \
-            }                                                                                \
-        }                                                                                    \
-        _Pragma("unroll") for (int r_ = 0; r_ < KL; ++r_) {                                  \
-            const int p_ = 64 * r_ + lane;                                                   \
-            if (p_ < K2) {                                                                   \
-                LV[qg_ * K2 + p_] = key_value(lk_[r_]);                                      \
-                LI[qg_ * K2 + p_] = key_index(lk_[r_]);                                      \
-            }                                                                                \
-        }                                                                                    \
-        if (SUMM) {                                                                          \
-            const bool sv_ = !exact_ && L.mode[j_] == 0u;                                    \
-            float p_[4] = {f32_from_order_bits(list_hi_at<KL>(lk_, rk1 - 1)),                \
-                           f32_from_order_bits(list_hi_at<KL>(lk_, rk2 - 1)),                \
-                           f32_from_order_bits(list_hi_at<KL>(lk_, rk3 - 1)),                \
-                           f32_from_order_bits(list_hi_at<KL>(lk_, k - 1))};                 \
-            if (lane == 0) {                                                                 \
-                _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_)                             \
-                    if (sv_ && p_[i_] < inf) p_[i_] = round_up_f((double)p_[i_] + (double)L.eps[j_]); \
-                SUMM[slot * nq + qg_] = make_float4(p_[0], p_[1], p_[2], p_[3]);             \
-            }                                                                                \
-        }                                                                                    \
-        if (lane == 0) {                                                                     \
-            if (SHARED_R && R_ < inf) {                                                      \
-                /* published without waiting for the old value: other segments' */           \
-                /* bounds reach this one at its next refresh */                              \
-                __hip_atomic_fetch_min(&SHARED_R[qg_], __float_as_uint(R_), __ATOMIC_RELAXED, \
-                                       __HIP_MEMORY_SCOPE_AGENT);                            \
-            }                                                                                \
-            L.thr[j_] = fminf(L.thr[j_], screen_threshold<COS>(R_, L.qs[j_], L.eps[j_]));    \
-        }                                                                                    \
-        if (jl == j_) cntr = 0u;                                                             \
-    } while (0)
-
-    // ---- k = 1: every queued pair of the wave evaluated in lane-parallel
+    // ---- flush: every queued pair of the wave evaluated in lane-parallel
     //      batches, kept with a 64-bit LDS atomicMin on (value, index) ----
-#define MLRS_FLUSH_K1()                                                                      \
+#define MLRS_FLUSH()                                                                      \
     do {                                                                                     \
         const uint32_t c_ = (lane < QPW) ? cntr : 0u;                                        \
         uint32_t incl_ = c_;                                                                 \
@@ -721,9 +383,7 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
                 _Pragma("unroll") for (int m_ = QPW / 2; m_ >= 1; m_ >>= 1) if (L.off[j_ + m_] <= e_) \
                     j_ += m_;                                                                \
                 const uint32_t t_ = L.qidx[j_][e_ - L.off[j_]];                              \
-                const float ya_ = row_operand<ARM>(a, t_);                                   \
-                const float v_ = exact_f32<ARM, VEC4>(Q + (qwave + j_) * d, X + (int64_t)t_ * d, d, \
-                                                       L.qa[j_], ya_);                       \
+                const float v_ = exact_f32<ARM, VEC4>(Q + (qwave + j_) * d, X + (int64_t)t_ * d, d); \
                 if (v_ == v_)                                                                \
                     atomicMin(&L.best[j_], ((unsigned long long)__float_as_uint(v_) << 32) | t_); \
             }                                                                                \
@@ -736,147 +396,59 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
                 const unsigned int old_ = atomicMin(&SHARED_R[qmine], __float_as_uint(R_));  \
                 R_ = fminf(R_, __uint_as_float(old_));                                       \
             }                                                                                \
-            L.thr[lane] = fminf(L.thr[lane], screen_threshold<COS>(R_, L.qs[lane], L.eps[lane])); \
+            L.thr[lane] = fminf(L.thr[lane], screen_threshold(R_, L.qs[lane], L.eps[lane])); \
         }                                                                                    \
     } while (0)
 
     float4 pf[PF];
     float pfn = 0.0f;
-    // Direct fill of tile T0 into DST: wave w's instruction i fills chunks
-    // 64 (w PF + i) .. + 63 of the contiguous tile; chunk f is position f % CPR
-    // of row f / CPR, which holds the row's column chunk position ^ (row & 15).
-    // Rows past the segment are not loaded (their values are masked out of the
-    // screen); the row norms go through a register as in the staged path.
-    // pair layout: lane l loads chunk l % 32 of slot row 16 (l / 32)
-    const uint32_t pair_off = (uint32_t)(16 * (lane >> 5) * DP + 4 * (lane & 31));
-    auto direct_load = [&](float (&dst)[TILE_FL], uint32_t t0) {
-        if constexpr (DIRECT && PAIRS) {
-            // slots 4w .. 4w + 3: lane l loads chunk l % 32 of row slot + 16 (l / 32)
-            if (FULLW && t_end32 - t0 >= (uint32_t)kBn) {
-                // unpadded rows, whole tile (t0 + kBn could wrap): a
-                // wave-uniform row base plus the lane's constant offset, so no
-                // per-slot runtime strides are kept (they were scalar
-                // registers spilled to VGPR lanes, read back every tile)
-                const float* base = X + (int64_t)(t0 + (uint32_t)(4 * w)) * DP;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    global_to_lds16(base + (uint32_t)(i * DP + pair_off), &dst[(4 * w + i) * SLOT]);
-            } else {
-                const int rl = 16 * (lane >> 5);
-                const float* xw = X + (int64_t)(t0 + (uint32_t)(4 * w)) * d + (int64_t)rl * d + 4 * (lane & 31);
-                const int di = (int)d;
-                if (4 * (lane & 31) < di) {
-                    if (t_end32 - t0 >= (uint32_t)kBn) {  // whole tile (t0 + kBn could wrap)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) global_to_lds16(xw + i * di, &dst[(4 * w + i) * SLOT]);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (t0 + (uint32_t)(4 * w + i + rl) < t_end32)
-                                global_to_lds16(xw + i * di, &dst[(4 * w + i) * SLOT]);
-                    }
-                }
-            }
-        } else if constexpr (DIRECT) {
-            // rows w, w + WV, ... of the tile: this wave's first row
-            // (wave-uniform) + the lane's chunk
-            const float* xw = X + (int64_t)(t0 + (uint32_t)w) * d + 4 * lane;
-            const int di = (int)d;
-            if (lane < CPR && 4 * lane < di) {
-                if (t_end32 - t0 >= (uint32_t)kBn) {  // whole tile (t0 + kBn could wrap)
-#pragma unroll
-                    for (int i = 0; i < RPW; ++i)
-                        if (kBn % WV == 0 || w + WV * i < kBn)
-                            global_to_lds16(xw + (int64_t)WV * i * di, &dst[(w + WV * i) * STRIDE]);
-                } else {
-#pragma unroll
-                    for (int i = 0; i < RPW; ++i)
-                        if ((kBn % WV == 0 || w + WV * i < kBn) && t0 + (uint32_t)(w + WV * i) < t_end32)
-                            global_to_lds16(xw + (int64_t)WV * i * di, &dst[(w + WV * i) * STRIDE]);
-                }
-            }
-        }
-        // the tile's row norms, one per lane of wave 0 (the three-block-list
-        // kernel tests the wave index and the lane, which measured faster
-        // there: c2k128 25.04 -> 24.51 ms; the others test tid)
-        if (KL > 1 ? (w == 0 && lane < kBn) : (tid < kBn)) {
-            const uint32_t t = t0 + (uint32_t)(KL > 1 ? lane : tid);
-            if (COS)
-                pfn = (t < t_end32) ? XSCALE[t] : 0.0f;
-            else
-                pfn = (t < t_end32) ? XSQ[t] : inf;
-        }
-    };
-    // the tile at T0: into registers (staged) or straight into DST (direct)
-    auto load_tile = [&](float (&dst)[TILE_FL], int64_t t0) {
-        if constexpr (DIRECT)
-            direct_load(dst, (uint32_t)t0);
-        else
-            MLRS_PREFETCH(t0);
-    };
-    if (t_begin < t_end) load_tile(tileA, t_begin);
+    if (t_begin < t_end) MLRS_PREFETCH(t_begin);
     __syncthreads();  // per-wave LDS init visible to the wave
-    // Sign-bit screen (below): Euclidean waves whose valid queries are all in
-    // screen-value mode (L.mode 0: no screen sum can overflow), where a NaN
-    // screen value comes only from a row holding a NaN, whose exact value is
-    // NaN and never kept, so the screen may drop it.  Used by the k = 1 and
-    // three-block-list kernels; the k <= 64 narrow kernel and the wide shape
-    // measured no faster with it (c2 +0.9%).
-    constexpr bool kSignScreen = !COS && !W16 && (K1 || KL > 1);
+    // Sign-bit screen (below): waves whose valid queries all have mode 0 (no
+    // screen sum can overflow), where a NaN screen value comes only from a row
+    // holding a NaN, whose exact value is NaN and never kept, so the screen may
+    // drop it.  The wide shape measured no faster with it.
+    constexpr bool kSignScreen = !W16;
     const bool nan_free =
         kSignScreen && __builtin_amdgcn_ballot_w64(lane < QPW && qvalid && L.mode[lane] != 0u) == 0;
 
     float thr = L.thr[jl];
-    const float eps2 = 2.0f * L.eps[jl];  // k = 1 tightening (exact doubling)
-    // k = 1: a lower bound on the screen values of the rows in query jl's
-    // queue.  A NaN screen value can hide a finite exact value only where a
-    // sum may overflow, so queries without screen-value mode (L.mode) keep
-    // -inf and never drop queued rows; with it, NaN screen values come from
+    const float eps2 = 2.0f * L.eps[jl];  // exact doubling
+    // A lower bound on the screen values of the rows in query jl's queue.  A NaN screen value can hide a finite exact value only where a
+    // sum may overflow, so queries of mode 1 keep
+    // -inf and never drop queued rows; otherwise NaN screen values come from
     // rows holding a NaN, whose exact values are NaN and never kept.
     const float qlo0 = (L.mode[jl] == 0u) ? inf : -inf;
     float qlo = qlo0;
     int tiles = 0;
-    // One tile: CUR holds (or receives from the staging registers) the rows
-    // at T0, the next tile is loaded towards NXT.
-    auto tile_step = [&](float (&cur)[TILE_FL], float* __restrict__ tncur, float (&nxt)[TILE_FL],
-                         int64_t t0) {
-        // publish the tile: the staged registers are stored into CUR; the
-        // direct loads into CUR are waited for, and the barrier makes every
-        // wave's visible (and ends every wave's reads of NXT)
-        if constexpr (DIRECT) {
-            __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-        } else {
+    // One tile: CUR receives the rows at T0 from the staging registers, which
+    // then take the next tile.
+    auto tile_step = [&](float (&cur)[TILE_FL], float* __restrict__ tncur, int64_t t0) {
 #pragma unroll
-            for (int p = 0; p < PF; ++p) {
-                const int f = tid + NT * p;
-                if (f < TILE_F4) {
-                    const int r = f / (DP / 4);
-                    const int c4 = f % (DP / 4);
-                    *reinterpret_cast<float4*>(&cur[0] + chunk_at(r, c4)) = pf[p];
-                }
+        for (int p = 0; p < PF; ++p) {
+            const int f = tid + NT * p;
+            if (f < TILE_F4) {
+                const int r = f / (DP / 4);
+                const int c4 = f % (DP / 4);
+                *reinterpret_cast<float4*>(&cur[0] + chunk_at(r, c4)) = pf[p];
             }
         }
-        if (KL > 1 ? (w == 0 && lane < kBn) : (tid < kBn)) tncur[KL > 1 ? lane : tid] = pfn;
+        if (tid < kBn) tncur[tid] = pfn;
         __syncthreads();
-        if (!SINGLE && t_end32 - (uint32_t)t0 > (uint32_t)kBn) load_tile(nxt, t0 + kBn);
+        if (t_end32 - (uint32_t)t0 > (uint32_t)kBn) MLRS_PREFETCH(t0 + kBn);
 
         // The lane's tile values: narrow, acc[r] = row row_of(r); wide, r < 4
         // in acc0 (the first 16-row half) and r >= 4 in acc1.
         f32x16 acc;
         f32x4 acc0, acc1;
         if constexpr (!W16) {
-            if (!COS) {
 #pragma unroll
-                for (int g4 = 0; g4 < 4; ++g4) {
-                    float4 n4 = *reinterpret_cast<const float4*>(&tncur[8 * g4 + 4 * h]);
-                    acc[4 * g4 + 0] = n4.x;
-                    acc[4 * g4 + 1] = n4.y;
-                    acc[4 * g4 + 2] = n4.z;
-                    acc[4 * g4 + 3] = n4.w;
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+            for (int g4 = 0; g4 < 4; ++g4) {
+                float4 n4 = *reinterpret_cast<const float4*>(&tncur[8 * g4 + 4 * h]);
+                acc[4 * g4 + 0] = n4.x;
+                acc[4 * g4 + 1] = n4.y;
+                acc[4 * g4 + 2] = n4.z;
+                acc[4 * g4 + 3] = n4.w;
             }
             // A operands double-buffered: the next group's LDS read is issued
             // before the current group's four MFMAs (the scheduling barriers keep
@@ -895,26 +467,13 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
                 __builtin_amdgcn_sched_barrier(0);
                 av = an;
             }
-            if (COS) {
-                // rows scaled by -1/||x_t|| after the contraction (the scales ride
-                // in tnorm), so the prefetched loads need no arithmetic before the
-                // next tile's LDS store
-#pragma unroll
-                for (int g4 = 0; g4 < 4; ++g4) {
-                    const float4 s4 = *reinterpret_cast<const float4*>(&tncur[8 * g4 + 4 * h]);
-                    acc[4 * g4 + 0] *= s4.x;
-                    acc[4 * g4 + 1] *= s4.y;
-                    acc[4 * g4 + 2] *= s4.z;
-                    acc[4 * g4 + 3] *= s4.w;
-                }
-            }
         } else {
             const float4 n0 = *reinterpret_cast<const float4*>(&tncur[4 * h]);
             const float4 n1 = *reinterpret_cast<const float4*>(&tncur[16 + 4 * h]);
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                acc0[r] = COS ? 0.0f : (&n0.x)[r];
-                acc1[r] = COS ? 0.0f : (&n1.x)[r];
+                acc0[r] = (&n0.x)[r];
+                acc1[r] = (&n1.x)[r];
             }
             // A operands: this lane's rows jl and 16 + jl, its quarter's chunk
             // i, one group ahead; each chunk feeds eight MFMAs (four k-steps
@@ -943,27 +502,14 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
                 av0 = an0;
                 av1 = an1;
             }
-            if (COS) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    acc0[r] *= (&n0.x)[r];
-                    acc1[r] *= (&n1.x)[r];
-                }
-            }
-        }
-        if constexpr (SINGLE) {
-            // every wave's chain has read the tile (and its norms): refill it
-            // under this tile's screen
-            __syncthreads();
-            if (t_end32 - (uint32_t)t0 > (uint32_t)kBn) load_tile(nxt, t0 + kBn);
         }
         auto val = [&](int r) -> float {
             if constexpr (W16) return r < 4 ? acc0[r] : acc1[r - 4];
             else return acc[r];
         };
 
-        // ---- k = 1: tighten with this tile's smallest expansion value ----
-        if (K1 && !COS) {  // the k = 1 kernel (every k = 1 search launches it)
+        // ---- tighten with this tile's smallest expansion value ----
+        {
             float m = inf;
 #pragma unroll
             for (int r = 0; r < SH::vals; ++r) m = fminf(m, val(r));  // NaN ignored; past-end rows are +inf
@@ -975,18 +521,16 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
                 const float s_ = m + eps2;
                 thr = fminf(thr, s_ + (__builtin_fabsf(s_) * 0x1p-23f + 0x1p-126f));
             }
-            if constexpr (K1) {
-                // Rows queued on earlier tiles whose screen values all exceed
-                // the tightened threshold cannot be the nearest row (nor tie
-                // with it): the queue restarts before this tile's rows join it.
-                // Each new running minimum used to leave its predecessors queued
-                // (about ln(tiles) rows per query at each flush).
-                if (qlo > thr) {
-                    cntr = 0u;
-                    qlo = inf;
-                }
-                qlo = fminf(qlo, m);
+            // Rows queued on earlier tiles whose screen values all exceed
+            // the tightened threshold cannot be the nearest row (nor tie
+            // with it): the queue restarts before this tile's rows join it.
+            // Each new running minimum used to leave its predecessors queued
+            // (about ln(tiles) rows per query at each flush).
+            if (qlo > thr) {
+                cntr = 0u;
+                qlo = inf;
             }
+            qlo = fminf(qlo, m);
         }
 
         // ---- screen: value r of the lane is tile row row_of(r) for query jl.
@@ -1037,136 +581,44 @@ __global__ __launch_bounds__(GramShape<(NG > 16)>::threads,
             }
             uint32_t pos = cntr + before;
             const uint32_t tb = (uint32_t)t0;
-            if (K1) {
-                while (m) {
-                    const int r = __builtin_ctz(m);
-                    m &= m - 1;
-                    L.qidx[jl][pos++] = tb + (uint32_t)row_of(r);
-                }
-            } else {
-                // one iteration per admitted row of the lane (usually one)
-                while (m) {
-                    const int r = __builtin_ctz(m);
-                    m &= m - 1;
-                    QIw[pos * QPW + jl] = tb + (uint32_t)row_of(r);
-                    if constexpr (W16) QVw[pos * QPW + jl] = pick8(acc0, acc1, r);
-                    else QVw[pos * QPW + jl] = pick16(acc, r);
-                    ++pos;
-                }
+            while (m) {
+                const int r = __builtin_ctz(m);
+                m &= m - 1;
+                L.qidx[jl][pos++] = tb + (uint32_t)row_of(r);
             }
             cntr += total;
         }
         // ---- flush queries whose queue could overflow on the next tile ----
-        uint64_t mask = __builtin_amdgcn_ballot_w64(lane < QPW && cntr > (uint32_t)kFlushAt);
-        if (mask) {
+        if (__builtin_amdgcn_ballot_w64(lane < QPW && cntr > (uint32_t)kFlushAt)) {
             if (lane < QPW) L.thr[lane] = fminf(L.thr[lane], thr);
-            if (K1) {
-                MLRS_FLUSH_K1();
-            } else {
-                // the queued screen values were stored by other lanes of this wave
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                while (mask) {
-                    const int j = __builtin_ctzll(mask);
-                    mask &= mask - 1;
-                    MLRS_FLUSH(j);
-                }
-            }
+            MLRS_FLUSH();
             thr = L.thr[jl];
         }
         // ---- pick up thresholds tightened by other strips of these queries ----
-        rotate_wave_priority((uint32_t)tiles + 1u, GramOcc<NG, K1, KL, VEC4>::wgs);
-        if (SHARED_R && (++tiles % share_every(K1, KL, W16)) == 0) {
+        rotate_wave_priority((uint32_t)tiles + 1u, gram_f32_wgs_per_cu(NG));
+        if (SHARED_R && (++tiles % kShareEvery) == 0) {
             if (lane < QPW && qvalid) {
-                float R = __uint_as_float(SHARED_R[qmine]);
-                if (nsum > 0) {
-                    // the smallest T with at least k pairs <= T over the
-                    // segment summaries: the four smallest (value, rank
-                    // increment) pairs, accumulated in order
-                    float b0 = inf, b1 = inf, b2 = inf, b3 = inf;
-                    int i0 = 0, i1 = 0, i2 = 0, i3 = 0;
-                    const int inc[4] = {rk1, rk2 - rk1, rk3 - rk2, k - rk3};
-                    for (int64_t s0 = 0; s0 < nsum; s0 += 4) {
-                        // four summaries in flight, then folded in
-                        float4 v4s[4];
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-                            v4s[u] = (s0 + u < nsum) ? SUMM[(s0 + u) * nq + qmine] : make_float4(inf, inf, inf, inf);
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            const float4 v4 = v4s[i >> 2];
-                            const float v = ((i & 3) == 0) ? v4.x : ((i & 3) == 1) ? v4.y : ((i & 3) == 2) ? v4.z : v4.w;
-                            const int n = inc[i & 3];
-                            const bool c0 = v < b0, c1 = v < b1, c2 = v < b2, c3 = v < b3;
-                            b3 = c2 ? b2 : (c3 ? v : b3);
-                            i3 = c2 ? i2 : (c3 ? n : i3);
-                            b2 = c1 ? b1 : (c2 ? v : b2);
-                            i2 = c1 ? i1 : (c2 ? n : i2);
-                            b1 = c0 ? b0 : (c1 ? v : b1);
-                            i1 = c0 ? i0 : (c1 ? n : i1);
-                            b0 = c0 ? v : b0;
-                            i0 = c0 ? n : i0;
-                        }
-                    }
-                    float T = inf;
-                    int got = i0;
-                    if (got >= k) {
-                        T = b0;
-                    } else {
-                        got += i1;
-                        if (got >= k) {
-                            T = b1;
-                        } else {
-                            got += i2;
-                            if (got >= k) {
-                                T = b2;
-                            } else {
-                                got += i3;
-                                if (got >= k) T = b3;
-                            }
-                        }
-                    }
-                    R = fminf(R, T);
-                }
-                L.thr[lane] = fminf(fminf(L.thr[lane], thr), screen_threshold<COS>(R, L.qs[lane], L.eps[lane]));
+                const float R = __uint_as_float(SHARED_R[qmine]);
+                L.thr[lane] = fminf(fminf(L.thr[lane], thr), screen_threshold(R, L.qs[lane], L.eps[lane]));
             }
             thr = L.thr[jl];
         }
     };
-    if constexpr (SINGLE) {
-        for (int64_t t0 = t_begin; t0 < t_end; t0 += kBn) tile_step(tileA, tnA, tileA, t0);
-    } else {
-        for (int64_t t0 = t_begin; t0 < t_end; t0 += 2 * kBn) {
-            tile_step(tileA, tnA, tileB, t0);
-            if (t0 + kBn < t_end) tile_step(tileB, tnB, tileA, t0 + kBn);
-        }
+    for (int64_t t0 = t_begin; t0 < t_end; t0 += 2 * kBn) {
+        tile_step(tileA, tnA, t0);
+        if (t0 + kBn < t_end) tile_step(tileB, tnB, t0 + kBn);
     }
 
     // ---- final flush of every non-empty queue ----
-    {
-        uint64_t mask = __builtin_amdgcn_ballot_w64(lane < QPW && cntr > 0u);
-        if (K1) {
-            if (mask) MLRS_FLUSH_K1();
-        } else {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            while (mask) {
-                const int j = __builtin_ctzll(mask);
-                mask &= mask - 1;
-                MLRS_FLUSH(j);
-            }
-        }
-    }
-#undef MLRS_FLUSH_K1
+    if (__builtin_amdgcn_ballot_w64(lane < QPW && cntr > 0u)) MLRS_FLUSH();
 #undef MLRS_FLUSH
-#undef MLRS_EXACT_AT
 #undef MLRS_PREFETCH
 #undef MLRS_PF_SRC
 #undef MLRS_PF_ROW
 #undef MLRS_PF_ON
 
-    // ---- k = 1: the kept pair becomes this segment's one-entry list ----
-    if (K1 && lane < QPW && qvalid) {
+    // ---- the kept pair is this segment's ----
+    if (lane < QPW && qvalid) {
         const unsigned long long b = L.best[lane];
         LV[qmine] = __uint_as_float((uint32_t)(b >> 32));
         LI[qmine] = (uint32_t)b;
@@ -1207,9 +659,9 @@ hipError_t launch_ng(const GramArgs32& a, int arm, hipStream_t s) {
     dim3 grid((unsigned)StreamSplit(a.nq, a.nt, a.qpb, kBn, a.grid_wgs).G);
     const dim3 block(GramShape<(NG > 16)>::threads);
     if (arm == ARM_EUCLID_MULADD)
-        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM_EUCLID_MULADD, false, VEC4, true, 1>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM_EUCLID_MULADD, VEC4>), grid, block, 0, s, a);
     else
-        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM_EUCLID_FMA, false, VEC4, true, 1>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((knn_gram_f32_kernel<NG, ARM_EUCLID_FMA, VEC4>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
@@ -1232,22 +684,19 @@ hipError_t launch_d(const GramArgs32& a, int arm, hipStream_t s) {
 int gram_f32_queries_per_block(int64_t d) { return d > 128 ? kQpbWide : kQpbNarrow; }
 
 
-void gram_f32_split(int64_t nq, int64_t nt, int64_t d, int k, int cus, bool vec4, int64_t* grid_wgs, int* nslots) {
+void gram_f32_split(int64_t nq, int64_t nt, int64_t d, int cus, int64_t* grid_wgs, int* nslots) {
     const int64_t qpb = gram_f32_queries_per_block(d);
     const StreamSplit full(nq, nt, qpb, kBn, 1);
     // one resident round (gram_f32_wgs_per_cu workgroups per CU), but at
     // least 16 tiles each
-    const int per_cu = gram_f32_wgs_per_cu((int)((d + 7) / 8), k == 1, k <= 64 ? 1 : 3, vec4);
-    int64_t g0 = per_cu * (int64_t)(cus > 0 ? cus : 1);
+    int64_t g0 = gram_f32_wgs_per_cu((int)((d + 7) / 8)) * (int64_t)(cus > 0 ? cus : 1);
     if (g0 > full.T / 16) g0 = full.T / 16;
     if (g0 < 1) g0 = 1;
     *grid_wgs = g0;
     *nslots = (int)StreamSplit(nq, nt, qpb, kBn, g0).nslots();
 }
 
-int gram_f32_max_k() { return kKcap; }
 int gram_f32_max_d() { return 256; }
-int gram_f32_rows_per_tile() { return kBn; }
 
 hipError_t launch_gram_f32_prep(const GramArgs32& a, hipStream_t s) {
     if (!a.shared_r) return hipSuccess;

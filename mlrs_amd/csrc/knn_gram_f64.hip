@@ -1,14 +1,6 @@
-// Fused f64 Gram-MFMA kNN with exact rescoring (gfx950).
-//
-// The f64 counterpart of knn_gram_f32.hip: serves every cpu arm
-// (direct / metric / knn_host, Euclidean and cosine) for d <= 256, k <= 128,
-// replacing the materialized-matrix paths tiled_distance_topk /
-// tiled_metric_distance_topk (crates/mlrs-algos/src/neighbors/nearest.rs:
-// 1058-1512) and the host scan of knn_host_topk (crates/mlrs-backend/src/
-// prims/knn_host.rs:418-851) for f64.
-//
-// Launched for the k-means assignment only (k = 1, ARM_EUCLID_MULADD); searches
-// are knn_groupmin's.
+// Fused f64 Gram-MFMA nearest row with exact rescoring (gfx950): the k-means
+// assignment (argmin_dist_rows, crates/mlrs-kernels/src/kmeans.rs:284-310) in
+// f64, d <= 256.
 //
 // Shape of one workgroup: 4 waves x 16 queries = 64 queries, walking one
 // segment of index rows 16 at a time with v_mfma_f64_16x16x4f64.
@@ -16,13 +8,14 @@
 //    dimension is split into four contiguous quarters of NS columns: at
 //    k-step s, group g supplies column g*NS + s of both operands, so each
 //    lane's A operand is a contiguous run of its tile row (ds_read_b128
-//    feeds two k-steps) and its B operand (the query, pre-scaled by -2 for
-//    Euclidean) is held in VGPRs for the whole segment.
+//    feeds two k-steps) and its B operand (the query, pre-scaled by -2) is
+//    held in VGPRs for the whole segment.
 //  * The MFMA result layout is D[l/16 + 4r][l%16], r = 0..3: lane l scores
 //    tile rows g, g+4, g+8, g+12 against its query.
-//  * The screen, the per-query queues, the exact rescoring in the reference
-//    arm's operation order, the (value, index) lists and the stream-K split
-//    with a shared per-query bound are those of the f32 kernel, in double.
+//  * The screen, the per-query queues, the exact rescoring in the arm's
+//    operation order and the stream-K split with a shared per-query bound are
+//    those of the f32 kernel, in double; the bound starts from a sample of the
+//    rows (knn_seed_f64_kernel).
 // The thresholds are computed in double with a margin for their own
 // rounding folded into the error bound (the f32 kernel rounds up in double
 // instead).
@@ -37,7 +30,6 @@ constexpr int kWaves = 4;
 constexpr int kQpw = 16;               // queries per wave (MFMA N dimension)
 constexpr int kQpb = kWaves * kQpw;    // queries per workgroup
 constexpr int kBn = 16;                // index rows per tile (MFMA M dimension)
-constexpr int kKcap = 128;             // largest k kept
 constexpr int kQcap = 48;              // queued candidates per query (two workgroups still fit a CU's LDS)
 constexpr int kFlushAt = kQcap - kBn;  // flush when a queue may overflow on the next tile
 constexpr int kShareEvery = 32;        // tiles between reads of the shared bound
@@ -48,34 +40,23 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 struct WaveLds64 {
     uint32_t qidx[kQpw][kQcap];
     double thr[kQpw];
-    double qa[kQpw];   // exact arm's query operand (squared or reciprocal norm)
-    double qs[kQpw];   // screen operand: ||q||^2 (Euclidean) or ||q|| (cosine)
+    double qs[kQpw];   // ||q||^2
     double eps[kQpw];  // screen error bound
-    uint32_t mode[kQpw];  // 0 = screen-value list, 1 = exact list
 };
 
-constexpr unsigned long long kInfBits64 = 0x7FF0000000000000ull;
-
-template <bool COS>
 __device__ __forceinline__ double screen_threshold64(double R, double qs, double eps) {
     const double inf = __builtin_huge_val();
     if (!(R < inf)) return inf;
-    // Euclidean: R widened by a relative 2^-48, so that every pair whose root
-    // equals the root of a value <= R passes too (the X-vs-X graph ranks by
-    // the root, and sqrt maps at most a few consecutive doubles to one)
-    if (!COS) return ((R + __builtin_fabs(R) * 0x1p-48) - qs) + eps;
-    if (qs == 0.0) return inf;  // a zero query ties every row: never screened
-    return ((R + eps) - 1.0) * qs;
+    return ((R + __builtin_fabs(R) * 0x1p-48) - qs) + eps;
 }
 
 // Exact value of one (query, row) pair in the arm's operation order; loads
-// issued U 16-byte pairs at a time when rows are 16-byte aligned (inside the
-// Gram kernel U = 2: the d = 256 kernel holds 128 VGPRs of query operand;
-// the merge kernel has registers for more in flight).
-template <int ARM, bool VEC2, int U = 2>
-__device__ __forceinline__ double exact_f64(const double* __restrict__ q, const double* __restrict__ y,
-                                            int64_t d, double qa, double ya) {
-    if (!VEC2) return exact_pair<double, ARM>(q, y, d, qa, ya);
+// issued two 16-byte pairs at a time when rows are 16-byte aligned (the d = 256
+// kernel holds 128 VGPRs of query operand).
+template <bool VEC2>
+__device__ __forceinline__ double exact_f64(const double* __restrict__ q, const double* __restrict__ y, int64_t d) {
+    if (!VEC2) return exact_pair<double, ARM_EUCLID_MULADD>(q, y, d, 0.0, 0.0);
+    constexpr int U = 2;
     const double2* q2 = reinterpret_cast<const double2*>(q);
     const double2* y2 = reinterpret_cast<const double2*>(y);
     const int n2 = (int)(d >> 1);
@@ -97,35 +78,15 @@ __device__ __forceinline__ double exact_f64(const double* __restrict__ q, const 
         for (int u = 0; u < U; ++u) {
             if (c + u >= n2) break;
             const double e0a = a[u].x, e1a = a[u].y, e0b = b[u].x, e1b = b[u].y;
-            if (ARM == ARM_EUCLID_FMA) {
-                const double d0 = e0a - e0b, d1 = e1a - e1b;
-                acc = __builtin_fma(d0, d0, acc);
-                acc = __builtin_fma(d1, d1, acc);
-            } else if (ARM == ARM_EUCLID_MULADD) {
-                const double d0 = e0a - e0b, d1 = e1a - e1b;
-                acc = acc + d0 * d0;
-                acc = acc + d1 * d1;
-            } else if (ARM == ARM_COS_FOLD) {
-                acc = __builtin_fma(e0a, e0b, acc);
-                acc = __builtin_fma(e1a, e1b, acc);
-            } else {  // ARM_COS_HOST: mul + add
-                acc = acc + e0a * e0b;
-                acc = acc + e1a * e1b;
-            }
+            const double d0 = e0a - e0b, d1 = e1a - e1b;
+            acc = acc + d0 * d0;
+            acc = acc + d1 * d1;
         }
     }
-    if (ARM == ARM_COS_FOLD) {
-        const double denom = __builtin_sqrt(qa * ya);
-        const double sim = (denom > 0.0) ? acc / denom : 0.0;
-        return clamp02<double>(1.0 - sim);
-    }
-    if (ARM == ARM_COS_HOST) return clamp02<double>(1.0 - acc * qa * ya);
     return acc;
 }
 
-// KL: 64-entry blocks of a (segment, query) list during a flush (1 for
-// k <= 64, 3 for k <= 128: k + 32 entries).
-template <int NS, int ARM, bool COS, bool VEC2, int KL>
+template <int NS, bool VEC2>
 __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
     constexpr int DP = 4 * NS;             // padded feature count
     constexpr int STRIDE = DP + 2;         // LDS row stride (doubles): rows 16 bytes apart in the banks
@@ -154,13 +115,8 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
     const double* __restrict__ X = a.x;
     const double* __restrict__ QSQ = a.qsq;
     const double* __restrict__ XSQ = a.xsq;
-    const double* __restrict__ QINV = a.qinv;
-    const double* __restrict__ XINV = a.xinv;
-    const double* __restrict__ XSCALE = a.xscale;
     unsigned long long* __restrict__ SHARED_R = a.shared_r;
     const int64_t nq = a.nq, nt = a.nt, d = a.d;
-    const int k = a.k;
-    const int K2 = gram_list_cap(k);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform: tile rows and LDS slots in SGPRs
@@ -168,9 +124,6 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
     const int jl = lane & 15;  // query of the lane within the wave
     WaveLds64& L = wl[w];
     const double inf = __builtin_huge_val();
-    // screen values of this wave's queued pairs, [query][queue position]
-    double* __restrict__ QVw = a.qval + ((int64_t)blockIdx.x * kWaves + w) * (kQpw * kQcap);
-
     // ---- work split (StreamSplit), as in the f32 kernel ----
     const StreamSplit sp(nq, nt, kQpb, kBn, a.grid_wgs);
     const int64_t wg = xcd_grouped_wg(blockIdx.x, gridDim.x);
@@ -180,8 +133,8 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
     sp.decode(u, panel, qblock, tile0, left);
     const int64_t tile1 = tile0 + ((left < u_hi - u) ? left : (u_hi - u));
     const int64_t slot = sp.slot(wg, panel, qblock);
-    double* __restrict__ LV = a.part_val + slot * nq * K2;
-    uint32_t* __restrict__ LI = a.part_idx + slot * nq * K2;
+    double* __restrict__ LV = a.part_val + slot * nq;
+    uint32_t* __restrict__ LI = a.part_idx + slot * nq;
 
     const int64_t qwave = qblock * kQpb + w * kQpw;
     const int64_t qmine = qwave + jl;
@@ -195,42 +148,22 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
     if (lane < kQpw) {
         const double qsq = qvalid ? QSQ[qmine] : 0.0;
         L.thr[lane] = qvalid ? inf : -inf;
-        if (!COS) {
-            L.qs[lane] = qsq;
-            L.qa[lane] = 0.0;
-            L.eps[lane] = a.eps_rel * (qsq + a.stats->xsq_max64) + a.eps_abs;
-        } else {
-            L.qs[lane] = __builtin_sqrt(qsq);
-            L.qa[lane] = (ARM == ARM_COS_HOST) ? (qvalid ? QINV[qmine] : 0.0) : qsq;
-            L.eps[lane] = a.eps_abs;
-        }
-        // Screen-value lists need |screen distance - exact| <= eps for every
-        // pair: norms well inside the double range (a nonzero query for
-        // cosine), and k > 1 (a one-entry list has no room for near ties).
-        bool sv = qvalid && k > 1 && (qsq + a.stats->xsq_max64 <= 0x1p1020) && (L.eps[lane] < inf);
-        if (COS) sv = sv && (L.qs[lane] > 0.0);
-        L.mode[lane] = sv ? 0u : 1u;
-    }
-    for (int j = 0; j < kQpw; ++j) {
-        const int64_t qg = qwave + j;
-#pragma unroll
-        for (int r = 0; r < KL; ++r) {
-            const int p = 64 * r + lane;
-            if (qg < nq && p < K2) {
-                LV[qg * K2 + p] = inf;
-                LI[qg * K2 + p] = kSentinelIdx;
-            }
+        L.qs[lane] = qsq;
+        L.eps[lane] = a.eps_rel * (qsq + a.stats->xsq_max64) + a.eps_abs;
+        if (qvalid) {
+            LV[qmine] = inf;
+            LI[qmine] = kSentinelIdx;
         }
     }
     if (SHARED_R && lane < kQpw && qvalid) {
         const double R0 = __longlong_as_double((long long)SHARED_R[qmine]);
-        L.thr[lane] = fmin(L.thr[lane], screen_threshold64<COS>(R0, L.qs[lane], L.eps[lane]));
+        L.thr[lane] = fmin(L.thr[lane], screen_threshold64(R0, L.qs[lane], L.eps[lane]));
     }
 
     // ---- query operand: qreg[s] = scale * q[g*NS + s] ----
     double qreg[NS];
     {
-        const double scale = COS ? 1.0 : -2.0;
+        const double scale = -2.0;
         const double* qp = Q + qmine * d;
         if (VEC2) {  // 16-byte loads, all issued before use (NS and d even)
 #pragma unroll
@@ -281,124 +214,40 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
         pfp += kBn * d;                                                                      \
         if (tid < kBn) {                                                                     \
             const uint32_t t = t0_ + (uint32_t)tid;                                          \
-            if (COS)                                                                         \
-                pfn = (t < t_end32) ? XSCALE[t] : 0.0;                                       \
-            else                                                                             \
-                pfn = (t < t_end32) ? XSQ[t] : inf;                                          \
+            pfn = (t < t_end32) ? XSQ[t] : inf;                                              \
         }                                                                                    \
     } while (0)
 
-// Flush: one query's queue sorted and merged into its list.  Screen-value
-// mode: a queued pair enters with its screen value mapped back to a
-// distance, within eps of its exact value; the list keeps the K2 smallest and
-// the segment's bound is its k-th + eps.  A pair whose screen value is NaN,
-// and every pair of an exact-mode query, is evaluated exactly in the arm's
-// operation order.  When a discarded pair lies within 2 eps of the k-th, the
-// old list and the queue are re-evaluated exactly and the query's list stays
-// exact from then on.
-#define MLRS_EXACT64_AT(T_)                                                                  \
-    exact_f64<ARM, VEC2>(Q + qg_ * d, X + (int64_t)(T_) * d, d, L.qa[j_],                    \
-                         (ARM == ARM_COS_FOLD) ? XSQ[(T_)] : (ARM == ARM_COS_HOST) ? XINV[(T_)] : 0.0)
+// Flush: one query's queued rows evaluated exactly, the best of them against
+// the segment's best pair (in memory).
 #define MLRS_FLUSH64(J)                                                                      \
     do {                                                                                     \
         const int j_ = (J);                                                                  \
         const int64_t qg_ = qwave + j_;                                                      \
-        const uint32_t n_ = bcast_u(cntr, j_);                                                \
-        const bool exact_ = L.mode[j_] != 0u;                                                \
-        double lv_[KL];                                                                      \
-        uint32_t li_[KL];                                                                    \
-        _Pragma("unroll") for (int r_ = 0; r_ < KL; ++r_) {                                  \
-            const int p_ = 64 * r_ + lane;                                                   \
-            lv_[r_] = (p_ < K2) ? LV[qg_ * K2 + p_] : inf;                                   \
-            li_[r_] = (p_ < K2) ? LI[qg_ * K2 + p_] : kSentinelIdx;                          \
-        }                                                                                    \
+        const uint32_t n_ = bcast_u(cntr, j_);                                               \
         double e_ = inf;                                                                     \
         uint32_t t_ = kSentinelIdx;                                                          \
         if ((uint32_t)lane < n_) {                                                           \
             t_ = L.qidx[j_][lane];                                                           \
-            const double s_ = exact_ ? 0.0 : QVw[j_ * kQcap + lane];                         \
-            if (exact_ || s_ != s_)                                                          \
-                e_ = MLRS_EXACT64_AT(t_);                                                    \
-            else                                                                             \
-                e_ = COS ? 1.0 + s_ / L.qs[j_] : s_ + L.qs[j_];                              \
-            if (e_ != e_) {                                                                  \
+            e_ = exact_f64<VEC2>(Q + qg_ * d, X + (int64_t)t_ * d, d);                       \
+            if (e_ != e_) { /* NaN is never admitted */                                      \
                 e_ = inf;                                                                    \
                 t_ = kSentinelIdx;                                                           \
             }                                                                                \
         }                                                                                    \
         wave_sort64<double>(e_, t_, lane);                                                   \
-        const uint32_t oi_ = li_[0];                                                         \
-        double dm_;                                                                          \
-        if constexpr (KL == 1)                                                               \
-            dm_ = wave_merge64_drop<double>(lv_[0], li_[0], e_, t_, lane);                   \
-        else                                                                                 \
-            dm_ = wave_merge_blocks_drop<double, KL>(lv_, li_, e_, t_, lane);                \
-        double R_ = list_value_at<double, KL>(lv_, k - 1);                                   \
-        /* the smallest exact value the list drops (exact lists only) */                     \
-        double dx_ = exact_ ? ((K2 < 64 * KL) ? list_value_at<double, KL>(lv_, K2) : dm_) : inf; \
-        if (!exact_) {                                                                       \
-            const double dr_ = (K2 < 64 * KL) ? list_value_at<double, KL>(lv_, K2) : dm_;    \
-            double w_ = R_ + 2.0 * L.eps[j_];                                                \
-            w_ += __builtin_fabs(w_) * 0x1p-40;                                              \
-            if (dr_ < inf && dr_ <= w_) {                                                    \
-              if constexpr (KL == 1) {                                                       \
-                double x1_ = inf, x2_ = inf;                                                 \
-                uint32_t i1_ = oi_, i2_ = t_;                                                \
-                if (i1_ != kSentinelIdx) x1_ = MLRS_EXACT64_AT(i1_);                         \
-                if (i2_ != kSentinelIdx) x2_ = MLRS_EXACT64_AT(i2_);                         \
-                if (x1_ != x1_) { x1_ = inf; i1_ = kSentinelIdx; }                           \
-                if (x2_ != x2_) { x2_ = inf; i2_ = kSentinelIdx; }                           \
-                wave_sort64<double>(x1_, i1_, lane);                                         \
-                wave_sort64<double>(x2_, i2_, lane);                                         \
-                dx_ = wave_merge64_drop<double>(x1_, i1_, x2_, i2_, lane);                   \
-                lv_[0] = x1_;                                                                \
-                li_[0] = i1_;                                                                \
-              } else {                                                                       \
-                /* the old list (still in memory) and the queue, exactly */                  \
-                _Pragma("unroll") for (int r_ = 0; r_ < KL; ++r_) {                          \
-                    lv_[r_] = inf;                                                           \
-                    li_[r_] = kSentinelIdx;                                                  \
-                }                                                                            \
-                _Pragma("unroll") for (int r_ = 0; r_ <= KL; ++r_) {                         \
-                    uint32_t i_ = kSentinelIdx;                                              \
-                    if (r_ < KL) {                                                           \
-                        const int p_ = 64 * r_ + lane;                                       \
-                        if (p_ < K2) i_ = LI[qg_ * K2 + p_];                                 \
-                    } else if ((uint32_t)lane < n_) {                                        \
-                        i_ = L.qidx[j_][lane];                                               \
-                    }                                                                        \
-                    double x_ = inf;                                                         \
-                    if (i_ != kSentinelIdx) x_ = MLRS_EXACT64_AT(i_);                        \
-                    if (x_ != x_) { x_ = inf; i_ = kSentinelIdx; }                           \
-                    wave_sort64<double>(x_, i_, lane);                                       \
-                    dx_ = fmin(dx_, wave_merge_blocks_drop<double, KL>(lv_, li_, x_, i_, lane)); \
-                }                                                                            \
-              }                                                                              \
-                if (K2 < 64 * KL) dx_ = fmin(dx_, list_value_at<double, KL>(lv_, K2));       \
-                R_ = list_value_at<double, KL>(lv_, k - 1);                                  \
-                if (lane == 0) L.mode[j_] = 1u;                                              \
-            } else if (R_ < inf) {                                                           \
-                R_ = R_ + L.eps[j_];                                                         \
-            }                                                                                \
-        }                                                                                    \
-        _Pragma("unroll") for (int r_ = 0; r_ < KL; ++r_) {                                  \
-            const int p_ = 64 * r_ + lane;                                                   \
-            if (p_ < K2) {                                                                   \
-                LV[qg_ * K2 + p_] = lv_[r_];                                                 \
-                LI[qg_ * K2 + p_] = li_[r_];                                                 \
-            }                                                                                \
-        }                                                                                    \
-        /* a dropped exact value whose root may equal the k-th's: the merge */               \
-        /* cannot rank that root's ties by index, the root fill will */                      \
-        if (a.root_flag && lane == 0 && dx_ < inf && dx_ <= R_ + __builtin_fabs(R_) * 0x1p-48) \
-            a.root_flag[qg_] = 1u;                                                           \
         if (lane == 0) {                                                                     \
-            if (SHARED_R && R_ < inf && R_ >= 0.0) {                                         \
+            double R_ = LV[qg_];                                                             \
+            if (pair_less<double>(e_, t_, R_, LI[qg_])) {                                    \
+                LV[qg_] = R_ = e_;                                                           \
+                LI[qg_] = t_;                                                                \
+            }                                                                                \
+            if (SHARED_R && R_ < inf) {                                                      \
                 const unsigned long long old_ =                                              \
                     atomicMin(&SHARED_R[qg_], (unsigned long long)__double_as_longlong(R_)); \
                 R_ = fmin(R_, __longlong_as_double((long long)old_));                        \
             }                                                                                \
-            L.thr[j_] = fmin(L.thr[j_], screen_threshold64<COS>(R_, L.qs[j_], L.eps[j_]));   \
+            L.thr[j_] = fmin(L.thr[j_], screen_threshold64(R_, L.qs[j_], L.eps[j_]));        \
         }                                                                                    \
         if (jl == j_) cntr = 0u;                                                             \
     } while (0)
@@ -445,10 +294,7 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
         }
         if (tid < kBn) {
             const uint32_t t = t0 + (uint32_t)tid;
-            if (COS)
-                pfn = (t < t_end32) ? XSCALE[t] : 0.0;
-            else
-                pfn = (t < t_end32) ? XSQ[t] : inf;
+            pfn = (t < t_end32) ? XSQ[t] : inf;
         }
     };
     if (DIRECT && d < DP) {
@@ -496,7 +342,7 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
         f64x4 acc0, acc1;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            acc0[r] = COS ? 0.0 : tncur[g + 4 * r];
+            acc0[r] = tncur[g + 4 * r];
             acc1[r] = 0.0;
         }
         // A operand: this lane's tile row jl, columns g*NS + s; one 16-byte
@@ -516,13 +362,6 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
         f64x4 acc;
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[r] = acc0[r] + acc1[r];
-        if (COS) {
-            // rows scaled by -1/||x_t|| after the contraction (the scales ride
-            // in tnorm), so the prefetched loads need no arithmetic until the
-            // LDS store after the MFMAs
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r] *= tncur[g + 4 * r];
-        }
         if (more) {
             if (DIRECT) {
                 if (tid < kBn) tnnxt[tid] = pfn;
@@ -555,7 +394,6 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
             for (int r = 0; r < 4; ++r) {
                 if (m & (1u << r)) {
                     L.qidx[jl][pos] = (uint32_t)t0 + (uint32_t)(g + 4 * r);
-                    QVw[jl * kQcap + pos] = acc[r];
                     ++pos;
                 }
             }
@@ -564,7 +402,7 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
         uint64_t mask = __builtin_amdgcn_ballot_w64(lane < kQpw && cntr > (uint32_t)kFlushAt);
         if (mask) {
             if (lane < kQpw) L.thr[lane] = fmin(L.thr[lane], thr);
-            // the queued screen values were stored by other lanes of this wave
+            // the queued rows were stored by other lanes of this wave
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
             while (mask) {
@@ -578,7 +416,7 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
         if (SHARED_R && (++tiles % kShareEvery) == 0) {
             if (lane < kQpw && qvalid) {
                 const double R = __longlong_as_double((long long)SHARED_R[qmine]);
-                L.thr[lane] = fmin(fmin(L.thr[lane], thr), screen_threshold64<COS>(R, L.qs[lane], L.eps[lane]));
+                L.thr[lane] = fmin(fmin(L.thr[lane], thr), screen_threshold64(R, L.qs[lane], L.eps[lane]));
             }
             thr = L.thr[jl];
         }
@@ -601,7 +439,6 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
         }
     }
 #undef MLRS_FLUSH64
-#undef MLRS_EXACT64_AT
 #undef MLRS_STORE64
 #undef MLRS_PREFETCH64
     u += tile1 - tile0;
@@ -609,133 +446,55 @@ __global__ __launch_bounds__(256, 2) void knn_gram_f64_kernel(GramArgs64 a) {
     }
 }
 
-// Merge the per-segment lists of one query per wave and emit the output
-// transform (boundary sqrt, identity, or the k-means pair with the centre-0
-// NaN rule of argmin_dist_rows, crates/mlrs-kernels/src/kmeans.rs:284-310).
-// Every list entry's value lies within eps of its pair's exact value (exact
-// entries equal it) and the segments hold disjoint index rows, so with V the
-// k-th smallest value over all lists a pair can be among the k best only if
-// its value is <= V + 2 eps: exactly those pairs are evaluated in the arm's
-// operation order and ranked by (exact value, index), NaN never admitted.
-// EMIT_ROOT_RANKED ranks by (sqrt(exact value), index) instead: every pair
-// whose root equals the k-th root lies within V + 2 eps too (its aggregate
-// exceeds the k-th by a relative 2^-50 at most), and the kernel's screen and
-// drops keep all of them listed unless root_flag says otherwise.
-template <int ARM, bool VEC2>
+// A query's best pair over its segments, and the output transform: the k-means
+// pair with the centre-0 NaN rule of argmin_dist_rows
+// (crates/mlrs-kernels/src/kmeans.rs:284-310), the boundary sqrt or identity.
 __global__ __launch_bounds__(256) void knn_merge_f64_kernel(GramArgs64 a) {
-    __shared__ uint32_t cand[4][128];
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    const int64_t qg = (int64_t)blockIdx.x * 4 + wv;
+    const int64_t qg = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (qg >= a.nq) return;
-    const int k = a.k;
-    const int K2 = gram_list_cap(k);
-    const int64_t d = a.d;
     const double inf = __builtin_huge_val();
     const StreamSplit sp(a.nq, a.nt, kQpb, kBn, a.grid_wgs);
     const int64_t nsl = sp.slots_of(qg / kQpb);
-    double uv = inf;
-    uint32_t ui = kSentinelIdx;
-    for (int64_t s = 0; s < nsl; ++s) {
-        double v = inf;
-        uint32_t ix = kSentinelIdx;
-        if (lane < K2) {
-            const int64_t o = (s * a.nq + qg) * K2 + lane;
-            v = a.part_val[o];
-            ix = a.part_idx[o];
+    double lv = a.part_val[qg];
+    uint32_t li = a.part_idx[qg];
+    for (int64_t s = 1; s < nsl; ++s) {
+        const double v = a.part_val[s * a.nq + qg];
+        const uint32_t ix = a.part_idx[s * a.nq + qg];
+        if (pair_less<double>(v, ix, lv, li)) {
+            lv = v;
+            li = ix;
         }
-        wave_merge64<double>(uv, ui, v, ix, lane);
     }
-    const double qsq = a.qsq[qg];
-    const bool cos = (ARM == ARM_COS_FOLD || ARM == ARM_COS_HOST);
-    const double eps = cos ? a.eps_abs : a.eps_rel * (qsq + a.stats->xsq_max64) + a.eps_abs;
-    double W = bcast_f(uv, k - 1) + 2.0 * eps;
-    W += __builtin_fabs(W) * 0x1p-40;
-    const double qa = (ARM == ARM_COS_HOST) ? a.qinv[qg] : qsq;
-    double lv = inf;
-    uint32_t li = kSentinelIdx;
-    uint32_t nc = 0;
-    auto evaluate = [&](uint32_t count) {
-        double e = inf;
-        uint32_t t = kSentinelIdx;
-        if ((uint32_t)lane < count) {
-            t = cand[wv][lane];
-            const double ya = (ARM == ARM_COS_FOLD) ? a.xsq[t] : (ARM == ARM_COS_HOST) ? a.xinv[t] : 0.0;
-            e = exact_f64<ARM, VEC2, 8>(a.q + qg * d, a.x + (int64_t)t * d, d, qa, ya);
-            if (e != e) {
-                e = inf;
-                t = kSentinelIdx;
-            } else if (a.mode == EMIT_ROOT_RANKED) {
-                e = __builtin_sqrt(e);  // ranked by (root, index)
+    if (a.mode == EMIT_KMEANS) {
+        if (!(a.qsq[qg] < inf) || !(a.xsq[0] < inf)) {
+            const double e0 = exact_pair<double, ARM_EUCLID_MULADD>(a.q + qg * a.d, a.x, a.d, 0.0, 0.0);
+            if (e0 != e0) {
+                lv = e0;
+                li = 0;
             }
         }
-        wave_sort64<double>(e, t, lane);
-        wave_merge64<double>(lv, li, e, t, lane);
-    };
-    for (int64_t s = 0; s < nsl; ++s) {
-        bool in = false;
-        uint32_t ix = kSentinelIdx;
-        if (lane < K2) {
-            const int64_t o = (s * a.nq + qg) * K2 + lane;
-            ix = a.part_idx[o];
-            in = (ix != kSentinelIdx) && !(a.part_val[o] > W);
-        }
-        const uint64_t bal = __builtin_amdgcn_ballot_w64(in);
-        const uint32_t pre = (uint32_t)__builtin_popcountll(bal & ((1ull << lane) - 1ull));
-        if (in) cand[wv][nc + pre] = ix;
-        nc += (uint32_t)__builtin_popcountll(bal);
-        if (nc >= 64) {
-            evaluate(64);
-            const uint32_t rest = nc - 64;
-            const uint32_t mv = ((uint32_t)lane < rest) ? cand[wv][64 + lane] : 0u;
-            if ((uint32_t)lane < rest) cand[wv][lane] = mv;
-            nc = rest;
-        }
+        a.out_val[qg] = lv;
+    } else {
+        a.out_val[qg] = (a.mode == EMIT_SQRT) ? __builtin_sqrt(lv) : lv;
     }
-    if (nc > 0) evaluate(nc);
-    if (lane < k) {
-        const int64_t o = qg * k + lane;
-        if (a.mode == EMIT_KMEANS) {
-            if (!(a.qsq[qg] < inf) || !(a.xsq[0] < inf)) {
-                const double e0 = exact_pair<double, ARM_EUCLID_MULADD>(a.q + qg * a.d, a.x, a.d, 0.0, 0.0);
-                if (e0 != e0) {
-                    lv = e0;
-                    li = 0;
-                }
-            }
-            a.out_val[o] = lv;
-        } else {
-            a.out_val[o] = (a.mode == EMIT_SQRT) ? __builtin_sqrt(lv) : lv;
-        }
-        a.out_idx[o] = (li == kSentinelIdx) ? 0u : li;
-    }
+    a.out_idx[qg] = (li == kSentinelIdx) ? 0u : li;
 }
 
-// Initial per-query bound: the k-th smallest exact value over an evenly
-// spaced sample of index rows (seed_kth_block): any k distinct rows bound the
-// final k-th value from above, so each segment's screen starts tight instead
-// of at +inf.
-// SB: 64-entry blocks of the running sample list (k <= 64 SB).
-template <int ARM, int SB>
+// Initial per-query bound: the smallest exact value over an evenly spaced
+// sample of index rows (seed_kth_block), so that each segment's screen starts
+// tight instead of at +inf.
 __global__ __launch_bounds__(256) void knn_seed_f64_kernel(GramArgs64 a, int64_t nsamp) {
-    const double* qop = (ARM == ARM_COS_FOLD) ? a.qsq : a.qinv;
-    const double* yop = (ARM == ARM_COS_FOLD) ? a.xsq : a.xinv;
-    seed_kth_block<double, ARM, unsigned long long, SB>(a.q, a.x, a.nq, a.nt, a.d, a.k, nsamp, qop, yop,
-                                                        a.shared_r);
-}
-
-__global__ void fill_u64_kernel(unsigned long long* p, int64_t n, unsigned long long v) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+    seed_kth_block<double, ARM_EUCLID_MULADD, unsigned long long, 1>(a.q, a.x, a.nq, a.nt, a.d, 1, nsamp, nullptr,
+                                                                     nullptr, a.shared_r);
 }
 
 template <int NS>
 hipError_t launch_ns(const GramArgs64& a, bool vec2, hipStream_t s) {
     dim3 grid((unsigned)StreamSplit(a.nq, a.nt, kQpb, kBn, a.grid_wgs).G);
     if (vec2)
-        hipLaunchKernelGGL((knn_gram_f64_kernel<NS, ARM_EUCLID_MULADD, false, true, 1>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((knn_gram_f64_kernel<NS, true>), grid, dim3(256), 0, s, a);
     else
-        hipLaunchKernelGGL((knn_gram_f64_kernel<NS, ARM_EUCLID_MULADD, false, false, 1>), grid, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((knn_gram_f64_kernel<NS, false>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -756,22 +515,18 @@ void gram_f64_split(int64_t nq, int64_t nt, int cus, int64_t* grid_wgs, int* nsl
     *nslots = (int)StreamSplit(nq, nt, kQpb, kBn, g0).nslots();
 }
 
-int gram_f64_max_k() { return kKcap; }
 int gram_f64_max_d() { return kMaxD; }
 
 hipError_t launch_gram_f64_prep(const GramArgs64& a, hipStream_t s) {
-    const int64_t nsamp = gram_seed_rows(a.nt, a.k);
-    if (nsamp >= a.k)
-        hipLaunchKernelGGL((knn_seed_f64_kernel<ARM_EUCLID_MULADD, 1>),
-                           dim3((unsigned)((a.nq + kSeedQpb - 1) / kSeedQpb)), dim3(256), 0, s, a, nsamp);
-    else
-        hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a.shared_r, a.nq,
-                           kInfBits64);
+    // 512 rows, or the whole index
+    const int64_t nsamp = a.nt < 512 ? a.nt : 512;
+    hipLaunchKernelGGL(knn_seed_f64_kernel, dim3((unsigned)((a.nq + kSeedQpb - 1) / kSeedQpb)), dim3(256), 0, s, a,
+                       nsamp);
     return hipGetLastError();
 }
 
 hipError_t launch_gram_f64(const GramArgs64& a, int arm, hipStream_t s) {
-    if (a.k != 1 || arm != ARM_EUCLID_MULADD) return hipErrorInvalidValue;
+    if (arm != ARM_EUCLID_MULADD) return hipErrorInvalidValue;
     const bool vec2 = rows_vec2(a);
     // k-steps per lane group, even (one 16-byte LDS read feeds two)
     const int64_t ns = ((a.d + 3) / 4 + 1) / 2 * 2;
@@ -783,11 +538,7 @@ hipError_t launch_gram_f64(const GramArgs64& a, int arm, hipStream_t s) {
 }
 
 hipError_t launch_gram_f64_merge(const GramArgs64& a, hipStream_t s) {
-    const dim3 grid((unsigned)((a.nq + 3) / 4));
-    if (rows_vec2(a))
-        hipLaunchKernelGGL((knn_merge_f64_kernel<ARM_EUCLID_MULADD, true>), grid, dim3(256), 0, s, a);
-    else
-        hipLaunchKernelGGL((knn_merge_f64_kernel<ARM_EUCLID_MULADD, false>), grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL(knn_merge_f64_kernel, dim3((unsigned)((a.nq + 255) / 256)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -101,65 +101,24 @@ struct GramArgs32 {
     int mode;          // EmitMode
     const float* qsq;  // query row_sumsq
     const float* xsq;  // index row_sumsq
-    const float* xscale;  // cosine: -1/||x_t|| (0 for zero rows)
-    const float* qinv;    // knn_host cosine: query reciprocal norms (0 for zero rows)
-    const float* xinv;    // knn_host cosine: index reciprocal norms
     const NormStats* stats;
-    double eps_rel;    // Euclidean screen bound: eps = eps_rel*(||q||^2 + max||x||^2) + eps_abs
-    double eps_abs;    // cosine screen bound (absolute)
+    double eps_rel, eps_abs;  // screen bound: eps = eps_rel*(||q||^2 + max||x||^2) + eps_abs
     int64_t grid_wgs;  // the G0 the StreamSplit is built from (<= one resident round)
-    int nslots;        // list slots per query (StreamSplit::nslots)
+    int nslots;        // pairs kept per query (StreamSplit::nslots)
     int qpb;           // queries per workgroup: gram_f32_queries_per_block(d)
-    float* part_val;   // [nslots][nq][gram_list_cap(k)] lists, one per (segment, query)
+    float* part_val;   // [nslots][nq] best pairs, one per (segment, query)
     uint32_t* part_idx;
-    float* qval;       // [grid_wgs][4 waves][2][2048]: screen values, then index rows, of the queued pairs (k > 1)
-    float4* summ;      // [nslots][nq]: per-(segment, query) list summaries (k > 1), or null
-    float* out_val;    // [nq][k]
+    float* qval;       // the resident kernel's queues (gram_f32_k1_resident_queue_bytes)
+    float* out_val;    // [nq]
     uint32_t* out_idx;
-    unsigned int* shared_r;  // [nq] best known exact k-th value per query (float bits), or null
+    unsigned int* shared_r;  // [nq] best known exact value per query (float bits), or null
 };
 
-// Entries of one (segment, query) list of the Gram kernels: the k best plus
-// room for the pairs whose screen values lie within the error window of the
-// k-th (k = 1 keeps the single best pair, exactly): one 64-entry block for
-// k <= 64, k + 32 (at most 160, three blocks) above.
-__host__ __device__ inline int gram_list_cap(int k) {
-    return k == 1 ? 1 : k <= 64 ? (k + 32 < 64 ? k + 32 : 64) : k + 32;
-}
+// G0 and the pairs kept per query of the Gram kernel's split.
+void gram_f32_split(int64_t nq, int64_t nt, int64_t d, int cus, int64_t* grid_wgs, int* nslots);
 
-// Queued (screen value, index row) pairs of the f32 Gram kernel, 2 words
-// each, per workgroup of 4 waves: narrow shape 32 queries x 64 (k <= 64) or
-// 128 (k > 64) entries; the wide shape's 16 x 128 fits either.
-inline size_t gram_f32_qval_elems(int64_t grid_wgs, int k) {
-    return (size_t)grid_wgs * 4 * 32 * (k > 64 ? 128 : 64) * 2;
-}
-// The f64 kernel's queued screen values: 4 waves x 16 queries x 48 entries.
-inline size_t gram_f64_qval_elems(int64_t grid_wgs) { return (size_t)grid_wgs * 4 * 16 * 48; }
-
-// Index rows the seed launch samples for k > 1 (evenly spaced): 64 k, at
-// most 2048 and at most nt / 512 (the seed's exact vector work stays near
-// 0.2% of the scan's), but at least 512, so the k-th of the sample sits near
-// the same quantile for every k (at k = 128, 512 rows left the bound near the
-// 25% quantile).  Measured: c2 (1M rows, k = 32) steps fastest with the
-// 1953-row cap (1024 rows: +0.1 ms; 4096: the kernel gains 0.1 ms more but
-// the seed launch costs more), k = 128 likewise (4096 and 8192 rows cut the
-// scan by 0.6 and 1.1 ms and cost more in the seed), d256 (200k rows) with
-// 512; never more than the index.
-inline int64_t gram_seed_rows(int64_t nt, int k) {
-    int64_t n = 64 * (int64_t)k;
-    if (n > 2048) n = 2048;
-    if (n > nt / 512) n = nt / 512;
-    if (n < 512) n = 512;
-    return nt < n ? nt : n;
-}
-
-// G0, launched workgroups and per-query list slots of the Gram kernel's split.
-// vec4: the launch's 16-byte row test (d % 4 == 0, both bases 16-byte aligned),
-// which picks the kernel and with it the workgroups per CU the split assumes.
-void gram_f32_split(int64_t nq, int64_t nt, int64_t d, int k, int cus, bool vec4, int64_t* grid_wgs, int* nslots);
-
-// Three launches per assignment (k = 1, ARM_EUCLID_MULADD): prep (the shared
-// per-query bound reset), the Gram kernel, the strip merge + output transform.
+// Three launches (k = 1, the Euclidean arms): prep (the shared per-query bound
+// reset), the Gram kernel, the strip merge + output transform.
 hipError_t launch_gram_f32_prep(const GramArgs32& a, hipStream_t s);
 hipError_t launch_gram_f32(const GramArgs32& a, int arm, hipStream_t s);
 // k = 1 Euclidean searches whose index fits a few workgroups' LDS
@@ -175,11 +134,9 @@ hipError_t launch_gram_f32_k1_resident(const GramArgs32& a, int arm, int cus, fl
 size_t gram_f32_k1_resident_queue_bytes(int cus);
 hipError_t launch_gram_f32_k1_resident_merge(const GramArgs32& a, int nchunks, hipStream_t s);
 hipError_t launch_gram_f32_merge(const GramArgs32& a, hipStream_t s);
-int gram_f32_max_k();
 int gram_f32_max_d();
 // 128 queries per workgroup for d <= 128 (32 per wave), 64 above (16 per wave)
 int gram_f32_queries_per_block(int64_t d);
-int gram_f32_rows_per_tile();
 
 struct GramArgs64 {
     const double* q;
@@ -187,28 +144,18 @@ struct GramArgs64 {
     const double* x;
     int64_t nt;
     int64_t d;
-    int k;
     int mode;             // EmitMode
     const double* qsq;    // query row_sumsq
     const double* xsq;    // index row_sumsq
-    const double* qinv;   // knn_host cosine: query reciprocal norms
-    const double* xinv;   // knn_host cosine: index reciprocal norms
-    const double* xscale; // cosine: -1/||x_t|| (0 for zero rows)
     const NormStats* stats;
-    double eps_rel;       // Euclidean screen bound: eps = eps_rel*(||q||^2 + max||x||^2) + eps_abs
-    double eps_abs;       // cosine screen bound (absolute)
+    double eps_rel, eps_abs;  // as GramArgs32
     int64_t grid_wgs;
     int nslots;
-    double* part_val;     // [nslots][nq][gram_list_cap(k)]
+    double* part_val;     // [nslots][nq]
     uint32_t* part_idx;
-    double* qval;         // [grid_wgs][4 waves][16 queries][48]: screen values of the queued pairs
-    double* out_val;      // [nq][k]
+    double* out_val;      // [nq]
     uint32_t* out_idx;
-    unsigned long long* shared_r;  // [nq] best known exact k-th value per query (double bits)
-    // EMIT_ROOT_RANKED only, else null: [nq], set to 1 where an exact list
-    // dropped a pair whose root may equal the k-th root (the merge cannot
-    // then rank that root's ties by index)
-    unsigned int* root_flag;
+    unsigned long long* shared_r;  // [nq] best known exact value per query (double bits)
 };
 
 void gram_f64_split(int64_t nq, int64_t nt, int cus, int64_t* grid_wgs, int* nslots);
@@ -217,7 +164,6 @@ void gram_f64_split(int64_t nq, int64_t nt, int cus, int64_t* grid_wgs, int* nsl
 hipError_t launch_gram_f64_prep(const GramArgs64& a, hipStream_t s);
 hipError_t launch_gram_f64(const GramArgs64& a, int arm, hipStream_t s);
 hipError_t launch_gram_f64_merge(const GramArgs64& a, hipStream_t s);
-int gram_f64_max_k();
 int gram_f64_max_d();
 
 // Row norms: sq[r] = row_sumsq (separate multiply/add, ascending column),
