@@ -78,9 +78,12 @@ inline int gm_chunks(int64_t d) {
 }
 // Two query blocks per workgroup read every LDS tile for twice the products
 // (one block keeps the LDS at about 80% of its rate), but leave half the
-// workgroups.  One block / two, us per search: 1M x 10k, d = 128: 8649 / 8091;
-// 60k x 60k, d = 50: 2338 / 2127; 50k x 5k, d = 50: 197 / 192; 10k x 1k, d = 64:
-// 49 / 51.  Past 128 columns two blocks' operands do not fit the registers.
+// workgroups.  One block / two, us per f32 search of k = 10 at d = 32, 64, 128:
+// 2^25.6 pairs: 71.9 / 70.8, 87.8 / 87.4, 127.6 / 128.3; 10k x 10k (2^26.6):
+// 103.1 / 104.4, 135.0 / 133.0, 206.5 / 210.6; 50k x 5k (2^27.9): 142.5 / 133.6,
+// 187.8 / 179.8, 287.3 / 281.5; 200k x 5k (2^29.9): 463 / 398, 588 / 527, 883 / 842:
+// the line stands where they are equal.  Past 128 columns two blocks' operands do
+// not fit the registers.
 inline bool gm_two_blocks(int nk, int64_t nq, int64_t nt) {
     return nk <= 16 && nq > kGmQpb && (double)nq * (double)nt >= 0x1p26;
 }

@@ -857,9 +857,18 @@ __global__ __launch_bounds__(256, gm_select_waves(ARM, KL)) void gm_select_wave_
     L.emit(ov, oi, k, mode, a.last, lane);
 }
 
+// A wave per query where there are queries enough to fill the chip with four
+// times fewer workgroups, and few groups to read; longer lists take more of the
+// wave's serial work.  A search, us, wave / workgroup per query, f32, d = 64:
+//   k = 10: 10k x 500: 49.2 / 48.7, 10k x 1k: 51.2 / 53.7, 10k x 2k: 60.5 / 77.3,
+//   100k x 500: 100.9 / 96.5, 100k x 1k: 121 / 120, 100k x 4k: 241 / 271,
+//   260k x 2k (16,250 groups): 293 / 298, 520k x 2k: 556 / 563, 1M x 2k: 1084 / 1044;
+//   k = 50: 10k x 1k: 86 / 75, 10k x 2k: 97 / 112, 100k x 1k: 160 / 140,
+//   100k x 2k: 200 / 207, 260k x 2k: 346 / 362, 1M x 2k: 1132 / 1094
+//   (f64: 10k x 1k: 113 / 97, 10k x 2k: 141 / 154).
 template <typename T, typename TS, int ARM, int KL>
 void gm_select_launch(const GmSelectArgs<TS>& a, hipStream_t s) {
-    if (KL == 1 && a.nq >= 1000 && 2 * a.ntp <= 16384)
+    if (KL == 1 && a.nq >= (a.k <= 16 ? 1000 : 2000) && 2 * a.ntp <= 16384)
         hipLaunchKernelGGL((gm_select_wave_kernel<T, TS, ARM, KL>), dim3((unsigned)((a.nq + 3) / 4)), dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((gm_select_kernel<T, TS, ARM, KL>), dim3((unsigned)a.nq), dim3(256), 0, s, a);
