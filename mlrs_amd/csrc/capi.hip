@@ -509,10 +509,9 @@ int32_t kmeans_generic(const T* x, int64_t n, const T* c, int64_t kc, int64_t d,
 // ---------------------------------------------------------------------------
 // fast paths
 // ---------------------------------------------------------------------------
-// Below about 4e9 multiply-adds the whole exact distance matrix is cheaper
-// than the fused kernel's fixed costs (a few flush round trips per segment
-// and query): c1's 1k x 10k x 64 search takes 0.05 ms of exact tiles against
-// 0.5 ms fused on an MI355X.
+// Searches up to about 4e9 multiply-adds: the nearest-row kernels' fixed costs do
+// not pay, and the allocation-free entry point's limit (noalloc_admits) never
+// bound them.
 static bool small_search(int64_t nq, int64_t nt, int64_t d) {
     return (double)nq * (double)nt * (double)d <= 4294967296.0;
 }

@@ -2,14 +2,18 @@
 // and cosine arms (d <= 256, k <= 128), f32 and f64, in two passes.
 //
 //  scan    (knn_groupmin_scan.hpp) every (query, row) pair gets a screen value
-//          on the f16 matrix cores from operands of two halves, and only the minimum over each group of
-//          16 index rows is written: 4 bytes for 16 pairs.
+//          on the f16 matrix cores from operands of two halves, and only the
+//          minimum over each group of 16 index rows is written: 4 bytes for 16
+//          pairs.
 //  select  (knn_groupmin.hip) per query: T, the k-th smallest group minimum,
 //          bounds the k-th screen value (k groups hold k distinct rows at or
 //          below it), so with the screen's error bounded (gm_bound) every row
-//          of the answer lies in a group whose minimum is not far above T.  The rows of
-//          those groups (about k of them) are evaluated exactly, in the
-//          reference arm's operation order, and ranked by (value, index).
+//          of the answer lies in a group whose minimum is not far above T.
+//          The rows of those groups (about k of them) are evaluated exactly, in
+//          the reference arm's operation order, and ranked by (value, index).
+//  precise (knn_groupmin_precise.hip) f64 values only: the queries whose
+//          candidates the screen leaves too many, scanned again in f64 and
+//          selected for by those minima.  Usually there are none.
 //
 // The screen is the same whatever the element type: it only decides which pairs
 // are evaluated, never a result.  It works on a copy of the index, made per
@@ -26,9 +30,11 @@
 // 50, k = 15: 14.1, 3.69, 2.13; 50k x 5k, d = 50, k = 15, f32: 1.33, 0.32, 0.19; 10k
 // x 1k, d = 64, k = 10, f32: 0.090, 0.056, 0.049.
 // What it is bad at: points whose neighbours the screen cannot tell apart
-// (clusters a hundredth of their spacing wide and less, where every row of a
-// query's cluster is evaluated): 200k x 5k, d = 128 in 100 such clusters take
-// 10.7 ms in f32 and 20 in f64.
+// (clusters a fiftieth of their spacing wide and less).  f32 searches, and f64
+// ones too small for the precise scan, evaluate every row of a query's cluster:
+// 20k x 2k, d = 64, k = 10 in five clusters take 0.57 and 0.79 ms, where exact tiles
+// and a selection took 0.22 and 0.42; 100k x 10k, k = 15, f32 15.7 (13.8 with
+// per-row admission).
 //
 // Rows whose screen value cannot be trusted (norms near the ends of the f32
 // range, NaN under the fold arm) are "forced": their screen value is +inf and

@@ -10,9 +10,10 @@
 // about half as many roundings as the f32 chain made.  A workgroup is 4 waves of 32 queries; each wave
 // holds its queries in VGPRs as the B operand (d / 2 registers: two halves of 16 bits per column), and the index
 // is walked in 32-row tiles through two LDS buffers with one barrier per tile.
-// A lane ends a tile with 16 values of one query (its half of the tile's rows)
-// and keeps their minimum: eight v_min3 for up to 128 MFMAs, where a screen
-// with per-row admission issued about 110 vector instructions.  Four tiles'
+// A lane ends a tile with 16 values of one query (its half of the tile's rows),
+// unscales them (a multiplication and a multiply-add each, 32 instructions per
+// query block) and keeps their minimum (eight v_min3), beside 3 / 16 MFMAs a
+// column and query block, 48 at most.  Four tiles'
 // minima make one 16-byte store.  No state outlives a tile, so the (query
 // block, four tiles) units are cut into equal ranges, one per resident
 // workgroup, panel by panel (StreamSplit) so that workgroups of an XCD stream

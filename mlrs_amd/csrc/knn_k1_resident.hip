@@ -32,7 +32,7 @@
 // The results are the fused kernel's, bit for bit: a screen with a bounded
 // error and the same exact rescoring.
 // Bound by the vector instructions of a tile (the unscaling, the minimum and the
-// screen, about 70) beside its 24 MFMAs per 64 columns.  5M x 1024, d = 64: 5.54 ms
+// screen, about 70) beside its 12 MFMAs per 64 columns.  5M x 1024, d = 64: 5.54 ms
 // with f32 MFMA (74% of that peak), 2.63 ms.
 #include "knn_common.hpp"
 #include "knn_kernels.hpp"

@@ -188,3 +188,25 @@ def test_clusters_the_screen_does_not_resolve(dtype, metric, limit):
     centres = 20.0 * torch.rand((20, 128), generator=g, device=DEV, dtype=dtype) - 10.0
     xt, xq = (centres[torch.randint(0, 20, (x.shape[0],), generator=g, device=DEV)] + 0.01 * x for x in (xt, xq))
     assert _ms(_search(name, xq, xt, 16, metric)) < limit * plain
+
+
+@pytest.mark.parametrize("metric", [2, 3])
+def test_metric_sets(metric):
+    """Two sets of queries of the exact tiles' minima."""
+    nt, nq = 300_000, 2_500
+    xt, xq = _rows(nt, nt, 4), _rows(nq, nq, 4)
+    xt[nt - 3] = xt[1]
+    xt[7, 0], xt[8, 1] = float("nan"), float("inf")
+    xq[0] = xq[nq - 1] = xt[1]
+    xq[nq - 2, 0] = float("inf")
+    free, bound = (_search(n, xq, xt, 9, metric)() for n in ("mlrs_knn_topk_f32", "mlrs_knn_topk_f32_noalloc"))
+    torch.cuda.synchronize()
+    assert torch.equal(free[1], bound[1])
+    assert torch.equal(free[0].view(torch.int32), bound[0].view(torch.int32))
+    at = [0, 1, nq // 2, nq - 3, nq - 2, nq - 1]
+    prims.force_path("generic")
+    try:
+        dist, idx = prims.knn_topk(xq[at].contiguous(), xt, 9, "manhattan" if metric == 2 else "chebyshev")
+    finally:
+        prims.force_path("auto")
+    assert torch.equal(idx, bound[1][at].long()) and torch.equal(dist, bound[0][at])
