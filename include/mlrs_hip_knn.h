@@ -454,8 +454,9 @@ int32_t mlrs_release_workspace(void);
 /*
  * Measurement hook (no counterpart in the reference; for benchmarks).
  * While enabled, every call records a pair of HIP events on its own stream
- * around the launch of its dominant kernel (the Gram-MFMA kernel, the low-d
- * ALU kernel, or the generic path's distance tile; k-means fit also times
+ * around the launch of its dominant kernel (the group-minimum scan or tiles,
+ * the resident or Gram kernel, the low-d ALU kernel, or the generic path's
+ * distance tile; k-means fit also times
  * its centroid-sum pass).  mlrs_timing_read waits for the recorded events,
  * picks the name with the largest summed time, and returns that sum, the
  * number of launches timed under the name and the name; enabling again
@@ -481,12 +482,12 @@ int32_t mlrs_probe_peak(int32_t kind, int32_t waves_per_simd, double *tflops, vo
 /*
  * Kernel-family override (no counterpart in the reference; for tests and
  * benchmarks).  Every family returns the same bits, so this only changes
- * speed: 0 = automatic choice (default); 1 = the fused Gram-MFMA kernels
- * wherever they serve the shape (d <= 256, k <= 128; the f32 knn_host
- * cosine arm only at d > 128; k-means: d <= 256);
- * 2 = the
- * low-d ALU kernel wherever it serves the shape (f32 and f64, Euclidean
- * and cosine, d <= 16, k <= 32); 3 = the generic exact-tile path.  A family that does not serve
+ * speed: 0 = automatic choice (default); 1 = the matrix-core kernels wherever
+ * they serve the shape (Euclidean and cosine searches with d <= 256 and k <=
+ * 128: the group-minimum search, the resident one for k = 1; k-means: d <= 256);
+ * 2 = the low-d ALU kernel wherever it serves the shape (f32 and f64, Euclidean
+ * and cosine, d <= 16, k <= 32); 3 = the generic exact-tile path.  A family that
+ * does not serve
  * a shape falls back to the automatic choice.  radius_neighbors: 1 = the
  * matrix-core screen wherever it serves (f32 Euclidean / cosine, d <= 128),
  * 3 = the host-scan kernel.  Process-wide.

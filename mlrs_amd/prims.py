@@ -98,7 +98,7 @@ _PATHS = {"auto": 0, "fused": 1, "lowd": 2, "generic": 3}
 
 def force_path(name):
     """Kernel-family override for tests and benchmarks (mlrs_force_path):
-    "auto" (default), "fused" (Gram-MFMA), "lowd" (low-d ALU) or "generic"
+    "auto" (default), "fused" (matrix cores), "lowd" (low-d ALU) or "generic"
     (exact tiles + selection).  Every family returns the same bits."""
     if name not in _PATHS:
         raise ValueError("unknown kernel family %r (expected one of %s)" % (name, sorted(_PATHS)))
