@@ -554,7 +554,9 @@ static SearchKind cheapest_search(int64_t nq, int64_t nt, int64_t d, int64_t k, 
         1e-3 * q * (0.3 + batches * (f64 ? 1.5 + 0.019 * D : 1.25 + 0.008 * D));
     double exact = HUGE_VAL;
     if (k <= 64)
-        exact = (cos ? 33.0 + (f64 ? 0.002 : 0.006) * std::min(q, 1000.0) : 27.0) + std::max(0.0, D - 60.0) * (gram ? 0.12 : 0.08) * (f64 ? 1.5 : 1.0) + 2.4e-3 * (double)nt + 1e-3 * q * (f64 ? 1.8 : 1.5) +
+        exact = (cos ? 33.0 + (f64 ? 0.002 : 0.006) * std::min(q, 1000.0) : 27.0) +
+                std::max(0.0, D - 60.0) * (gram ? 0.12 : 0.08) * (f64 ? 1.5 : 1.0) + 2.4e-3 * (double)nt +
+                1e-3 * q * (f64 ? 1.8 : 1.5) +
                 mpairs * (gram ? (f64 ? 2.2 + 0.1 * D : 0.9 + 0.045 * D) : (f64 ? 2.6 + 0.066 * D : 0.9 + 0.036 * D));
     double lowd = HUGE_VAL;
     if (lowd_ok && k <= 16) {

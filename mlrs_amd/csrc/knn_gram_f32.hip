@@ -414,10 +414,11 @@ void knn_gram_f32_kernel(GramArgs32 a) {
 
     float thr = L.thr[jl];
     const float eps2 = 2.0f * L.eps[jl];  // exact doubling
-    // A lower bound on the screen values of the rows in query jl's queue.  A NaN screen value can hide a finite exact value only where a
-    // sum may overflow, so queries of mode 1 keep
-    // -inf and never drop queued rows; otherwise NaN screen values come from
-    // rows holding a NaN, whose exact values are NaN and never kept.
+    // A lower bound on the screen values of the rows in query jl's queue.  A NaN
+    // screen value can hide a finite exact value only where a sum may overflow,
+    // so queries of mode 1 keep -inf and never drop queued rows; otherwise NaN
+    // screen values come from rows holding a NaN, whose exact values are NaN and
+    // never kept.
     const float qlo0 = (L.mode[jl] == 0u) ? inf : -inf;
     float qlo = qlo0;
     int tiles = 0;

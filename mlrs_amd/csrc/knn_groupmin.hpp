@@ -63,7 +63,8 @@ struct GmStats {
 struct GmScanArgs {
     // Operand rows hold, per 16 columns, the high halves of the first and the
     // last eight, then the low halves: 64 bytes, counted as 16 floats.
-    const float* q;     // [queries, rounded up to the launch's 128 or 256][DP] query operand: -q or -q / ||q||, scaled and split; zeros past nq
+    const float* q;     // [queries, rounded up to the launch's 128 or 256][DP] query operand:
+                        // -q or -q / ||q||, scaled and split; zeros past nq
     const float* x;     // index rows, scaled and split, row stride ldx (a multiple of 16)
     const float* bias;  // [tiles * 32] Euclidean ||x||^2 less its share of the error, cosine 0; +inf for rows left out
     const float* xinv;  // [tiles * 32] what undoes the row's scale

@@ -379,9 +379,10 @@ struct GmProbe {
         return s;
     }
     // What no row of the answer exceeds, given that none has a minimum above
-    // thr: its exact value is then at most thr + base, eps and the factor take the roundings of that sum and of the exact value; the
-    // operands hold 2^-22 of their elements, a distance of at most 2^-20 of
-    // (||q|| + ||x||), ||x|| <= ||q|| + the distance.
+    // thr: its exact value is then at most thr + base, eps and the factor take
+    // the roundings of that sum and of the exact value; the operands hold 2^-22 of
+    // their elements, a distance of at most 2^-20 of (||q|| + ||x||), ||x|| <= ||q||
+    // + the distance.
     static __device__ __forceinline__ float limit(float thr, float base, float qn, float eps) {
         if (!(thr < __builtin_huge_valf())) return __builtin_huge_valf();
         const float D = (COS ? 2.0f : 1.0f) * (thr + base + eps);
